@@ -354,7 +354,7 @@ int smoe_decode_glu_mlp(const void* X, int64_t sxm, const int64_t* experts, int6
       sw1e % 8 || sw1n % 8 || sw2e % 8 || sw2n % 8 || !al16(X) || !al16(W1) || !al16(W2) || !al16(H))
     return SMOE_ERR_UNSUPPORTED;
   DecodeArgs a{X, sxm, experts, set, sek, gates, sgt, sgk, W1, sw1e, sw1n, b1, sb1e, sb1n, W2, sw2e, sw2n,
-               b2, sb2e, sb2n, H, shm, OUT, som, (int)T, k, (int)d, (int)F, E, act};
+               b2, sb2e, sb2n, H, shm, OUT, som, (int)T, k, (int)d, (int)F, E, act, 65535u / (unsigned)k + 1u};
   return launch_decode_glu_mlp(a, dtype, (hipStream_t)stream);
 }
 

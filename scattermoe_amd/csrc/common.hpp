@@ -233,6 +233,7 @@ struct DecodeArgs {
   void* H; int64_t shm;                              // (T*k, F) workspace: hidden rows in slot order
   void* OUT; int64_t som;                            // (T, d)
   int T, k, d, F, E, act;
+  unsigned k_inv;                                    // ceil(65536 / k): slot i belongs to token (i * k_inv) >> 16
 };
 int launch_decode_glu_mlp(const DecodeArgs& a, int dtype, hipStream_t st);
 
