@@ -23,7 +23,7 @@
 //                tokens: 1.68 -> 1.37 ms for the two forward launches; neutral at 4096, 2 % slower at 8192)
 //   GM_S2S       row super-tiles per raster band of scatter2scatter (4: +3 % on the layer-2 shaped launches)
 //   GM_XTY       the same for groupXtY (4: 1-2 % over unbanded on all three training workloads)
-static constexpr int ROWS32_BELOW = 24, ROWS64_BELOW = 52, ROWS128_BELOW = 112, ROWS256_BELOW = 224;
+static constexpr int ROWS32_BELOW = 16, ROWS64_BELOW = 52, ROWS128_BELOW = 112, ROWS256_BELOW = 224;
 static constexpr int ROWS128W_BELOW = 136;   // wide launches: 128 x 256 ring tiles for 52..135 rows per expert, 256 x 256 from there
 static constexpr int GM_RING = 8;
 static constexpr int STRIPE_BELOW = 1024;
@@ -370,12 +370,14 @@ __device__ __forceinline__ void issue_slice_tail(const AOp& A, const BOp& B, uns
   }
 }
 
-template <int BM_, int BN_, int WM_, int WN_, int NS_ = 2, bool RS_ = false>
+// WG_: workgroups per CU the registers have to leave room for (LDS permitting)
+template <int BM_, int BN_, int WM_, int WN_, int NS_ = 2, bool RS_ = false, int WG_ = 1>
 struct Tile {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_;
   static constexpr int NS = NS_;                      // LDS stages (2: double buffer, more: ring)
   static constexpr bool RS = RS_;                     // operands travel global -> registers -> LDS (mainloop_rs)
   static constexpr int NW = WM * WN, NT = NW * 64;
+  static constexpr int WAVES_PER_SIMD = WG_ * NW / 4 > 0 ? WG_ * NW / 4 : 1;
   static constexpr int WTM = BM / WM, WTN = BN / WN;
   static constexpr int FM = WTM / 32, FN = WTN / 32;
   static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile must be a multiple of the 32x32 MFMA");
@@ -1276,13 +1278,13 @@ static Raster make_striped(int64_t m_tiles, int n_tiles, int gm) {
 // scatter2scatter
 // =====================================================================================================
 template <typename T, class TL, bool B_TR>
-__global__ __launch_bounds__(TL::NT) void s2s_mfma_kernel(S2SArgs a, Raster rast) {
+__global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2SArgs a, Raster rast) {
   typedef DirectOp<TL::BM, TL::NT> AOp;
   // Ring classes serve launches with at most a tile row or two per expert: (nearly) every weight element is read
   // once, and with the non-temporal hint it does not push the token rows, which every workgroup of a tile row reads,
   // out of the L2s (hint extended from the 32-/64-row classes to all ring classes: Mixtral layer forward at 256 /
   // 384 / 448 tokens 0.539 -> 0.505 / 0.559 -> 0.526 / 0.711 -> 0.688 ms, neutral from 768 tokens on)
-  constexpr bool W_ONCE = TL::NS > 2;
+  constexpr bool W_ONCE = TL::NS > 2 || TL::BM < 256;
   typedef typename std::conditional<B_TR, TransOp<TL::BN, TL::NT, W_ONCE>, DirectOp<TL::BN, TL::NT, W_ONCE>>::type BOp;
   constexpr int STAGE = AOp::LDS_BYTES + BOp::LDS_BYTES;
   __shared__ __attribute__((aligned(16))) char lds[TL::NS * STAGE];
@@ -1660,6 +1662,48 @@ static int launch_main(const S2SArgs& a, bool b_tr, hipStream_t st) {
   return launch_tails<T>(a, b_tr, st);
 }
 
+static bool glu_fwd_pieces(const S2SArgs& a) {
+  return a.glu != 1 || (((((uintptr_t)a.Y | (uintptr_t)a.H) & 15) == 0) && ((a.sym | a.shm | a.N) & 7) == 0);
+}
+
+// Fewer than 52 rows per expert: a stream over the weights of the experts that are hit, tiles of 64 or 32 rows.  What
+// counts is weight bytes in flight across the chip, and that the filling of one tile's ring hides behind the stream of
+// another: a workgroup that has the CU to itself (six 20 KB stages, the only form until now) leaves the memory idle
+// while it looks its tile up, fills its ring and stores its result, for a tile of 512 KB (128 columns x 2048) about a
+// fifth of its time.  Hence two or three workgroups per CU with shallower rings wherever the launch has that many.
+// Measured (us, one 32 x 128 x 6 workgroup per CU -> now; weights streamed at):
+//   128 experts x 12 rows, layer 1 of d = 2048, F = 768: 162 -> 140 (5.7 TB/s); layer 2: 91 -> 70 (5.7 TB/s)
+//   32 experts x 6 rows, 2880 -> 2 x 2880 (N-contiguous): 169 -> 157 (6.8 TB/s); 2880 -> 2880: 88 -> 82
+//   8 experts x 8 rows, layer 1 of d = 4096, F = 14336: 289 -> 275; 64 experts x 8 rows, 1024 -> 2 x 512: 29 -> 24
+//   128 experts x 40 rows (64-row tiles, five stages -> three): 178 -> 156 and 106 -> 79
+template <typename T>
+static int dispatch_few_rows(const S2SArgs& a, bool b_tr, hipStream_t st) {
+  const int64_t avg = a.L / a.E;
+  const int bn = a.glu == 1 ? 64 : 128;                                   // output columns of a 128-wide tile
+  const int64_t cols = (a.N + bn - 1) / bn, wgs = std::min<int64_t>(a.L, a.E) * cols;
+  // Three two-stage workgroups per CU where that makes one round of what would be 1.5 rounds of two per CU
+  // (us, two x three stages -> three x two: 64 x 11 tiles of K = 2048 80 -> 67, 16 x 44 74 -> 66, 32 x 23 of K = 2880
+  // 89 -> 82, 16 x 44 of K = 4096 137 -> 124; with fewer tiles two stages are too few: 256 of K = 14336 147 -> 211)
+  if (wgs > 2 * NUM_CU && wgs <= 3 * NUM_CU) return launch_s2s<T, Tile<64, 128, 2, 2, 2, false, 3>>(a, b_tr, st);
+  const bool few = b_tr ? wgs < NUM_CU : wgs <= NUM_CU;                   // up to one workgroup per CU: deep rings
+  if (avg >= (few ? 24 : ROWS32_BELOW)) {
+    if (few) return launch_s2s<T, Tile<64, 128, 2, 2, 5>>(a, b_tr, st);
+    return launch_s2s<T, Tile<64, 128, 2, 2, 3, false, 2>>(a, b_tr, st);
+  }
+  // 32-row tiles have one column block per wave: the fused forward GLU only in its LDS-staged form (16-byte pieces)
+  if (!glu_fwd_pieces(a)) return SMOE_ERR_UNSUPPORTED;
+  if (!b_tr) {
+    // K-contiguous weights: half-width tiles while 128-wide ones would not give every CU two workgroups (44 x 8 tiles
+    // of K = 1024: 25 -> 17 us, 22 x 16 of K = 2048: 47 -> 39, 8 x 8 of K = 2816: 18 -> 16), and where 128-wide
+    // columns do not divide evenly among the 8 XCDs (12 columns: 152 -> 140 us; 45 or 16: even)
+    if (wgs < 192) return launch_s2s<T, Tile<32, 64, 1, 2, 6>>(a, b_tr, st);
+    if (wgs < 2 * NUM_CU || cols * 4 <= (cols + 7) / 8 * 8 * 3) return launch_s2s<T, Tile<32, 64, 1, 2, 4, false, 3>>(a, b_tr, st);
+  } else if (few) {
+    return launch_s2s<T, Tile<32, 128, 1, 4, 6>>(a, b_tr, st);
+  }
+  return launch_s2s<T, Tile<32, 128, 1, 4, 3, false, 2>>(a, b_tr, st);
+}
+
 template <typename T>
 static int dispatch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
   // the gpt-oss epilogues exist only in their LDS-staged form (16-byte pieces)
@@ -1684,19 +1728,12 @@ static int dispatch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
   const bool wide = (int64_t)a.E * ((a.N + (a.glu == 1 ? 127 : 255)) / (a.glu == 1 ? 128 : 256)) >= 2 * NUM_CU;
   if (wide && avg >= ROWS128W_BELOW) return launch_main<T>(a, b_tr, st);
   if (wide && avg >= ROWS64_BELOW) return launch_s2s<T, Tile<128, 256, 2, 4, 3>>(a, b_tr, st);
-  // Below that the launch is a stream over the weights: ring-buffered classes, tile height by rows per expert
+  // Below that the launch is a stream over the weights: tile height by rows per expert
   if (avg >= ROWS128_BELOW) return launch_s2s<T, Tile<256, 128, 4, 2, 3>>(a, b_tr, st);
-  if (avg >= ROWS32_BELOW && avg < ROWS64_BELOW) return launch_s2s<T, Tile<64, 128, 2, 2, 5>>(a, b_tr, st);
+  if (avg < ROWS64_BELOW) return dispatch_few_rows<T>(a, b_tr, st);
   // With one column block per wave the fused forward GLU exists only in its LDS-staged form (16-byte pieces)
-  if (a.glu == 1 && !((((uintptr_t)a.Y | (uintptr_t)a.H) & 15) == 0 && ((a.sym | a.shm | a.N) & 7) == 0))
-    return SMOE_ERR_UNSUPPORTED;
-  if (avg >= ROWS64_BELOW) return launch_s2s<T, Tile<128, 128, 2, 4, 3>>(a, b_tr, st);
-  // With few output columns the 128-wide tiles do not give every CU a workgroup, and what counts is bytes in
-  // flight across the chip: narrower tiles (K-contiguous weights only) restore the count.
-  const int64_t wgs128 = max_tiles(a.L, a.E, 32) * ((a.N + 127) / 128);
-  if (!b_tr && wgs128 < 96) return launch_s2s<T, Tile<32, 32, 1, 1, 8>>(a, b_tr, st);
-  if (!b_tr && wgs128 < 192) return launch_s2s<T, Tile<32, 64, 1, 2, 6>>(a, b_tr, st);
-  return launch_s2s<T, Tile<32, 128, 1, 4, 6>>(a, b_tr, st);
+  if (!glu_fwd_pieces(a)) return SMOE_ERR_UNSUPPORTED;
+  return launch_s2s<T, Tile<128, 128, 2, 4, 3>>(a, b_tr, st);
 }
 
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
