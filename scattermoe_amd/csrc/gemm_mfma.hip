@@ -16,15 +16,13 @@
 
 // Tunables (measured on the Mixtral-shape workload unless noted):
 //   ROWS*_BELOW  average rows per expert under which the 32-, 64-, 128- and 256-row ring-buffered tile classes
-//                are used (weight-streaming regime, Mixtral expert shapes with 64..1536 tokens; from there on
-//                the 256x256 two-stage tile)
+//                are used (weight-streaming regime; see dispatch_s2s)
 //   GM_RING      tile rows that visit a tile column back to back in the ring classes' order (1: -15 %, 4: -4 %)
 //   STRIPE_BELOW average rows per expert under which the 256x256 class uses that order too (Mixtral shape, 1536
 //                tokens: 1.68 -> 1.37 ms for the two forward launches; neutral at 4096, 2 % slower at 8192)
 //   GM_S2S       row super-tiles per raster band of scatter2scatter (4: +3 % on the layer-2 shaped launches)
 //   GM_XTY       the same for groupXtY (4: 1-2 % over unbanded on all three training workloads)
 static constexpr int ROWS32_BELOW = 16, ROWS64_BELOW = 52, ROWS128_BELOW = 112, ROWS256_BELOW = 224;
-static constexpr int ROWS128W_BELOW = 136;   // wide launches: 128 x 256 ring tiles for 52..135 rows per expert, 256 x 256 from there
 static constexpr int GM_RING = 8;
 static constexpr int STRIPE_BELOW = 1024;
 static constexpr int GM_S2S = 4;
@@ -376,6 +374,9 @@ struct Tile {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_;
   static constexpr int NS = NS_;                      // LDS stages (2: double buffer, more: ring)
   static constexpr bool RS = RS_;                     // operands travel global -> registers -> LDS (mainloop_rs)
+  static constexpr int WG = WG_;
+  // the same tile with U blocks of 32 rows per wave
+  template <int U> using Height = Tile<U * 32 * WM_, BN_, WM_, WN_, NS_, RS_, WG_>;
   static constexpr int NW = WM * WN, NT = NW * 64;
   static constexpr int WAVES_PER_SIMD = WG_ * NW / 4 > 0 ? WG_ * NW / 4 : 1;
   static constexpr int WTM = BM / WM, WTN = BN / WN;
@@ -457,70 +458,97 @@ __device__ __forceinline__ void mainloop(AOp& A, BOp& B, int klen, char* lds, bo
           __builtin_amdgcn_sched_group_barrier(0x100, BOp::DS_PER_FRAG, 0);
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, TL::FM * TL::FN - TL::FM - TL::FN, 0);
+        if constexpr (TL::FM * TL::FN > TL::FM + TL::FN)
+          __builtin_amdgcn_sched_group_barrier(0x008, TL::FM * TL::FN - TL::FM - TL::FN, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
 
-// Main loop of the one-wave-per-SIMD class (4 waves, 128 x 128 wave tiles): operands travel global -> registers ->
-// LDS.  A burst of loads at the top of a slice holds the waves that issue it off the matrix pipe until the memory
-// pipeline has taken all of them (it takes one 1 KB wave-load per ~17 cycles and CU), and loads spread over the
-// slice leave the late ones too little time to land when LDS is the only place they can land in: here every
-// thread's 16 pieces of a slice sit in registers for up to two slices, which LDS has no room for.
+// Main loop of the one-wave-per-SIMD class (4 waves, wave tiles of up to 128 x 128): operands travel global ->
+// registers -> LDS.  A burst of loads at the top of a slice holds the waves that issue it off the matrix pipe until
+// the memory pipeline has taken all of them (it takes one 1 KB wave-load per ~17 cycles and CU), and loads spread over
+// the slice leave the late ones too little time to land when LDS is the only place they can land in: here every
+// thread's pieces of a slice (16 in a 256 x 256 tile) sit in registers for up to two slices, which LDS has no room for.
 //   set S = (kt + 1) & 1 holds slice kt + 1: its pieces are written to the other LDS stage during steps 0-2 of
-//   slice kt (ds_write_b128, second half of each step) and each is reloaded with slice kt + 3 one step later
-//   (pieces 12-15 in step 0 of the next slice), one load per 4 MFMAs throughout;
+//   slice kt (ds_write_b128, spread evenly: behind every third MFMA) and each is reloaded with slice kt + 3 one step
+//   later (the last quarter of them in step 0 of the next slice), one load per 4 MFMAs throughout;
 //   one barrier per slice, after step 2: behind it the fragments of step 0 of slice kt + 1 are read while the
 //   MFMAs of step 3 run.
 // Whole 64-deep slices only, at least two of them (the launcher checks); loads past the end re-read the last slice.
-template <typename T, class TL, class AOp, class BOp, int P, int KS>
+//
+// A thread's pieces of a slice in the order they are written and reloaded: the operands alternate while the row
+// operand (the smaller one in a tile of fewer than 256 rows) has pieces left.
+template <class TL, class AOp, class BOp>
+struct RsPlan {
+  static_assert(AOp::R <= BOp::R && BOp::R == 8, "the column operand is the larger one");
+  static constexpr int N = AOp::R + BOp::R;                       // pieces per thread and slice
+  static constexpr int NM = TL::FM * TL::FN;                      // MFMAs per step
+  static constexpr int L = (N + 3) / 4;                           // loads per step (step 0: what is left)
+  static_assert(N <= 3 * NM, "at most one LDS write behind an MFMA");
+  static constexpr bool is_b(int q) { return q >= 2 * AOp::R || (q & 1); }
+  static constexpr int index(int q) { return q < 2 * AOp::R ? q >> 1 : q - AOp::R; }
+  // pieces written before MFMA g of steps 0-2
+  static constexpr int written(int g) { return N * (g + 1) / (3 * NM); }
+  static_assert(written(0) == 0 && written(3 * NM) == N, "every piece is written once");
+  static_assert(written(NM) >= L && written(2 * NM) >= 2 * L && N >= 3 * L, "a piece is reloaded after it has been written");
+  // fragments of the next step read behind MFMA m: one behind each, the surplus of small tiles behind the first
+  static constexpr int NF = TL::FM + TL::FN, FIRST = NF > NM ? NF - NM + 1 : 1;
+  static constexpr int frags_before(int m) { return m == 0 ? 0 : FIRST + m - 1 < NF ? FIRST + m - 1 : NF; }
+  static constexpr int loads_before(int n, int m) { return n * m / NM; }
+};
+
+template <typename T, class TL, class AOp, class BOp, int P, int KS, int N>
 __device__ __forceinline__ void rs_step(const AOp& A, const BOp& B, const char* __restrict__ cur, char* __restrict__ nxt,
                                         int k2, int k3, int kend, int wm, int wn,
-                                        f32x16 (&acc)[TL::FM][TL::FN], i32x4 (&g)[2][16],
+                                        f32x16 (&acc)[TL::FM][TL::FN], i32x4 (&g)[2][N],
                                         i32x4 (&fa)[2][TL::FM], i32x4 (&fb)[2][TL::FN]) {
-  constexpr int FM = TL::FM, FN = TL::FN, NM = FM * FN;
-  static_assert(NM == 16 && FM + FN <= 8, "pipeline below is laid out for 16 MFMAs per step");
+  typedef RsPlan<TL, AOp, BOp> Plan;
+  constexpr int FM = TL::FM, FN = TL::FN, NM = Plan::NM;
   constexpr int S = P ^ 1;
   constexpr int c = KS & 1, n = c ^ 1;
   // LDS traffic of the step in the order it is to be issued in (the compiler keeps reads and writes of LDS in
-  // program order): one fragment of the next step behind each of the first FM + FN MFMAs - from the stage being
-  // multiplied, in step 3 from the stage just filled - and one piece written behind every third MFMA of steps 0-2
-  // (pieces 0-4, 5-10, 11-15).
-  constexpr int W0[5] = {0, 5, 11, 16, 16};
+  // program order): the fragments of the next step behind the first MFMAs - from the stage being multiplied, in
+  // step 3 from the stage just filled - and the pieces of steps 0-2 spread evenly.
   const char* src = KS < 3 ? cur : (const char*)nxt;
   constexpr int fstep = KS < 3 ? KS + 1 : 0;
 #pragma unroll
   for (int m = 0; m < NM; ++m) {
-    if (m < FM) fa[n][m] = AOp::frag(src, wm * TL::WTM + m * 32, fstep);
-    else if (m < FM + FN) fb[n][m - FM] = BOp::frag(src + AOp::LDS_BYTES, wn * TL::WTN + (m - FM) * 32, fstep);
-    if ((KS * NM + m) % 3 == 1 && KS < 3) {
-      const int q = (KS * NM + m) / 3;
-      if (q & 1) lds_write16(nxt + AOp::LDS_BYTES + B.piece_lds(q >> 1), g[S][q]);
-      else lds_write16(nxt + A.piece_lds(q >> 1), g[S][q]);
+#pragma unroll
+    for (int f = Plan::frags_before(m); f < Plan::frags_before(m + 1); ++f) {
+      if (f < FM) fa[n][f] = AOp::frag(src, wm * TL::WTM + f * 32, fstep);
+      else fb[n][f - FM] = BOp::frag(src + AOp::LDS_BYTES, wn * TL::WTN + (f - FM) * 32, fstep);
+    }
+    if (KS < 3 && Plan::written(KS * NM + m + 1) > Plan::written(KS * NM + m)) {
+      const int q = Plan::written(KS * NM + m);
+      if (Plan::is_b(q)) lds_write16(nxt + AOp::LDS_BYTES + B.piece_lds(Plan::index(q)), g[S][q]);
+      else lds_write16(nxt + A.piece_lds(Plan::index(q)), g[S][q]);
     }
   }
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = Mfma<T>::run(fb[c][j], fa[c][i], acc[i][j]);
-  static_assert(W0[1] == 5 && W0[2] == 11, "pieces per step follow from one write per three MFMAs");
-  // pieces loaded in this step: 12-15 of the other set (slice kt + 2), then 0-3, 4-7, 8-11 of this one (slice kt + 3)
+  // pieces loaded in this step: the last ones of the other set (slice kt + 2), then a third each of the others of
+  // this one (slice kt + 3)
+  constexpr int SET = KS == 0 ? P : S;
+  constexpr int q0 = KS == 0 ? 3 * Plan::L : (KS - 1) * Plan::L, nl = KS == 0 ? N - 3 * Plan::L : Plan::L;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    constexpr int SET = KS == 0 ? P : S;
-    const int q = KS == 0 ? 12 + u : (KS - 1) * 4 + u;
+  for (int q = q0; q < q0 + nl; ++q) {
     const int k0 = KS == 0 ? k2 : k3;
-    g[SET][q] = (q & 1) ? B.load_piece(k0, kend, q >> 1) : A.load_piece(k0, kend, q >> 1);
+    g[SET][q] = Plan::is_b(q) ? B.load_piece(k0, kend, Plan::index(q)) : A.load_piece(k0, kend, Plan::index(q));
   }
 #pragma unroll
   for (int m = 0; m < NM; ++m) {
     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    if (m < FM) __builtin_amdgcn_sched_group_barrier(0x100, AOp::DS_PER_FRAG, 0);
-    else if (m < FM + FN) __builtin_amdgcn_sched_group_barrier(0x100, BOp::DS_PER_FRAG, 0);
-    if ((KS * NM + m) % 3 == 1 && KS < 3) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-    if (m % 4 == 3) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+#pragma unroll
+    for (int f = Plan::frags_before(m); f < Plan::frags_before(m + 1); ++f) {
+      if (f < FM) __builtin_amdgcn_sched_group_barrier(0x100, AOp::DS_PER_FRAG, 0);
+      else __builtin_amdgcn_sched_group_barrier(0x100, BOp::DS_PER_FRAG, 0);
+    }
+    if (KS < 3 && Plan::written(KS * NM + m + 1) > Plan::written(KS * NM + m)) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+    if (Plan::loads_before(nl, m + 1) > Plan::loads_before(nl, m)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
   }
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (KS == 2) {
@@ -530,23 +558,25 @@ __device__ __forceinline__ void rs_step(const AOp& A, const BOp& B, const char* 
   }
 }
 
-template <typename T, class TL, class AOp, class BOp, int P>
+template <typename T, class TL, class AOp, class BOp, int P, int N>
 __device__ __forceinline__ void rs_slice(const AOp& A, const BOp& B, const char* cur, char* nxt,
                                          int kt, int last_k0, int kend, int wm, int wn,
-                                         f32x16 (&acc)[TL::FM][TL::FN], i32x4 (&g)[2][16],
+                                         f32x16 (&acc)[TL::FM][TL::FN], i32x4 (&g)[2][N],
                                          i32x4 (&fa)[2][TL::FM], i32x4 (&fb)[2][TL::FN]) {
   const int k2 = min((kt + 2) * BK, last_k0), k3 = min((kt + 3) * BK, last_k0);
   __builtin_amdgcn_sched_barrier(0);
-  rs_step<T, TL, AOp, BOp, P, 0>(A, B, cur, nxt, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_step<T, TL, AOp, BOp, P, 1>(A, B, cur, nxt, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_step<T, TL, AOp, BOp, P, 2>(A, B, cur, nxt, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_step<T, TL, AOp, BOp, P, 3>(A, B, cur, nxt, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_step<T, TL, AOp, BOp, P, 0, N>(A, B, cur, nxt, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_step<T, TL, AOp, BOp, P, 1, N>(A, B, cur, nxt, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_step<T, TL, AOp, BOp, P, 2, N>(A, B, cur, nxt, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_step<T, TL, AOp, BOp, P, 3, N>(A, B, cur, nxt, k2, k3, kend, wm, wn, acc, g, fa, fb);
 }
 
 template <typename T, class TL, class AOp, class BOp>
 __device__ __forceinline__ void mainloop_rs(const AOp& A, const BOp& B, int klen, char* lds,
                                             f32x16 (&acc)[TL::FM][TL::FN]) {
-  static_assert(AOp::R == 8 && BOp::R == 8 && BK == 64, "16 pieces per thread and slice");
+  typedef RsPlan<TL, AOp, BOp> Plan;
+  constexpr int N = Plan::N;
+  static_assert(BK == 64, "four steps per slice");
   constexpr int STAGE = AOp::LDS_BYTES + BOp::LDS_BYTES;
   const int wave = threadIdx.x >> 6;
   const int wm = wave / TL::WN, wn = wave % TL::WN;
@@ -554,20 +584,23 @@ __device__ __forceinline__ void mainloop_rs(const AOp& A, const BOp& B, int klen
   // zeros is multiplied (no branch around the loop: 256 accumulator registers would have to be merged behind it).
   const int nk = max(1, (klen + BK - 1) / BK);
   const int last_k0 = (nk - 1) * BK;
-  i32x4 g[2][16];
+  i32x4 g[2][N];
   i32x4 fa[2][TL::FM], fb[2][TL::FN];
   const int k1 = min(BK, last_k0), k2 = min(2 * BK, last_k0);
+  auto load = [&](int k0, int q) {
+    return Plan::is_b(q) ? B.load_piece(k0, klen, Plan::index(q)) : A.load_piece(k0, klen, Plan::index(q));
+  };
 #pragma unroll
-  for (int q = 0; q < 16; ++q) g[0][q] = (q & 1) ? B.load_piece(0, klen, q >> 1) : A.load_piece(0, klen, q >> 1);
+  for (int q = 0; q < N; ++q) g[0][q] = load(0, q);
 #pragma unroll
-  for (int q = 0; q < 16; ++q) g[1][q] = (q & 1) ? B.load_piece(k1, klen, q >> 1) : A.load_piece(k1, klen, q >> 1);
+  for (int q = 0; q < N; ++q) g[1][q] = load(k1, q);
 #pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    if (q & 1) lds_write16(lds + AOp::LDS_BYTES + B.piece_lds(q >> 1), g[0][q]);
-    else lds_write16(lds + A.piece_lds(q >> 1), g[0][q]);
+  for (int q = 0; q < N; ++q) {
+    if (Plan::is_b(q)) lds_write16(lds + AOp::LDS_BYTES + B.piece_lds(Plan::index(q)), g[0][q]);
+    else lds_write16(lds + A.piece_lds(Plan::index(q)), g[0][q]);
   }
 #pragma unroll
-  for (int q = 0; q < 12; ++q) g[0][q] = (q & 1) ? B.load_piece(k2, klen, q >> 1) : A.load_piece(k2, klen, q >> 1);
+  for (int q = 0; q < 3 * Plan::L; ++q) g[0][q] = load(k2, q);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
@@ -575,18 +608,18 @@ __device__ __forceinline__ void mainloop_rs(const AOp& A, const BOp& B, int klen
   for (int i = 0; i < TL::FM; ++i) fa[0][i] = AOp::frag(lds, wm * TL::WTM + i * 32, 0);
 #pragma unroll
   for (int j = 0; j < TL::FN; ++j) fb[0][j] = BOp::frag(lds + AOp::LDS_BYTES, wn * TL::WTN + j * 32, 0);
-  // The second stage starts 64 KB into LDS, beyond what the offset field of an LDS instruction can add: its
-  // addresses are formed from a base of their own (kept from being folded into constants), not with one
+  // The second stage starts 64 KB into LDS (in a 256-row tile), beyond what the offset field of an LDS instruction can
+  // add: its addresses are formed from a base of their own (kept from being folded into constants), not with one
   // vector-ALU instruction per access.
   unsigned second = STAGE;
   asm volatile("" : "+v"(second));
   char* lds1 = lds + second;
   int kt = 0;
   for (; kt + 1 < nk; kt += 2) {
-    rs_slice<T, TL, AOp, BOp, 0>(A, B, lds, lds1, kt, last_k0, klen, wm, wn, acc, g, fa, fb);
-    rs_slice<T, TL, AOp, BOp, 1>(A, B, lds1, lds, kt + 1, last_k0, klen, wm, wn, acc, g, fa, fb);
+    rs_slice<T, TL, AOp, BOp, 0, N>(A, B, lds, lds1, kt, last_k0, klen, wm, wn, acc, g, fa, fb);
+    rs_slice<T, TL, AOp, BOp, 1, N>(A, B, lds1, lds, kt + 1, last_k0, klen, wm, wn, acc, g, fa, fb);
   }
-  if (kt < nk) rs_slice<T, TL, AOp, BOp, 0>(A, B, lds, lds1, kt, last_k0, klen, wm, wn, acc, g, fa, fb);
+  if (kt < nk) rs_slice<T, TL, AOp, BOp, 0, N>(A, B, lds, lds1, kt, last_k0, klen, wm, wn, acc, g, fa, fb);
 }
 
 // Main loop of the small-row (decode) tile class: memory bound, so what matters is bytes in flight.  The
@@ -918,7 +951,7 @@ __device__ __forceinline__ void epilogue_staged(const f32x16 (&acc)[TL::FM][TL::
   }, sbias);
   // In groups: the row offsets of a group, then its pieces, are read from LDS back to back before the first of its
   // stores (written as one conditional store per piece, every piece would wait for two LDS round trips of its own)
-  constexpr int GRP = PP >= 16 ? 16 : PP;
+  constexpr int GRP = PP % 16 == 0 ? 16 : PP % 8 == 0 ? 8 : PP;
   static_assert(PP % GRP == 0, "groups must divide the pieces");
 #pragma unroll
   for (int q0 = 0; q0 < PP; q0 += GRP) {
@@ -961,7 +994,7 @@ __device__ __forceinline__ void epilogue_glu_fwd_staged(const f32x16 (&acc)[TL::
     T* pre = (T*)a.Y;
     T* hid = (T*)a.H;
     // a group's LDS reads are issued back to back ahead of its arithmetic and stores (see epilogue_staged)
-    constexpr int GRP = PP >= 8 ? 8 : PP;
+    constexpr int GRP = PP % 8 == 0 ? 8 : PP % 4 == 0 ? 4 : PP;
     static_assert(PP % GRP == 0, "groups must divide the pieces");
     // which half holds the gate is the same for the whole launch: one copy of the loop for each case instead of a
     // select per element (the accumulators are in LDS by now, so the branch has nothing to carry)
@@ -1015,7 +1048,7 @@ __device__ __forceinline__ void epilogue_glu_bwd_staged(const f32x16 (&acc)[TL::
                                                         int row0, int rows, int n0, char* lds, float* sbias = nullptr) {
   typedef T T8 __attribute__((ext_vector_type(8)));
   constexpr int CPR = TL::BN / 8, PIECES = TL::BM * CPR, PP = PIECES / TL::NT;
-  constexpr int GRP = PP >= 8 ? 4 : (PP >= 2 ? PP / 2 : 1);       // pieces per group, two groups in flight
+  constexpr int GRP = PP % 8 == 0 ? 4 : PP % 4 == 0 ? 2 : (PP >= 2 ? PP / 2 : 1);    // pieces per group, two in flight
   static_assert(PIECES % TL::NT == 0 && (PP == 1 || PP % (2 * GRP) == 0), "pieces must divide evenly");
   stage_accumulators<T, TL>(acc, lds, [](int) { return 0.0f; }, sbias);
   const int F = a.N;
@@ -1100,7 +1133,7 @@ __device__ __forceinline__ void epilogue_oss_fwd_staged(const f32x16 (&acc)[TL::
   }, sbias);
   T* pre = (T*)a.Y;
   T* hid = (T*)a.H;
-  constexpr int GRP = PP >= 16 ? 16 : PP;               // LDS reads of a group back to back (see epilogue_staged)
+  constexpr int GRP = PP % 16 == 0 ? 16 : PP % 8 == 0 ? 8 : PP;      // LDS reads of a group back to back (see epilogue_staged)
   static_assert(PP % GRP == 0, "groups must divide the pieces");
 #pragma unroll
   for (int q0 = 0; q0 < PP; q0 += GRP) {
@@ -1137,7 +1170,7 @@ __device__ __forceinline__ void epilogue_oss_bwd_staged(const f32x16 (&acc)[TL::
                                                         int row0, int rows, int n0, char* lds, float* sbias = nullptr) {
   typedef T T8 __attribute__((ext_vector_type(8)));
   constexpr int CPR = TL::BN / 8, PIECES = TL::BM * CPR, PP = PIECES / TL::NT;
-  constexpr int GRP = PP >= 8 ? 4 : (PP >= 2 ? PP / 2 : 1);       // pieces per group, two groups in flight
+  constexpr int GRP = PP % 8 == 0 ? 4 : PP % 4 == 0 ? 2 : (PP >= 2 ? PP / 2 : 1);    // pieces per group, two in flight
   static_assert(PIECES % TL::NT == 0 && (PP == 1 || PP % (2 * GRP) == 0), "pieces must divide evenly");
   stage_accumulators<T, TL>(acc, lds, [](int) { return 0.0f; }, sbias);
   const int F = a.N;
@@ -1277,63 +1310,32 @@ static Raster make_striped(int64_t m_tiles, int n_tiles, int gm) {
 // =====================================================================================================
 // scatter2scatter
 // =====================================================================================================
+// What the workgroup of an output tile knows before it starts on it.
+struct S2STile {
+  int e, row0, rows;            // expert, first row (grouped order) and number of rows
+  int n_tile, n0;               // tile column and its first output column
+  int m_loc, n_loc;             // place inside the super tile
+  int part, klen;               // contraction part and its length
+  int64_t slot, own_row;        // this thread's row of the tables (thread m < BM: row m of the tile)
+};
+
+// One output tile; TL::BM >= rows.
 template <typename T, class TL, bool B_TR>
-__global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2SArgs a, Raster rast) {
+__device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int n_tiles, char* lds, int64_t* sDst,
+                                         const int* sSrc, float* sBias) {
   typedef DirectOp<TL::BM, TL::NT> AOp;
   // Ring classes serve launches with at most a tile row or two per expert: (nearly) every weight element is read
   // once, and with the non-temporal hint it does not push the token rows, which every workgroup of a tile row reads,
   // out of the L2s (hint extended from the 32-/64-row classes to all ring classes: Mixtral layer forward at 256 /
   // 384 / 448 tokens 0.539 -> 0.505 / 0.559 -> 0.526 / 0.711 -> 0.688 ms, neutral from 768 tokens on)
-  constexpr bool W_ONCE = TL::NS > 2 || TL::BM < 256;
+  constexpr bool W_ONCE = TL::NS > 2 || TL::WG > 1;
   typedef typename std::conditional<B_TR, TransOp<TL::BN, TL::NT, W_ONCE>, DirectOp<TL::BN, TL::NT, W_ONCE>>::type BOp;
-  constexpr int STAGE = AOp::LDS_BYTES + BOp::LDS_BYTES;
-  __shared__ __attribute__((aligned(16))) char lds[TL::NS * STAGE];
-  __shared__ int64_t sDst[TL::BM];
-  __shared__ int sSrc[TL::BM];
-  __shared__ __attribute__((aligned(16))) float sBias[TL::RS ? TL::BN : 4];
-
-  // Contraction parts (the class of the experts' last tiles only): the grid is `ksplit` copies of the raster, copy
-  // c multiplies the c-th part of the contraction (a raster is a multiple of 8 workgroups, so the XCD of a workgroup
-  // is still its first index modulo 8)
   constexpr bool CAN_SPLIT = TL::BM == 128 && TL::BN == 256 && TL::NS == 3;
-  // (the parts are the grid's second dimension; no division here: the compiler would do it in the vector unit and
-  // everything derived from it, loop counters and LDS addresses included, would leave the scalar registers)
-  const int part = CAN_SPLIT ? (int)blockIdx.y : 0;
-  const int klen = CAN_SPLIT && a.ksplit > 1 ? a.k_part : a.K;
-  const int k_first = part * klen;
-  int m_tile, n_tile, m_loc, n_loc;
-  if (!rast.map(blockIdx.x, m_tile, n_tile, m_loc, n_loc)) return;
-  int e, row0, rows;
-  if (a.tail_mode == 2) {
-    // one tile row per expert: the rows its last 256-row tile would hold, when there are at most BM of them
-    e = m_tile;
-    if (!find_remainder<256>(a.off, a.E, e, TL::BM, row0, rows)) return;
-  } else if (m_tile >= a.m_count ||
-             !find_tile<TL::BM>(a.off, a.E, a.m_begin + m_tile, e, row0, rows, a.tail_mode == 1 ? REMAINDER_ROWS : 0)) {
-    return;
-  }
-  // first output column of the tile; the fused forward GLU tile holds BN/2 columns of each half
-  const int n0 = a.glu == 1 ? n_tile * (TL::BN / 2) : n_tile * TL::BN;
-
-  // Row tables, one tile row per thread.  The main loop needs only the source rows; where the output rows go is
-  // stored after it, so that a launch whose input is grouped and whose output is not (layer-2 forward, layer-1
-  // input gradient) does not wait for the index vector before its first operand loads.
-  static_assert(TL::BM <= TL::NT, "one row of the tables per thread");
-  int64_t slot = 0;                                         // idx[n] where it is needed, else unused
-  int64_t own_row = 0;
-  {
-    const int m = threadIdx.x;
-    if (m < TL::BM) {
-      const int mm = m < rows ? m : rows - 1;               // tail rows re-read the last valid row
-      own_row = row0 + mm;
-      if (!a.x_grouped || !a.y_grouped) slot = a.idx[own_row];
-      sSrc[m] = a.x_grouped ? (int)own_row : (int)(slot / a.fan_out);
-    }
-  }
-  __syncthreads();
+  const int e = t.e, row0 = t.row0, rows = t.rows, n0 = t.n0;
+  const int k_first = CAN_SPLIT ? t.part * t.klen : 0;
 
   AOp A;
-  A.rot = TL::RS ? 0 : (n_loc * AOp::R / Raster::SN) % AOp::R;      // the row panel has SN sharers
+  A.rot = TL::RS ? 0 : (t.n_loc * AOp::R / Raster::SN) % AOp::R;    // the row panel has SN sharers
   // Lane offsets are 32-bit: grouped input rows are taken relative to the tile's first row (so that the input may
   // be of any size), gathered ones relative to the start of the token matrix.
   const int64_t sxm = a.sxm;
@@ -1341,7 +1343,7 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
   const char* Xb = (const char*)a.X + ((int64_t)src0 * sxm + k_first) * 2;
   A.init(Xb, [&](int row) { return (int64_t)(sSrc[row] - src0) * sxm * 2; });
   BOp B;
-  B.rot = TL::RS ? 0 : (m_loc * BOp::R / Raster::SM) % BOp::R;      // the column panel has SM sharers
+  B.rot = TL::RS ? 0 : (t.m_loc * BOp::R / Raster::SM) % BOp::R;    // the column panel has SM sharers
   const char* Wb = (const char*)a.W + ((int64_t)e * a.swe + (int64_t)k_first * (B_TR ? a.swk : 1)) * 2;
   if (a.glu == 1) {
     // tile column tc -> weight column: wave block tc / WTN, first half of the block from [0, F), second from [F, 2F)
@@ -1374,7 +1376,7 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
   if constexpr (TL::RS) mainloop_rs<T, TL, AOp, BOp>(A, B, a.K, lds, acc);
-  else if constexpr (TL::NS > 2) mainloop_ring<T, TL, AOp, BOp>(A, B, klen, lds, acc);
+  else if constexpr (TL::NS > 2) mainloop_ring<T, TL, AOp, BOp>(A, B, t.klen, lds, acc);
   else mainloop<T, TL, AOp, BOp, false>(A, B, a.K, lds, false, acc, rs);
 
   if constexpr (CAN_SPLIT) {
@@ -1383,7 +1385,7 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
       // wave); splitk_reduce_kernel knows which output element each of them belongs to.
       typedef float f32x4_t __attribute__((ext_vector_type(4)));
       f32x4_t* P = (f32x4_t*)a.partial +
-                   (((int64_t)e * rast.n_tiles + n_tile) * a.ksplit + part) * (TL::FM * TL::FN * 4 * TL::NT);
+                   (((int64_t)e * n_tiles + t.n_tile) * a.ksplit + t.part) * (TL::FM * TL::FN * 4 * TL::NT);
 #pragma unroll
       for (int i = 0; i < TL::FM; ++i)
 #pragma unroll
@@ -1397,6 +1399,7 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
   }
 
   {
+    int64_t slot = t.slot, own_row = t.own_row;
     asm volatile("" : "+v"(slot), "+v"(own_row));           // not looked at before this point
     const int m = threadIdx.x;
     if (m < TL::BM) sDst[m] = m < rows ? (a.y_grouped ? own_row : slot) * a.sym : -1;
@@ -1427,6 +1430,67 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
     epilogue_oss_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds);      // alignment checked by the launcher
   } else {
     epilogue_oss_bwd_staged<T, TL>(acc, a, row0, rows, n0, lds);
+  }
+}
+
+template <typename T, class TL, bool B_TR>
+__global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2SArgs a, Raster rast) {
+  constexpr int STAGE = (TL::BM + TL::BN) * 128;
+  __shared__ __attribute__((aligned(16))) char lds[TL::NS * STAGE];
+  __shared__ int64_t sDst[TL::BM];
+  __shared__ int sSrc[TL::BM];
+  __shared__ __attribute__((aligned(16))) float sBias[TL::RS ? TL::BN : 4];
+
+  // Contraction parts (the class of the experts' last tiles only): the grid is `ksplit` copies of the raster, copy
+  // c multiplies the c-th part of the contraction (a raster is a multiple of 8 workgroups, so the XCD of a workgroup
+  // is still its first index modulo 8)
+  constexpr bool CAN_SPLIT = TL::BM == 128 && TL::BN == 256 && TL::NS == 3;
+  // (the parts are the grid's second dimension; no division here: the compiler would do it in the vector unit and
+  // everything derived from it, loop counters and LDS addresses included, would leave the scalar registers)
+  S2STile t;
+  t.part = CAN_SPLIT ? (int)blockIdx.y : 0;
+  t.klen = CAN_SPLIT && a.ksplit > 1 ? a.k_part : a.K;
+  int m_tile;
+  if (!rast.map(blockIdx.x, m_tile, t.n_tile, t.m_loc, t.n_loc)) return;
+  if (a.tail_mode == 2) {
+    // one tile row per expert: the rows its last 256-row tile would hold, when there are at most BM of them
+    t.e = m_tile;
+    if (!find_remainder<256>(a.off, a.E, t.e, TL::BM, t.row0, t.rows)) return;
+  } else if (m_tile >= a.m_count ||
+             !find_tile<TL::BM>(a.off, a.E, a.m_begin + m_tile, t.e, t.row0, t.rows, a.tail_mode == 1 ? REMAINDER_ROWS : 0)) {
+    return;
+  }
+  // first output column of the tile; the fused forward GLU tile holds BN/2 columns of each half
+  t.n0 = a.glu == 1 ? t.n_tile * (TL::BN / 2) : t.n_tile * TL::BN;
+
+  // Row tables, one tile row per thread.  The main loop needs only the source rows; where the output rows go is
+  // stored after it, so that a launch whose input is grouped and whose output is not (layer-2 forward, layer-1
+  // input gradient) does not wait for the index vector before its first operand loads.
+  static_assert(TL::BM <= TL::NT, "one row of the tables per thread");
+  t.slot = 0;                                               // idx[n] where it is needed, else unused
+  t.own_row = 0;
+  {
+    const int m = threadIdx.x;
+    if (m < TL::BM) {
+      const int mm = m < t.rows ? m : t.rows - 1;           // tail rows re-read the last valid row
+      t.own_row = t.row0 + mm;
+      if (!a.x_grouped || !a.y_grouped) t.slot = a.idx[t.own_row];
+      sSrc[m] = a.x_grouped ? (int)t.own_row : (int)(t.slot / a.fan_out);
+    }
+  }
+  __syncthreads();
+  if constexpr (TL::BM == 256 && TL::BN == 256) {
+    // An expert's last tile is partly filled: it is multiplied at the height of its rows, in steps of 64 (which keep
+    // the four waves, or the eight, equally busy), not as a whole tile.  (Same sums in the same order.)
+    // Mixtral training shape (16.5 tiles per expert): step -1.3 %; what it mostly buys is that such tiles need no launch
+    // of their own any more (see cut_tails).
+    const int h = (t.rows + 63) >> 6;
+    if (h == 4) s2s_tile<T, TL, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
+    else if (h == 3) s2s_tile<T, typename TL::template Height<3>, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
+    else if (h == 2) s2s_tile<T, typename TL::template Height<2>, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
+    else s2s_tile<T, typename TL::template Height<1>, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
+  } else {
+    s2s_tile<T, TL, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
   }
 }
 
@@ -1502,15 +1566,9 @@ static int launch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
   return launch_status("s2s_mfma_kernel");
 }
 
-// Launches of only a few rounds of 256 x 256 tiles (one tile per CU and round) lose up to a whole round to the
-// partly filled last one; tiles of half the width take HALF_WIDTH_COST of the time and round off finer.  The
-// number of tile rows is only known on the device; the host prices both classes with its expectation for rows
-// spread evenly over the experts (binomial spread around the mean).  A wrong guess costs speed only.  Mixtral
-// expert shapes, layer 1 + layer 2 forward: 896 tokens 912 -> 833 us, 1984..2112 tokens -3 %, nothing lost
-// anywhere between 800 and 3136 tokens.
 static constexpr int NUM_CU = 256;
-static constexpr double HALF_WIDTH_COST = 0.58;
-// expected number of 256-row tiles, rounded; `skip_small`: without the experts' last tiles of at most that many rows
+// expected number of 256-row tiles for rows spread evenly over the experts (binomial spread around the mean), rounded;
+// `skip_small`: without the experts' last tiles of at most that many rows
 static double expected_row_tiles(int64_t L, int E, int skip_small = 0) {
   const double avg = (double)L / E, sd = sqrt(avg * (1.0 - 1.0 / E)) + 1e-9;
   auto above = [&](double x) { return 0.5 * erfc((x - avg) / (sd * 1.41421356)); };      // P(rows > x)
@@ -1525,15 +1583,6 @@ static double expected_row_tiles(int64_t L, int E, int skip_small = 0) {
   }
   return nearbyint(per_expert * E);
 }
-static bool half_width_wins(const S2SArgs& a) {
-  const int cols = a.glu == 1 ? 128 : 256;               // output columns of a 256-wide tile
-  const int64_t n_full = (a.N + cols - 1) / cols, n_half = (a.N + cols / 2 - 1) / (cols / 2);
-  if (max_tiles(a.L, a.E, 256) * n_full > 4 * NUM_CU) return false;
-  const double m = expected_row_tiles(a.L, a.E);
-  if (m * n_full < 96) return false;                     // far below one round: nothing to win, keep the default
-  const double full = ceil(m * n_full / NUM_CU), half = ceil(m * n_half / NUM_CU) * HALF_WIDTH_COST;
-  return half < 0.95 * full;
-}
 
 // A launch of a few whole rounds plus a remainder of up to half a round pays a whole round for the remainder.
 // Such a product is cut by tile rows: the whole rounds stay with the 256 x 256 class, the remaining tile rows go
@@ -1541,9 +1590,12 @@ static bool half_width_wins(const S2SArgs& a) {
 // rows of the first launch, 0 when the product is not split.  Plain products only (no fused unit behind them).
 // Mixtral shape, 16384 tokens (8.25 rounds in the launches with 4096 output columns): layer-2 forward
 // 3.47 -> 3.34 ms, layer-1 input gradient 7.03 -> 6.68 ms; 128 x 128 tiles for the remainder were slower
-// (four times the workgroups at 0.75 of the time).
+// (four times the workgroups at 0.75 of the time).  With few tile rows per expert the heights of the partly filled
+// tiles decide, not their number (one launch is then as fast or faster: 32 experts x 262 rows, 5760 -> 2880
+// 484 -> 456 us; 8 experts x 500 rows, 14336 -> 4096 631 -> 605), with many it pays (8 x 1000 rows 916 -> 884).
+static constexpr int TAIL_SPLIT_MIN_AVG_ROWS = 640;
 static int tail_split(const S2SArgs& a) {
-  if (a.glu != 0 || a.m_begin != 0) return 0;
+  if (a.glu != 0 || a.m_begin != 0 || a.L / a.E < TAIL_SPLIT_MIN_AVG_ROWS) return 0;
   const int64_t n_full = (a.N + 255) / 256;
   const int64_t upper = max_tiles(a.L, a.E, 256);
   if (upper * n_full > 26 * NUM_CU) return 0;
@@ -1576,21 +1628,18 @@ static int launch_main_class(const S2SArgs& a, bool b_tr, hipStream_t st) {
   return launch_s2s<T, Tile<256, 256, 2, 4>>(a, b_tr, st);
 }
 
-// A partly filled tile costs what a full one costs, and every expert ends in one (its row count modulo 256).  Products
-// with few tile rows per expert that are large enough to carry a second launch leave the last tiles of at most 128
-// rows to a launch of 128 x 256 tiles, one tile row per expert (which experts have such a tile is known only on the
-// device: the second launch covers all of them and the others' workgroups exit).  Same bits as one launch: every
-// class adds up an output element in the same order.  Measured per training step, same box: 32 experts with skewed
-// loads, 1024 rows on average (a fifth of the tile rows partly filled, several experts below 128 rows) 5.76 -> 5.51 ms;
-// 128 experts of 2048 +- 45 rows 8.01 -> 7.97 ms; 8 experts of 4096 rows 29.36 -> 29.58 ms (the second launch costs
-// what it saves): taken below 1536 rows per expert.
-// With many rows per expert and few tile columns that second launch has too few workgroups for the chip and every one
-// of them walks the whole contraction (8 experts x 16 tile columns: 64 to 128 workgroups, as long as a full tile).
-// Plain products with a caller workspace then cut the contraction of those tiles into parts, one workgroup each
-// (tail_ksplit), and a small launch adds the parts up: float32 partial sums in a fixed order, so the result is the
-// same on every run, but no longer the same bits as the unsplit product (its additions are grouped differently).
+// Products with many rows per expert and few tile columns (8 experts x 4096 rows x 16 tile columns) run in whole rounds
+// of full tiles; the experts' last tiles of at most 128 rows would add a round of 64 to 128 workgroups that each walk
+// the whole contraction.  With a caller workspace they are left to a launch of 128 x 256 tiles, one tile row per expert
+// (which experts have such a tile is known only on the device: the launch covers all of them and the others'
+// workgroups exit), with the contraction cut into parts, one workgroup each (tail_ksplit), and a small launch adds the
+// parts up: float32 partial sums in a fixed order, so the result is the same on every run, but not the same bits as
+// the unsplit product (its additions are grouped differently).  Everywhere else the last tiles stay with the others,
+// at the height of their rows: next to the expert's other tiles they find the weights in the L2, which a launch of
+// their own reads again (8 experts x 250 rows, 14336 -> 4096 505 -> 335 us, 4096 -> 2 x 14336 738 -> 636;
+// 32 experts x 400 rows, 2880 -> 2 x 2880 541 -> 468; 128 x 250 rows, 2048 -> 2 x 768 301 -> 276).
 static constexpr double REMAINDER_MIN_FLOP = 2e11;
-static constexpr int REMAINDER_MAX_AVG_ROWS = 1536;
+static constexpr int REMAINDER_MIN_AVG_ROWS = 1536;
 static constexpr int KSPLIT_MAX = 8;
 static constexpr int KSPLIT_MIN_SLICES = 16;      // 64-deep slices a part must keep
 static constexpr int64_t SPLITK_TILE_FLOATS = 128 * 256;
@@ -1607,14 +1656,14 @@ static int tail_ksplit_for(int64_t K, int64_t N, int E, int glu) {
 }
 static int64_t splitk_floats(int64_t N, int E, int ks) { return (int64_t)E * ((N + 255) / 256) * ks * SPLITK_TILE_FLOATS; }
 static int tail_ksplit(const S2SArgs& a) {
-  if (a.L / a.E < REMAINDER_MAX_AVG_ROWS) return 1;      // enough last tiles to fill the chip as they are
+  if (a.L / a.E < REMAINDER_MIN_AVG_ROWS) return 1;
   const int ks = tail_ksplit_for(a.K, a.N, a.E, a.glu);
   if (ks <= 1 || a.partial == nullptr || a.partial_floats < splitk_floats(a.N, a.E, ks)) return 1;
   return ks;
 }
 
 int64_t s2s_workspace_floats(int64_t L, int64_t K, int64_t N, int E, int dtype) {
-  if ((dtype != SMOE_BF16 && dtype != SMOE_F16) || E <= 0 || L / E < REMAINDER_MAX_AVG_ROWS) return 0;
+  if ((dtype != SMOE_BF16 && dtype != SMOE_F16) || E <= 0 || L / E < REMAINDER_MIN_AVG_ROWS) return 0;
   if (2.0 * (double)L * K * N < REMAINDER_MIN_FLOP) return 0;
   const int ks = tail_ksplit_for(K, N, E, 0);
   return ks > 1 ? splitk_floats(N, E, ks) : 0;
@@ -1623,7 +1672,7 @@ int64_t s2s_workspace_floats(int64_t L, int64_t K, int64_t N, int E, int dtype) 
 static bool cut_tails(const S2SArgs& a) {
   const bool whole = a.m_begin == 0 && a.m_count == 0x7fffffff && a.tail_mode == 0;
   if (!whole || 2.0 * (double)a.L * a.K * (a.glu == 1 ? 2.0 * a.N : (double)a.N) < REMAINDER_MIN_FLOP) return false;
-  return a.L / a.E < REMAINDER_MAX_AVG_ROWS || tail_ksplit(a) > 1;
+  return tail_ksplit(a) > 1;
 }
 
 template <typename T>
@@ -1634,21 +1683,20 @@ static int launch_tails(const S2SArgs& a, bool b_tr, hipStream_t st) {
   rest.ksplit = tail_ksplit(a);
   rest.k_part = a.K / rest.ksplit;
   if (const int rc = launch_s2s<T, TailTile>(rest, b_tr, st)) return rc;
-  if (rest.ksplit <= 1) return 0;
   const int n_tiles = (a.N + 255) / 256;
   hipLaunchKernelGGL(splitk_reduce_kernel<T>, dim3((unsigned)n_tiles, (unsigned)a.E), dim3(512), 0, st, rest, n_tiles);
   return launch_status("splitk_reduce_kernel");
 }
 
-// A whole product in the 256-row classes: the experts' sparsely filled last tiles apart (cut_tails), the rest as
-// whole rounds of 256 x 256 tiles plus a remainder of 256 x 128 tiles (tail_split) or as one launch.
+// A whole product in the 256-row classes: one launch, or whole rounds of 256 x 256 tiles plus a remainder of 256 x 128
+// tiles (tail_split), the experts' sparsely filled last tiles apart (cut_tails).
 template <typename T>
 static int launch_main(const S2SArgs& a, bool b_tr, hipStream_t st) {
   S2SArgs m = a;
   const bool tails = cut_tails(a);
   if (tails) m.tail_mode = 1;
   int rc;
-  if (const int m_first = a.L / a.E >= ROWS256_BELOW ? tail_split(m) : 0) {
+  if (const int m_first = tail_split(m)) {
     S2SArgs first = m, rest = m;
     first.m_count = m_first;
     rest.m_begin = m_first;
@@ -1662,6 +1710,7 @@ static int launch_main(const S2SArgs& a, bool b_tr, hipStream_t st) {
   return launch_tails<T>(a, b_tr, st);
 }
 
+static constexpr int MAIN_MIN_TILES = 160;
 static bool glu_fwd_pieces(const S2SArgs& a) {
   return a.glu != 1 || (((((uintptr_t)a.Y | (uintptr_t)a.H) & 15) == 0) && ((a.sym | a.shm | a.N) & 7) == 0);
 }
@@ -1715,21 +1764,21 @@ static int dispatch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
   // the backward gated epilogues address a tile's output rows with 32-bit byte offsets from its first row
   if ((a.glu == 2 || a.glu == 4) && a.sym * 2 * 256 >= 0xffffffffLL) return SMOE_ERR_UNSUPPORTED;
   const int64_t avg = a.L / a.E;
-  if (avg >= ROWS256_BELOW) {
-    S2SArgs m = a;
-    if (cut_tails(a)) m.tail_mode = 1;
-    if (tail_split(m) != 0 || !half_width_wins(a)) return launch_main<T>(a, b_tr, st);
-  }
-  // Wide launches (enough 256-wide tile columns to fill the chip twice even with one tile row per expert, e.g.
-  // Mixtral layer 1) move half as many token rows per weight byte with 256-wide tiles as with 128-wide ones:
-  // the 256 x 256 class from 136 rows per expert on (544..832 Mixtral tokens: layer 1 -9..-11 % against the
-  // 256 x 128 ring), 128 x 256 ring tiles below (experts of about one 128-row tile: 448 tokens 518 -> 373 us,
-  // 512 tokens 520 -> 455 us).  Launches with few tile columns (Mixtral layer 2) are faster in the classes below.
-  const bool wide = (int64_t)a.E * ((a.N + (a.glu == 1 ? 127 : 255)) / (a.glu == 1 ? 128 : 256)) >= 2 * NUM_CU;
-  if (wide && avg >= ROWS128W_BELOW) return launch_main<T>(a, b_tr, st);
-  if (wide && avg >= ROWS64_BELOW) return launch_s2s<T, Tile<128, 256, 2, 4, 3>>(a, b_tr, st);
-  // Below that the launch is a stream over the weights: tile height by rows per expert
+  // 256 x 256 tiles, each at the height of its rows, from 112 rows per expert on if one tile row per expert gives most
+  // CUs a workgroup (us against the 256 x 128 and 128-row ring classes: 32 experts x 125 rows, 2880 -> 2 x 2880
+  // 269 -> 214, 5760 -> 2880 286 -> 254; 8 x 140, 4096 -> 11264 210 -> 181; 128 x 188, 2048 -> 768 with its gated unit's
+  // gradient 168 -> 144; with half as many tiles as CUs, 8 x 188, 14336 -> 4096, 263 -> 288, even below 160 rows), from
+  // 52 rows on where it makes one round of what the 128-row tiles do in two (16 x 90, 2048 -> 2 x 1408 56 -> 42), and
+  // whatever the number of tiles from 224 rows on.
+  const int64_t tiles = (int64_t)a.E * ((a.N + (a.glu == 1 ? 127 : 255)) / (a.glu == 1 ? 128 : 256));
+  if (avg >= ROWS256_BELOW || (avg >= ROWS128_BELOW && tiles >= MAIN_MIN_TILES) ||
+      (avg >= ROWS64_BELOW && tiles > NUM_CU / 2 && tiles <= NUM_CU))
+    return launch_main<T>(a, b_tr, st);
+  // Below that the launch is a stream over the weights: tile height by rows per expert.  Launches with enough 256-wide
+  // tile columns to fill the chip twice move half as many token rows per weight byte with 256-wide tiles as with
+  // 128-wide ones (experts of about one 128-row tile, Mixtral layer 1: 448 tokens 518 -> 373 us).
   if (avg >= ROWS128_BELOW) return launch_s2s<T, Tile<256, 128, 4, 2, 3>>(a, b_tr, st);
+  if (avg >= ROWS64_BELOW && tiles >= 2 * NUM_CU) return launch_s2s<T, Tile<128, 256, 2, 4, 3>>(a, b_tr, st);
   if (avg < ROWS64_BELOW) return dispatch_few_rows<T>(a, b_tr, st);
   // With one column block per wave the fused forward GLU exists only in its LDS-staged form (16-byte pieces)
   if (!glu_fwd_pieces(a)) return SMOE_ERR_UNSUPPORTED;
