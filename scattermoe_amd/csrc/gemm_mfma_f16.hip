@@ -1,0 +1,9 @@
+// fp16 instantiation of the MFMA kernels (gemm_mfma.hpp).
+#include "gemm_mfma.hpp"
+
+namespace smoe {
+
+int dispatch_s2s_f16(const S2SArgs& a, bool b_tr, hipStream_t st) { return dispatch_s2s<f16_t>(a, b_tr, st); }
+int dispatch_xty_f16(const XtYArgs& a, bool rs_form, hipStream_t st) { return dispatch_xty<f16_t>(a, rs_form, st); }
+
+}  // namespace smoe
