@@ -5,6 +5,7 @@
 namespace smoe {
 
 int dispatch_s2s_f16(const S2SArgs& a, bool b_tr, hipStream_t st);
+int dispatch_xty_bf16(const XtYArgs& a, bool rs_form, hipStream_t st);
 int dispatch_xty_f16(const XtYArgs& a, bool rs_form, hipStream_t st);
 
 int64_t s2s_workspace_floats(int64_t L, int64_t K, int64_t N, int E, int dtype) {
@@ -61,7 +62,7 @@ bool try_xty_mfma(const XtYArgs& a, int dtype, hipStream_t st, int& rc) {
   const bool out16 = (((uintptr_t)a.DW & 15) == 0) && ((a.sdwe | (a.sdwk == 1 ? a.sdwn : a.sdwk) | (a.sdwk == 1 ? a.K : a.N)) & 7) == 0;
   const bool db_in_loop = a.Db != nullptr && a.sdwk == 1;
   const bool rs_form = a.idx == nullptr && !db_in_loop && out16 && a.L / a.E >= RS_XTY_MIN_ROWS;
-  rc = dtype == SMOE_BF16 ? dispatch_xty<bf16_t>(a, rs_form, st) : dispatch_xty_f16(a, rs_form, st);
+  rc = dtype == SMOE_BF16 ? dispatch_xty_bf16(a, rs_form, st) : dispatch_xty_f16(a, rs_form, st);
   return true;
 }
 

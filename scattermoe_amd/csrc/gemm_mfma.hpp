@@ -405,8 +405,19 @@ __device__ __forceinline__ void mainloop(AOp& A, BOp& B, int klen, char* lds, bo
   A.fetch_rows(BK, klen);            // gathered operands: row indices of the slice after the one just issued
   B.fetch_rows(BK, klen);
   for (int kt = 0; kt < nk; ++kt) {
-    char* cur = lds + (kt & 1) * STAGE;
-    const unsigned nxt = lds_u + ((kt + 1) & 1) * STAGE;
+    char* cur = lds + (TL::NS == 1 ? 0 : (kt & 1) * STAGE);
+    const unsigned nxt = lds_u + (TL::NS == 1 ? 0 : ((kt + 1) & 1) * STAGE);
+    if (TL::NS == 1 && kt > 0) {
+      // one stage: slice kt is requested once everyone is done with slice kt - 1; the other workgroups of the CU
+      // multiply meanwhile
+      __syncthreads();
+      A.take_rows(kt);
+      B.take_rows(kt);
+      if (kt < nfull) issue_slice(A, B, lds_u, kt * BK);
+      else issue_slice_tail(A, B, lds_u, kt * BK, klen);
+      A.fetch_rows((kt + 1) * BK, klen);
+      B.fetch_rows((kt + 1) * BK, klen);
+    }
     __builtin_amdgcn_s_waitcnt(0);   // this thread's direct loads of slice kt have landed in LDS
     if (tail && kt == nfull) {
       A.zero_tail(cur, kt * BK, klen);
@@ -415,13 +426,15 @@ __device__ __forceinline__ void mainloop(AOp& A, BOp& B, int klen, char* lds, bo
     A.stage_rows(kt + 1);
     B.stage_rows(kt + 1);
     __syncthreads();                 // ... everyone's have, and everyone is done reading `nxt`
-    A.take_rows(kt + 1);
-    B.take_rows(kt + 1);
-    if (kt + 1 < nfull) issue_slice(A, B, nxt, (kt + 1) * BK);
-    else if (tail && kt + 1 == nfull) issue_slice_tail(A, B, nxt, (kt + 1) * BK, klen);
-    if (kt + 2 < nk) {
-      A.fetch_rows((kt + 2) * BK, klen);
-      B.fetch_rows((kt + 2) * BK, klen);
+    if constexpr (TL::NS > 1) {
+      A.take_rows(kt + 1);
+      B.take_rows(kt + 1);
+      if (kt + 1 < nfull) issue_slice(A, B, nxt, (kt + 1) * BK);
+      else if (tail && kt + 1 == nfull) issue_slice_tail(A, B, nxt, (kt + 1) * BK, klen);
+      if (kt + 2 < nk) {
+        A.fetch_rows((kt + 2) * BK, klen);
+        B.fetch_rows((kt + 2) * BK, klen);
+      }
     }
     const char* ta = cur;
     const char* tb = cur + AOp::LDS_BYTES;
@@ -750,7 +763,6 @@ template <typename T, class TL, typename BF>
 __device__ __forceinline__ void stage_accumulators(const f32x16 (&acc)[TL::FM][TL::FN], char* lds, BF bias_of,
                                                    float* sbias) {
   typedef T T4 __attribute__((ext_vector_type(4)));
-  static_assert(TL::BM * TL::BN * 2 <= TL::NS * (TL::BM + TL::BN) * 128, "staged tile must fit the operand buffers");
   const int wave = threadIdx.x >> 6, l = lane_id();
   const int wm = wave / TL::WN, wn = wave % TL::WN;
   // One wave per SIMD: the additions per column come from LDS (written here, one column per thread), so that the
@@ -1437,6 +1449,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
 template <typename T, class TL, bool B_TR>
 __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2SArgs a, Raster rast) {
   constexpr int STAGE = (TL::BM + TL::BN) * 128;
+  static_assert(TL::BM * TL::BN * 2 <= TL::NS * STAGE, "staged tile must fit the operand buffers");
   __shared__ __attribute__((aligned(16))) char lds[TL::NS * STAGE];
   __shared__ int64_t sDst[TL::BM];
   __shared__ int sSrc[TL::BM];
@@ -1801,11 +1814,12 @@ struct XtYPlan {
 };
 
 template <typename T, class TL, bool GA, bool GB>
-__global__ __launch_bounds__(TL::NT) void xty_mfma_kernel(XtYPlan a, Raster rast, int p_tiles) {
+__global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void xty_mfma_kernel(XtYPlan a, Raster rast, int p_tiles) {
   typedef TransOp<TL::BM, TL::NT, false, GA> AOp;
   typedef TransOp<TL::BN, TL::NT, false, GB> BOp;
   constexpr int STAGE = AOp::LDS_BYTES + BOp::LDS_BYTES;
-  __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
+  constexpr int STAGED = TL::BM * TL::BN * 2;          // the output tile on its way out
+  __shared__ __attribute__((aligned(16))) char lds[TL::NS * STAGE > STAGED ? TL::NS * STAGE : STAGED];
   __shared__ int64_t sDst[TL::BM];
   __shared__ unsigned sRows[2 * 64];       // row offsets of a gathered operand (see TransOp)
   __shared__ __attribute__((aligned(16))) float sBias[TL::RS ? TL::BN : 4];
@@ -1876,7 +1890,17 @@ __global__ __launch_bounds__(256) void colsum_kernel(const T* __restrict__ DY, i
   const int r_lo = e ? (int)off[e - 1] : 0, r_hi = (int)off[e];
   float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (n < N) {
-    for (int r = r_lo + rg; r < r_hi; r += 8) {
+    int r = r_lo + rg;
+    for (; r + 56 < r_hi; r += 64) {                   // eight loads in flight: a load at a time is all latency
+      T8 v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = *(const T8*)(DY + (int64_t)(r + 8 * u) * ld + n);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s[q] += to_f32(v[u][q]);
+    }
+    for (; r < r_hi; r += 8) {
       const T8 v = *(const T8*)(DY + (int64_t)r * ld + n);
 #pragma unroll
       for (int q = 0; q < 8; ++q) s[q] += to_f32(v[q]);
@@ -1930,8 +1954,29 @@ static int launch_xty(const XtYArgs& a, hipStream_t st) {
   return rc;
 }
 
+// Which tiles a weight gradient is cut into.  A 256 x 256 tile has a CU to itself and the memory idles while it is
+// looked up, waits for its first slice and is stored; with few rows per expert that is most of its time.  Small tiles
+// (128 x 128, one 32 KB stage, four workgroups per CU; the stores of one run under the loads and products of the
+// others) pay for it with twice the operand traffic through LDS, so they win below a number of rows (both sides
+// measured alone, us: 32 experts 2880 x 5760, 100 / 188 / 300 / 400 rows each: 314 -> 225, 407 -> 335, 493 -> 455,
+// 594 -> 579; 128 experts 2048 x 1536: 223 -> 168, 286 -> 242, 371 -> 364, 462 -> 477; 8 experts 14336 x 4096:
+// 257 -> 191, 316 -> 270, 390 -> 370, 480 -> 489.  Inside a training step, at its lower clock: 32 x 188 rows, 2880 x 2880
+// 248 -> 212; even at 280).  Gathered rows chain two more memory accesses in front of every slice, which small tiles
+// repeat too often (32 experts 400 -> 372, 128 experts 276 -> 279): they keep the large ones.
+static constexpr int XTY_SMALL_ROWS = 256;
+// The same small tiles, whatever the number of rows, where the 256 x 256 ones leave the chip idle: at most 5/8 of a
+// round of one per CU, or a second round up to 9/16 full (1600 rows per expert, plain / gathered, us: 128 tiles
+// 56 -> 38 / 45 -> 37, 160 tiles 59 -> 50 / 51 -> 48, 320 tiles 102 -> 77 / 96 -> 84, 384 tiles 105 -> 90 / 100 -> 90;
+// but 192 tiles 56 -> 57 / 48 -> 58, 256 tiles 64 -> 60 / 55 -> 61, 512 tiles 110 -> 112 / 105 -> 116).
+static bool xty_idle_chip(const XtYArgs& a) {
+  const int64_t tiles = (int64_t)a.E * ((a.N + 255) / 256) * ((a.K + 255) / 256);
+  return tiles <= 160 || (tiles > 256 && tiles <= 400);
+}
+
 template <typename T>
 static int dispatch_xty(const XtYArgs& a, bool rs_form, hipStream_t st) {
+  typedef Tile<128, 128, 2, 2, 1, false, 4> Small;
+  if (xty_idle_chip(a) || (a.idx == nullptr && a.L / a.E <= XTY_SMALL_ROWS)) return launch_xty<T, Small>(a, st);
   if (rs_form) return launch_xty<T, Tile<256, 256, 2, 2, 2, true>>(a, st);
   return launch_xty<T, Tile<256, 256, 2, 4>>(a, st);
 }

@@ -4,6 +4,5 @@
 namespace smoe {
 
 int dispatch_s2s_f16(const S2SArgs& a, bool b_tr, hipStream_t st) { return dispatch_s2s<f16_t>(a, b_tr, st); }
-int dispatch_xty_f16(const XtYArgs& a, bool rs_form, hipStream_t st) { return dispatch_xty<f16_t>(a, rs_form, st); }
 
 }  // namespace smoe

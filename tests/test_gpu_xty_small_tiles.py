@@ -1,0 +1,62 @@
+"""Weight gradients in small tiles (128 x 128, one operand stage): expert loads on both sides
+of every slice boundary, output sizes that are no whole number of tiles, both output layouts, with and without
+gathered rows and bias gradient, an output whose rows are not 16-byte aligned."""
+import pytest
+import torch
+
+from scattermoe_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+LOADS = [1, 63, 64, 65, 0, 127, 128, 129, 191, 192, 193, 256, 300, 320, 31, 0]
+
+
+def _check(got, want, mass, n, dtype):
+    """One rounding to the storage type, float32 sums of n products of total magnitude `mass` in any order."""
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    bound = unit * want.abs() + n * 2.0 ** -24 * mass + 2.0 ** -24
+    assert bool(((got.double() - want).abs() <= bound).all())
+
+
+# 16 experts of 139 rows on average: few rows (512 output tiles of 256 x 256 and more); 64-wide sizes: few tiles
+@pytest.mark.parametrize("K,N", [(2056, 1048), (1536, 1544), (200, 136), (64, 520)])
+@pytest.mark.parametrize("layout", ["nk", "kn"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_against_float64(K, N, layout, dtype):
+    g = torch.Generator(device=DEV).manual_seed(K + N)
+    E, L, k = len(LOADS), sum(LOADS), 2
+    loads = LOADS if L % k == 0 else LOADS[:-2] + [LOADS[-2] + 1, 0]
+    L = sum(loads)
+    experts = torch.repeat_interleave(torch.arange(E, device=DEV), torch.tensor(loads, device=DEV))
+    experts = experts[torch.randperm(L, generator=g, device=DEV)].view(L // k, k)
+    eid, idx, off = ops.route(experts, E)
+    X = torch.randn(L // k, K, generator=g, device=DEV).to(dtype)
+    DY = torch.randn(L, N, generator=g, device=DEV).to(dtype)
+    like = torch.empty(E, K, N, dtype=dtype, device=DEV) if layout == "kn" else None
+    Xg = ops.group(X, idx, fan_out=k)
+    DW, Db = ops.group_bwd_W(DY, Xg, off, E, has_bias=True, like=like)
+    DWg, Dbg = ops.group_bwd_W(DY, X, off, E, has_bias=True, like=like, gather=(idx, k))
+    assert torch.equal(DW, DWg) and torch.equal(Db, Dbg)
+    DWg, Dbg = torch.empty_like(DW), torch.empty_like(Db)
+    assert ops._backend.xty_gathered(DY, X, idx, k, DWg, Dbg, off, E)          # rows looked up inside the launch
+    assert torch.equal(DW, DWg) and torch.equal(Db, Dbg)
+    ends = [0] + off.tolist()
+    for e in range(E):
+        x, y = Xg[ends[e]:ends[e + 1]].double(), DY[ends[e]:ends[e + 1]].double()
+        n = x.size(0)
+        _check(DW[e], x.t() @ y, x.abs().t() @ y.abs(), n, dtype)
+        _check(Db[e], y.sum(0), y.abs().sum(0), n, dtype)
+
+
+def test_unaligned_output():
+    """An output two bytes off a 16-byte boundary takes the plain stores; the same bits."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    E, n, K, N = 4, 100, 136, 72
+    off = torch.arange(1, E + 1, device=DEV) * n
+    X = torch.randn(E * n, K, generator=g, device=DEV).bfloat16()
+    DY = torch.randn(E * n, N, generator=g, device=DEV).bfloat16()
+    DW, _ = ops.group_bwd_W(DY, X, off, E)
+    buf = torch.zeros(E * N * K + 2, device=DEV, dtype=torch.bfloat16)
+    out = buf[1:-1].view(E, N, K)
+    ops._xty_launch(E, out.permute(0, 2, 1), None, DY, X, off)
+    assert torch.equal(out.permute(0, 2, 1), DW) and buf[0] == 0 and buf[-1] == 0
