@@ -142,6 +142,86 @@ __device__ __forceinline__ bool find_tile(const int64_t* __restrict__ off, int E
   return false;
 }
 
+// The same for launches whose workgroups take all output tiles in an order that keeps together what shares operands:
+// expert by expert, inside an expert column by column (of `n_tiles`), the expert's tile rows of a column side by side.
+// The XCD of a workgroup is `pid` % 8; the order is cut into 8 R chunks of equal length and XCD x takes the chunks
+// x, x + 8, ... (in turn from either end).  How many tiles there are is known only here, from `off`: R = 1, or with
+// `rounds` as many as there are rounds of 256 tiles.  A grid of chunked_grid() workgroups covers every tile.
+// Returns 1: this workgroup's tile; 0: none; -1: the experts differ in tile rows by more than a quarter (and not only in
+// having none), so that equal numbers of tiles are not equal work: another order has to be taken (the same answer in
+// every workgroup).
+template <int BM>
+__device__ __forceinline__ int find_tile_chunked(const int64_t* __restrict__ off, int E, int pid, int n_tiles,
+                                                 bool rounds, int& expert, int& row_start, int& rows, int& column) {
+  const int lane = lane_id();
+  auto load = [&](int e0, int& lo, int& hi, int& nt) {        // experts e0 .. e0 + 63, one per lane
+    const int e = e0 + lane;
+    lo = hi = 0;
+    if (e < E) {
+      hi = (int)off[e];
+      lo = e ? (int)off[e - 1] : 0;
+    }
+    nt = (hi - lo + BM - 1) / BM;
+  };
+  auto scan = [&](int nt) {                                   // inclusive sums
+    int incl = nt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      int v = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += v;
+    }
+    return incl;
+  };
+  int lo, hi, nt;
+  load(0, lo, hi, nt);
+  const int ref = __builtin_amdgcn_readfirstlane(nt);
+  bool many = nt > 1, differs = lane < E && 4 * abs(nt - ref) > ref;
+  for (int e0 = 64; e0 < E; e0 += 64) {
+    int l_, h_, n_;
+    load(e0, l_, h_, n_);
+    many |= n_ > 1;
+    differs |= e0 + lane < E && 4 * abs(n_ - ref) > ref;
+  }
+  if (__ballot(many) && __ballot(differs)) return -1;
+  int incl = scan(nt);
+  int total = __builtin_amdgcn_readlane(incl, 63);
+  for (int e0 = 64; e0 < E; e0 += 64) {
+    int l_, h_, n_;
+    load(e0, l_, h_, n_);
+    total += __builtin_amdgcn_readlane(scan(n_), 63);
+  }
+  const unsigned tiles = (unsigned)total * n_tiles;
+  const unsigned R = rounds && tiles >= 384 ? (tiles + 128) / 256 : 1;
+  const unsigned len = __builtin_amdgcn_readfirstlane((tiles + 8 * R - 1) / (8 * R));
+  if (len == 0) return 0;
+  const unsigned x = pid & 7, i = (unsigned)pid >> 3, c = i / len;
+  const unsigned l = (c * 8 + ((c & 1) ? 7 - x : x)) * len + (i - c * len);
+  if (c >= R || l >= tiles) return 0;
+  int before = 0;                                             // tile rows of the experts before this group
+  for (int e0 = 0;;) {
+    const unsigned cum = before + incl;
+    const unsigned long long hit = __ballot(cum * n_tiles > l);
+    if (hit) {
+      const int src = __ffsll((long long)hit) - 1;
+      const int lo_s = __builtin_amdgcn_readlane(lo, src), hi_s = __builtin_amdgcn_readlane(hi, src);
+      const unsigned nt_s = __builtin_amdgcn_readlane(nt, src);
+      const unsigned in_expert = l - (__builtin_amdgcn_readlane((int)cum, src) - nt_s) * n_tiles;
+      column = __builtin_amdgcn_readfirstlane(in_expert / nt_s);
+      expert = e0 + src;
+      row_start = lo_s + __builtin_amdgcn_readfirstlane(in_expert - column * nt_s) * BM;
+      rows = min(BM, hi_s - row_start);
+      return 1;
+    }
+    before += __builtin_amdgcn_readlane(incl, 63);
+    e0 += 64;
+    if (e0 >= E) return 0;
+    load(e0, lo, hi, nt);
+    incl = scan(nt);
+  }
+}
+// Workgroups of such a launch of at most `tiles` tiles: 8 R chunks round up by less than 8 R <= tiles / 32 + 8.
+static inline int64_t chunked_grid(int64_t tiles) { return (tiles + tiles / 32 + 16 + 7) / 8 * 8; }
+
 // The rows that find_tile<BM>(..., skip_small) leaves out, as one tile per expert: the last n % BM rows of expert e
 // when there are between 1 and `small` of them.
 template <int BM>

@@ -26,6 +26,16 @@
 static constexpr int ROWS32_BELOW = 16, ROWS64_BELOW = 52, ROWS128_BELOW = 112, ROWS256_BELOW = 224;
 static constexpr int GM_RING = 8;
 static constexpr int STRIPE_BELOW = 1024;
+// Whole launches below this many rows per expert are taken in chunks of neighbouring tiles per XCD (find_tile_chunked)
+// where the experts' loads are even: an XCD then reads the token rows of its own experts only (column stripes: all rows,
+// eight times over the fabric) and streams through one contiguous piece of the weights.  One chunk per XCD where the
+// launch is a stream over the weights, else as many as there are rounds, so that the XCDs stay at neighbouring experts.
+// Whole layers, us, stripes or super tiles -> chunks: 128 experts d = 2048, F = 768, forward of 60 / 200 / 2000 / 6000 /
+// 10000 tokens 216 -> 205, 238 -> 227, 380 -> 350, 694 -> 677, 1032 -> 982; 32 experts d = F = 2880, 48 tokens 261 ->
+// 252, training step of 1501 / 3000 tokens 1617 -> 1574, 2653 -> 2525; 8 experts d = 4096, F = 14336, training step of
+// 6000 tokens 11996 -> 11728.  Uneven loads keep the other order (taken in chunks, loads falling as 1 / rank^1.8: 1607 -> 1681).
+// Above 2048 rows per expert: even (128 experts x 2048 rows 8538 -> 8546).
+static constexpr int CHUNK_BELOW = 3072;
 static constexpr int GM_S2S = 4;
 static constexpr int GM_XTY = 4;
 static constexpr int XTY_GATHER_MAX_N = 6144;   // widest dY for which groupXtY gathers the rows of X itself
@@ -1252,6 +1262,7 @@ struct Raster {
   static constexpr int SM = 8, SN = 4;
   int m_tiles, n_tiles, m_supers, n_supers, supers, gm;
   int striped;                             // 1: column-striped order of the memory-bound classes (see make_striped)
+  int chunked = 0;                         // 1, 2: order of find_tile_chunked (2: in rounds) before this one
   int64_t grid_size;                       // host side only: number of workgroups (may exceed what a launch takes)
   __host__ int64_t grid() const { return grid_size; }
   // (ml, nl): position of the tile inside its super tile
@@ -1465,8 +1476,16 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
   t.part = CAN_SPLIT ? (int)blockIdx.y : 0;
   t.klen = CAN_SPLIT && a.ksplit > 1 ? a.k_part : a.K;
   int m_tile;
-  if (!rast.map(blockIdx.x, m_tile, t.n_tile, t.m_loc, t.n_loc)) return;
-  if (a.tail_mode == 2) {
+  int found = -1;
+  if (rast.chunked) {
+    t.m_loc = t.n_loc = 0;
+    found = find_tile_chunked<TL::BM>(a.off, a.E, blockIdx.x, rast.n_tiles, rast.chunked == 2, t.e, t.row0, t.rows, t.n_tile);
+    if (found == 0) return;
+  }
+  if (found < 0 && !rast.map(blockIdx.x, m_tile, t.n_tile, t.m_loc, t.n_loc)) return;
+  if (found > 0) {
+    // looked up above
+  } else if (a.tail_mode == 2) {
     // one tile row per expert: the rows its last 256-row tile would hold, when there are at most BM of them
     t.e = m_tile;
     if (!find_remainder<256>(a.off, a.E, t.e, TL::BM, t.row0, t.rows)) return;
@@ -1566,7 +1585,13 @@ static int launch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
   // With only a few tile rows per expert no weight panel is shared by the tile rows of a super tile; the striped
   // order at least keeps the tile rows of one expert together on one XCD.
   const bool striped = TL::NS > 2 || a.L / a.E < STRIPE_BELOW;
-  const Raster r = striped ? make_striped(m_tiles, n_tiles, GM_RING) : make_raster(m_tiles, n_tiles, GM_S2S);
+  Raster r = striped ? make_striped(m_tiles, n_tiles, GM_RING) : make_raster(m_tiles, n_tiles, GM_S2S);
+  const bool whole = a.m_begin == 0 && a.m_count == 0x7fffffff && a.tail_mode == 0;
+  const int64_t chunked = chunked_grid(m_tiles * n_tiles);
+  if (whole && a.L / a.E < CHUNK_BELOW && chunked <= 0x7fffffffLL) {
+    r.chunked = TL::NS > 2 || TL::WG > 1 || a.L / a.E < ROWS256_BELOW ? 1 : 2;
+    r.grid_size = std::max(r.grid_size, chunked);
+  }
   const int64_t grid = r.grid();
   const unsigned parts = a.ksplit > 1 ? (unsigned)a.ksplit : 1u;
   if (grid > 0x7fffffffLL || m_tiles > 0x7fffffffLL) { set_error("smoe_scatter2scatter: grid too large"); return SMOE_ERR_RANGE; }
