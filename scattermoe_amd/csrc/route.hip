@@ -7,6 +7,8 @@
 //   hist    : per-chunk LDS histogram                       -> counts[chunk][E]
 //   scan    : exclusive scan over (expert-major, chunk)     -> bases[chunk][E], off[E]
 //   scatter : stable rank inside the chunk + base           -> eid_out, idx_out
+// (us, all three, chunks ranked by 16 waves in one pass instead of 4 waves in two: 31992 rows of 128 experts 26.9 -> 13.6,
+// 32768 of 8 18.7 -> 11.1, 262144 of 128 33.9 -> 20.6)
 // The result is independent of scheduling: every output position is a pure function of the input.
 #include "common.hpp"
 #include <mutex>
@@ -14,11 +16,10 @@
 namespace smoe {
 
 static constexpr int kRouteThreads = 256;
-static constexpr int kRouteWaves = kRouteThreads / 64;
 static constexpr int kRouteChunk = 4096;       // elements per block
 static constexpr int kRouteMaxE = 2048;        // LDS: (waves+1) * E ints
-static constexpr int kRouteFusedMax = 16384;   // rows one workgroup of 1024 threads sorts by itself (32768 rows take it
-                                               // 33 us, the three launches 28 us) ...
+static constexpr int kRouteFusedMax = 16384;   // rows one workgroup of 1024 threads sorts by itself, without a
+                                               // workspace (the three launches: 10 us and more) ...
 static constexpr int kRouteFusedMaxE = 512;    // ... for at most this many experts (17 * E ints of LDS)
 
 template <typename I>
@@ -41,72 +42,76 @@ __device__ __forceinline__ int bits_for(int E) {
   return nbits;
 }
 
-// Per-wave histogram of the wave's contiguous segment of the chunk.  wave w owns
-// [chunk_lo + w*seg, chunk_lo + (w+1)*seg) ∩ [0, L).
-template <typename I>
-__device__ __forceinline__ void wave_histogram(const I* __restrict__ ids, int64_t seg_lo, int64_t seg_hi,
-                                               int E, int* __restrict__ hist_w) {
+// A wave's contiguous segment of at most IT * 64 rows, read once: key[u] is the id of row seg_lo + 64 u + lane (-1: no
+// row, or an id that is no expert), loc[u] its rank among the wave's rows of that expert.  hist_w (zero on entry) ends
+// as the wave's histogram: equal ids of 64 rows are found by match_any and added by one lane, whose returned value is
+// the number of such rows before these (a wave's LDS operations complete in order), so neither many lanes on one
+// counter nor a second counting pass is needed to place the rows.
+template <typename I, int IT>
+__device__ __forceinline__ void wave_rank(const I* __restrict__ ids, int64_t seg_lo, int64_t seg_hi, int E, int nbits,
+                                          int* __restrict__ hist_w, int (&key)[IT], int (&loc)[IT]) {
   const int lane = lane_id();
-  for (int64_t p = seg_lo + lane; p < seg_hi; p += 64) {
-    const int e = load_id(ids, p);
-    if ((unsigned)e < (unsigned)E) atomicAdd(&hist_w[e], 1);
+  const unsigned long long lt = (1ull << lane) - 1ull;
+#pragma unroll
+  for (int u = 0; u < IT; ++u) {
+    const int64_t p = seg_lo + u * 64 + lane;
+    key[u] = p < seg_hi ? load_id(ids, p) : -1;
+  }
+#pragma unroll
+  for (int u = 0; u < IT; ++u) {
+    const bool ok = (unsigned)key[u] < (unsigned)E;
+    key[u] = ok ? key[u] : -1;
+    loc[u] = 0;
+    if (seg_lo + u * 64 < seg_hi) {
+      const unsigned long long same = match_any(ok ? key[u] : 0, nbits, ok);
+      const int leader = __ffsll((long long)same) - 1;   // -1 only for lanes with ok == false
+      int first = 0;
+      if (ok && lane == leader) first = atomicAdd(&hist_w[key[u]], __popcll(same));
+      first = __shfl(first, leader < 0 ? 0 : leader, 64);
+      loc[u] = first + __popcll(same & lt);
+    }
   }
 }
 
-// Stable scatter of one wave's segment.  base_w[e] holds the output position of the wave's next row
-// of expert e and is advanced as rounds of 64 consecutive elements are placed.
-template <typename I>
-__device__ __forceinline__ void wave_scatter(const I* __restrict__ ids, int64_t seg_lo, int64_t seg_hi,
-                                             int E, int nbits, int* __restrict__ base_w,
-                                             int64_t* __restrict__ eid_out, int64_t* __restrict__ idx_out) {
-  const int lane = lane_id();
-  const unsigned long long lt = (1ull << lane) - 1ull;
-  for (int64_t p0 = seg_lo; p0 < seg_hi; p0 += 64) {
-    const int64_t p = p0 + lane;
-    const bool in = p < seg_hi;
-    int e = in ? load_id(ids, p) : 0;
-    const bool ok = in && (unsigned)e < (unsigned)E;
-    if (!ok) e = 0;
-    const unsigned long long same = match_any(e, nbits, ok);
-    const int rank = __popcll(same & lt);
-    const int leader = __ffsll((long long)same) - 1;   // -1 only for lanes with ok == false
-    int first = 0;
-    if (ok && lane == leader) first = atomicAdd(&base_w[e], __popcll(same));
-    first = __shfl(first, leader < 0 ? 0 : leader, 64);
-    if (ok) {
-      const int pos = first + rank;
-      eid_out[pos] = (int64_t)e;
-      idx_out[pos] = p;
-    }
+// hist[w][e], w < W -> number of rows of expert e in the waves before w (from `run` on); returns the end.
+// All counters are read before the first is written: 16 LDS round trips one after the other otherwise.
+template <int W>
+__device__ __forceinline__ int prefix_over_waves(int* __restrict__ hist, int E, int e, int run) {
+  int c[W];
+#pragma unroll
+  for (int w = 0; w < W; ++w) c[w] = hist[w * E + e];
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    hist[w * E + e] = run;
+    run += c[w];
   }
+  return run;
 }
 
 // ---- single-launch path: whole input in one block ------------------------------------------------
-template <typename I, int THREADS>
+// Bound by latency (one read of the ids, LDS counters, four barriers) and, written row by row, by one CU's rate of
+// scattered 8-byte stores: the sorted rows are put together in LDS and written out in whole lines.
+// us, two passes over the ids by 4 waves (up to 4096 rows) or 16, rows written one by one -> now:
+// 1554 rows of 8 experts 6.6 -> 3.8, 1600 of 128 8.6 -> 4.6, 6004 of 32 8.4 -> 7.8, 16384 of 128 23.2 -> 19.3.
+template <typename I, int THREADS, int IT>
 __global__ __launch_bounds__(THREADS) void route_fused_kernel(
     const I* __restrict__ ids, int L, int E, int64_t* __restrict__ eid_out,
     int64_t* __restrict__ idx_out, int64_t* __restrict__ off_out) {
-  constexpr int kRouteThreads = THREADS, kRouteWaves = THREADS / 64;      // this kernel's own block shape
-  extern __shared__ int lds[];          // [kRouteWaves][E] wave histograms/bases, then [E] totals
-  int* hist = lds;
-  int* total = lds + kRouteWaves * E;
+  constexpr int W = THREADS / 64, EMAX = W == 16 ? kRouteFusedMaxE : kRouteMaxE;
+  static_assert(THREADS * IT <= 65536 && EMAX <= 65536, "row and expert share a word");
+  __shared__ int hist[W * EMAX];        // [W][E] wave histograms, then the wave's first place within the expert
+  __shared__ int total[EMAX];           // [E] rows of the expert, then its first place
+  __shared__ unsigned sorted[THREADS * IT];
+  __shared__ int n_valid;
   const int tid = threadIdx.x, w = tid >> 6;
-  for (int i = tid; i < (kRouteWaves + 1) * E; i += kRouteThreads) lds[i] = 0;
+  for (int i = tid; i < W * E; i += THREADS) hist[i] = 0;
   __syncthreads();
-  const int seg = (L + kRouteWaves - 1) / kRouteWaves;
-  const int64_t lo = min((int64_t)w * seg, (int64_t)L), hi = min(lo + seg, (int64_t)L);
-  wave_histogram(ids, lo, hi, E, hist + w * E);
+  const int seg = ((L + W - 1) / W + 63) / 64 * 64;      // at most IT * 64 (the launcher's choice)
+  const int lo = min(w * seg, L), hi = min(lo + seg, L);
+  int key[IT], loc[IT];
+  wave_rank<I, IT>(ids, lo, hi, E, bits_for(E), hist + w * E, key, loc);
   __syncthreads();
-  // per expert: exclusive prefix over waves, total count
-  for (int e = tid; e < E; e += kRouteThreads) {
-    int run = 0;
-    for (int ww = 0; ww < kRouteWaves; ++ww) {
-      const int c = hist[ww * E + e];
-      hist[ww * E + e] = run;
-      run += c;
-    }
-    total[e] = run;
-  }
+  for (int e = tid; e < E; e += THREADS) total[e] = prefix_over_waves<W>(hist, E, e, 0);
   __syncthreads();
   // exclusive scan of totals over experts (wave 0, 64 experts per step), inclusive offsets out
   if (w == 0) {
@@ -127,29 +132,36 @@ __global__ __launch_bounds__(THREADS) void route_fused_kernel(
       }
       carry += __shfl(incl, 63, 64);
     }
+    if (lane == 0) n_valid = carry;
   }
   __syncthreads();
-  for (int i = tid; i < kRouteWaves * E; i += kRouteThreads) hist[i] += total[i % E];
+#pragma unroll
+  for (int u = 0; u < IT; ++u)
+    if (key[u] >= 0)
+      sorted[total[key[u]] + hist[w * E + key[u]] + loc[u]] = (unsigned)key[u] << 16 | (unsigned)(lo + u * 64 + lane_id());
   __syncthreads();
-  wave_scatter(ids, lo, hi, E, bits_for(E), hist + w * E, eid_out, idx_out);
+  for (int i = tid; i < n_valid; i += THREADS) {
+    eid_out[i] = (int64_t)(sorted[i] >> 16);
+    idx_out[i] = (int64_t)(sorted[i] & 0xffff);
+  }
 }
 
 // ---- three-launch path ------------------------------------------------------------------------------
-template <typename I>
-__global__ __launch_bounds__(kRouteThreads) void route_hist_kernel(
+template <typename I, int THREADS>
+__global__ __launch_bounds__(THREADS) void route_hist_kernel(
     const I* __restrict__ ids, int64_t L, int E, int* __restrict__ counts /*[nchunk][E]*/) {
   extern __shared__ int lds[];  // [E]
   const int tid = threadIdx.x;
-  for (int i = tid; i < E; i += kRouteThreads) lds[i] = 0;
+  for (int i = tid; i < E; i += THREADS) lds[i] = 0;
   __syncthreads();
   const int64_t lo = (int64_t)blockIdx.x * kRouteChunk;
   const int64_t hi = min(lo + kRouteChunk, L);
-  for (int64_t p = lo + tid; p < hi; p += kRouteThreads) {
+  for (int64_t p = lo + tid; p < hi; p += THREADS) {
     const int e = load_id(ids, p);
     if ((unsigned)e < (unsigned)E) atomicAdd(&lds[e], 1);
   }
   __syncthreads();
-  for (int i = tid; i < E; i += kRouteThreads) counts[(int64_t)blockIdx.x * E + i] = lds[i];
+  for (int i = tid; i < E; i += THREADS) counts[(int64_t)blockIdx.x * E + i] = lds[i];
 }
 
 // One block of 16 waves.  counts[c][e] -> exclusive position of chunk c's first row of expert e.
@@ -159,6 +171,26 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(int* __restrict__ coun
                                                          int64_t* __restrict__ off_out) {
   extern __shared__ int total[];  // [E]
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  // many experts, few chunks: an expert per thread, eight chunks' counters in flight (a wave per expert would walk
+  // E / 16 experts one memory round trip after the other)
+  const bool by_thread = E >= 64 && nchunk <= 64;
+  auto over_chunks = [&](int e, auto use) {
+    for (int c0 = 0; c0 < nchunk; c0 += 8) {
+      int v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = c0 + u < nchunk ? counts[(int64_t)(c0 + u) * E + e] : 0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (c0 + u < nchunk) use(c0 + u, v[u]);
+    }
+  };
+  if (by_thread) {
+    for (int e = tid; e < E; e += 1024) {
+      int run = 0;
+      over_chunks(e, [&](int, int v) { run += v; });
+      total[e] = run;
+    }
+  } else
   for (int e = w; e < E; e += 16) {
     int run = 0;
     for (int c0 = 0; c0 < nchunk; c0 += 64) {
@@ -195,32 +227,43 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(int* __restrict__ coun
     }
   }
   __syncthreads();
+  if (by_thread) {
+    for (int e = tid; e < E; e += 1024) {
+      int run = total[e];
+      over_chunks(e, [&](int c, int v) {
+        counts[(int64_t)c * E + e] = run;
+        run += v;
+      });
+    }
+    return;
+  }
   for (int64_t i = tid; i < (int64_t)nchunk * E; i += blockDim.x) counts[i] += total[i % E];
 }
 
-template <typename I>
-__global__ __launch_bounds__(kRouteThreads) void route_scatter_kernel(
+template <typename I, int THREADS>
+__global__ __launch_bounds__(THREADS) void route_scatter_kernel(
     const I* __restrict__ ids, int64_t L, int E, const int* __restrict__ bases /*[nchunk][E]*/,
     int64_t* __restrict__ eid_out, int64_t* __restrict__ idx_out) {
-  extern __shared__ int lds[];  // [kRouteWaves][E]
+  constexpr int W = THREADS / 64, SEG = kRouteChunk / W, IT = SEG / 64;
+  extern __shared__ int lds[];  // [W][E]
   const int tid = threadIdx.x, w = tid >> 6;
-  for (int i = tid; i < kRouteWaves * E; i += kRouteThreads) lds[i] = 0;
+  for (int i = tid; i < W * E; i += THREADS) lds[i] = 0;
   __syncthreads();
-  constexpr int seg = kRouteChunk / kRouteWaves;
   const int64_t chunk_lo = (int64_t)blockIdx.x * kRouteChunk;
-  const int64_t lo = min(chunk_lo + (int64_t)w * seg, L), hi = min(lo + seg, L);
-  wave_histogram(ids, lo, hi, E, lds + w * E);
+  const int64_t lo = min(chunk_lo + (int64_t)w * SEG, L), hi = min(lo + SEG, L);
+  int key[IT], loc[IT];
+  wave_rank<I, IT>(ids, lo, hi, E, bits_for(E), lds + w * E, key, loc);
   __syncthreads();
-  for (int e = tid; e < E; e += kRouteThreads) {
-    int run = bases[(int64_t)blockIdx.x * E + e];
-    for (int ww = 0; ww < kRouteWaves; ++ww) {
-      const int c = lds[ww * E + e];
-      lds[ww * E + e] = run;
-      run += c;
+  for (int e = tid; e < E; e += THREADS) prefix_over_waves<W>(lds, E, e, bases[(int64_t)blockIdx.x * E + e]);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < IT; ++u) {
+    if (key[u] >= 0) {
+      const int pos = lds[w * E + key[u]] + loc[u];
+      eid_out[pos] = (int64_t)key[u];
+      idx_out[pos] = lo + u * 64 + lane_id();
     }
   }
-  __syncthreads();
-  wave_scatter(ids, lo, hi, E, bits_for(E), lds + w * E, eid_out, idx_out);
 }
 
 size_t route_workspace_bytes(int64_t L, int E) {
@@ -231,28 +274,29 @@ size_t route_workspace_bytes(int64_t L, int E) {
 template <typename I>
 static int launch_route_t(const I* ids, int64_t L, int E, int64_t* eid_out, int64_t* idx_out,
                           int64_t* off_out, void* ws, hipStream_t st) {
-  if (L <= kRouteChunk) {
-    const size_t lds = (size_t)(kRouteWaves + 1) * E * sizeof(int);
-    hipLaunchKernelGGL((route_fused_kernel<I, kRouteThreads>), dim3(1), dim3(kRouteThreads), lds, st, ids, (int)L, E,
-                       eid_out, idx_out, off_out);
+  auto fused = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(threads), 0, st, ids, (int)L, E, eid_out, idx_out, off_out);
     return launch_status("route_fused_kernel");
-  }
-  if (L <= kRouteFusedMax && E <= kRouteFusedMaxE) {
-    // one workgroup of 16 waves: a launch costs more than sorting 2048 rows per wave does
-    const size_t lds = (size_t)(1024 / 64 + 1) * E * sizeof(int);
-    hipLaunchKernelGGL((route_fused_kernel<I, 1024>), dim3(1), dim3(1024), lds, st, ids, (int)L, E,
-                       eid_out, idx_out, off_out);
-    return launch_status("route_fused_kernel");
-  }
+  };
+  // 16 waves need 17 E ints of LDS; with more experts, and for a row per thread, 4 waves
+  if (L <= kRouteThreads) return fused(&route_fused_kernel<I, kRouteThreads, 1>, kRouteThreads);
+  if (L <= kRouteChunk && E <= kRouteFusedMaxE) return fused(&route_fused_kernel<I, 1024, 4>, 1024);
+  if (L <= kRouteChunk) return fused(&route_fused_kernel<I, kRouteThreads, 16>, kRouteThreads);
+  // one workgroup of 16 waves: a launch costs more than ranking 1024 rows per wave does
+  if (L <= kRouteFusedMax / 2 && E <= kRouteFusedMaxE) return fused(&route_fused_kernel<I, 1024, 8>, 1024);
+  if (L <= kRouteFusedMax && E <= kRouteFusedMaxE) return fused(&route_fused_kernel<I, 1024, 16>, 1024);
   const int nchunk = (int)cdiv64(L, kRouteChunk);
   int* counts = (int*)ws;
-  hipLaunchKernelGGL(route_hist_kernel<I>, dim3(nchunk), dim3(kRouteThreads), (size_t)E * sizeof(int), st,
-                     ids, L, E, counts);
+  hipLaunchKernelGGL((route_hist_kernel<I, 1024>), dim3(nchunk), dim3(1024), (size_t)E * sizeof(int), st, ids, L, E,
+                     counts);
   hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(1024), (size_t)E * sizeof(int), st, counts, nchunk,
                      E, off_out);
-  hipLaunchKernelGGL(route_scatter_kernel<I>, dim3(nchunk), dim3(kRouteThreads),
-                     (size_t)kRouteWaves * E * sizeof(int), st, ids, L, E, (const int*)counts, eid_out,
-                     idx_out);
+  auto scatter = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(nchunk), dim3(threads), (size_t)(threads / 64) * E * sizeof(int), st, ids, L, E,
+                       (const int*)counts, eid_out, idx_out);
+  };
+  if (E <= kRouteFusedMaxE) scatter(&route_scatter_kernel<I, 1024>, 1024);
+  else scatter(&route_scatter_kernel<I, kRouteThreads>, kRouteThreads);
   return launch_status("route_scatter_kernel");
 }
 
