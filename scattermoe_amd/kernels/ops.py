@@ -576,14 +576,16 @@ def _xty_gathered_launch(E, DW, Db, DY, X, idx, fan_out, expert_offsets):
     # 1637 -> 1609 us).  The copy costs 4 K bytes per row against 2 K N flops, so narrow dY keeps the lookups from
     # fewer rows on (N = 1536: 128 rows 1143 -> 1147, 188 rows 1329 -> 1343).
     few_rows = DY.size(0) <= min(256, DY.size(1) // 16) * E
-    if (not few_rows and DY.is_cuda and hasattr(_backend, "xty_gathered")
-            and DY.dtype in (torch.bfloat16, torch.float16)):
+    lookups = DY.is_cuda and hasattr(_backend, "xty_gathered") and DY.dtype in (torch.bfloat16, torch.float16)
+    if lookups and not few_rows:
         _same_dtype("group_bwd_W", DY, X, DW, Db)
         if _backend.xty_gathered(DY, X, _as_i64(idx).contiguous(), fan_out, DW, Db,
                                  _as_i64(expert_offsets).contiguous(), E):
             return
     Xg = torch.empty((idx.size(0), X.size(1)), dtype=X.dtype, device=X.device)
-    _group_launch(X, Xg, None, fan_out, idx, True)            # `idx` is the routing's index vector
+    # The copy in place of lookups takes any index vector, as they do; a copy by source row would leave the rows of a
+    # repeated index unwritten.
+    _group_launch(X, Xg, None, fan_out, idx, not (lookups and few_rows))
     _xty_launch(E, DW, Db, DY, Xg, expert_offsets)
 
 

@@ -60,3 +60,18 @@ def test_unaligned_output():
     out = buf[1:-1].view(E, N, K)
     ops._xty_launch(E, out.permute(0, 2, 1), None, DY, X, off)
     assert torch.equal(out.permute(0, 2, 1), DW) and buf[0] == 0 and buf[-1] == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gather_takes_any_index_vector(dtype):
+    """`gather` stands for group() over the same index vector, also where that repeats rows and leaves others out."""
+    g = torch.Generator(device=DEV).manual_seed(7)
+    E, n, K, N, k = 4, 20, 136, 512, 2
+    off = torch.arange(1, E + 1, device=DEV) * n
+    X = torch.randn(E * n // k, K, generator=g, device=DEV).to(dtype)
+    DY = torch.randn(E * n, N, generator=g, device=DEV).to(dtype)
+    idx = torch.randint(0, E * n, (E * n,), generator=g, device=DEV)
+    torch.full((E * n * K,), float("nan"), device=DEV, dtype=dtype)        # what a later allocation would find
+    DW, Db = ops.group_bwd_W(DY, X, off, E, has_bias=True, gather=(idx, k))
+    want, want_b = ops.group_bwd_W(DY, X[idx // k], off, E, has_bias=True)
+    assert torch.equal(DW, want) and torch.equal(Db, want_b)
