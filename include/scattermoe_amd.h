@@ -66,8 +66,9 @@ const char* smoe_last_error(void);
  *   expert_idxs  L unsorted ids in [0,E), contiguous, dtype `idx_dtype` (SMOE_I64 ...)
  *   eid_out/idx_out  L int64 each;  off_out  E int64
  *   workspace    device scratch of at least smoe_route_workspace_bytes(L,E) bytes (may be NULL iff that is 0)
- * Ids outside [0,E) are undefined behaviour in the reference; here such rows are dropped from the
- * histogram and the outputs are unspecified (no out-of-bounds access happens).
+ * Ids outside [0,E) are undefined behaviour in the reference; here such rows are dropped: the off_out[E-1] rows that
+ * are left come first, the places behind them hold eid E and idx -1, and the launches that take these vectors skip
+ * them (no out-of-bounds access happens; output rows that belong to a dropped slot are unspecified).
  */
 size_t smoe_route_workspace_bytes(int64_t L, int E);
 int smoe_route(const void* expert_idxs, int idx_dtype, int64_t L, int E,
@@ -146,6 +147,7 @@ int smoe_scatter2scatter_ws(const void* X, int64_t sxm, int64_t sxk,
  * Replaces scattermoe/kernels/ops.py:377-410 (group / op scattermoe::group), kernel ops.py:413-457.
  *   Y[n, :] = A[idx[n] / fan_out, :] * (coeff ? coeff[idx[n]] : 1)      n in [0,L)
  *   A (L/fan_out, K) strides sam,sak;  coeff (L) contiguous or NULL;  Y (L,K) strides sym,syk
+ * A row of Y whose index entry lies outside [0, L) is left unwritten.
  */
 int smoe_group(const void* A, int64_t sam, int64_t sak, const void* coeff,
                void* Y, int64_t sym, int64_t syk, const int64_t* idx,

@@ -3,6 +3,7 @@
 //   Y[n, :] = A[idx[n] / fan_out, :] * coeff[idx[n]]
 // Pure HBM traffic: one wave moves one row in 16-byte pieces when rows are contiguous and aligned,
 // element-wise otherwise.  The product is formed in fp32 and rounded once to the tensor dtype.
+// A row whose index lies outside [0, L) is left unwritten.
 #include "common.hpp"
 
 namespace smoe {
@@ -22,6 +23,7 @@ __global__ __launch_bounds__(kGroupThreads) void group_kernel(GroupArgs a) {
   for (int64_t n = (int64_t)blockIdx.x * kGroupRowsPerBlock + wave; n < a.L;
        n += (int64_t)gridDim.x * kGroupRowsPerBlock) {
     const int64_t i = a.idx[n];
+    if ((uint64_t)i >= (uint64_t)a.L) continue;      // no slot: the place of a row that the routing dropped
     const int64_t src = i / a.fan_out;
     const float c = coeff ? to_f32(coeff[i]) : 1.0f;
     const T* __restrict__ s = A + src * a.sam;

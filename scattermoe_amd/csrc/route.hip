@@ -88,6 +88,17 @@ __device__ __forceinline__ int prefix_over_waves(int* __restrict__ hist, int E, 
   return run;
 }
 
+// The places behind the last valid row (as many as there are ids that are no expert): an id past the experts and an
+// index that is no slot, which every launch that reads the vectors skips.  Unwritten they would hold what the memory
+// held before: an address to nowhere, or a slot that has a place already.
+__device__ __forceinline__ void fill_dropped(int64_t first, int64_t step, int64_t L, int E, int64_t* __restrict__ eid_out,
+                                             int64_t* __restrict__ idx_out) {
+  for (int64_t i = first; i < L; i += step) {
+    eid_out[i] = (int64_t)E;
+    idx_out[i] = -1;
+  }
+}
+
 // ---- single-launch path: whole input in one block ------------------------------------------------
 // Bound by latency (one read of the ids, LDS counters, four barriers) and, written row by row, by one CU's rate of
 // scattered 8-byte stores: the sorted rows are put together in LDS and written out in whole lines.
@@ -144,6 +155,7 @@ __global__ __launch_bounds__(THREADS) void route_fused_kernel(
     eid_out[i] = (int64_t)(sorted[i] >> 16);
     idx_out[i] = (int64_t)(sorted[i] & 0xffff);
   }
+  fill_dropped(n_valid + tid, THREADS, L, E, eid_out, idx_out);
 }
 
 // ---- three-launch path ------------------------------------------------------------------------------
@@ -167,9 +179,11 @@ __global__ __launch_bounds__(THREADS) void route_hist_kernel(
 // One block of 16 waves.  counts[c][e] -> exclusive position of chunk c's first row of expert e.
 // A wave takes the experts e = wave, wave + 16, ...; its lanes take 64 chunks at a time (wave-wide scan, carry
 // between the groups of 64), so the walk over the chunks of an expert is 64 wide instead of serial.
-__global__ __launch_bounds__(1024) void route_scan_kernel(int* __restrict__ counts, int nchunk, int E,
+__global__ __launch_bounds__(1024) void route_scan_kernel(int* __restrict__ counts, int nchunk, int64_t L, int E,
+                                                         int64_t* __restrict__ eid_out, int64_t* __restrict__ idx_out,
                                                          int64_t* __restrict__ off_out) {
   extern __shared__ int total[];  // [E]
+  __shared__ int n_valid;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   // many experts, few chunks: an expert per thread, eight chunks' counters in flight (a wave per expert would walk
   // E / 16 experts one memory round trip after the other)
@@ -225,8 +239,10 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(int* __restrict__ coun
       }
       carry += __shfl(incl, 63, 64);
     }
+    if (lane == 0) n_valid = carry;
   }
   __syncthreads();
+  fill_dropped((int64_t)n_valid + tid, 1024, L, E, eid_out, idx_out);
   if (by_thread) {
     for (int e = tid; e < E; e += 1024) {
       int run = total[e];
@@ -289,8 +305,8 @@ static int launch_route_t(const I* ids, int64_t L, int E, int64_t* eid_out, int6
   int* counts = (int*)ws;
   hipLaunchKernelGGL((route_hist_kernel<I, 1024>), dim3(nchunk), dim3(1024), (size_t)E * sizeof(int), st, ids, L, E,
                      counts);
-  hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(1024), (size_t)E * sizeof(int), st, counts, nchunk,
-                     E, off_out);
+  hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(1024), (size_t)E * sizeof(int), st, counts, nchunk, L,
+                     E, eid_out, idx_out, off_out);
   auto scatter = [&](auto kernel, int threads) {
     hipLaunchKernelGGL(kernel, dim3(nchunk), dim3(threads), (size_t)(threads / 64) * E * sizeof(int), st, ids, L, E,
                        (const int*)counts, eid_out, idx_out);
