@@ -75,3 +75,21 @@ def test_gather_takes_any_index_vector(dtype):
     DW, Db = ops.group_bwd_W(DY, X, off, E, has_bias=True, gather=(idx, k))
     want, want_b = ops.group_bwd_W(DY, X[idx // k], off, E, has_bias=True)
     assert torch.equal(DW, want) and torch.equal(Db, want_b)
+
+
+@pytest.mark.parametrize("n,N,dtype", [(400, 512, torch.bfloat16), (20, 6400, torch.bfloat16), (400, 6400, torch.float16),
+                                       (20, 512, torch.float32), (400, 512, torch.float32)])
+@pytest.mark.parametrize("k", [2, 4])
+def test_gather_takes_any_index_vector_on_every_route(n, N, dtype, k):
+    """The same where the rows are looked up inside the launch (n = 400, N = 512) and where the launch declines lookups
+    (dY beyond 6144 columns, float32)."""
+    g = torch.Generator(device=DEV).manual_seed(n + N)
+    E, K = 4, 136
+    off = torch.arange(1, E + 1, device=DEV) * n
+    X = torch.randn(E * n // k, K, generator=g, device=DEV).to(dtype)
+    DY = torch.randn(E * n, N, generator=g, device=DEV).to(dtype)
+    idx = torch.randint(0, E * n, (E * n,), generator=g, device=DEV)
+    torch.full((E * n * K,), float("nan"), device=DEV, dtype=dtype)
+    DW, Db = ops.group_bwd_W(DY, X, off, E, has_bias=True, gather=(idx, k))
+    want, want_b = ops.group_bwd_W(DY, X[idx // k], off, E, has_bias=True)
+    assert torch.equal(DW, want) and torch.equal(Db, want_b)
