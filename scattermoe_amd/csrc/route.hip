@@ -22,8 +22,13 @@ static constexpr int kRouteFusedMax = 16384;   // rows one workgroup of 1024 thr
                                                // workspace (the three launches: 10 us and more) ...
 static constexpr int kRouteFusedMaxE = 512;    // ... for at most this many experts (17 * E ints of LDS)
 
+// Id i, -1 when it is no expert (compared at its full width: the low half of a 64-bit id may look like one).
 template <typename I>
-__device__ __forceinline__ int load_id(const I* p, int64_t i) { return (int)p[i]; }
+__device__ __forceinline__ int load_id(const I* p, int64_t i, int E) {
+  const I v = p[i];
+  if constexpr (sizeof(I) == 8) return (uint64_t)v < (uint64_t)E ? (int)v : -1;
+  return (unsigned)(int)v < (unsigned)E ? (int)v : -1;
+}
 
 // Lanes of the wave that hold the same key as this lane (keys < 2^nbits), inactive lanes excluded.
 __device__ __forceinline__ unsigned long long match_any(int key, int nbits, bool active) {
@@ -55,12 +60,11 @@ __device__ __forceinline__ void wave_rank(const I* __restrict__ ids, int64_t seg
 #pragma unroll
   for (int u = 0; u < IT; ++u) {
     const int64_t p = seg_lo + u * 64 + lane;
-    key[u] = p < seg_hi ? load_id(ids, p) : -1;
+    key[u] = p < seg_hi ? load_id(ids, p, E) : -1;
   }
 #pragma unroll
   for (int u = 0; u < IT; ++u) {
-    const bool ok = (unsigned)key[u] < (unsigned)E;
-    key[u] = ok ? key[u] : -1;
+    const bool ok = key[u] >= 0;
     loc[u] = 0;
     if (seg_lo + u * 64 < seg_hi) {
       const unsigned long long same = match_any(ok ? key[u] : 0, nbits, ok);
@@ -169,8 +173,8 @@ __global__ __launch_bounds__(THREADS) void route_hist_kernel(
   const int64_t lo = (int64_t)blockIdx.x * kRouteChunk;
   const int64_t hi = min(lo + kRouteChunk, L);
   for (int64_t p = lo + tid; p < hi; p += THREADS) {
-    const int e = load_id(ids, p);
-    if ((unsigned)e < (unsigned)E) atomicAdd(&lds[e], 1);
+    const int e = load_id(ids, p, E);
+    if (e >= 0) atomicAdd(&lds[e], 1);
   }
   __syncthreads();
   for (int i = tid; i < E; i += THREADS) counts[(int64_t)blockIdx.x * E + i] = lds[i];

@@ -33,6 +33,23 @@ def test_places_behind_the_last_row(L, E):
     assert torch.equal(ops.offsets_from_sorted(eid, E), off)
 
 
+@pytest.mark.parametrize("L", [7, 3000, 40000])
+def test_ids_beyond_32_bits(L):
+    """Their low half may look like an expert; the two-launch decode step (L = 7) and the routing agree on them."""
+    E, d, F = 16, 64, 64
+    ids = torch.arange(L, device=DEV) % E
+    far = torch.arange(L, device=DEV) % 3 == 0
+    wide = torch.where(far, ids + torch.where(ids % 2 == 0, 1 << 32, -(1 << 40)), ids)
+    got, want = ops.route(wide, E), ops.route(torch.where(far, -1, ids), E)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    if L == 7:
+        g = torch.Generator(device=DEV).manual_seed(1)
+        r = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()
+        x, p, w1, w2 = r(1, d), r(1, L), r(E, 2 * F, d), r(E, d, F)
+        a, b = (ops.decode_glu_mlp(x, p, e.view(1, L), w1, None, w2, None) for e in (wide, torch.where(far, -1, ids)))
+        assert a is not None and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype,K", [(torch.bfloat16, 136), (torch.bfloat16, 133), (torch.float32, 136)])
 @pytest.mark.parametrize("coeff", [False, True])
 def test_group_leaves_rows_without_a_slot(dtype, K, coeff):
