@@ -3,13 +3,14 @@
 The kernels issue their direct-to-LDS loads from inline assembly with the base address in scalar registers.  On
 gfx9-family hardware a vector memory instruction must not read a scalar register within five wait states of a
 vector instruction (v_readfirstlane) writing it; the compiler keeps that distance for its own instructions but does
-not look into assembly blocks, and a load that reads a stale base faults the GPU.  The test compiles the file to
-assembly and looks at the six instructions in front of every load of an assembly block."""
+not look into assembly blocks, and a load that reads a stale base faults the GPU.  The test compiles every
+source of the MFMA kernels to assembly and looks at the six instructions in front of every load of an assembly block."""
 import os
 import re
 import shutil
 import subprocess
 import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 
@@ -58,13 +59,26 @@ def test_scanner_sees_a_hazard_and_its_fix():
     assert _hazards(bad)[1] and not _hazards(good)[1]
 
 
+def _sources():
+    """Every compiled source that instantiates the MFMA kernels."""
+    names = [n for n in _build.SOURCES if "gemm_mfma.hpp" in open(os.path.join(_build.CSRC, n)).read()]
+    assert len(names) >= 3
+    return names
+
+
 @pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="needs hipcc")
 def test_no_inline_assembly_load_reads_a_freshly_written_scalar_base():
+    names = _sources()
     with tempfile.TemporaryDirectory() as tmp:
-        out = os.path.join(tmp, "gemm_mfma.s")
-        cmd = [_build._hipcc()] + _build.HIPCC_FLAGS + ["-S", "--cuda-device-only", "-o", out,
-                                                       os.path.join(_build.CSRC, "gemm_mfma.hip")]
-        subprocess.run(cmd, check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
-        loads, found = _hazards(open(out).read())
-    assert loads > 100, "no inline-assembly loads found: the scan is looking at the wrong text"
-    assert not found, found[:5]
+        def assembly(name):
+            out = os.path.join(tmp, name + ".s")
+            cmd = [_build._hipcc()] + _build.HIPCC_FLAGS + ["-S", "--cuda-device-only", "-o", out,
+                                                           os.path.join(_build.CSRC, name)]
+            subprocess.run(cmd, check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+            return open(out).read()
+        with ThreadPoolExecutor(max_workers=len(names)) as pool:      # side by side: a minute, not three
+            texts = list(pool.map(assembly, names))
+    for name, text in zip(names, texts):
+        loads, found = _hazards(text)
+        assert loads > 100, "%s: no inline-assembly loads found: the scan is looking at the wrong text" % name
+        assert not found, (name, found[:5])
