@@ -130,14 +130,15 @@ __device__ __forceinline__ bool find_tile(const int64_t* __restrict__ off, int E
     const unsigned long long hit = __ballot(cum > t);
     if (hit) {
       const int src = __ffsll((long long)hit) - 1;
-      const int lo_s = __shfl(lo, src, 64), hi_s = __shfl(hi, src, 64);
-      const int first = __shfl(cum - nt, src, 64);
+      // readlane: the answer stays in scalar registers (a shuffle's would hold vector registers across the main loop)
+      const int lo_s = __builtin_amdgcn_readlane(lo, src), hi_s = __builtin_amdgcn_readlane(hi, src);
+      const int first = __builtin_amdgcn_readlane(cum - nt, src);
       expert = e0 + src;
       row_start = lo_s + (t - first) * BM;
       rows = min(BM, hi_s - row_start);
       return true;
     }
-    tiles_before += __shfl(incl, 63, 64);
+    tiles_before += __builtin_amdgcn_readlane(incl, 63);
   }
   return false;
 }

@@ -1340,7 +1340,7 @@ struct S2STile {
   int n_tile, n0;               // tile column and its first output column
   int m_loc, n_loc;             // place inside the super tile
   int part, klen;               // contraction part and its length
-  int64_t slot, own_row;        // this thread's row of the tables (thread m < BM: row m of the tile)
+  int slot;                     // thread m < BM: slot of row m of the tile, where one is needed
 };
 
 // One output tile; TL::BM >= rows.
@@ -1355,6 +1355,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   constexpr bool W_ONCE = TL::NS > 2 || TL::WG > 1;
   typedef typename std::conditional<B_TR, TransOp<TL::BN, TL::NT, W_ONCE>, DirectOp<TL::BN, TL::NT, W_ONCE>>::type BOp;
   constexpr bool CAN_SPLIT = TL::BM == 128 && TL::BN == 256 && TL::NS == 3;
+  const int glu = TL::RS ? __builtin_amdgcn_readfirstlane(a.glu) : -1;      // (as for the tile in s2s_mfma_kernel)
   const int e = t.e, row0 = t.row0, rows = t.rows, n0 = t.n0;
   const int k_first = CAN_SPLIT ? t.part * t.klen : 0;
 
@@ -1369,7 +1370,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   BOp B;
   B.rot = TL::RS ? 0 : (t.m_loc * BOp::R / Raster::SM) % BOp::R;    // the column panel has SM sharers
   const char* Wb = (const char*)a.W + ((int64_t)e * a.swe + (int64_t)k_first * (B_TR ? a.swk : 1)) * 2;
-  if (a.glu == 1) {
+  if ((TL::RS ? glu : a.glu) == 1) {
     // tile column tc -> weight column: wave block tc / WTN, first half of the block from [0, F), second from [F, 2F)
     const int F = a.N;
     auto wcol = [&](int tc) {
@@ -1423,20 +1424,20 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   }
 
   {
-    int64_t slot = t.slot, own_row = t.own_row;
-    asm volatile("" : "+v"(slot), "+v"(own_row));           // not looked at before this point
+    int slot = t.slot;
+    asm volatile("" : "+v"(slot));                          // not looked at before this point
     const int m = threadIdx.x;
-    if (m < TL::BM) sDst[m] = m < rows ? (a.y_grouped ? own_row : slot) * a.sym : -1;
+    if (m < TL::BM) sDst[m] = m < rows ? (int64_t)(a.y_grouped ? row0 + m : slot) * a.sym : -1;
   }
   __syncthreads();
   const T* bias = a.b ? (const T*)a.b + (int64_t)e * a.sbe : nullptr;
   // 16-byte pieces need every row start 16-byte aligned; otherwise the lane-wise epilogues are used (the
   // one-wave-per-SIMD class is only launched on aligned outputs)
   if constexpr (TL::RS) {
-    if (a.glu == 0) epilogue_staged<T, TL>(acc, (T*)a.Y, sDst, n0, a.N, bias, a.sbn, lds, sBias);
-    else if (a.glu == 1) epilogue_glu_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds, sBias);
-    else if (a.glu == 2) epilogue_glu_bwd_staged<T, TL>(acc, a, row0, rows, n0, lds, sBias);
-    else if (a.glu == 3) epilogue_oss_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds, sBias);
+    if (glu == 0) epilogue_staged<T, TL>(acc, (T*)a.Y, sDst, n0, a.N, bias, a.sbn, lds, sBias);
+    else if (glu == 1) epilogue_glu_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds, sBias);
+    else if (glu == 2) epilogue_glu_bwd_staged<T, TL>(acc, a, row0, rows, n0, lds, sBias);
+    else if (glu == 3) epilogue_oss_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds, sBias);
     else epilogue_oss_bwd_staged<T, TL>(acc, a, row0, rows, n0, lds, sBias);
   } else if (a.glu == 0) {
     const bool al16 = (((uintptr_t)a.Y & 15) == 0) && ((a.sym | a.N) & 7) == 0;
@@ -1493,6 +1494,12 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
              !find_tile<TL::BM>(a.off, a.E, a.m_begin + m_tile, t.e, t.row0, t.rows, a.tail_mode == 1 ? REMAINDER_ROWS : 0)) {
     return;
   }
+  if constexpr (TL::RS) {      // (one scalar value each, said so: ten registers of this form go to scratch memory otherwise)
+    t.e = __builtin_amdgcn_readfirstlane(t.e);
+    t.row0 = __builtin_amdgcn_readfirstlane(t.row0);
+    t.rows = __builtin_amdgcn_readfirstlane(t.rows);
+    t.n_tile = __builtin_amdgcn_readfirstlane(t.n_tile);
+  }
   // first output column of the tile; the fused forward GLU tile holds BN/2 columns of each half
   t.n0 = a.glu == 1 ? t.n_tile * (TL::BN / 2) : t.n_tile * TL::BN;
 
@@ -1500,23 +1507,21 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
   // stored after it, so that a launch whose input is grouped and whose output is not (layer-2 forward, layer-1
   // input gradient) does not wait for the index vector before its first operand loads.
   static_assert(TL::BM <= TL::NT, "one row of the tables per thread");
-  t.slot = 0;                                               // idx[n] where it is needed, else unused
-  t.own_row = 0;
+  t.slot = 0;                                               // idx[n] (< L, an int) where it is needed, else unused
   {
     const int m = threadIdx.x;
     if (m < TL::BM) {
-      const int mm = m < t.rows ? m : t.rows - 1;           // tail rows re-read the last valid row
-      t.own_row = t.row0 + mm;
-      if (!a.x_grouped || !a.y_grouped) t.slot = a.idx[t.own_row];
-      sSrc[m] = a.x_grouped ? (int)t.own_row : (int)(t.slot / a.fan_out);
+      const int row = t.row0 + (m < t.rows ? m : t.rows - 1);      // tail rows re-read the last valid row
+      if (!a.x_grouped || !a.y_grouped) t.slot = (int)a.idx[row];
+      sSrc[m] = a.x_grouped ? row : (int)((unsigned)t.slot / (unsigned)a.fan_out);
     }
   }
   __syncthreads();
   if constexpr (TL::BM == 256 && TL::BN == 256) {
     // An expert's last tile is partly filled: it is multiplied at the height of its rows, in steps of 64 (which keep
     // the four waves, or the eight, equally busy), not as a whole tile.  (Same sums in the same order.)
-    // Mixtral training shape (16.5 tiles per expert): step -1.3 %; what it mostly buys is that such tiles need no launch
-    // of their own any more (see cut_tails).
+    // What it buys is that such tiles need no launch of their own any more (see cut_tails); a training step with many
+    // tiles per expert is the same with it (Mixtral shape, 16.5 tiles per expert).
     const int h = (t.rows + 63) >> 6;
     if (h == 4) s2s_tile<T, TL, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
     else if (h == 3) s2s_tile<T, typename TL::template Height<3>, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);

@@ -66,19 +66,56 @@ def _sources():
     return names
 
 
-@pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="needs hipcc")
-def test_no_inline_assembly_load_reads_a_freshly_written_scalar_base():
+needs_hipcc = pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"),
+                                 reason="needs hipcc")
+
+
+@pytest.fixture(scope="module")
+def assembly():
+    """File name -> generated assembly of the sources that instantiate the MFMA kernels."""
     names = _sources()
     with tempfile.TemporaryDirectory() as tmp:
-        def assembly(name):
+        def compile_(name):
             out = os.path.join(tmp, name + ".s")
             cmd = [_build._hipcc()] + _build.HIPCC_FLAGS + ["-S", "--cuda-device-only", "-o", out,
                                                            os.path.join(_build.CSRC, name)]
             subprocess.run(cmd, check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
             return open(out).read()
-        with ThreadPoolExecutor(max_workers=len(names)) as pool:      # side by side: a minute, not three
-            texts = list(pool.map(assembly, names))
-    for name, text in zip(names, texts):
+        with ThreadPoolExecutor(max_workers=len(names)) as pool:      # side by side
+            return dict(zip(names, pool.map(compile_, names)))
+
+
+@needs_hipcc
+def test_no_inline_assembly_load_reads_a_freshly_written_scalar_base(assembly):
+    for name, text in assembly.items():
         loads, found = _hazards(text)
         assert loads > 100, "%s: no inline-assembly loads found: the scan is looking at the wrong text" % name
         assert not found, (name, found[:5])
+
+
+def _scratch_of_kernels(text):
+    """(name, bytes of scratch memory per lane) of every kernel of an assembly listing, from its metadata."""
+    out = []
+    for block in text.split("\n  - .agpr_count:")[1:]:
+        name, size = (re.search(r"\.%s:\s+(\S+)" % k, block).group(1) for k in ("name", "private_segment_fixed_size"))
+        out.append((name, int(size)))
+    return out
+
+
+def _tile(name):
+    """The Tile<...> arguments in a kernel's mangled name: (BM, BN, WM, WN, NS, RS, ...)."""
+    m = re.search(r"4TileI((?:L[ib]\d+E)+)E", name)
+    return tuple(int(v) for v in re.findall(r"L[ib](\d+)E", m.group(1))) if m else ()
+
+
+@needs_hipcc
+def test_the_one_wave_per_simd_form_fits_its_registers(assembly):
+    """256 accumulators and two register sets of operands leave that form little room; what does not fit goes to scratch
+    memory, for every thread of every tile.  Three registers at the most, none of them in the path of a full tile."""
+    seen = 0
+    for name, text in assembly.items():
+        for kernel, scratch in _scratch_of_kernels(text):
+            if "s2s_mfma_kernel" in kernel and _tile(kernel)[:6] == (256, 256, 2, 2, 2, 1):
+                seen += 1
+                assert scratch <= 12, (name, kernel, scratch)
+    assert seen == 4
