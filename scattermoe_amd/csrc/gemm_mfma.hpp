@@ -237,7 +237,9 @@ struct TransOp {
   // GATHER only
   const int64_t* rows; // wave-uniform: index vector, already offset to the first contraction row
   unsigned fan;
-  unsigned colb[R];    // byte offset of this thread's piece inside its contraction row
+  unsigned colb;       // byte offset of this thread's pieces inside their contraction rows (the rows of its load slots
+                       // differ by multiples of 4, which the swizzle does not see)
+  static_assert(!GATHER || NT / CPR % 4 == 0, "one column offset per thread");
   unsigned next_row;   // thread t < 64: index of contraction row t of the slice after the one being issued
   unsigned* srow;      // LDS, [2][64]: byte offsets of the rows of the slice to be issued next, by slice parity
   // contraction row inside a slice that load slot j of this thread carries
@@ -258,7 +260,7 @@ struct TransOp {
       const int p = rnd(j) * NT + t;
       const int kr = p / CPR, phys = p % CPR;
       const int cc = ((((phys >> 2) ^ (kr & 3)) << 2) | (phys & 3));      // logical 16-byte piece of the row
-      if constexpr (GATHER) colb[j] = (unsigned)col_of(cc * 8) * 2;
+      if constexpr (GATHER) colb = (unsigned)col_of(cc * 8) * 2;
       else off[j] = (unsigned)(kr * ld_bytes) + (unsigned)col_of(cc * 8) * 2;
     }
   }
@@ -296,7 +298,7 @@ struct TransOp {
   __device__ __forceinline__ void take_rows(int slice) {
     if constexpr (GATHER) {
 #pragma unroll
-      for (int j = 0; j < R; ++j) off[j] = srow[(slice & 1) * 64 + slot_row(j)] + colb[j];
+      for (int j = 0; j < R; ++j) off[j] = srow[(slice & 1) * 64 + slot_row(j)] + colb;
     }
   }
   __device__ __forceinline__ void issue_one(unsigned tile, int k0, int j) const {

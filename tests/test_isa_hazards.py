@@ -109,13 +109,14 @@ def _tile(name):
 
 
 @needs_hipcc
-def test_the_one_wave_per_simd_form_fits_its_registers(assembly):
-    """256 accumulators and two register sets of operands leave that form little room; what does not fit goes to scratch
-    memory, for every thread of every tile.  Three registers at the most, none of them in the path of a full tile."""
+def test_kernels_fit_their_registers(assembly):
+    """What does not fit goes to scratch memory, for every thread of every tile.  Five registers at the most (gathered
+    rows in 128 x 128 tiles, four workgroups per CU), three in the one-wave-per-SIMD form of scatter2scatter, which has
+    256 accumulators and two register sets of operands, and none of those in the path of a full tile."""
     seen = 0
     for name, text in assembly.items():
         for kernel, scratch in _scratch_of_kernels(text):
-            if "s2s_mfma_kernel" in kernel and _tile(kernel)[:6] == (256, 256, 2, 2, 2, 1):
-                seen += 1
-                assert scratch <= 12, (name, kernel, scratch)
+            one_wave = "s2s_mfma_kernel" in kernel and _tile(kernel)[:6] == (256, 256, 2, 2, 2, 1)
+            seen += one_wave
+            assert scratch <= (12 if one_wave else 20), (name, kernel, scratch)
     assert seen == 4
