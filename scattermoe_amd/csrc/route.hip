@@ -22,13 +22,9 @@ static constexpr int kRouteFusedMax = 16384;   // rows one workgroup of 1024 thr
                                                // workspace (the three launches: 10 us and more) ...
 static constexpr int kRouteFusedMaxE = 512;    // ... for at most this many experts (17 * E ints of LDS)
 
-// Id i, -1 when it is no expert (compared at its full width: the low half of a 64-bit id may look like one).
+// An id is compared at its full width: the low half of a 64-bit id that is no expert may look like one.
 template <typename I>
-__device__ __forceinline__ int load_id(const I* p, int64_t i, int E) {
-  const I v = p[i];
-  if constexpr (sizeof(I) == 8) return (uint64_t)v < (uint64_t)E ? (int)v : -1;
-  return (unsigned)(int)v < (unsigned)E ? (int)v : -1;
-}
+__device__ __forceinline__ bool is_expert(I id, int E) { return (uint64_t)(int64_t)id < (uint64_t)E; }
 
 // Lanes of the wave that hold the same key as this lane (keys < 2^nbits), inactive lanes excluded.
 __device__ __forceinline__ unsigned long long match_any(int key, int nbits, bool active) {
@@ -57,14 +53,16 @@ __device__ __forceinline__ void wave_rank(const I* __restrict__ ids, int64_t seg
                                           int* __restrict__ hist_w, int (&key)[IT], int (&loc)[IT]) {
   const int lane = lane_id();
   const unsigned long long lt = (1ull << lane) - 1ull;
+  I id[IT];                             // all loads ahead of the first comparison: one memory round trip, not IT of them
 #pragma unroll
   for (int u = 0; u < IT; ++u) {
     const int64_t p = seg_lo + u * 64 + lane;
-    key[u] = p < seg_hi ? load_id(ids, p, E) : -1;
+    id[u] = p < seg_hi ? ids[p] : (I)0;
   }
 #pragma unroll
   for (int u = 0; u < IT; ++u) {
-    const bool ok = key[u] >= 0;
+    const bool ok = seg_lo + u * 64 + lane < seg_hi && is_expert(id[u], E);
+    key[u] = ok ? (int)id[u] : -1;
     loc[u] = 0;
     if (seg_lo + u * 64 < seg_hi) {
       const unsigned long long same = match_any(ok ? key[u] : 0, nbits, ok);
@@ -173,8 +171,8 @@ __global__ __launch_bounds__(THREADS) void route_hist_kernel(
   const int64_t lo = (int64_t)blockIdx.x * kRouteChunk;
   const int64_t hi = min(lo + kRouteChunk, L);
   for (int64_t p = lo + tid; p < hi; p += THREADS) {
-    const int e = load_id(ids, p, E);
-    if (e >= 0) atomicAdd(&lds[e], 1);
+    const I id = ids[p];
+    if (is_expert(id, E)) atomicAdd(&lds[(int)id], 1);
   }
   __syncthreads();
   for (int i = tid; i < E; i += THREADS) counts[(int64_t)blockIdx.x * E + i] = lds[i];
