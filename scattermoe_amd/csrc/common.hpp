@@ -143,14 +143,26 @@ __device__ __forceinline__ bool find_tile(const int64_t* __restrict__ off, int E
   return false;
 }
 
+// Largest of the wave's values, in a scalar register: six row shifts and row broadcasts (lanes without a source keep
+// their own value).
+__device__ __forceinline__ int wave_max(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x111, 0xf, 0xf, false));       // row_shr 1, 2, 4, 8
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x112, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x114, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x118, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));       // lane 15 of a row to the next row
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));       // lane 31 to the upper half
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 // The same for launches whose workgroups take all output tiles in an order that keeps together what shares operands:
 // expert by expert, inside an expert column by column (of `n_tiles`), the expert's tile rows of a column side by side.
 // The XCD of a workgroup is `pid` % 8; the order is cut into 8 R chunks of equal length and XCD x takes the chunks
 // x, x + 8, ... (in turn from either end).  How many tiles there are is known only here, from `off`: R = 1, or with
 // `rounds` as many as there are rounds of 256 tiles.  A grid of chunked_grid() workgroups covers every tile.
-// Returns 1: this workgroup's tile; 0: none; -1: the experts differ in tile rows by more than a quarter (and not only in
-// having none), so that equal numbers of tiles are not equal work: another order has to be taken (the same answer in
-// every workgroup).
+// Returns 1: this workgroup's tile; 0: none; -1: the experts that have rows differ in tile rows by more than a quarter of
+// the most, so that equal numbers of tiles are not equal work: another order has to be taken (the same answer in every
+// workgroup, and for the same loads in any order).
 template <int BM>
 __device__ __forceinline__ int find_tile_chunked(const int64_t* __restrict__ off, int E, int pid, int n_tiles,
                                                  bool rounds, int& expert, int& row_start, int& rows, int& column) {
@@ -175,15 +187,17 @@ __device__ __forceinline__ int find_tile_chunked(const int64_t* __restrict__ off
   };
   int lo, hi, nt;
   load(0, lo, hi, nt);
-  const int ref = __builtin_amdgcn_readfirstlane(nt);
-  bool many = nt > 1, differs = lane < E && 4 * abs(nt - ref) > ref;
+  int most = nt, least = nt > 0 ? nt : 0x7fffffff;            // tile rows of an expert that has any
   for (int e0 = 64; e0 < E; e0 += 64) {
     int l_, h_, n_;
     load(e0, l_, h_, n_);
-    many |= n_ > 1;
-    differs |= e0 + lane < E && 4 * abs(n_ - ref) > ref;
+    most = max(most, n_);
+    if (n_ > 0) least = min(least, n_);
   }
-  if (__ballot(many) && __ballot(differs)) return -1;
+  if (__ballot(most > 1)) {
+    most = wave_max(most);
+    if (4 * (most + wave_max(-least)) > most) return -1;
+  }
   int incl = scan(nt);
   int total = __builtin_amdgcn_readlane(incl, 63);
   for (int e0 = 64; e0 < E; e0 += 64) {

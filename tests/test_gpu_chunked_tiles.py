@@ -17,6 +17,15 @@ def _loads(kind, E, rows):
         return [0 if e % 3 == 1 else rows - e % 4 for e in range(E)]
     if kind == "one_more":                   # the last expert: another tile row
         return [rows] * (E - 1) + [rows + 256]
+    if kind in ("first_low", "first_high"):  # three and four tile rows of 256: even, whichever comes first
+        low = [E // 2] if kind == "first_high" else [0]
+        return [3 * 256 - 5 if e in low else 4 * 256 - e % 9 for e in range(E)]
+    if kind == "heights":                    # one tile row of 256 each, a few rows to all of them
+        return [60 + (190 * e) // (E - 1) for e in range(E)]
+    if kind == "heights_gaps":               # the same, every fourth expert without rows, loads falling
+        return [0 if e % 4 == 2 else 250 - (190 * e) // (E - 1) for e in range(E)]
+    if kind == "tile_rows_gaps":             # two tile rows each, the first and every third expert without rows
+        return [0 if e % 3 == 0 else rows - e % 4 for e in range(E)]
     return [rows * 4] + [max(1, rows // 8)] * (E - 1)       # uneven
 
 
@@ -29,6 +38,18 @@ def _loads(kind, E, rows):
 ])
 @pytest.mark.parametrize("n_contig", [False, True])
 def test_plain_and_gated(E, rows, K, N, n_contig, kind):
+    _check_plain_and_gated(E, rows, K, N, n_contig, kind)
+
+
+@pytest.mark.parametrize("kind", ["first_low", "first_high", "heights", "heights_gaps", "tile_rows_gaps"])
+@pytest.mark.parametrize("E,rows,K,N", [(32, 500, 264, 2568), (66, 500, 264, 1032), (17, 500, 1856, 648)])
+@pytest.mark.parametrize("n_contig", [False, True])
+def test_loads_at_the_rule(E, rows, K, N, n_contig, kind):
+    """Loads that count as even whatever expert comes first, and those whose tile rows agree while their heights do not."""
+    _check_plain_and_gated(E, rows, K, N, n_contig, kind)
+
+
+def _check_plain_and_gated(E, rows, K, N, n_contig, kind):
     g = torch.Generator(device=DEV).manual_seed(E + rows)
     loads = _loads(kind, E, rows)
     L = sum(loads)
