@@ -2,7 +2,7 @@
 
 The kernels issue their direct-to-LDS loads from inline assembly with the base address in scalar registers.  On
 gfx9-family hardware a vector memory instruction must not read a scalar register within five wait states of a
-vector instruction (v_readfirstlane) writing it; the compiler keeps that distance for its own instructions but does
+vector instruction (v_readfirstlane, v_readlane) writing it; the compiler keeps that distance for its own instructions but does
 not look into assembly blocks, and a load that reads a stale base faults the GPU.  The test compiles every
 source of the MFMA kernels to assembly and looks at the six instructions in front of every load of an assembly block."""
 import os
@@ -19,6 +19,7 @@ from scattermoe_amd import _build
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 VMEM = re.compile(r"\b(global_load|buffer_load|global_store|buffer_store)\w*\b")
 SBASE = re.compile(r"\bs\[(\d+):(\d+)\]")
+VALU_TO_SGPR = re.compile(r"v_\w+ s(?:(\d+)|\[(\d+):(\d+)\])")      # a vector instruction whose destination is scalar
 
 
 def _hazards(text):
@@ -46,8 +47,8 @@ def _hazards(text):
                 continue
             nop = re.match(r"s_nop (\d+)", t)
             states += int(nop.group(1)) + 1 if nop else 1
-            w = re.match(r"v_readfirstlane_b32 s(\d+)", t)
-            if w and int(w.group(1)) in regs and states <= 5:
+            w = VALU_TO_SGPR.match(t)
+            if w and states <= 5 and regs & set(range(int(w[1] or w[2]), int(w[1] or w[3]) + 1)):
                 found.append((i + 1, t, line.strip()))
                 break
     return loads, found
@@ -57,6 +58,9 @@ def test_scanner_sees_a_hazard_and_its_fix():
     bad = "\tv_readfirstlane_b32 s2, v20\n\t;;#ASMSTART\n\tglobal_load_dword v1, v2, s[2:3]\n\t;;#ASMEND\n"
     good = "\tv_readfirstlane_b32 s2, v20\n\t;;#ASMSTART\n\ts_nop 4\n\tglobal_load_dword v1, v2, s[2:3]\n\t;;#ASMEND\n"
     assert _hazards(bad)[1] and not _hazards(good)[1]
+    for writer in ("v_readlane_b32 s3, v20, s9", "v_cmp_lt_u32_e64 s[2:3], v1, v2", "v_readlane_b32 s2, v20, 63"):
+        assert _hazards(bad.replace("v_readfirstlane_b32 s2, v20", writer))[1], writer
+    assert not _hazards(bad.replace("v_readfirstlane_b32 s2, v20", "v_readlane_b32 s4, v20, s2"))[1]
 
 
 def _sources():
