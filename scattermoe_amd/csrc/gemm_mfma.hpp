@@ -2000,15 +2000,35 @@ static constexpr int XTY_SMALL_ROWS = 256;
 // round of one per CU, or a second round up to 9/16 full (1600 rows per expert, plain / gathered, us: 128 tiles
 // 56 -> 38 / 45 -> 37, 160 tiles 59 -> 50 / 51 -> 48, 320 tiles 102 -> 77 / 96 -> 84, 384 tiles 105 -> 90 / 100 -> 90;
 // but 192 tiles 56 -> 57 / 48 -> 58, 256 tiles 64 -> 60 / 55 -> 61, 512 tiles 110 -> 112 / 105 -> 116).
-static bool xty_idle_chip(const XtYArgs& a) {
-  const int64_t tiles = (int64_t)a.E * ((a.N + 255) / 256) * ((a.K + 255) / 256);
-  return tiles <= 160 || (tiles > 256 && tiles <= 400);
+// They request every operand byte twice as often, so they lose once the operands are no longer served from the 256 MB
+// memory-side cache, or the rows are so many that the large tiles' shorter loop outweighs the idle CUs (us, 256 x 256
+// with one wave per SIMD -> small, whole products of E x (N, K) by rows per expert):
+//   second round: 8 x (1536, 1536) 4096 rows 200 -> 183, 6000 rows (295 MB) 283 -> 286, 8192 rows 372 -> 397;
+//     4 x (2048, 2304) 8192 rows (143 MB) 366 -> 365; 8 x (1536, 2048) 4096 rows 216 -> 205, 8192 rows 410 -> 479;
+//     2 x (3072, 4096) 5000 rows 262 -> 244, 8192 rows (235 MB) 406 -> 425; 4 x (2560, 2560), 400 tiles, 1024 rows
+//     67 -> 60, 2048 rows 109 -> 111, 3072 rows 150 -> 166, 4096 rows 205 -> 220, 8192 rows 390 -> 579
+//   129 to 160 tiles: 8 x (1024, 1280) 6000 rows 153 -> 142, 8192 rows (302 MB) 205 -> 216; 17 x (512, 1024) 5000 rows
+//     130 -> 114, 6000 rows (313 MB) 155 -> 160; 16 x (768, 768) 8192 rows (402 MB) 177 -> 216
+//   up to 128 tiles: 8 x (1024, 1024) 16384 rows (537 MB) 402 -> 349, 12 x (512, 1024) 16384 rows 399 -> 348, but experts
+//     of few tiles stream too much per product: 32 x (512, 512) 4096 rows 93 -> 73, 8192 rows (537 MB) 171 -> 183
+//     (gathered, against eight waves: 219 -> 199)
+// and for experts of one or two tiles beside many others: 128 x (256, 256) 512 / 1600 rows 19 -> 20, 42 -> 49; 53 x (256, 768)
+// 1024 / 2048 rows 33 -> 36, 54 -> 66; 64 x (256, 512) 2048 rows 49 -> 40.
+static bool xty_idle_chip(const XtYArgs& a, bool rs_form) {
+  const int64_t per_expert = (int64_t)((a.N + 255) / 256) * ((a.K + 255) / 256), tiles = a.E * per_expert;
+  const int64_t rows = a.L / a.E;
+  const bool cached = (int64_t)a.L * (a.N + a.K) * 2 <= (256ll << 20);
+  if (tiles <= 128) return cached ? per_expert > 1 || tiles <= 64 : per_expert >= 6 || !rs_form;
+  if (per_expert < 4) return false;
+  if (tiles <= 160) return cached;
+  if (tiles <= 256 || tiles > 400) return false;
+  return rows <= (tiles > 384 ? 1536 : !cached ? 3072 : tiles > 320 ? 5120 : 8192);
 }
 
 template <typename T>
 static int dispatch_xty(const XtYArgs& a, bool rs_form, hipStream_t st) {
   typedef Tile<128, 128, 2, 2, 1, false, 4> Small;
-  if (xty_idle_chip(a) || (a.idx == nullptr && a.L / a.E <= XTY_SMALL_ROWS)) return launch_xty<T, Small>(a, st);
+  if (xty_idle_chip(a, rs_form) || (a.idx == nullptr && a.L / a.E <= XTY_SMALL_ROWS)) return launch_xty<T, Small>(a, st);
   if (rs_form) return launch_xty<T, Tile<256, 256, 2, 2, 2, true>>(a, st);
   return launch_xty<T, Tile<256, 256, 2, 4>>(a, st);
 }

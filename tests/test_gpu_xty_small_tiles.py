@@ -48,6 +48,31 @@ def test_against_float64(K, N, layout, dtype):
         _check(Db[e], y.sum(0), y.abs().sum(0), n, dtype)
 
 
+# both sides of the lines between small and 256 x 256 tiles where the chip would idle: at most 128 output tiles of 256 x 256
+# (operands of 17 MB; of 270 MB with six tiles per expert, with four, with one), up to 160, a second round (400 tiles at the
+# last row count of small tiles and the first of large ones); always rows enough for the one-wave-per-SIMD form
+@pytest.mark.parametrize("E,rows,K,N", [(4, 2100, 520, 1040), (16, 8200, 520, 512), (32, 8200, 512, 512), (80, 2064, 256, 256),
+                                        (40, 2100, 512, 512), (2, 1536, 2560, 5120), (2, 1537, 2560, 5120),
+                                        (2, 2064, 2560, 5120)])
+def test_many_rows(E, rows, K, N):
+    g = torch.Generator(device=DEV).manual_seed(rows + K)
+    loads = [rows + (37 if e % 2 else -37) for e in range(E)]
+    off = torch.tensor(loads, device=DEV).cumsum(0)
+    L, dtype = sum(loads), torch.bfloat16
+    X = torch.randn(L, K, generator=g, device=DEV).to(dtype)
+    DY = torch.randn(L, N, generator=g, device=DEV).to(dtype)
+    idx = torch.randperm(L, generator=g, device=DEV)
+    DW, _ = ops.group_bwd_W(DY, X[idx], off, E)
+    DWg, Db = ops.group_bwd_W(DY, X, off, E, has_bias=True, gather=(idx, 1))
+    assert torch.equal(DW, DWg)
+    lo = 0
+    for e, n in enumerate(loads):
+        x, y = X[idx[lo:lo + n]].double(), DY[lo:lo + n].double()
+        _check(DW[e], x.t() @ y, x.abs().t() @ y.abs(), n, dtype)
+        _check(Db[e], y.sum(0), y.abs().sum(0), n, dtype)
+        lo += n
+
+
 def test_unaligned_output():
     """An output two bytes off a 16-byte boundary takes the plain stores; the same bits."""
     g = torch.Generator(device=DEV).manual_seed(5)
