@@ -21,8 +21,8 @@ SHAPES = [
     (520, 8, 2, 320, 1000),      # 130 rows/expert: ring-buffered 256x128 tiles
     (160, 8, 3, 448, 72),        # 60 rows/expert: ring-buffered 128x128 tiles, F < one tile
     (130, 8, 2, 320, 200),       # ~32 rows/expert: 64-row ring tiles
-    (40, 8, 2, 192, 136),        # 10 rows/expert: no fused forward kernel (falls back), fused backward
-    (960, 8, 2, 64, 2048),       # 240 rows/expert, about half a round of 256-row tiles: half-width tiles chosen
+    (40, 8, 2, 192, 136),        # 10 rows/expert: ring-buffered 32-row tiles
+    (960, 8, 2, 64, 2048),       # 240 rows/expert, half a round of 256-row tiles
     (1600, 32, 2, 64, 2048),     # 100 rows/expert and 512 wide tiles: 128x256 ring tiles
     (2560, 32, 2, 64, 2048),     # 160 rows/expert and 512 wide tiles: 256x256 tiles below their usual threshold
 ]

@@ -40,12 +40,12 @@ SHAPES = [
     (160, 8, 3, 448, 72),        # 60 rows/expert: ring-buffered 128x128 tiles, N < one tile
     (300, 8, 2, 200, 328),       # 75 rows/expert: 128x128 ring tiles with contraction and column tails
     (130, 8, 2, 448, 200),       # ~32 rows/expert: 64-row ring tiles
-    (3, 8, 2, 64, 256),          # decode-like: a handful of rows (ring-buffered 32-row tiles)
+    (3, 8, 2, 64, 256),          # decode-like: a handful of rows (row-dot kernel; 32-row ring tiles for N-contiguous weights)
     (40, 8, 2, 200, 264),        # 10 rows/expert: 32-row tiles with contraction and column tails
     (9, 4, 2, 1096, 136),        # 32-row tiles, contraction longer than the ring (17 full slices + tail)
-    (40, 8, 2, 200, 1288),       # enough 128-wide tiles to pick the 64-wide ring class for K-contiguous weights
+    (40, 8, 2, 200, 1288),       # ring-buffered 32-row tiles, 64 columns wide for K-contiguous weights
     (2048, 32, 4, 192, 328),     # E = 32 with skew: tiny and empty experts
-    (960, 8, 2, 64, 4096),       # 240 rows/expert, about half a round of 256x256 tiles: half-width tiles chosen
+    (960, 8, 2, 64, 4096),       # 240 rows/expert, half a round of 256x256 tiles
     (1600, 32, 2, 64, 4096),     # 100 rows/expert and 512 wide tiles: 128x256 ring tiles
     (2560, 32, 2, 64, 4096),     # 160 rows/expert and 512 wide tiles: 256x256 tiles below their usual threshold
 ]
@@ -178,12 +178,11 @@ def _routing_with_counts(counts, k, seed):
 
 @pytest.mark.parametrize("x_grouped,y_grouped", [(False, True), (True, False), (True, True)])
 def test_s2s_last_tiles_of_few_rows_in_their_own_launch(x_grouped, y_grouped):
-    """A large product with fewer than 1536 rows per expert leaves every expert's last tile of at most 128 rows to a
-    second launch of 128-row tiles.  Row counts chosen for each case of the tile lookup: a last tile of 100 rows
-    (second launch), of 200 rows (stays), none (exact multiple of 256), an expert without rows, one of 60 rows
-    (only the second launch sees it), last tiles of exactly 128 and of 129 rows, and one of 1 row.  Every row must
-    be written once, to the oracle's values, and with the same bits as the launches over the column halves, which
-    are too small to be split.  (30 tile columns: 3.75 rounds, so the product is not cut by whole rounds instead.)"""
+    """A large product with fewer than 1536 rows per expert keeps every expert's last tile in its one launch, at the
+    height of its rows: last tiles of 1, 60, 100, 128, 129 and 200 rows, none (exact multiple of 256), an expert
+    without rows, one of 60 rows only.  Every row must be written once, to the oracle's values, and with the same bits
+    as the launches over the column halves.  (30 tile columns: the product is not cut by whole rounds either.  The
+    products that do leave last tiles to a launch of their own: test_s2s_split_contraction_at_every_last_tile.)"""
     counts, k, K, N = LAST_TILE_COUNTS, 2, 2048, 7680
     E, L = len(counts), sum(counts)
     eid, idx, off, g = _routing_with_counts(counts, k, seed=11)
@@ -269,6 +268,36 @@ def test_s2s_last_tiles_with_split_contraction(x_grouped, y_grouped, w_layout, d
     assert torch.equal(via_ops, got)
 
 
+@pytest.mark.parametrize("w_layout", ["k_contig", "n_contig"])
+@pytest.mark.parametrize("x_grouped,y_grouped", [(False, True), (True, False), (True, True)])
+def test_s2s_split_contraction_at_every_last_tile(x_grouped, y_grouped, w_layout):
+    """The cases of the tile lookups around such a launch: last tiles of 1, 128 (split) and of 129, 200 rows (not), none,
+    an expert without rows, one of 60 rows only.  Against float32 products on the GPU, and against the product without
+    workspace as above."""
+    counts, K, N = [2049, 1664, 1921, 1480, 2560, 0, 4232, 60], 4096, 2048
+    E, L, dtype = len(counts), sum(counts), torch.bfloat16
+    assert L // E >= 1536 and 2 * L * K * N >= 2e11
+    eid, idx, off, g = _routing_with_counts(counts, 1, seed=23)
+    X = torch.randn(L, K, generator=g).to(dtype).to(DEV)
+    W = (torch.randn(E, N, K, generator=g) * 0.03).to(dtype).to(DEV).permute(0, 2, 1)
+    b = torch.randn(E, N, generator=g).to(dtype).to(DEV)
+    W = W.contiguous() if w_layout == "n_contig" else W
+    idx = idx.to(DEV)
+    args = (X, W, b, eid.to(DEV), idx, off.to(DEV), 1, x_grouped, y_grouped)
+    got, plain = _s2s_through_the_c_abi(*args, workspace=True), _s2s_through_the_c_abi(*args, workspace=False)
+    lo = differ = 0
+    for e, c in enumerate(counts):
+        src, dst = (torch.arange(lo, lo + c, device=DEV) if grouped else idx[lo:lo + c] for grouped in (x_grouped, y_grouped))
+        _close(got[dst], X[src].float() @ W[e].float() + b[e].float(), scale=0.03 * K ** 0.5)
+        split = c % 256 if c % 256 <= 128 else 0
+        assert torch.equal(got[dst[:c - split]], plain[dst[:c - split]]), c
+        a, p = got[dst[c - split:]].float(), plain[dst[c - split:]].float()
+        assert bool(((a - p).abs() <= 2.0 ** -7 * p.abs() + 1e-4).all()), c       # float32 regrouping, as above
+        differ += int((a != p).sum())
+        lo += c
+    assert differ > 0, "no last tile was added up in parts"
+
+
 def test_s2s_workspace_that_is_too_small_or_misaligned_is_not_used():
     """smoe_scatter2scatter_ws with less workspace than it asks for, or with a workspace that is not 16-byte aligned,
     is exactly smoe_scatter2scatter: same bits, nothing written to the workspace."""
@@ -303,9 +332,9 @@ def test_s2s_workspace_that_is_too_small_or_misaligned_is_not_used():
 
 @pytest.mark.parametrize("act", ["SILU", "GPT_OSS"])
 def test_fused_gated_products_with_last_tiles_in_their_own_launch(act):
-    """The same row counts through the products that carry the gated unit in their epilogue (forward: saved
-    pre-activations and hidden rows; backward: gradient of the pre-activations), against the plain product followed
-    by the elementwise pass, which is checked above."""
+    """The row counts of test_s2s_last_tiles_of_few_rows_in_their_own_launch through the products that carry the gated
+    unit in their epilogue, one launch each (forward: saved pre-activations and hidden rows; backward: gradient of the
+    pre-activations), against the plain product followed by the elementwise pass, which is checked above."""
     counts, k, d, F = LAST_TILE_COUNTS, 2, 2048, 4096
     E, L = len(counts), sum(counts)
     eid, idx, off, g = _routing_with_counts(counts, k, seed=12)
