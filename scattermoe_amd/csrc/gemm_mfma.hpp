@@ -34,12 +34,16 @@ static constexpr int STRIPE_BELOW = 1024;
 // 10000 tokens 216 -> 205, 238 -> 227, 380 -> 350, 694 -> 677, 1032 -> 982; 32 experts d = F = 2880, 48 tokens 261 ->
 // 252, training step of 1501 / 3000 tokens 1617 -> 1574, 2653 -> 2525; 8 experts d = 4096, F = 14336, training step of
 // 6000 tokens 11996 -> 11728.  Uneven loads keep the other order (taken in chunks, loads falling as 1 / rank^1.8: 1607 -> 1681).
+// Even is judged by tile rows: experts of one tile row each may still differ in its height.  One launch with loads of 60 to
+// 250 rows, experts in no order, chunks against stripes: 32 experts 2880 -> 2880 147 / 161, 2880 -> 2 x 2880 240 / 265;
+// 64, 2048 -> 2048 144 / 152; 128, 2048 -> 1536 198 / 229, 768 -> 2048 122 / 128; with the experts sorted by load (the heavy
+// ones then share an XCD) 161 / 154, 261 / 263, 150 / 159, 229 / 229, 138 / 124.
 // Above 2048 rows per expert: even (128 experts x 2048 rows 8538 -> 8546).
 static constexpr int CHUNK_BELOW = 3072;
 static constexpr int GM_S2S = 4;
 static constexpr int GM_XTY = 4;
 static constexpr int XTY_GATHER_MAX_N = 6144;   // widest dY for which groupXtY gathers the rows of X itself
-static constexpr int REMAINDER_ROWS = 128;      // an expert's last tile of at most this many rows goes to a launch of 128-row tiles
+static constexpr int REMAINDER_ROWS = 128;      // last tiles of at most this many rows leave a product that cuts them off (cut_tails)
 #include <type_traits>
 #include <algorithm>
 #include <math.h>
@@ -1756,7 +1760,7 @@ static bool glu_fwd_pieces(const S2SArgs& a) {
 
 // Fewer than 52 rows per expert: a stream over the weights of the experts that are hit, tiles of 64 or 32 rows.  What
 // counts is weight bytes in flight across the chip, and that the filling of one tile's ring hides behind the stream of
-// another: a workgroup that has the CU to itself (six 20 KB stages, the only form until now) leaves the memory idle
+// another: a workgroup that has the CU to itself (six 20 KB stages) leaves the memory idle
 // while it looks its tile up, fills its ring and stores its result, for a tile of 512 KB (128 columns x 2048) about a
 // fifth of its time.  Hence two or three workgroups per CU with shallower rings wherever the launch has that many.
 // Measured (us, one 32 x 128 x 6 workgroup per CU -> now; weights streamed at):
@@ -1773,7 +1777,10 @@ static int dispatch_few_rows(const S2SArgs& a, bool b_tr, hipStream_t st) {
   // (us, two x three stages -> three x two: 64 x 11 tiles of K = 2048 80 -> 67, 16 x 44 74 -> 66, 32 x 23 of K = 2880
   // 89 -> 82, 16 x 44 of K = 4096 137 -> 124; with fewer tiles two stages are too few: 256 of K = 14336 147 -> 211)
   if (wgs > 2 * NUM_CU && wgs <= 3 * NUM_CU) return launch_s2s<T, Tile<64, 128, 2, 2, 2, false, 3>>(a, b_tr, st);
-  const bool few = b_tr ? wgs < NUM_CU : wgs <= NUM_CU;                   // up to one workgroup per CU: deep rings
+  // Up to one workgroup per CU: deep rings.  At exactly one per CU N-contiguous weights are faster in two shallow ones
+  // (us, deep -> shallow, 256 tiles: 8 x 30 rows, K = 14336 150 -> 141, K = 2048 27 -> 25; 32 x 30 rows, K = 2880 35 -> 33),
+  // K-contiguous ones only with a short contraction (149 -> 153, 33.8 -> 32.7, 33.2 -> 32.2): deep.
+  const bool few = b_tr ? wgs < NUM_CU : wgs <= NUM_CU;
   if (avg >= (few ? 24 : ROWS32_BELOW)) {
     if (few) return launch_s2s<T, Tile<64, 128, 2, 2, 5>>(a, b_tr, st);
     return launch_s2s<T, Tile<64, 128, 2, 2, 3, false, 2>>(a, b_tr, st);
@@ -1783,7 +1790,10 @@ static int dispatch_few_rows(const S2SArgs& a, bool b_tr, hipStream_t st) {
   if (!b_tr) {
     // K-contiguous weights: half-width tiles while 128-wide ones would not give every CU two workgroups (44 x 8 tiles
     // of K = 1024: 25 -> 17 us, 22 x 16 of K = 2048: 47 -> 39, 8 x 8 of K = 2816: 18 -> 16), and where 128-wide
-    // columns do not divide evenly among the 8 XCDs (12 columns: 152 -> 140 us; 45 or 16: even)
+    // columns do not divide evenly among the 8 XCDs, as the stripes of uneven loads have to, at most 3/4 of the last
+    // row of eight in use (128 experts of K = 2048, uneven / evenly loaded, which take chunks: 9 columns 127 -> 116 /
+    // 118 -> 106, 12 columns 164 -> 146 / 133 -> 131, 17 columns 214 -> 194 / 180 -> 179; 16 columns 213 -> 185 /
+    // 165 -> 168, 32 columns 375 -> 356 / 329 -> 329: evenly loaded decides, being the ordinary case)
     if (wgs < 192) return launch_s2s<T, Tile<32, 64, 1, 2, 6>>(a, b_tr, st);
     if (wgs < 2 * NUM_CU || cols * 4 <= (cols + 7) / 8 * 8 * 3) return launch_s2s<T, Tile<32, 64, 1, 2, 4, false, 3>>(a, b_tr, st);
   } else if (few) {

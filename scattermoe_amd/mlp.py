@@ -77,7 +77,7 @@ class _GatedMLP(torch.autograd.Function):
             dpre = ops.scatter2scatter_glu_bwd(dy, w2.permute(0, 2, 1), pre, eid, idx, act=act, expert_offsets=off,
                                                alpha=ctx.alpha, limit=ctx.limit)
             if need_w1 or need_b1:
-                # the weight gradient reads the rows of x through idx: no gathered copy of x is made
+                # rows of x by idx: looked up inside the launch, or copied ahead of it where that is faster
                 d_w1, d_b1 = ops.group_bwd_W(DY=dpre, X=x, expert_offsets=off, E=E, has_bias=b1 is not None, like=w1,
                                              gather=(idx, k))
                 d_w1 = d_w1 if need_w1 else None

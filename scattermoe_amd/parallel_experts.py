@@ -97,8 +97,8 @@ class ParallelLinear(torch.autograd.Function):
 
         d_w = d_b = None
         if need_w or need_b:
-            # ungrouped input: the weight gradient reads the rows of x through idx (the reference gathers a copy
-            # of x first, parallel_experts.py:95-99)
+            # ungrouped input: the rows of x by idx, looked up inside the launch or, where that is faster, copied
+            # ahead of it (the reference always gathers a copy, parallel_experts.py:95-99)
             d_w, d_b = ops.group_bwd_W(DY=dy, X=x, expert_offsets=off, E=E, has_bias=bias is not None, like=W,
                                        gather=None if grouped_in else (idx, k))
             if not need_w:
