@@ -1754,6 +1754,16 @@ static int launch_main(const S2SArgs& a, bool b_tr, hipStream_t st) {
 }
 
 static constexpr int MAIN_MIN_TILES = 160;
+// Products whose 256 x 128 tiles fit one round of a workgroup per CU take those: the 256 x 256 ones would leave half of
+// the chip idle for as long (us, 256 x 256 -> 256 x 128: 4 experts x 332 rows, 1280 -> 3328 36 -> 26; 8 x 1829,
+// 10752 -> 448 224 -> 172; 32 x 438, 7616 -> 384 151 -> 118; 16 x 572, 10624 -> 448 191 -> 157; over 509 launches of
+// 224 to 4000 rows per expert, a quarter of them at this line, 5.5 % on average; a second round of them loses).  The line
+// is drawn for even loads: uneven ones go by column stripes, where a column's tiles share the 32 CUs of an XCD and may
+// take two rounds (8 x 584 rows on average, 4640 -> 1272, 21 tile rows in ten columns 109 -> 168).
+static bool one_round_of_halves(const S2SArgs& a) {
+  const int cols = a.glu == 1 ? 64 : 128;
+  return expected_row_tiles(a.L, a.E) * ((a.N + cols - 1) / cols) <= NUM_CU;
+}
 static bool glu_fwd_pieces(const S2SArgs& a) {
   return a.glu != 1 || (((((uintptr_t)a.Y | (uintptr_t)a.H) & 15) == 0) && ((a.sym | a.shm | a.N) & 7) == 0);
 }
@@ -1818,8 +1828,9 @@ static int dispatch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
   // 269 -> 214, 5760 -> 2880 286 -> 254; 8 x 140, 4096 -> 11264 210 -> 181; 128 x 188, 2048 -> 768 with its gated unit's
   // gradient 168 -> 144; with half as many tiles as CUs, 8 x 188, 14336 -> 4096, 263 -> 288, even below 160 rows), from
   // 52 rows on where it makes one round of what the 128-row tiles do in two (16 x 90, 2048 -> 2 x 1408 56 -> 42), and
-  // whatever the number of tiles from 224 rows on.
+  // from 224 rows on whatever the number of tiles, unless half-width ones fit one round.
   const int64_t tiles = (int64_t)a.E * ((a.N + (a.glu == 1 ? 127 : 255)) / (a.glu == 1 ? 128 : 256));
+  if (avg >= ROWS256_BELOW && one_round_of_halves(a)) return launch_s2s<T, Tile<256, 128, 4, 2, 3>>(a, b_tr, st);
   if (avg >= ROWS256_BELOW || (avg >= ROWS128_BELOW && tiles >= MAIN_MIN_TILES) ||
       (avg >= ROWS64_BELOW && tiles > NUM_CU / 2 && tiles <= NUM_CU))
     return launch_main<T>(a, b_tr, st);
