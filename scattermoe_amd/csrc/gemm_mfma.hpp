@@ -2014,9 +2014,21 @@ static int launch_xty(const XtYArgs& a, hipStream_t st) {
 // measured alone, us: 32 experts 2880 x 5760, 100 / 188 / 300 / 400 rows each: 314 -> 225, 407 -> 335, 493 -> 455,
 // 594 -> 579; 128 experts 2048 x 1536: 223 -> 168, 286 -> 242, 371 -> 364, 462 -> 477; 8 experts 14336 x 4096:
 // 257 -> 191, 316 -> 270, 390 -> 370, 480 -> 489.  Inside a training step, at its lower clock: 32 x 188 rows, 2880 x 2880
-// 248 -> 212; even at 280).  Gathered rows chain two more memory accesses in front of every slice, which small tiles
-// repeat too often (32 experts 400 -> 372, 128 experts 276 -> 279): they keep the large ones.
+// 248 -> 212; even at 280).  Gathered rows as well: 34 random launches of 128 to 256 rows per expert 256 x 256 -> small
+// 1.23 times as fast.
 static constexpr int XTY_SMALL_ROWS = 256;
+// But with few rows per expert the launch is all stores.  Output rows that are no whole number of 64-byte pieces (the unit
+// memory is written in) share one at every tile edge; twice the edges cost more than small tiles save, in launches of more than
+// 512 large tiles: 50 random ones of 2 to 96 rows per expert 256 x 256 -> small 0.92 times as fast (161 of whole pieces 1.28;
+// us: 16 experts x 22 rows, (11024, 2416) 278 -> 311, 128 x 34, (1064, 4144) 384 -> 475).
+static constexpr int XTY_STORE_ROWS = 96, XTY_STORE_TILES = 512;
+static bool xty_few_rows(const XtYArgs& a) {
+  const int64_t rows = a.L / a.E, tiles = (int64_t)a.E * ((a.N + 255) / 256) * ((a.K + 255) / 256);
+  if (rows > XTY_SMALL_ROWS) return false;
+  const int64_t pitch = a.sdwk == 1 ? a.sdwn : a.sdwk;                    // elements between output rows
+  const bool pieces = ((uintptr_t)a.DW & 63) == 0 && ((pitch | a.sdwe) & 31) == 0;
+  return pieces || rows >= XTY_STORE_ROWS || tiles <= XTY_STORE_TILES;
+}
 // The same small tiles, whatever the number of rows, where the 256 x 256 ones leave the chip idle: at most 5/8 of a
 // round of one per CU, or a second round up to 9/16 full (1600 rows per expert, plain / gathered, us: 128 tiles
 // 56 -> 38 / 45 -> 37, 160 tiles 59 -> 50 / 51 -> 48, 320 tiles 102 -> 77 / 96 -> 84, 384 tiles 105 -> 90 / 100 -> 90;
@@ -2049,7 +2061,7 @@ static bool xty_idle_chip(const XtYArgs& a, bool rs_form) {
 template <typename T>
 static int dispatch_xty(const XtYArgs& a, bool rs_form, hipStream_t st) {
   typedef Tile<128, 128, 2, 2, 1, false, 4> Small;
-  if (xty_idle_chip(a, rs_form) || (a.idx == nullptr && a.L / a.E <= XTY_SMALL_ROWS)) return launch_xty<T, Small>(a, st);
+  if (xty_idle_chip(a, rs_form) || xty_few_rows(a)) return launch_xty<T, Small>(a, st);
   if (rs_form) return launch_xty<T, Tile<256, 256, 2, 2, 2, true>>(a, st);
   return launch_xty<T, Tile<256, 256, 2, 4>>(a, st);
 }

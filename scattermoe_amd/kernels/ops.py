@@ -572,13 +572,15 @@ def _xty_launch(E, DW, Db, DY, X, expert_offsets):
 def _xty_gathered_launch(E, DW, Db, DY, X, idx, fan_out, expert_offsets):
     """groupXtY over X[idx // fan_out]: one launch that reads the rows of X through idx where the library has one,
     else the gathered copy and the plain launch."""
-    # Few rows per expert: the small tiles of the plain launch and a copy are faster than lookups inside the launch
-    # (whole training step of d = F = 2880, 32 experts, top-4, 50 / 100 / 188 rows per expert: 949 -> 922, 1227 -> 1207,
-    # 1637 -> 1609 us).  The copy costs 4 K bytes per row against 2 K N flops, so narrow dY keeps the lookups from
-    # fewer rows on (N = 1536: 128 rows 1143 -> 1147, 188 rows 1329 -> 1343).
-    few_rows = DY.size(0) <= min(256, DY.size(1) // 16) * E
+    # A dW with N contiguous takes the gathered rows as its row operand; wide launches of few rows are then faster over a
+    # copy (32 random ones of more than 512 tiles of 256 x 256, up to 256 rows per expert, N from 2048: 1.04 times as
+    # fast, 0.94 to 1.17; d = F = 2880, 32 experts, 50 / 188 rows: 219 -> 201, 377 -> 369 us).  Everything else looks the rows
+    # up inside the launch: of up to 512 tiles the copy's launch is what counts (20 rows: 11 us against 19), and with K
+    # contiguous the copy is never faster (87 random launches 0.93; 128 experts x 100 rows, 2048 x 1536 201 against 249 us).
+    copy_rows = (DW.stride(2) == 1 and DY.size(0) <= 256 * E and DY.size(1) >= 2048
+                 and E * DY.size(1) * X.size(1) > 512 * 256 * 256)
     lookups = DY.is_cuda and hasattr(_backend, "xty_gathered") and DY.dtype in (torch.bfloat16, torch.float16)
-    if lookups and not few_rows:
+    if lookups and not copy_rows:
         _same_dtype("group_bwd_W", DY, X, DW, Db)
         if _backend.xty_gathered(DY, X, _as_i64(idx).contiguous(), fan_out, DW, Db,
                                  _as_i64(expert_offsets).contiguous(), E):

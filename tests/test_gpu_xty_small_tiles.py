@@ -102,6 +102,31 @@ def test_gather_takes_any_index_vector(dtype):
     assert torch.equal(DW, want) and torch.equal(Db, want_b)
 
 
+# dW on both sides of the lines between small and large tiles (output rows of whole 64-byte pieces or not, more than 512 tiles
+# or not) and between lookups and a copy of the rows (N or K contiguous, wide or not): the same bits on every route
+@pytest.mark.parametrize("layout", ["nk", "kn"])
+@pytest.mark.parametrize("E,rows,K,N", [(64, 90, 520, 2056), (64, 90, 544, 2080), (64, 100, 520, 2056), (16, 20, 1544, 6144),
+                                        (64, 250, 768, 776), (4, 20, 264, 2056)])
+def test_routes_of_few_rows(E, rows, K, N, layout):
+    g = torch.Generator(device=DEV).manual_seed(rows + K)
+    loads = [rows + (7 if e % 2 else -7) for e in range(E)]
+    off = torch.tensor(loads, device=DEV).cumsum(0)
+    L, dtype = sum(loads), torch.bfloat16
+    X = torch.randn(L // 2, K, generator=g, device=DEV).to(dtype)
+    DY = torch.randn(L, N, generator=g, device=DEV).to(dtype)
+    idx = torch.randperm(L, generator=g, device=DEV)
+    like = torch.empty(E, K, N, dtype=dtype, device=DEV) if layout == "kn" else None
+    DW, Db = ops.group_bwd_W(DY, X[idx // 2], off, E, has_bias=True, like=like)
+    DWg, Dbg = ops.group_bwd_W(DY, X, off, E, has_bias=True, like=like, gather=(idx, 2))
+    assert torch.equal(DW, DWg) and torch.equal(Db, Dbg)
+    lo = 0
+    for e, n in enumerate(loads):
+        x, y = X[idx[lo:lo + n] // 2].double(), DY[lo:lo + n].double()
+        _check(DW[e], x.t() @ y, x.abs().t() @ y.abs(), n, dtype)
+        _check(Db[e], y.sum(0), y.abs().sum(0), n, dtype)
+        lo += n
+
+
 @pytest.mark.parametrize("n,N,dtype", [(400, 512, torch.bfloat16), (20, 6400, torch.bfloat16), (400, 6400, torch.float16),
                                        (20, 512, torch.float32), (400, 512, torch.float32)])
 @pytest.mark.parametrize("k", [2, 4])
