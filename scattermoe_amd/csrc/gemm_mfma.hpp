@@ -1785,8 +1785,10 @@ static int dispatch_few_rows(const S2SArgs& a, bool b_tr, hipStream_t st) {
   const int64_t cols = (a.N + bn - 1) / bn, wgs = std::min<int64_t>(a.L, a.E) * cols;
   // Three two-stage workgroups per CU where that makes one round of what would be 1.5 rounds of two per CU
   // (us, two x three stages -> three x two: 64 x 11 tiles of K = 2048 80 -> 67, 16 x 44 74 -> 66, 32 x 23 of K = 2880
-  // 89 -> 82, 16 x 44 of K = 4096 137 -> 124; with fewer tiles two stages are too few: 256 of K = 14336 147 -> 211)
-  if (wgs > 2 * NUM_CU && wgs <= 3 * NUM_CU) return launch_s2s<T, Tile<64, 128, 2, 2, 2, false, 3>>(a, b_tr, st);
+  // 89 -> 82, 16 x 44 of K = 4096 137 -> 124; with fewer tiles two stages are too few: 256 of K = 14336 147 -> 211), while
+  // no expert is expected to need a second tile row, which would be a second round (three standard deviations; 32 x 23 of
+  // K = 2880, two x three -> three x two: 40 rows per expert 91 -> 89, 44 rows 90 -> 89, 49 rows 113 -> 130)
+  if (wgs > 2 * NUM_CU && wgs <= 3 * NUM_CU && avg + 3 * sqrt((double)avg) < 64) return launch_s2s<T, Tile<64, 128, 2, 2, 2, false, 3>>(a, b_tr, st);
   // Up to one workgroup per CU: deep rings.  At exactly one per CU N-contiguous weights are faster in two shallow ones
   // (us, deep -> shallow, 256 tiles: 8 x 30 rows, K = 14336 150 -> 141, K = 2048 27 -> 25; 32 x 30 rows, K = 2880 35 -> 33),
   // K-contiguous ones only with a short contraction (149 -> 153, 33.8 -> 32.7, 33.2 -> 32.2): deep.
