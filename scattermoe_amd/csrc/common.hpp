@@ -162,8 +162,11 @@ __device__ __forceinline__ int wave_max(int v) {
 // `rounds` as many as there are rounds of 256 tiles.  A grid of chunked_grid() workgroups covers every tile.
 // Returns 1: this workgroup's tile; 0: none; -1: the experts that have rows differ in tile rows by more than a quarter of
 // the most, so that equal numbers of tiles are not equal work: another order has to be taken (the same answer in every
-// workgroup, and for the same loads in any order).
-template <int BM>
+// workgroup, and for the same loads in any order).  HEIGHTS: tiles cost their rows in blocks of 64, so loads whose blocks
+// differ by no more are even too: around a multiple of BM rows most experts end in a tile that others don't have
+// (us, stripes -> chunks, 32 experts x 238 rows, one of them 270, 2880 -> 2 x 2880 325 -> 273, 2880 -> 2880 218 -> 151;
+// 128 x 238, 16 of them 270, 2048 -> 2 x 768 290 -> 265, 768 -> 2048 159 -> 155).
+template <int BM, bool HEIGHTS>
 __device__ __forceinline__ int find_tile_chunked(const int64_t* __restrict__ off, int E, int pid, int n_tiles,
                                                  bool rounds, int& expert, int& row_start, int& rows, int& column) {
   const int lane = lane_id();
@@ -187,17 +190,21 @@ __device__ __forceinline__ int find_tile_chunked(const int64_t* __restrict__ off
   };
   int lo, hi, nt;
   load(0, lo, hi, nt);
-  int most = nt, least = nt > 0 ? nt : 0x7fffffff;            // tile rows of an expert that has any
+  // tile rows, and blocks of 64 rows, of an expert that has any
+  auto blocks = [](int l_, int h_) { return (h_ - l_ + 63) >> 6; };
+  int most = nt, least = nt > 0 ? nt : 0x7fffffff, most_b = blocks(lo, hi), least_b = hi > lo ? most_b : 0x7fffffff;
   for (int e0 = 64; e0 < E; e0 += 64) {
     int l_, h_, n_;
     load(e0, l_, h_, n_);
     most = max(most, n_);
-    if (n_ > 0) least = min(least, n_);
+    most_b = max(most_b, blocks(l_, h_));
+    if (n_ > 0) least = min(least, n_), least_b = min(least_b, blocks(l_, h_));
   }
-  if (__ballot(most > 1)) {
-    most = wave_max(most);
-    if (4 * (most + wave_max(-least)) > most) return -1;
-  }
+  auto differ = [](int most_, int least_) {                   // by more than a quarter of the most
+    most_ = wave_max(most_);
+    return 4 * (most_ + wave_max(-least_)) > most_;
+  };
+  if (__ballot(most > 1) && differ(most, least) && (!HEIGHTS || differ(most_b, least_b))) return -1;
   int incl = scan(nt);
   int total = __builtin_amdgcn_readlane(incl, 63);
   for (int e0 = 64; e0 < E; e0 += 64) {

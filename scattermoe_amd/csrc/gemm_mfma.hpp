@@ -34,8 +34,8 @@ static constexpr int STRIPE_BELOW = 1024;
 // 10000 tokens 216 -> 205, 238 -> 227, 380 -> 350, 694 -> 677, 1032 -> 982; 32 experts d = F = 2880, 48 tokens 261 ->
 // 252, training step of 1501 / 3000 tokens 1617 -> 1574, 2653 -> 2525; 8 experts d = 4096, F = 14336, training step of
 // 6000 tokens 11996 -> 11728.  Uneven loads keep the other order (taken in chunks, loads falling as 1 / rank^1.8: 1607 -> 1681).
-// Even is judged by tile rows: experts of one tile row each may still differ in its height.  One launch with loads of 60 to
-// 250 rows, experts in no order, chunks against stripes: 32 experts 2880 -> 2880 147 / 161, 2880 -> 2 x 2880 240 / 265;
+// Even is judged by tile rows or blocks of 64: experts of one tile row each may still differ in its height.  One launch with
+// loads of 60 to 250 rows, experts in no order, chunks against stripes: 32 experts 2880 -> 2880 147 / 161, 2880 -> 2 x 2880 240 / 265;
 // 64, 2048 -> 2048 144 / 152; 128, 2048 -> 1536 198 / 229, 768 -> 2048 122 / 128; with the experts sorted by load (the heavy
 // ones then share an XCD) 161 / 154, 261 / 263, 150 / 159, 229 / 229, 138 / 124.
 // Above 2048 rows per expert: even (128 experts x 2048 rows 8538 -> 8546).
@@ -1486,7 +1486,8 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
   int found = -1;
   if (rast.chunked) {
     t.m_loc = t.n_loc = 0;
-    found = find_tile_chunked<TL::BM>(a.off, a.E, blockIdx.x, rast.n_tiles, rast.chunked == 2, t.e, t.row0, t.rows, t.n_tile);
+    found = find_tile_chunked<TL::BM, TL::BM == 256 && TL::BN == 256>(a.off, a.E, blockIdx.x, rast.n_tiles, rast.chunked == 2,
+                                                                      t.e, t.row0, t.rows, t.n_tile);
     if (found == 0) return;
   }
   if (found < 0 && !rast.map(blockIdx.x, m_tile, t.n_tile, t.m_loc, t.n_loc)) return;

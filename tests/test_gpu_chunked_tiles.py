@@ -24,6 +24,10 @@ def _loads(kind, E, rows):
         return [60 + (190 * e) // (E - 1) for e in range(E)]
     if kind == "heights_gaps":               # the same, every fourth expert without rows, loads falling
         return [0 if e % 4 == 2 else 250 - (190 * e) // (E - 1) for e in range(E)]
+    if kind == "blocks":                     # a multiple of 256 between them: another tile row, another block of 64
+        return [rows // 256 * 256 - e % 5 + (20 if e % 3 == 0 else 0) for e in range(E)]
+    if kind == "blocks_gaps":                # the same, the last expert without rows
+        return [0 if e == E - 1 else rows // 256 * 256 - e % 5 + (20 if e == 0 else 0) for e in range(E)]
     if kind == "tile_rows_gaps":             # two tile rows each, the first and every third expert without rows
         return [0 if e % 3 == 0 else rows - e % 4 for e in range(E)]
     return [rows * 4] + [max(1, rows // 8)] * (E - 1)       # uneven
@@ -41,11 +45,14 @@ def test_plain_and_gated(E, rows, K, N, n_contig, kind):
     _check_plain_and_gated(E, rows, K, N, n_contig, kind)
 
 
-@pytest.mark.parametrize("kind", ["first_low", "first_high", "heights", "heights_gaps", "tile_rows_gaps"])
-@pytest.mark.parametrize("E,rows,K,N", [(32, 500, 264, 2568), (66, 500, 264, 1032), (17, 500, 1856, 648)])
+@pytest.mark.parametrize("kind", ["first_low", "first_high", "heights", "heights_gaps", "tile_rows_gaps", "blocks",
+                                  "blocks_gaps"])
+@pytest.mark.parametrize("E,rows,K,N", [(32, 500, 264, 2568), (66, 500, 264, 1032), (17, 500, 1856, 648),
+                                        (130, 530, 264, 264), (64, 300, 264, 2056)])
 @pytest.mark.parametrize("n_contig", [False, True])
 def test_loads_at_the_rule(E, rows, K, N, n_contig, kind):
-    """Loads that count as even whatever expert comes first, and those whose tile rows agree while their heights do not."""
+    """Loads that count as even whatever expert comes first, those whose tile rows agree while their heights do
+    not, and those whose tile rows differ while their blocks of 64 rows hardly do."""
     _check_plain_and_gated(E, rows, K, N, n_contig, kind)
 
 
