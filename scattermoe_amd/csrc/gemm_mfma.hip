@@ -54,7 +54,8 @@ bool try_xty_mfma(const XtYArgs& a, int dtype, hipStream_t st, int& rc) {
   // traffic per row against 2 K N flops, i.e. a share of the kernel time that shrinks with N.  Measured per training
   // step: N = 1536 (Qwen-like, top-8) 9.12 -> 8.90 ms, N = 5760 (gpt-oss-like) 6.07 -> 6.03 ms, N = 28672 (Mixtral)
   // 31.3 -> 31.5 ms: wide layers keep the separate pass.
-  if (a.idx != nullptr && a.N > XTY_GATHER_MAX_N) return false;
+  // (The kernel that holds one operand looks every row up once per unit: always.)
+  if (a.idx != nullptr && a.N > XTY_GATHER_MAX_N && !xty_held(a)) return false;
   // One-wave-per-SIMD form: needs the LDS-staged epilogue; no gathered operand, no bias gradient in the main loop.
   // Both operands are read transposed (two LDS reads per fragment), which leaves less to win than in
   // scatter2scatter: Mixtral shape (4096 rows per expert) 3.28 -> 3.12 and 6.35 -> 6.20 ms, 2048 rows per expert

@@ -1867,24 +1867,15 @@ struct XtYPlan {
   // that holds X (Q when db_from_p, else P) reads its rows through idx; NULL: X is already in grouped order
   const int64_t* idx;
   int fan_out;
+  int64_t x_rows;                         // rows of the matrix X is gathered from
 };
 
+// One output tile: rows p0, columns q0 of expert e.
 template <typename T, class TL, bool GA, bool GB>
-__global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void xty_mfma_kernel(XtYPlan a, Raster rast, int p_tiles) {
+__device__ __forceinline__ void xty_tile(const XtYPlan& a, int e, int p0, int q0, char* lds, int64_t* sDst, unsigned* sRows,
+                                         float* sBias) {
   typedef TransOp<TL::BM, TL::NT, false, GA> AOp;
   typedef TransOp<TL::BN, TL::NT, false, GB> BOp;
-  constexpr int STAGE = AOp::LDS_BYTES + BOp::LDS_BYTES;
-  constexpr int STAGED = TL::BM * TL::BN * 2;          // the output tile on its way out
-  __shared__ __attribute__((aligned(16))) char lds[TL::NS * STAGE > STAGED ? TL::NS * STAGE : STAGED];
-  __shared__ int64_t sDst[TL::BM];
-  __shared__ unsigned sRows[2 * 64];       // row offsets of a gathered operand (see TransOp)
-  __shared__ __attribute__((aligned(16))) float sBias[TL::RS ? TL::BN : 4];
-
-  int m_tile, n_tile, m_loc, n_loc;
-  if (!rast.map(blockIdx.x, m_tile, n_tile, m_loc, n_loc)) return;
-  const int e = m_tile / p_tiles;
-  const int p0 = (m_tile % p_tiles) * TL::BM;
-  const int q0 = n_tile * TL::BN;
   const int r_lo = e ? (int)a.off[e - 1] : 0;
   const int r_hi = (int)a.off[e];
 
@@ -1909,7 +1900,7 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void xty_mfma_kernel(Xt
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
   }
-  const bool want_db = a.Db != nullptr && a.db_from_p && n_tile == 0;
+  const bool want_db = a.Db != nullptr && a.db_from_p && q0 == 0;
   if constexpr (TL::RS) mainloop_rs<T, TL, AOp, BOp>(A, B, r_hi - r_lo, lds, acc);      // no bias gradient, no gather
   else mainloop<T, TL, AOp, BOp, true>(A, B, r_hi - r_lo, lds, want_db, acc, rs);
 
@@ -1930,6 +1921,28 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void xty_mfma_kernel(Xt
     }
   }
 }
+
+// LDS of a workgroup: operand stages, later the output tile on its way out; row tables.
+template <class TL>
+struct XtYLds {
+  static constexpr int STAGES = TL::NS * (TL::BM + TL::BN) * 128, STAGED = TL::BM * TL::BN * 2;
+  __attribute__((aligned(16))) char lds[STAGES > STAGED ? STAGES : STAGED];
+  int64_t dst[TL::BM];
+  unsigned rows[2 * 64];                    // row offsets of a gathered operand (see TransOp)
+  __attribute__((aligned(16))) float bias[TL::RS ? TL::BN : 4];
+};
+
+template <typename T, class TL, bool GA, bool GB>
+__global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void xty_mfma_kernel(XtYPlan a, Raster rast, int p_tiles) {
+  __shared__ XtYLds<TL> s;
+  int m_tile, n_tile, m_loc, n_loc;
+  if (!rast.map(blockIdx.x, m_tile, n_tile, m_loc, n_loc)) return;
+  xty_tile<T, TL, GA, GB>(a, m_tile / p_tiles, (m_tile % p_tiles) * TL::BM, n_tile * TL::BN, s.lds, s.dst, s.rows, s.bias);
+}
+
+}  // namespace smoe
+#include "xty_rows.hpp"
+namespace smoe {
 
 // Bias gradient when dY is the column operand: column sums per expert segment.  A workgroup owns 256 columns of one
 // expert: 32 column threads (16 bytes = 8 columns each) x 8 row lanes; every thread adds up the rows r = lane
@@ -1974,8 +1987,7 @@ __global__ __launch_bounds__(256) void colsum_kernel(const T* __restrict__ DY, i
   }
 }
 
-template <typename T, class TL>
-static int launch_xty(const XtYArgs& a, hipStream_t st) {
+static XtYPlan xty_plan(const XtYArgs& a) {
   XtYPlan p;
   const bool k_contig = a.sdwk == 1;     // output rows = N index
   if (k_contig) {
@@ -1992,6 +2004,14 @@ static int launch_xty(const XtYArgs& a, hipStream_t st) {
   p.off = a.off; p.E = a.E;
   p.db_from_p = k_contig ? 1 : 0;
   p.idx = a.idx; p.fan_out = a.fan_out;
+  p.x_rows = a.L / (a.idx ? a.fan_out : 1);
+  return p;
+}
+
+template <typename T, class TL>
+static int launch_xty(const XtYArgs& a, hipStream_t st) {
+  const bool k_contig = a.sdwk == 1;
+  const XtYPlan p = xty_plan(a);
   const int p_tiles = (p.np + TL::BM - 1) / TL::BM;
   const int q_tiles = (p.nq + TL::BN - 1) / TL::BN;
   const Raster r = make_raster((int64_t)a.E * p_tiles, q_tiles, GM_XTY);
@@ -2001,13 +2021,7 @@ static int launch_xty(const XtYArgs& a, hipStream_t st) {
   else if (a.idx == nullptr) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, false>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r, p_tiles);
   else if (k_contig) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, true>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r, p_tiles);
   else hipLaunchKernelGGL((xty_mfma_kernel<T, TL, true, false>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r, p_tiles);
-  int rc = launch_status("xty_mfma_kernel");
-  if (rc == 0 && a.Db != nullptr && !k_contig) {
-    hipLaunchKernelGGL(colsum_kernel<T>, dim3((a.N + 255) / 256, a.E), dim3(256), 0, st, (const T*)a.DY,
-                       a.sdym, a.N, a.off, (T*)a.Db, a.sdbe, a.sdbn);
-    rc = launch_status("colsum_kernel");
-  }
-  return rc;
+  return launch_status("xty_mfma_kernel");
 }
 
 // Which tiles a weight gradient is cut into.  A 256 x 256 tile has a CU to itself and the memory idles while it is
@@ -2061,12 +2075,38 @@ static bool xty_idle_chip(const XtYArgs& a, bool rs_form) {
   return rows <= (tiles > 384 ? 1536 : !cached ? 3072 : tiles > 320 ? 5120 : 8192);
 }
 
+// One operand in registers, the other streamed past it (xty_rows.hpp), us against 128 x 128 tiles over 390 random launches with
+// output rows on whole lines.  From 96 rows per expert on: even loads of 110 to 220 rows 1.07 to 1.31 times as fast; below 64
+// 0.96 (both are bound by their stores there), 64 to 96 1.00 to 1.07.  Up to 224: experts beyond 256 rows go in tiles, two
+// workgroups per CU where a launch of nothing but tiles has four (even loads of 250 rows, half of them beyond: 0.95, 1190
+// rows 0.85).  At least 256 tiles of 256 x 256: smaller launches have too few units (16 x 142 rows, 1472 x 512 11 -> 13).
+// Uneven loads of such an average (1 / rank^0.84, 1 / rank^1.8): 0.95 and 1.2, the heavy experts then start first.
+static constexpr int XTY_HELD_MIN_ROWS = 96, XTY_HELD_MAX_ROWS = 224;
+static bool xty_held(const XtYArgs& a) {
+  const int64_t rows = a.L / a.E;
+  if (rows < XTY_HELD_MIN_ROWS || rows > XTY_HELD_MAX_ROWS) return false;
+  return (int64_t)a.E * ((a.N + 255) / 256) * ((a.K + 255) / 256) >= 256 && xty_rows_fits(xty_plan(a));
+}
+
 template <typename T>
 static int dispatch_xty(const XtYArgs& a, bool rs_form, hipStream_t st) {
   typedef Tile<128, 128, 2, 2, 1, false, 4> Small;
-  if (xty_idle_chip(a, rs_form) || xty_few_rows(a)) return launch_xty<T, Small>(a, st);
-  if (rs_form) return launch_xty<T, Tile<256, 256, 2, 2, 2, true>>(a, st);
-  return launch_xty<T, Tile<256, 256, 2, 4>>(a, st);
+  typedef Tile<256, 256, 2, 4> Large;
+  const bool small = xty_idle_chip(a, rs_form) || xty_few_rows(a);
+  int rc;
+  if (xty_held(a)) {
+    rc = launch_xty_rows<T>(xty_plan(a), a.L, st);
+  } else if (small) {
+    rc = launch_xty<T, Small>(a, st);
+  } else {
+    rc = rs_form ? launch_xty<T, Tile<256, 256, 2, 2, 2, true>>(a, st) : launch_xty<T, Large>(a, st);
+  }
+  if (rc == 0 && a.Db != nullptr && a.sdwk != 1) {
+    hipLaunchKernelGGL(colsum_kernel<T>, dim3((a.N + 255) / 256, a.E), dim3(256), 0, st, (const T*)a.DY,
+                       a.sdym, a.N, a.off, (T*)a.Db, a.sdbe, a.sdbn);
+    rc = launch_status("colsum_kernel");
+  }
+  return rc;
 }
 
 }  // namespace smoe

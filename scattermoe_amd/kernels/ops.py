@@ -577,7 +577,10 @@ def _xty_gathered_launch(E, DW, Db, DY, X, idx, fan_out, expert_offsets):
     # fast, 0.94 to 1.17; d = F = 2880, 32 experts, 50 / 188 rows: 219 -> 201, 377 -> 369 us).  Everything else looks the rows
     # up inside the launch: of up to 512 tiles the copy's launch is what counts (20 rows: 11 us against 19), and with K
     # contiguous the copy is never faster (87 random launches 0.93; 128 experts x 100 rows, 2048 x 1536 201 against 249 us).
-    copy_rows = (DW.stride(2) == 1 and DY.size(0) <= 256 * E and DY.size(1) >= 2048
+    # Nor is it where the rows held in registers are looked up once per workgroup (96 to 224 rows per expert, output rows on
+    # 128-byte lines: 188 rows, 2880 x 2880 / 5760, lookups 156 / 266 us, plain 154 / 255, the copy 9).
+    held = 96 * E <= DY.size(0) < 225 * E and (DW.stride(0) | DW.stride(1)) % 64 == 0
+    copy_rows = (DW.stride(2) == 1 and DY.size(0) <= 256 * E and DY.size(1) >= 2048 and not held
                  and E * DY.size(1) * X.size(1) > 512 * 256 * 256)
     lookups = DY.is_cuda and hasattr(_backend, "xty_gathered") and DY.dtype in (torch.bfloat16, torch.float16)
     if lookups and not copy_rows:
