@@ -159,7 +159,7 @@ __device__ __forceinline__ int wave_max(int v) {
 // expert by expert, inside an expert column by column (of `n_tiles`), the expert's tile rows of a column side by side.
 // The XCD of a workgroup is `pid` % 8; the order is cut into 8 R chunks of equal length and XCD x takes the chunks
 // x, x + 8, ... (in turn from either end).  How many tiles there are is known only here, from `off`: R = 1, or with
-// `rounds` as many as there are rounds of 256 tiles.  A grid of chunked_grid() workgroups covers every tile.
+// `round` > 0 as many as there are rounds of that many tiles (256 or more).  A grid of chunked_grid() workgroups covers every tile.
 // Returns 1: this workgroup's tile; 0: none; -1: the experts that have rows differ in tile rows by more than a quarter of
 // the most, so that equal numbers of tiles are not equal work: another order has to be taken (the same answer in every
 // workgroup, and for the same loads in any order).  HEIGHTS: tiles cost their rows in blocks of 64, so loads whose blocks
@@ -168,7 +168,7 @@ __device__ __forceinline__ int wave_max(int v) {
 // 128 x 238, 16 of them 270, 2048 -> 2 x 768 290 -> 265, 768 -> 2048 159 -> 155).
 template <int BM, bool HEIGHTS>
 __device__ __forceinline__ int find_tile_chunked(const int64_t* __restrict__ off, int E, int pid, int n_tiles,
-                                                 bool rounds, int& expert, int& row_start, int& rows, int& column) {
+                                                 int round, int& expert, int& row_start, int& rows, int& column) {
   const int lane = lane_id();
   auto load = [&](int e0, int& lo, int& hi, int& nt) {        // experts e0 .. e0 + 63, one per lane
     const int e = e0 + lane;
@@ -213,7 +213,7 @@ __device__ __forceinline__ int find_tile_chunked(const int64_t* __restrict__ off
     total += __builtin_amdgcn_readlane(scan(n_), 63);
   }
   const unsigned tiles = (unsigned)total * n_tiles;
-  const unsigned R = rounds && tiles >= 384 ? (tiles + 128) / 256 : 1;
+  const unsigned R = round && tiles >= round + round / 2u ? (tiles + round / 2u) / round : 1;
   const unsigned len = __builtin_amdgcn_readfirstlane((tiles + 8 * R - 1) / (8 * R));
   if (len == 0) return 0;
   const unsigned x = pid & 7, i = (unsigned)pid >> 3, c = i / len;

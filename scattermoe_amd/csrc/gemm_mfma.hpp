@@ -386,14 +386,16 @@ __device__ __forceinline__ void issue_slice_tail(const AOp& A, const BOp& B, uns
 }
 
 // WG_: workgroups per CU the registers have to leave room for (LDS permitting)
-template <int BM_, int BN_, int WM_, int WN_, int NS_ = 2, bool RS_ = false, int WG_ = 1>
+// PAIR_: two workgroups per CU that fill its LDS between them (mainloop_pair)
+template <int BM_, int BN_, int WM_, int WN_, int NS_ = 2, bool RS_ = false, int WG_ = 1, bool PAIR_ = false>
 struct Tile {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_;
   static constexpr int NS = NS_;                      // LDS stages (2: double buffer, more: ring)
   static constexpr bool RS = RS_;                     // operands travel global -> registers -> LDS (mainloop_rs)
   static constexpr int WG = WG_;
+  static constexpr bool PAIR = PAIR_;
   // the same tile with U blocks of 32 rows per wave
-  template <int U> using Height = Tile<U * 32 * WM_, BN_, WM_, WN_, NS_, RS_, WG_>;
+  template <int U> using Height = Tile<U * 32 * WM_, BN_, WM_, WN_, NS_, RS_, WG_, PAIR_>;
   static constexpr int NW = WM * WN, NT = NW * 64;
   static constexpr int WAVES_PER_SIMD = WG_ * NW / 4 > 0 ? WG_ * NW / 4 : 1;
   static constexpr int WTM = BM / WM, WTN = BN / WN;
@@ -650,6 +652,83 @@ __device__ __forceinline__ void mainloop_rs(const AOp& A, const BOp& B, int klen
     rs_slice<T, TL, AOp, BOp, 1, N>(A, B, lds1, lds, kt + 1, last_k0, klen, wm, wn, acc, g, fa, fb);
   }
   if (kt < nk) rs_slice<T, TL, AOp, BOp, 0, N>(A, B, lds, lds1, kt, last_k0, klen, wm, wn, acc, g, fa, fb);
+}
+
+// Main loop of the class with two workgroups of four waves per CU (256 x 128 tiles, wave tiles of up to 128 x 64).  Its
+// point is what happens outside the loop: a tile is looked up, waits for its first slice and is rounded and stored while
+// the other workgroup of the CU multiplies, which a 256 x 256 tile that has the CU to itself cannot hide (17 to 23 K cycles of
+// them against 2 400 to 2 900 per slice).  80 KB of LDS each: two stages of the row operand, one of the column operand, whose
+// fragments of a whole slice are read into registers (32 of them) ahead of the products, so that the next slice's pieces
+// can be on their way into the same stage while they run.  The burst of reads and the two barriers around it fall into the
+// other workgroup's products.
+// Whole 64-deep slices only (the launcher checks).
+static constexpr int PAIR_STAGE = 32 * 1024, PAIR_B = 2 * PAIR_STAGE, PAIR_LDS = PAIR_B + 16 * 1024;
+template <typename T, class TL, class AOp, class BOp>
+__device__ __forceinline__ void mainloop_pair(const AOp& A, const BOp& B, int klen, char* lds, f32x16 (&acc)[TL::FM][TL::FN]) {
+  static_assert(AOp::LDS_BYTES <= PAIR_STAGE && BOp::LDS_BYTES <= PAIR_LDS - PAIR_B, "LDS");
+  constexpr int KS = BK / 16, LOADS = AOp::R + BOp::R, PER_STEP = (LOADS + KS - 2) / (KS - 1);      // (all of them up front: 2 % slower)
+  const int wave = threadIdx.x >> 6;
+  const int wm = wave / TL::WN, wn = wave % TL::WN;
+  const unsigned lds_u = lds_address(lds);
+  const int nk = klen / BK;
+#pragma unroll
+  for (int j = 0; j < BOp::R; ++j) B.issue_one(lds_u + PAIR_B, 0, j);
+#pragma unroll
+  for (int j = 0; j < AOp::R; ++j) A.issue_one(lds_u, 0, j);
+  auto slice = [&](int kt, auto more) {
+    const unsigned par = (unsigned)(kt & 1) * PAIR_STAGE;
+    const char* ta = lds + par;
+    const char* tb = lds + PAIR_B;
+    const unsigned na = lds_u + (PAIR_STAGE - par);
+    // this thread's pieces of slice kt have landed, everyone's have, and everyone is done with slice kt - 1
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    i32x4 fa[2][TL::FM], fb[KS][TL::FN];
+#pragma unroll
+    for (int j = 0; j < TL::FN; ++j) fb[0][j] = BOp::frag(tb, wn * TL::WTN + j * 32, 0);
+#pragma unroll
+    for (int i = 0; i < TL::FM; ++i) fa[0][i] = AOp::frag(ta, wm * TL::WTM + i * 32, 0);
+#pragma unroll
+    for (int ks = 1; ks < KS; ++ks)
+#pragma unroll
+      for (int j = 0; j < TL::FN; ++j) fb[ks][j] = BOp::frag(tb, wn * TL::WTN + j * 32, ks);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // everyone has the column operand's fragments
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);                       // ahead of the other workgroup's reads (1 to 2 %)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int c = ks & 1, n = c ^ 1;
+      if constexpr (decltype(more)::value) {
+#pragma unroll
+        for (int q = ks * PER_STEP; q < (ks + 1) * PER_STEP && q < LOADS; ++q) {
+          if (q < BOp::R) B.issue_one(lds_u + PAIR_B, (kt + 1) * BK, q);
+          else A.issue_one(na, (kt + 1) * BK, q - BOp::R);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (ks + 1 < KS) {
+#pragma unroll
+        for (int i = 0; i < TL::FM; ++i) fa[n][i] = AOp::frag(ta, wm * TL::WTM + i * 32, ks + 1);
+      }
+#pragma unroll
+      for (int i = 0; i < TL::FM; ++i)
+#pragma unroll
+        for (int j = 0; j < TL::FN; ++j) acc[i][j] = Mfma<T>::run(fb[ks][j], fa[c][i], acc[i][j]);
+      if (ks + 1 < KS) {
+#pragma unroll
+        for (int i = 0; i < TL::FM; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x100, AOp::DS_PER_FRAG, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+        if constexpr (TL::FM * TL::FN > TL::FM) __builtin_amdgcn_sched_group_barrier(0x008, TL::FM * TL::FN - TL::FM, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+  };
+  for (int kt = 0; kt + 1 < nk; ++kt) slice(kt, std::true_type());
+  slice(nk - 1, std::false_type());
 }
 
 // Main loop of the small-row (decode) tile class: memory bound, so what matters is bytes in flight.  The
@@ -1272,6 +1351,7 @@ struct Raster {
   int64_t grid_size;                       // host side only: number of workgroups (may exceed what a launch takes)
   __host__ int64_t grid() const { return grid_size; }
   // (ml, nl): position of the tile inside its super tile
+  template <int SN_ = SN>
   __device__ __forceinline__ bool map(int pid, int& m, int& n, int& ml, int& nl) const {
     const int x = pid & 7, i = pid >> 3;
     if (striped) {
@@ -1287,8 +1367,8 @@ struct Raster {
     // The 8 supers of step j = i / 32 go to the 8 XCDs rotated by j: supers differ in how many of their tiles
     // exist (partial last column-super, empty tile rows), and a fixed assignment would give some XCDs the full
     // ones every time.
-    const int j = i / (SM * SN);
-    const int s = j * 8 + ((x + j) & 7), r = i % (SM * SN);
+    const int j = i / (SM * SN_);
+    const int s = j * 8 + ((x + j) & 7), r = i % (SM * SN_);
     if (s >= supers) return false;
     ml = r % SM;
     nl = r / SM;
@@ -1297,7 +1377,7 @@ struct Raster {
     const int rem = s - band * gm * n_supers;
     const int g = min(gm, m_supers - band * gm);
     m = (band * gm + rem % g) * SM + r % SM;
-    n = (rem / g) * SN + r / SM;
+    n = (rem / g) * SN_ + r / SM;
     return m < m_tiles && n < n_tiles;
   }
 };
@@ -1305,16 +1385,16 @@ struct Raster {
 // `gm`: row-supers per band.  A band's row panels (gm * 8 tiles) are reused by every column-super while the
 // column panels stream past once, so the band should be small enough for its row panels to stay in the
 // memory-side cache and large enough to keep all XCDs inside one band.
-static Raster make_raster(int64_t m_tiles, int n_tiles, int gm) {
+static Raster make_raster(int64_t m_tiles, int n_tiles, int gm, int sn = Raster::SN) {
   Raster r;
   r.m_tiles = (int)m_tiles;
   r.n_tiles = n_tiles;
   r.m_supers = (int)((m_tiles + Raster::SM - 1) / Raster::SM);
-  r.n_supers = (n_tiles + Raster::SN - 1) / Raster::SN;
+  r.n_supers = (n_tiles + sn - 1) / sn;
   r.striped = 0;
   r.gm = gm < 1 ? 1 : (gm > r.m_supers ? r.m_supers : gm);
   const int64_t supers = (int64_t)r.m_supers * r.n_supers;
-  r.grid_size = (supers + 7) / 8 * 8 * Raster::SM * Raster::SN;
+  r.grid_size = (supers + 7) / 8 * 8 * Raster::SM * sn;
   r.supers = supers > 0x7fffffffLL ? 0x7fffffff : (int)supers;   // such a grid is rejected by the launchers
   return r;
 }
@@ -1358,7 +1438,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   // once, and with the non-temporal hint it does not push the token rows, which every workgroup of a tile row reads,
   // out of the L2s (hint extended from the 32-/64-row classes to all ring classes: Mixtral layer forward at 256 /
   // 384 / 448 tokens 0.539 -> 0.505 / 0.559 -> 0.526 / 0.711 -> 0.688 ms, neutral from 768 tokens on)
-  constexpr bool W_ONCE = TL::NS > 2 || TL::WG > 1;
+  constexpr bool W_ONCE = TL::NS > 2 || (TL::WG > 1 && !TL::PAIR);
   typedef typename std::conditional<B_TR, TransOp<TL::BN, TL::NT, W_ONCE>, DirectOp<TL::BN, TL::NT, W_ONCE>>::type BOp;
   constexpr bool CAN_SPLIT = TL::BM == 128 && TL::BN == 256 && TL::NS == 3;
   const int glu = TL::RS ? __builtin_amdgcn_readfirstlane(a.glu) : -1;      // (as for the tile in s2s_mfma_kernel)
@@ -1366,7 +1446,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   const int k_first = CAN_SPLIT ? t.part * t.klen : 0;
 
   AOp A;
-  A.rot = TL::RS ? 0 : (t.n_loc * AOp::R / Raster::SN) % AOp::R;    // the row panel has SN sharers
+  A.rot = TL::RS ? 0 : (t.n_loc * AOp::R / (TL::PAIR ? 2 * Raster::SN : Raster::SN)) % AOp::R;    // the row panel has SN sharers
   // Lane offsets are 32-bit: grouped input rows are taken relative to the tile's first row (so that the input may
   // be of any size), gathered ones relative to the start of the token matrix.
   const int64_t sxm = a.sxm;
@@ -1407,6 +1487,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
   if constexpr (TL::RS) mainloop_rs<T, TL, AOp, BOp>(A, B, a.K, lds, acc);
+  else if constexpr (TL::PAIR) mainloop_pair<T, TL, AOp, BOp>(A, B, a.K, lds, acc);
   else if constexpr (TL::NS > 2) mainloop_ring<T, TL, AOp, BOp>(A, B, t.klen, lds, acc);
   else mainloop<T, TL, AOp, BOp, false>(A, B, a.K, lds, false, acc, rs);
 
@@ -1466,12 +1547,18 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
 
 template <typename T, class TL, bool B_TR>
 __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2SArgs a, Raster rast) {
+  // (a workgroup that shares its CU's LDS with one other keeps its row tables where operands are to come: the source rows in
+  // the second row stage, which is requested behind a barrier that follows their last reading, the output rows in the
+  // column stage)
   constexpr int STAGE = (TL::BM + TL::BN) * 128;
-  static_assert(TL::BM * TL::BN * 2 <= TL::NS * STAGE, "staged tile must fit the operand buffers");
-  __shared__ __attribute__((aligned(16))) char lds[TL::NS * STAGE];
-  __shared__ int64_t sDst[TL::BM];
-  __shared__ int sSrc[TL::BM];
-  __shared__ __attribute__((aligned(16))) float sBias[TL::RS ? TL::BN : 4];
+  static_assert(TL::BM * TL::BN * 2 <= (TL::PAIR ? PAIR_B : TL::NS * STAGE), "staged tile must fit the operand buffers");
+  __shared__ __attribute__((aligned(16))) char lds[TL::PAIR ? PAIR_LDS : TL::NS * STAGE];
+  __shared__ int64_t sDst_[TL::PAIR ? 1 : TL::BM];
+  __shared__ int sSrc_[TL::PAIR ? 1 : TL::BM];
+  __shared__ __attribute__((aligned(16))) float sBias_[TL::RS ? TL::BN : 4];
+  int64_t* sDst = TL::PAIR ? (int64_t*)(lds + PAIR_B) : sDst_;
+  int* sSrc = TL::PAIR ? (int*)(lds + PAIR_STAGE) : sSrc_;
+  float* sBias = TL::PAIR ? nullptr : sBias_;
 
   // Contraction parts (the class of the experts' last tiles only): the grid is `ksplit` copies of the raster, copy
   // c multiplies the c-th part of the contraction (a raster is a multiple of 8 workgroups, so the XCD of a workgroup
@@ -1486,11 +1573,12 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
   int found = -1;
   if (rast.chunked) {
     t.m_loc = t.n_loc = 0;
-    found = find_tile_chunked<TL::BM, TL::BM == 256 && TL::BN == 256>(a.off, a.E, blockIdx.x, rast.n_tiles, rast.chunked == 2,
+    found = find_tile_chunked<TL::BM, TL::BM == 256 && (TL::BN == 256 || TL::PAIR)>(a.off, a.E, blockIdx.x, rast.n_tiles,
+                                                                      rast.chunked == 2 ? TL::WG * 256 : 0,
                                                                       t.e, t.row0, t.rows, t.n_tile);
     if (found == 0) return;
   }
-  if (found < 0 && !rast.map(blockIdx.x, m_tile, t.n_tile, t.m_loc, t.n_loc)) return;
+  if (found < 0 && !rast.map<TL::PAIR ? 2 * Raster::SN : Raster::SN>(blockIdx.x, m_tile, t.n_tile, t.m_loc, t.n_loc)) return;
   if (found > 0) {
     // looked up above
   } else if (a.tail_mode == 2) {
@@ -1524,7 +1612,7 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
     }
   }
   __syncthreads();
-  if constexpr (TL::BM == 256 && TL::BN == 256) {
+  if constexpr (TL::BM == 256 && (TL::BN == 256 || TL::PAIR)) {
     // An expert's last tile is partly filled: it is multiplied at the height of its rows, in steps of 64 (which keep
     // the four waves, or the eight, equally busy), not as a whole tile.  (Same sums in the same order.)
     // What it buys is that such tiles need no launch of their own any more (see cut_tails); a training step with many
@@ -1597,11 +1685,11 @@ static int launch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
   // With only a few tile rows per expert no weight panel is shared by the tile rows of a super tile; the striped
   // order at least keeps the tile rows of one expert together on one XCD.
   const bool striped = TL::NS > 2 || a.L / a.E < STRIPE_BELOW;
-  Raster r = striped ? make_striped(m_tiles, n_tiles, GM_RING) : make_raster(m_tiles, n_tiles, GM_S2S);
+  Raster r = striped ? make_striped(m_tiles, n_tiles, GM_RING) : make_raster(m_tiles, n_tiles, GM_S2S, TL::PAIR ? 2 * Raster::SN : Raster::SN);
   const bool whole = a.m_begin == 0 && a.m_count == 0x7fffffff && a.tail_mode == 0;
   const int64_t chunked = chunked_grid(m_tiles * n_tiles);
   if (whole && a.L / a.E < CHUNK_BELOW && chunked <= 0x7fffffffLL) {
-    r.chunked = TL::NS > 2 || TL::WG > 1 || a.L / a.E < ROWS256_BELOW ? 1 : 2;
+    r.chunked = TL::NS > 2 || (TL::WG > 1 && !TL::PAIR) || a.L / a.E < ROWS256_BELOW ? 1 : 2;
     r.grid_size = std::max(r.grid_size, chunked);
   }
   const int64_t grid = r.grid();
@@ -1668,13 +1756,29 @@ static int tail_split(const S2SArgs& a) {
 // Both forms add up every output element in the same order: the same bits.
 static constexpr int RS_MIN_K = 1792;
 static constexpr int RS_XTY_MIN_ROWS = 2048;      // groupXtY: average rows per expert from which that form is used
-template <typename T>
-static int launch_main_class(const S2SArgs& a, bool b_tr, hipStream_t st) {
-  bool al16 = true;             // the one-wave-per-SIMD form has only the LDS-staged epilogues (16-byte pieces)
+// Whole slices, and output pieces of 16 bytes: what the one-wave-per-SIMD form and the paired tiles take.
+static bool whole_pieces(const S2SArgs& a) {
+  bool al16 = true;
   if (a.glu == 0) al16 = (((uintptr_t)a.Y & 15) == 0) && ((a.sym | a.N) & 7) == 0;
   else if (a.glu == 1) al16 = ((((uintptr_t)a.Y | (uintptr_t)a.H) & 15) == 0) && ((a.sym | a.shm | a.N) & 7) == 0;
   else if (a.glu == 2) al16 = ((((uintptr_t)a.aux | (uintptr_t)a.Y) & 15) == 0) && ((a.saux | a.sym | a.N) & 7) == 0;
-  if (al16 && a.K % BK == 0 && a.K >= RS_MIN_K)
+  return al16 && a.K % BK == 0;
+}
+// Contractions of fewer than 1792 go in 256 x 128 tiles, two workgroups per CU (mainloop_pair).  The shorter the contraction
+// the more of a 256 x 256 tile's time is what it does before and behind its loop; launches of one to three rounds gain most,
+// their rounds being half as long.  590 random launches of 112 to 4000 rows per expert, K and N from 256 to 6000, plain and
+// with every fused unit, against eight waves per 256 x 256 tile (us): K below 512 1.13 times as fast on average, below 1024
+// 1.10, from there 1.05, one in thirty more than 3 % slower; 256 to 768 tiles of 256 x 256 1.16.  16 experts x 1000 rows,
+// 1024 -> 1024 60 -> 48; 64 x 500, 512 -> 512 39 -> 34; 128 x 2048, 768 -> 2048 963 -> 943, 1536 -> 2048 1687 -> 1673.  (Both
+// forms are held by the power cap there: a launch of K = 64 takes what its stores take, and every slice adds 63 us, 1.1 PFLOP/s.)
+// Longer contractions: the one-wave-per-SIMD form reads half as much from LDS per product; K from 2048 0.97, 8 x 4096 rows,
+// 14336 -> 4096 2957 -> 3216.
+typedef Tile<256, 128, 2, 2, 2, false, 2, true> PairTile;
+static bool takes_pairs(const S2SArgs& a) { return a.K < RS_MIN_K && whole_pieces(a); }
+
+template <typename T>
+static int launch_main_class(const S2SArgs& a, bool b_tr, hipStream_t st) {
+  if (a.K >= RS_MIN_K && whole_pieces(a))
     return launch_s2s<T, Tile<256, 256, 2, 2, 2, true>>(a, b_tr, st);
   return launch_s2s<T, Tile<256, 256, 2, 4>>(a, b_tr, st);
 }
@@ -1736,6 +1840,7 @@ static int launch_tails(const S2SArgs& a, bool b_tr, hipStream_t st) {
 // tiles (tail_split), the experts' sparsely filled last tiles apart (cut_tails).
 template <typename T>
 static int launch_main(const S2SArgs& a, bool b_tr, hipStream_t st) {
+  if (takes_pairs(a)) return launch_s2s<T, PairTile>(a, b_tr, st);
   S2SArgs m = a;
   const bool tails = cut_tails(a);
   if (tails) m.tail_mode = 1;
@@ -1830,12 +1935,13 @@ static int dispatch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
   // CUs a workgroup (us against the 256 x 128 and 128-row ring classes: 32 experts x 125 rows, 2880 -> 2 x 2880
   // 269 -> 214, 5760 -> 2880 286 -> 254; 8 x 140, 4096 -> 11264 210 -> 181; 128 x 188, 2048 -> 768 with its gated unit's
   // gradient 168 -> 144; with half as many tiles as CUs, 8 x 188, 14336 -> 4096, 263 -> 288, even below 160 rows), from
-  // 52 rows on where it makes one round of what the 128-row tiles do in two (16 x 90, 2048 -> 2 x 1408 56 -> 42), and
+  // 52 rows on where it makes one round of what the 128-row tiles do in two (16 x 90, 2048 -> 2 x 1408 56 -> 42; paired
+  // tiles, of which twice as many make a round, up to two: 17 random launches of 52 to 112 rows 1.15 times as fast), and
   // from 224 rows on whatever the number of tiles, unless half-width ones fit one round.
   const int64_t tiles = (int64_t)a.E * ((a.N + (a.glu == 1 ? 127 : 255)) / (a.glu == 1 ? 128 : 256));
   if (avg >= ROWS256_BELOW && one_round_of_halves(a)) return launch_s2s<T, Tile<256, 128, 4, 2, 3>>(a, b_tr, st);
   if (avg >= ROWS256_BELOW || (avg >= ROWS128_BELOW && tiles >= MAIN_MIN_TILES) ||
-      (avg >= ROWS64_BELOW && tiles > NUM_CU / 2 && tiles <= NUM_CU))
+      (avg >= ROWS64_BELOW && tiles > NUM_CU / 2 && tiles <= (takes_pairs(a) ? 2 : 1) * NUM_CU))
     return launch_main<T>(a, b_tr, st);
   // Below that the launch is a stream over the weights: tile height by rows per expert.  Launches with enough 256-wide
   // tile columns to fill the chip twice move half as many token rows per weight byte with 256-wide tiles as with
