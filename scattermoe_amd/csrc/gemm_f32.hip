@@ -7,7 +7,8 @@
 // operands stored [k][row] so that an MFMA operand (lane = row, lanes 32..63 the second k) is one conflict-free
 // ds_read_b32.  Global loads are 16 bytes per thread, fetched into registers one slice ahead of the MFMAs; an
 // operand with contiguous contraction axis is transposed on its way into LDS.  The fp32 matrix pipe is 16 times
-// slower than the bf16 one, so this simple pipeline already keeps it busy.
+// slower than the bf16 one, so this simple pipeline already keeps it busy.  Launches of fewer such tiles than CUs go in
+// tiles of 32 x 32 instead (s2s_f32_small_kernel, xty_f32_small_kernel).
 //
 // Counterparts in the reference: _scatter2scatter (scattermoe/kernels/ops.py:50-118) and _groupXtY
 // (ops.py:242-366) with float32 tensors (where Triton would use TF32 products under ALLOW_TF32).
@@ -172,6 +173,121 @@ __global__ __launch_bounds__(FNT) void s2s_f32_kernel(S2SArgs a, int n_tiles) {
   }
 }
 
+// =====================================================================================================
+// Launches that 128 x 128 tiles leave most of the chip idle for
+// =====================================================================================================
+// A 128 x 128 tile is a chain of 1 us per 16-deep slice (32 products of 64 cycles per wave), whatever its rows; a layer of a few
+// hundred tokens is a dozen of them on 256 CUs.  Here a workgroup owns 32 x 32 outputs, its four waves a quarter of the
+// contraction each; every wave takes its operands from memory straight into the registers they are multiplied from, 32
+// contraction elements ahead, with no LDS and no barrier until the four partial sums meet in LDS, where they are added in
+// ascending order.  (2 x 2 waves of 32 x 32, the whole contraction each: 1.3 to 2.5 times slower up to 256 tiles of 128 x 128.)
+// Which contraction element an operand's register holds is free as long as both agree: lane half h of chunk c, register s holds
+// element 8 c + 4 h + s, so that an operand with contiguous contraction is one 16-byte load per lane and chunk.
+// us, 128 x 128 tiles -> 32 x 32 (8 experts): 64 rows each, 128 -> 256 21.8 -> 6.0, 256 -> 128 34.5 -> 6.9, weight gradient
+// 11.7 -> 5.8; 112 rows, 600 -> 1200 69 -> 32; 700 rows, 512 -> 512 62 -> 55; 34 rows, 100 -> 100 19.3 -> 5.1.
+static constexpr int SMALL = 32, SMALL_WAVES = FNT / 64;
+// The line: products up to 256 expected tiles of 128 x 128 (192 62 -> 55, 320 141 -> 129, 448 115 -> 118 and 96 -> 113), weight
+// gradients, of which both operands come a float per lane and load, up to 128 (64 13.5 -> 9.5 and, of 12 rows, 8.2 -> 7.9; 128
+// 17.0 -> 16.6, of 583 rows 57 -> 51; 192 21 -> 30).
+static constexpr int64_t S2S_SMALL_TILES = 256, XTY_SMALL_TILES = 128;
+
+template <bool KC>
+struct LaneOp {
+  static constexpr int CHUNKS = 4, STEP = 8 * CHUNKS;
+  const float* p;                        // this lane's row (KC) or column, at its half's first element
+  int64_t ld;                            // elements between contraction steps
+  __device__ __forceinline__ void init(const float* first, int64_t ld_) {
+    ld = KC ? 1 : ld_;
+    p = first + (lane_id() >> 5) * 4 * ld;
+  }
+  // contraction elements [k0, k0 + STEP); from `kend` on zeros (nothing is read there)
+  __device__ __forceinline__ void load(int k0, int kend, f32x4 (&v)[CHUNKS]) const {
+    const int h4 = (lane_id() >> 5) * 4;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int k = k0 + 8 * c + h4;
+      if constexpr (KC) {
+        v[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (k < kend) v[c] = *(const f32x4*)(p + k0 + 8 * c);
+      } else {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          v[c][s] = 0.0f;
+          if (k + s < kend) v[c][s] = p[(int64_t)(k0 + 8 * c + s) * ld];
+        }
+      }
+    }
+  }
+};
+
+template <class AOp, class BOp>
+__device__ __forceinline__ void lane_product(const AOp& A, const BOp& B, int k_lo, int k_hi, f32x16& acc) {
+  constexpr int CH = AOp::CHUNKS;
+  f32x4 a[CH], b[CH];
+  A.load(k_lo, k_hi, a);
+  B.load(k_lo, k_hi, b);
+  for (int k0 = k_lo; k0 < k_hi; k0 += AOp::STEP) {
+    f32x4 na[CH], nb[CH];
+    A.load(k0 + AOp::STEP, k_hi, na);
+    B.load(k0 + AOp::STEP, k_hi, nb);
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[c][s], b[c][s], acc, 0, 0, 0);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) a[c] = na[c], b[c] = nb[c];
+  }
+}
+
+// The tile's outputs: `emit(row, column, value)` for each.
+template <typename F>
+__device__ __forceinline__ void small_outputs(const f32x16& acc, float (*part)[SMALL][SMALL + 1], F emit) {
+  const int l = lane_id(), wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) part[wave][(r >> 2) * 8 + (l >> 5) * 4 + (r & 3)][l & 31] = acc[r];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int m = q * 8 + (threadIdx.x >> 5), n = threadIdx.x & 31;
+    emit(m, n, ((part[0][m][n] + part[1][m][n]) + part[2][m][n]) + part[3][m][n]);
+  }
+}
+// this wave's part of a contraction of `k` elements: whole chunks of 8
+__device__ __forceinline__ void small_part(int k, int& lo, int& hi) {
+  const int per = (k + 8 * SMALL_WAVES - 1) / (8 * SMALL_WAVES) * 8;
+  lo = min(k, (int)(threadIdx.x >> 6) * per);
+  hi = min(k, lo + per);
+}
+
+template <bool W_KC>
+__global__ __launch_bounds__(FNT) void s2s_f32_small_kernel(S2SArgs a, int n_tiles) {
+  __shared__ float part[SMALL_WAVES][SMALL][SMALL + 1];
+  const int m_tile = blockIdx.x / n_tiles, n0 = (blockIdx.x % n_tiles) * SMALL;
+  int e, row0, rows;
+  if (!find_tile<SMALL>(a.off, a.E, m_tile, e, row0, rows)) return;
+  const int r = lane_id() & 31;
+  int64_t src = row0 + min(r, rows - 1);                     // rows and columns beyond the last repeat it
+  if (!a.x_grouped) src = a.idx[src] / a.fan_out;
+  LaneOp<true> A;
+  A.init((const float*)a.X + src * a.sxm, 1);
+  LaneOp<W_KC> B;
+  const int nc = min(n0 + r, a.N - 1);
+  B.init((const float*)a.W + (int64_t)e * a.swe + (int64_t)nc * (W_KC ? a.swn : 1), a.swk);
+  f32x16 acc;
+#pragma unroll
+  for (int q = 0; q < 16; ++q) acc[q] = 0.0f;
+  int lo, hi;
+  small_part(a.K, lo, hi);
+  lane_product(A, B, lo, hi, acc);
+  const float* bias = a.b ? (const float*)a.b + (int64_t)e * a.sbe : nullptr;
+  small_outputs(acc, part, [&](int mm, int nn, float v) {
+    if (mm >= rows || n0 + nn >= a.N) return;
+    const int64_t row = row0 + mm;
+    if (bias) v += bias[(int64_t)(n0 + nn) * a.sbn];
+    ((float*)a.Y)[(a.y_grouped ? row : a.idx[row]) * a.sym + n0 + nn] = v;
+  });
+}
+
 static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 bool try_s2s_f32(const S2SArgs& a, hipStream_t st, int& rc) {
@@ -183,6 +299,15 @@ bool try_s2s_f32(const S2SArgs& a, hipStream_t st, int& rc) {
   else if (a.swn == 1 && a.swk % 4 == 0 && a.N % 4 == 0) w_kc = false;
   else return false;
   const int n_tiles = (a.N + FBN - 1) / FBN;
+  // (an expert's last tile is half full on average)
+  if ((cdiv64(a.L, FBM) + a.E / 2) * n_tiles <= S2S_SMALL_TILES) {
+    const int cols = (a.N + SMALL - 1) / SMALL;
+    const dim3 grid((unsigned)(max_tiles(a.L, a.E, SMALL) * cols));
+    if (w_kc) hipLaunchKernelGGL(s2s_f32_small_kernel<true>, grid, dim3(FNT), 0, st, a, cols);
+    else hipLaunchKernelGGL(s2s_f32_small_kernel<false>, grid, dim3(FNT), 0, st, a, cols);
+    rc = launch_status("s2s_f32_small_kernel");
+    return true;
+  }
   const int64_t grid = max_tiles(a.L, a.E, FBM) * n_tiles;
   if (grid > 0x7fffffffLL) { set_error("smoe_scatter2scatter: grid too large"); rc = SMOE_ERR_RANGE; return true; }
   if (w_kc) hipLaunchKernelGGL(s2s_f32_kernel<true>, dim3((unsigned)grid), dim3(FNT), 0, st, a, n_tiles);
@@ -259,6 +384,28 @@ __global__ __launch_bounds__(FNT) void xty_f32_kernel(XtYPlanF32 a, int p_tiles,
   }
 }
 
+__global__ __launch_bounds__(FNT) void xty_f32_small_kernel(XtYPlanF32 a, int p_tiles, int q_tiles) {
+  __shared__ float part[SMALL_WAVES][SMALL][SMALL + 1];
+  int t = blockIdx.x;
+  const int q0 = t % q_tiles * SMALL; t /= q_tiles;
+  const int p0 = t % p_tiles * SMALL, e = t / p_tiles;
+  const int r_lo = e ? (int)a.off[e - 1] : 0, r_hi = (int)a.off[e];
+  const int r = lane_id() & 31;
+  LaneOp<false> A, B;
+  A.init(a.P + (int64_t)r_lo * a.ldp + min(p0 + r, a.np - 1), a.ldp);
+  B.init(a.Q + (int64_t)r_lo * a.ldq + min(q0 + r, a.nq - 1), a.ldq);
+  f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+  int lo, hi;
+  small_part(r_hi - r_lo, lo, hi);
+  lane_product(A, B, lo, hi, acc);
+  float* O = a.OUT + (int64_t)e * a.soe;                     // an expert without rows: zeros
+  small_outputs(acc, part, [&](int pp, int qq, float v) {
+    if (p0 + pp < a.np && q0 + qq < a.nq) O[(int64_t)(p0 + pp) * a.sop + q0 + qq] = v;
+  });
+}
+
 // bias gradient: column sums of dY per expert segment.  A workgroup owns 256 columns of one expert: 64 column threads
 // (16 bytes = 4 columns each) x 4 row lanes; the 4 partial sums of a column are added in a fixed order.
 __global__ __launch_bounds__(256) void colsum_f32_kernel(const float* __restrict__ DY, int64_t ld, int N,
@@ -298,7 +445,12 @@ bool try_xty_f32(const XtYArgs& a, hipStream_t st, int& rc) {
   const int p_tiles = (p.np + FBM - 1) / FBM, q_tiles = (p.nq + FBN - 1) / FBN;
   const int64_t grid = (int64_t)a.E * p_tiles * q_tiles;
   if (grid > 0x7fffffffLL) { set_error("smoe_groupXtY: grid too large"); rc = SMOE_ERR_RANGE; return true; }
-  if (grid > 0) {
+  if (grid > 0 && grid <= XTY_SMALL_TILES) {
+    const int pt = (p.np + SMALL - 1) / SMALL, qt = (p.nq + SMALL - 1) / SMALL;
+    hipLaunchKernelGGL(xty_f32_small_kernel, dim3((unsigned)(a.E * pt * qt)), dim3(FNT), 0, st, p, pt, qt);
+    rc = launch_status("xty_f32_small_kernel");
+    if (rc != 0) return true;
+  } else if (grid > 0) {
     hipLaunchKernelGGL(xty_f32_kernel, dim3((unsigned)grid), dim3(FNT), 0, st, p, p_tiles, q_tiles);
     rc = launch_status("xty_f32_kernel");
     if (rc != 0) return true;
