@@ -1,5 +1,5 @@
 // float32 MFMA paths of scatter2scatter and groupXtY for gfx950: true fp32 products and fp32 accumulation
-// (v_mfma_f32_32x32x2_f32; gfx950 has no TF32 mode), for operands whose rows are 16-byte aligned.  Everything else
+// (v_mfma_f32_32x32x2_f32; gfx950 has no TF32 mode), for operands with one contiguous axis each.  Everything else
 // in float32 runs on the any-layout FMA kernels.
 //
 // One workgroup (4 waves, 2 x 2) owns one 128 x 128 output tile that never straddles two experts; each wave a
@@ -7,8 +7,8 @@
 // operands stored [k][row] so that an MFMA operand (lane = row, lanes 32..63 the second k) is one conflict-free
 // ds_read_b32.  Global loads are 16 bytes per thread, fetched into registers one slice ahead of the MFMAs; an
 // operand with contiguous contraction axis is transposed on its way into LDS.  The fp32 matrix pipe is 16 times
-// slower than the bf16 one, so this simple pipeline already keeps it busy.  Launches of fewer such tiles than CUs go in
-// tiles of 32 x 32 instead (s2s_f32_small_kernel, xty_f32_small_kernel).
+// slower than the bf16 one, so this simple pipeline already keeps it busy.  Launches of fewer such tiles than CUs, and
+// operands whose rows are not 16-byte aligned, go in tiles of 32 x 32 instead (s2s_f32_small_kernel, xty_f32_small_kernel).
 //
 // Counterparts in the reference: _scatter2scatter (scattermoe/kernels/ops.py:50-118) and _groupXtY
 // (ops.py:242-366) with float32 tensors (where Triton would use TF32 products under ALLOW_TF32).
@@ -183,13 +183,17 @@ __global__ __launch_bounds__(FNT) void s2s_f32_kernel(S2SArgs a, int n_tiles) {
 // ascending order.  (2 x 2 waves of 32 x 32, the whole contraction each: 1.3 to 2.5 times slower up to 256 tiles of 128 x 128.)
 // Which contraction element an operand's register holds is free as long as both agree: lane half h of chunk c, register s holds
 // element 8 c + 4 h + s, so that an operand with contiguous contraction is one 16-byte load per lane and chunk.
-// us, 128 x 128 tiles -> 32 x 32 (8 experts): 64 rows each, 128 -> 256 21.8 -> 6.0, 256 -> 128 34.5 -> 6.9, weight gradient
-// 11.7 -> 5.8; 112 rows, 600 -> 1200 69 -> 32; 700 rows, 512 -> 512 62 -> 55; 34 rows, 100 -> 100 19.3 -> 5.1.
+// us, 128 x 128 tiles -> 32 x 32 (8 experts): 64 rows each, 128 -> 256 22.7 -> 5.2, 256 -> 128 34.5 -> 6.6, weight gradient
+// 11.7 -> 5.3; 112 rows, 600 -> 1200 70 -> 36, 1200 -> 600 124 -> 35; 583 rows, 512 -> 512 62 -> 44; 34 rows, 100 -> 100
+// 19.5 -> 5.4.
 static constexpr int SMALL = 32, SMALL_WAVES = FNT / 64;
 // The line: products up to 256 expected tiles of 128 x 128 (192 62 -> 55, 320 141 -> 129, 448 115 -> 118 and 96 -> 113), weight
 // gradients, of which both operands come a float per lane and load, up to 128 (64 13.5 -> 9.5 and, of 12 rows, 8.2 -> 7.9; 128
-// 17.0 -> 16.6, of 583 rows 57 -> 51; 192 21 -> 30).
+// 17.2 -> 14.7, of 583 rows 58 -> 49; 192 21 -> 30).  Rows that are not 16-byte aligned: always, in place of the any-layout
+// kernels (8 x 410 rows, 682 -> 512 137 -> 45, its weight gradient 158 -> 51).
 static constexpr int64_t S2S_SMALL_TILES = 256, XTY_SMALL_TILES = 128;
+
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));      // 16-byte loads need dword alignment only
 
 template <bool KC>
 struct LaneOp {
@@ -202,20 +206,25 @@ struct LaneOp {
   }
   // contraction elements [k0, k0 + STEP); from `kend` on zeros (nothing is read there)
   __device__ __forceinline__ void load(int k0, int kend, f32x4 (&v)[CHUNKS]) const {
-    const int h4 = (lane_id() >> 5) * 4;
+    if (k0 + STEP <= kend) {
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-      const int k = k0 + 8 * c + h4;
-      if constexpr (KC) {
-        v[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (k < kend) v[c] = *(const f32x4*)(p + k0 + 8 * c);
-      } else {
+      for (int c = 0; c < CHUNKS; ++c) {
+        if constexpr (KC) {
+          v[c] = *(const f32x4_any*)(p + k0 + 8 * c);
+        } else {
+#pragma unroll
+          for (int s = 0; s < 4; ++s) v[c][s] = p[(int64_t)(k0 + 8 * c + s) * ld];
+        }
+      }
+    } else {
+      const int k = k0 + (lane_id() >> 5) * 4;
+#pragma unroll
+      for (int c = 0; c < CHUNKS; ++c)
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           v[c][s] = 0.0f;
-          if (k + s < kend) v[c][s] = p[(int64_t)(k0 + 8 * c + s) * ld];
+          if (k + 8 * c + s < kend) v[c][s] = p[(int64_t)(k0 + 8 * c + s) * ld];
         }
-      }
     }
   }
 };
@@ -228,8 +237,10 @@ __device__ __forceinline__ void lane_product(const AOp& A, const BOp& B, int k_l
   B.load(k_lo, k_hi, b);
   for (int k0 = k_lo; k0 < k_hi; k0 += AOp::STEP) {
     f32x4 na[CH], nb[CH];
-    A.load(k0 + AOp::STEP, k_hi, na);
-    B.load(k0 + AOp::STEP, k_hi, nb);
+    if (k0 + AOp::STEP < k_hi) {
+      A.load(k0 + AOp::STEP, k_hi, na);
+      B.load(k0 + AOp::STEP, k_hi, nb);
+    }
 #pragma unroll
     for (int c = 0; c < CH; ++c)
 #pragma unroll
@@ -291,20 +302,19 @@ __global__ __launch_bounds__(FNT) void s2s_f32_small_kernel(S2SArgs a, int n_til
 static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 bool try_s2s_f32(const S2SArgs& a, hipStream_t st, int& rc) {
-  if (a.glu != 0) return false;
-  if (a.sxk != 1 || a.syn != 1 || a.K % 4 != 0 || a.sxm % 4 != 0 || !al16(a.X) || !al16(a.W) || a.swe % 4 != 0)
-    return false;
-  bool w_kc;
-  if (a.swk == 1 && a.swn % 4 == 0) w_kc = true;
-  else if (a.swn == 1 && a.swk % 4 == 0 && a.N % 4 == 0) w_kc = false;
-  else return false;
+  if (a.glu != 0 || a.sxk != 1 || a.syn != 1 || (a.swk != 1 && a.swn != 1)) return false;
+  bool w_kc = a.swk == 1 && a.swn % 4 == 0;
+  const bool aligned = a.K % 4 == 0 && a.sxm % 4 == 0 && al16(a.X) && al16(a.W) && a.swe % 4 == 0 &&
+                       (w_kc || (a.swn == 1 && a.swk % 4 == 0 && a.N % 4 == 0));
   const int n_tiles = (a.N + FBN - 1) / FBN;
   // (an expert's last tile is half full on average)
-  if ((cdiv64(a.L, FBM) + a.E / 2) * n_tiles <= S2S_SMALL_TILES) {
+  if (!aligned || (cdiv64(a.L, FBM) + a.E / 2) * n_tiles <= S2S_SMALL_TILES) {
+    if (!aligned) w_kc = a.swk == 1;
     const int cols = (a.N + SMALL - 1) / SMALL;
-    const dim3 grid((unsigned)(max_tiles(a.L, a.E, SMALL) * cols));
-    if (w_kc) hipLaunchKernelGGL(s2s_f32_small_kernel<true>, grid, dim3(FNT), 0, st, a, cols);
-    else hipLaunchKernelGGL(s2s_f32_small_kernel<false>, grid, dim3(FNT), 0, st, a, cols);
+    const int64_t grid = max_tiles(a.L, a.E, SMALL) * cols;
+    if (grid > 0x7fffffffLL) return false;
+    if (w_kc) hipLaunchKernelGGL(s2s_f32_small_kernel<true>, dim3((unsigned)grid), dim3(FNT), 0, st, a, cols);
+    else hipLaunchKernelGGL(s2s_f32_small_kernel<false>, dim3((unsigned)grid), dim3(FNT), 0, st, a, cols);
     rc = launch_status("s2s_f32_small_kernel");
     return true;
   }
@@ -417,8 +427,14 @@ __global__ __launch_bounds__(256) void colsum_f32_kernel(const float* __restrict
   const int n = (blockIdx.x * 64 + c4) * 4;
   const int r_lo = e ? (int)off[e - 1] : 0, r_hi = (int)off[e];
   f32x4 s = {0.f, 0.f, 0.f, 0.f};
-  if (n < N)
-    for (int r = r_lo + rg; r < r_hi; r += 4) s += *(const f32x4*)(DY + (int64_t)r * ld + n);
+  if (n + 3 < N) {
+    for (int r = r_lo + rg; r < r_hi; r += 4) s += *(const f32x4_any*)(DY + (int64_t)r * ld + n);
+  } else {
+    for (int r = r_lo + rg; r < r_hi; r += 4)
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        if (n + q < N) s[q] += DY[(int64_t)r * ld + n + q];
+  }
 #pragma unroll
   for (int q = 0; q < 4; ++q) part[rg][c4 * 4 + q] = s[q];
   __syncthreads();
@@ -429,25 +445,30 @@ __global__ __launch_bounds__(256) void colsum_f32_kernel(const float* __restrict
 
 bool try_xty_f32(const XtYArgs& a, hipStream_t st, int& rc) {
   rc = 0;
-  if (a.sdyn != 1 || a.sxk != 1 || a.sdym % 4 != 0 || a.sxm % 4 != 0 || a.K % 4 != 0 || a.N % 4 != 0) return false;
-  if (!al16(a.DY) || !al16(a.X) || !al16(a.DW) || a.sdwe % 4 != 0) return false;
+  if (a.sdyn != 1 || a.sxk != 1 || (a.sdwk != 1 && a.sdwn != 1)) return false;
+  const bool nk = a.sdwk == 1;                     // output rows = N index, K contiguous; else rows = K index, N contiguous
+  const bool aligned = a.sdym % 4 == 0 && a.sxm % 4 == 0 && a.K % 4 == 0 && a.N % 4 == 0 && al16(a.DY) && al16(a.X) &&
+                       al16(a.DW) && a.sdwe % 4 == 0 && (nk ? a.sdwn : a.sdwk) % 4 == 0;
+  if (!aligned && a.E > 65535) return false;       // (the bias gradient's grid)
   XtYPlanF32 p;
-  if (a.sdwk == 1 && a.sdwn % 4 == 0) {            // output rows = N index, K contiguous
+  if (nk) {
     p.P = (const float*)a.DY; p.ldp = a.sdym; p.np = a.N;
     p.Q = (const float*)a.X; p.ldq = a.sxm; p.nq = a.K;
     p.sop = a.sdwn;
-  } else if (a.sdwn == 1 && a.sdwk % 4 == 0) {     // output rows = K index, N contiguous
+  } else {
     p.P = (const float*)a.X; p.ldp = a.sxm; p.np = a.K;
     p.Q = (const float*)a.DY; p.ldq = a.sdym; p.nq = a.N;
     p.sop = a.sdwk;
-  } else return false;
+  }
   p.OUT = (float*)a.DW; p.soe = a.sdwe; p.off = a.off;
   const int p_tiles = (p.np + FBM - 1) / FBM, q_tiles = (p.nq + FBN - 1) / FBN;
   const int64_t grid = (int64_t)a.E * p_tiles * q_tiles;
   if (grid > 0x7fffffffLL) { set_error("smoe_groupXtY: grid too large"); rc = SMOE_ERR_RANGE; return true; }
-  if (grid > 0 && grid <= XTY_SMALL_TILES) {
+  if (grid > 0 && (!aligned || grid <= XTY_SMALL_TILES)) {
     const int pt = (p.np + SMALL - 1) / SMALL, qt = (p.nq + SMALL - 1) / SMALL;
-    hipLaunchKernelGGL(xty_f32_small_kernel, dim3((unsigned)(a.E * pt * qt)), dim3(FNT), 0, st, p, pt, qt);
+    const int64_t small = (int64_t)a.E * pt * qt;
+    if (small > 0x7fffffffLL) return false;
+    hipLaunchKernelGGL(xty_f32_small_kernel, dim3((unsigned)small), dim3(FNT), 0, st, p, pt, qt);
     rc = launch_status("xty_f32_small_kernel");
     if (rc != 0) return true;
   } else if (grid > 0) {

@@ -29,7 +29,7 @@ def _inputs(K, N, k, seed=0):
 
 
 @pytest.mark.parametrize("n_contig", [False, True])
-@pytest.mark.parametrize("K,N", [(4, 4), (28, 36), (32, 32), (36, 64), (100, 100), (132, 28), (260, 96), (600, 132)])
+@pytest.mark.parametrize("K,N", [(4, 4), (28, 36), (32, 32), (36, 64), (100, 100), (132, 28), (260, 96), (600, 132), (1, 1), (3, 5), (35, 66), (101, 133), (682, 31)])
 def test_products(K, N, n_contig):
     g, E, L, eid, idx, off, X, W, b = _inputs(K, N, 4)
     W = W.contiguous() if n_contig else W
@@ -45,7 +45,7 @@ def test_products(K, N, n_contig):
 
 
 @pytest.mark.parametrize("layout", ["nk", "kn"])
-@pytest.mark.parametrize("K,N", [(4, 36), (32, 32), (100, 132), (128, 256)])
+@pytest.mark.parametrize("K,N", [(4, 36), (32, 32), (100, 132), (128, 256), (1, 3), (33, 35), (101, 682)])
 def test_weight_gradients(K, N, layout):
     g, E, L, eid, idx, off, X, W, b = _inputs(K, N, 1)
     DY = torch.randn(L, N, generator=g, device=DEV)
@@ -57,6 +57,27 @@ def test_weight_gradients(K, N, layout):
         _check(DW[e], x.t() @ y, x.abs().t() @ y.abs(), hi - lo)
         _check(Db[e], y.sum(0), y.abs().sum(0), hi - lo)
         lo = hi
+
+
+def test_unaligned_operands():
+    """Operands and outputs that begin one element into wider matrices; more tiles than the aligned ones may have."""
+    for K, N in ((68, 3300), (67, 3301)):
+        g, E, L, eid, idx, off, X, W, b = _inputs(K + 1, N + 1, 1)
+        X, W = X[:, 1:], W[:, 1:, 1:]
+        DY = torch.randn(L, N + 1, generator=g, device=DEV)[:, 1:]
+        out = torch.full((L, N + 1), 7.0, device=DEV)
+        ops.scatter2scatter(X, W, eid, idx, 1, x_grouped=True, y_grouped=True, expert_offsets=off, out=out[:, 1:])
+        dx = ops.scatter2scatter(DY, W.permute(0, 2, 1), eid, idx, 1, x_grouped=True, y_grouped=True, expert_offsets=off)
+        DW, Db = ops.group_bwd_W(DY, X, off, E, has_bias=True)
+        assert bool((out[:, 0] == 7.0).all())
+        lo = 0
+        for e, hi in enumerate(off.tolist()):
+            x, w, y = X[lo:hi].double(), W[e].double(), DY[lo:hi].double()
+            _check(out[lo:hi, 1:], x @ w, x.abs() @ w.abs(), K)
+            _check(dx[lo:hi], y @ w.t(), y.abs() @ w.t().abs(), N)
+            _check(DW[e], x.t() @ y, x.abs().t() @ y.abs(), hi - lo)
+            _check(Db[e], y.sum(0), y.abs().sum(0), hi - lo)
+            lo = hi
 
 
 def test_infinities_stay_with_their_rows():
