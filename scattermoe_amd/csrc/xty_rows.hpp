@@ -77,8 +77,10 @@ __device__ __forceinline__ void xty_rows_unit(const XtYPlan& a, int e, int r_lo,
   };
   auto rsrc_of = [&](auto gathered, const void* base, int64_t ld, int cols) {
     const bool g = decltype(gathered)::value;
-    const int64_t n = g ? a.x_rows : rows;
-    return buffer_rsrc((const char*)base + (g ? 0 : (int64_t)r_lo * ld * 2), n > 0 ? (unsigned)(((n - 1) * ld + cols) * 2) : 0u);
+    // (an expert without rows reads none, its lanes being out of any range; one row's range all the same, as the bounds
+    // check may take a step's scalar offset off the range and must not wrap around)
+    const int64_t n = max((int64_t)1, g ? a.x_rows : (int64_t)rows);
+    return buffer_rsrc((const char*)base + (g ? 0 : (int64_t)r_lo * ld * 2), (unsigned)(((n - 1) * ld + cols) * 2));
   };
 
   // ---- the held operand: two slices at a time through LDS, then as fragments in registers
