@@ -364,6 +364,109 @@ struct TransOp {
   }
 };
 
+// 16 bytes per lane from global memory into LDS through a buffer descriptor: as load_to_lds16, but a lane whose offset lies
+// beyond the descriptor's range reads zeros (the rows behind an expert's last one, without a branch and without a second
+// write to LDS).  `soff`: a scalar byte offset on top of the lanes' own.
+__device__ __forceinline__ void buffer_to_lds16(i32x4 rsrc, unsigned off, unsigned soff, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"(lds_addr), "v"(off), "s"(rsrc), "s"(soff)
+               : "memory", "m0");
+}
+__device__ __forceinline__ i32x4 buffer_rsrc(const void* base, unsigned bytes) {
+  const uint64_t v = (uint64_t)base;
+  i32x4 r = {(int)__builtin_amdgcn_readfirstlane((unsigned)v), (int)__builtin_amdgcn_readfirstlane((unsigned)(v >> 32)),
+             (int)__builtin_amdgcn_readfirstlane(bytes), 0x00020000};
+  asm volatile("s_nop 4" : "+s"(r));      // an assembly load may follow: five wait states behind the instructions above
+  return r;
+}
+
+// A lane offset that every descriptor of a weight gradient's gathered or short operand rejects, with any instruction or scalar offset on top of it (ranges stay
+// below 2 GiB: the launchers check).
+static constexpr unsigned OUT_OF_RANGE = 0x80000000u;
+// ---- operand with strided contraction axis whose contraction may end anywhere (weight gradients of mainloop_pair) --------
+// The LDS layout of TransOp, filled through a buffer descriptor that ends with the last contraction row: what lies behind it
+// reads as zeros, without a pass over LDS afterwards.  GATHER: row r of the operand is row rows[r] / fan of the source matrix;
+// lane t of every wave looks up row t of a slice, two slices ahead of its loads (fetch_rows, an ordinary load that the main
+// loop's wait covers), turns it into a byte offset while the slice before is multiplied (stage_rows), and the lanes pick the
+// offsets of their own pieces from each other (take_rows): no LDS, no barrier.
+template <int EXT, int NT, bool GATHER>
+struct RowsOp {
+  typedef TransOp<EXT, NT> Layout;
+  static constexpr int R = Layout::R, LDS_BYTES = Layout::LDS_BYTES, DS_PER_FRAG = Layout::DS_PER_FRAG, CPR = Layout::CPR;
+  static_assert(NT / CPR % 4 == 0, "one column offset per thread");
+  const char* base;        // wave-uniform: (contraction 0, column 0 of the tile); GATHER: of the source matrix
+  i32x4 rsrc;              // of the slice to be issued next
+  unsigned off[R];
+  unsigned ld, colb;       // bytes
+  int klen;
+  // GATHER only
+  const int64_t* rows;
+  unsigned fan, next_row, row_off;
+  __device__ __forceinline__ void init_cols(const char* b, int64_t ld_bytes, int valid_cols, int k) {
+    base = make_uniform(b);
+    ld = (unsigned)ld_bytes;
+    klen = k;
+    const int kr = (int)threadIdx.x / CPR, phys = (int)threadIdx.x % CPR;
+    const int tc = ((((phys >> 2) ^ (kr & 3)) << 2) | (phys & 3)) * 8;
+    colb = tc < valid_cols ? tc * 2 : 0;                   // (such columns only feed outputs that are never stored)
+  }
+  __device__ __forceinline__ void init(const char* b, int64_t ld_bytes, int valid_cols, int k) {
+    init_cols(b, ld_bytes, valid_cols, k);
+#pragma unroll
+    for (int j = 0; j < R; ++j) off[j] = (unsigned)((j * NT + (int)threadIdx.x) / CPR) * ld + colb;
+    take_rows(0);
+  }
+  // `span`: bytes from `b` to the end of the source matrix
+  __device__ __forceinline__ void init_gather(const char* b, int64_t ld_bytes, int valid_cols, int k, const int64_t* r,
+                                              int fan_out, unsigned span) {
+    init_cols(b, ld_bytes, valid_cols, k);
+    rows = r;
+    fan = (unsigned)fan_out;
+    next_row = 0;
+    rsrc = buffer_rsrc(base, span);
+    fetch_rows(0);
+    const unsigned first = next_row;
+    fetch_rows(BK);
+    const unsigned second = next_row;
+    fetch_rows(2 * BK);
+    const unsigned third = next_row;
+    next_row = first;
+    stage_rows(0);
+    take_rows(0);
+    next_row = second;
+    stage_rows(1);
+    next_row = third;
+  }
+  // row indices of the slice at contraction k0
+  __device__ __forceinline__ void fetch_rows(int k0) {
+    if constexpr (GATHER) {
+      const int r = k0 + lane_id();
+      if (r < klen) next_row = (unsigned)rows[r];
+    }
+  }
+  // what has been fetched becomes the offsets of slice number `slice`
+  __device__ __forceinline__ void stage_rows(int slice) {
+    if constexpr (GATHER) row_off = slice * BK + lane_id() < klen ? next_row / fan * ld : OUT_OF_RANGE;
+  }
+  // slice number `slice` is the next to be issued
+  __device__ __forceinline__ void take_rows(int slice) {
+    if constexpr (GATHER) {
+      asm volatile("" : "+v"(next_row));                   // (the compiler's wait for it: here, with nothing in flight)
+#pragma unroll
+      for (int j = 0; j < R; ++j)
+        off[j] = (unsigned)__builtin_amdgcn_ds_bpermute((j * NT + (int)threadIdx.x) / CPR * 4, (int)row_off) + colb;
+    } else {
+      const int left = klen - slice * BK;
+      rsrc = buffer_rsrc(base + (int64_t)slice * BK * ld, left > 0 ? (unsigned)min(left, BK) * ld : 0u);
+    }
+  }
+  __device__ __forceinline__ void issue_one(unsigned tile, int, int j) const {
+    buffer_to_lds16(rsrc, off[j], 0, tile + wave_uniform_id() * 1024 + j * NT * 16);
+  }
+  static __device__ __forceinline__ i32x4 frag(const char* tile, int b, int ks) { return Layout::frag(tile, b, ks); }
+};
+
 // One slice of both operands, load slots interleaved (A0 B0 A1 B1 ...) so that the rows each operand starts
 // with (see `rot`) are requested first.
 template <class AOp, class BOp>
@@ -661,16 +764,18 @@ __device__ __forceinline__ void mainloop_rs(const AOp& A, const BOp& B, int klen
 // fragments of a whole slice are read into registers (32 of them) ahead of the products, so that the next slice's pieces
 // can be on their way into the same stage while they run.  The burst of reads and the two barriers around it fall into the
 // other workgroup's products.
-// Whole 64-deep slices only (the launcher checks).
+// Whole 64-deep slices only (the launcher checks), or operands that read as zeros behind their last contraction row (RowsOp).
+// `rowsum` and rs as in mainloop.
 static constexpr int PAIR_STAGE = 32 * 1024, PAIR_B = 2 * PAIR_STAGE, PAIR_LDS = PAIR_B + 16 * 1024;
-template <typename T, class TL, class AOp, class BOp>
-__device__ __forceinline__ void mainloop_pair(const AOp& A, const BOp& B, int klen, char* lds, f32x16 (&acc)[TL::FM][TL::FN]) {
+template <typename T, class TL, class AOp, class BOp, bool ROWS>
+__device__ __forceinline__ void mainloop_pair(AOp& A, BOp& B, int klen, char* lds, bool rowsum, f32x16 (&acc)[TL::FM][TL::FN],
+                                              float (&rs)[TL::FM]) {
   static_assert(AOp::LDS_BYTES <= PAIR_STAGE && BOp::LDS_BYTES <= PAIR_LDS - PAIR_B, "LDS");
   constexpr int KS = BK / 16, LOADS = AOp::R + BOp::R, PER_STEP = (LOADS + KS - 2) / (KS - 1);      // (all of them up front: 2 % slower)
   const int wave = threadIdx.x >> 6;
   const int wm = wave / TL::WN, wn = wave % TL::WN;
   const unsigned lds_u = lds_address(lds);
-  const int nk = klen / BK;
+  const int nk = ROWS ? max(1, (klen + BK - 1) / BK) : klen / BK;      // (no rows: one slice of zeros)
 #pragma unroll
   for (int j = 0; j < BOp::R; ++j) B.issue_one(lds_u + PAIR_B, 0, j);
 #pragma unroll
@@ -683,6 +788,10 @@ __device__ __forceinline__ void mainloop_pair(const AOp& A, const BOp& B, int kl
     // this thread's pieces of slice kt have landed, everyone's have, and everyone is done with slice kt - 1
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (ROWS && decltype(more)::value) {
+      A.take_rows(kt + 1);
+      B.take_rows(kt + 1);
+    }
     i32x4 fa[2][TL::FM], fb[KS][TL::FN];
 #pragma unroll
     for (int j = 0; j < TL::FN; ++j) fb[0][j] = BOp::frag(tb, wn * TL::WTN + j * 32, 0);
@@ -705,6 +814,16 @@ __device__ __forceinline__ void mainloop_pair(const AOp& A, const BOp& B, int kl
           if (q < BOp::R) B.issue_one(lds_u + PAIR_B, (kt + 1) * BK, q);
           else A.issue_one(na, (kt + 1) * BK, q - BOp::R);
         }
+        if constexpr (ROWS) {
+          if (ks == 1) {
+            A.stage_rows(kt + 2);
+            B.stage_rows(kt + 2);
+          }
+          if (ks == KS - 1) {
+            A.fetch_rows((kt + 3) * BK);
+            B.fetch_rows((kt + 3) * BK);
+          }
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
       if (ks + 1 < KS) {
@@ -715,6 +834,10 @@ __device__ __forceinline__ void mainloop_pair(const AOp& A, const BOp& B, int kl
       for (int i = 0; i < TL::FM; ++i)
 #pragma unroll
         for (int j = 0; j < TL::FN; ++j) acc[i][j] = Mfma<T>::run(fb[ks][j], fa[c][i], acc[i][j]);
+      if (ROWS && rowsum) {
+#pragma unroll
+        for (int i = 0; i < TL::FM; ++i) rs[i] += Mfma<T>::sum8(fa[c][i]);
+      }
       if (ks + 1 < KS) {
 #pragma unroll
         for (int i = 0; i < TL::FM; ++i) {
@@ -1487,7 +1610,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
   if constexpr (TL::RS) mainloop_rs<T, TL, AOp, BOp>(A, B, a.K, lds, acc);
-  else if constexpr (TL::PAIR) mainloop_pair<T, TL, AOp, BOp>(A, B, a.K, lds, acc);
+  else if constexpr (TL::PAIR) mainloop_pair<T, TL, AOp, BOp, false>(A, B, a.K, lds, false, acc, rs);
   else if constexpr (TL::NS > 2) mainloop_ring<T, TL, AOp, BOp>(A, B, t.klen, lds, acc);
   else mainloop<T, TL, AOp, BOp, false>(A, B, a.K, lds, false, acc, rs);
 
@@ -1980,20 +2103,31 @@ struct XtYPlan {
 template <typename T, class TL, bool GA, bool GB>
 __device__ __forceinline__ void xty_tile(const XtYPlan& a, int e, int p0, int q0, char* lds, int64_t* sDst, unsigned* sRows,
                                          float* sBias) {
-  typedef TransOp<TL::BM, TL::NT, false, GA> AOp;
-  typedef TransOp<TL::BN, TL::NT, false, GB> BOp;
+  typedef std::conditional_t<TL::PAIR, RowsOp<TL::BM, TL::NT, GA>, TransOp<TL::BM, TL::NT, false, GA>> AOp;
+  typedef std::conditional_t<TL::PAIR, RowsOp<TL::BN, TL::NT, GB>, TransOp<TL::BN, TL::NT, false, GB>> BOp;
   const int r_lo = e ? (int)a.off[e - 1] : 0;
   const int r_hi = (int)a.off[e];
 
-  for (int m = threadIdx.x; m < TL::BM; m += TL::NT)
-    sDst[m] = (p0 + m < a.np) ? (int64_t)e * a.soe + (int64_t)(p0 + m) * a.sop : -1;
-  __syncthreads();
+  auto output_rows = [&] {
+    for (int m = threadIdx.x; m < TL::BM; m += TL::NT)
+      sDst[m] = (p0 + m < a.np) ? (int64_t)e * a.soe + (int64_t)(p0 + m) * a.sop : -1;
+    __syncthreads();
+  };
+  if constexpr (!TL::PAIR) output_rows();
 
   AOp A;
-  if constexpr (GA) A.init_gather((const char*)a.P + (int64_t)p0 * 2, a.ldp * 2, a.np - p0, a.idx + r_lo, a.fan_out, r_hi - r_lo, sRows);
+  if constexpr (TL::PAIR && GA)
+    A.init_gather((const char*)a.P + (int64_t)p0 * 2, a.ldp * 2, a.np - p0, r_hi - r_lo, a.idx + r_lo, a.fan_out,
+                  (unsigned)(((max(a.x_rows, (int64_t)1) - 1) * a.ldp + a.np - p0) * 2));
+  else if constexpr (TL::PAIR) A.init((const char*)a.P + ((int64_t)r_lo * a.ldp + p0) * 2, a.ldp * 2, a.np - p0, r_hi - r_lo);
+  else if constexpr (GA) A.init_gather((const char*)a.P + (int64_t)p0 * 2, a.ldp * 2, a.np - p0, a.idx + r_lo, a.fan_out, r_hi - r_lo, sRows);
   else A.init((const char*)a.P + ((int64_t)r_lo * a.ldp + p0) * 2, a.ldp * 2, a.np - p0);
   BOp B;           // (rotated load order measured 1.5 % slower here, so both operands keep rot = 0)
-  if constexpr (GB) B.init_gather((const char*)a.Q + (int64_t)q0 * 2, a.ldq * 2, a.nq - q0, a.idx + r_lo, a.fan_out, r_hi - r_lo, sRows);
+  if constexpr (TL::PAIR && GB)
+    B.init_gather((const char*)a.Q + (int64_t)q0 * 2, a.ldq * 2, a.nq - q0, r_hi - r_lo, a.idx + r_lo, a.fan_out,
+                  (unsigned)(((max(a.x_rows, (int64_t)1) - 1) * a.ldq + a.nq - q0) * 2));
+  else if constexpr (TL::PAIR) B.init((const char*)a.Q + ((int64_t)r_lo * a.ldq + q0) * 2, a.ldq * 2, a.nq - q0, r_hi - r_lo);
+  else if constexpr (GB) B.init_gather((const char*)a.Q + (int64_t)q0 * 2, a.ldq * 2, a.nq - q0, a.idx + r_lo, a.fan_out, r_hi - r_lo, sRows);
   else B.init((const char*)a.Q + ((int64_t)r_lo * a.ldq + q0) * 2, a.ldq * 2, a.nq - q0);
 
   f32x16 acc[TL::FM][TL::FN];
@@ -2008,9 +2142,11 @@ __device__ __forceinline__ void xty_tile(const XtYPlan& a, int e, int p0, int q0
   }
   const bool want_db = a.Db != nullptr && a.db_from_p && q0 == 0;
   if constexpr (TL::RS) mainloop_rs<T, TL, AOp, BOp>(A, B, r_hi - r_lo, lds, acc);      // no bias gradient, no gather
+  else if constexpr (TL::PAIR) mainloop_pair<T, TL, AOp, BOp, true>(A, B, r_hi - r_lo, lds, want_db, acc, rs);
   else mainloop<T, TL, AOp, BOp, true>(A, B, r_hi - r_lo, lds, want_db, acc, rs);
+  if constexpr (TL::PAIR) output_rows();                 // (into the column stage, which nobody reads any more)
 
-  if (TL::RS || ((((uintptr_t)a.OUT & 15) == 0) && ((a.soe | a.sop | a.nq) & 7) == 0))
+  if (TL::RS || TL::PAIR || ((((uintptr_t)a.OUT & 15) == 0) && ((a.soe | a.sop | a.nq) & 7) == 0))
     epilogue_staged<T, TL>(acc, (T*)a.OUT, sDst, q0, a.nq, nullptr, 0, lds, sBias);
   else
     epilogue<T, TL>(acc, (T*)a.OUT, sDst, q0, a.nq, nullptr, 0);
@@ -2038,12 +2174,85 @@ struct XtYLds {
   __attribute__((aligned(16))) float bias[TL::RS ? TL::BN : 4];
 };
 
+// Order of a launch's tiles: super tiles (Raster) while the experts' loads are alike.  A tile costs its expert's rows, and the
+// workgroup of index i runs on XCD i % 8 whatever else that one has to do: where an expert has more than twice the average
+// rows, every XCD takes an eighth of every expert's tiles, one contiguous piece in bands of `band` columns, the experts with
+// the most rows first.  In super tiles one XCD has all its CUs in the heaviest expert while others have none of its tiles
+// (us, super tiles -> this: 32 experts, 1 / rank^1.8 of 32768 rows, 2880 x 2880 256 x 256 tiles 877 -> 627, 256 x 128 915 ->
+// 582, 128 x 128 652 -> 591; 2880 x 5760 gathered 1541 -> 1266, 1576 -> 1290, 1385 -> 1293).  Even loads keep the super tiles:
+// an expert's rows shared by all XCDs are read by each of them (128 x 2048 rows, 2048 x 1536 1600 -> 1640; 64 x 400,
+// 1024 x 2048 138 -> 148).
+struct XtYOrder {
+  static constexpr int GROUPS = 4;         // more than 256 experts: always super tiles
+  Raster rast;
+  int p_tiles, q_tiles, band, chunk;       // chunk: tiles of an expert per XCD
+  template <int SN>
+  __device__ __forceinline__ bool map(const XtYPlan& a, int pid, int& e, int& m, int& n) const {
+    const int lane = lane_id();
+    int rows[GROUPS];
+    bool uneven = false;
+    if (a.E <= 64 * GROUPS) {
+      const int64_t L = a.off[a.E - 1];
+#pragma unroll
+      for (int g = 0; g < GROUPS; ++g) {
+        const int c = g * 64 + lane;
+        rows[g] = -1;
+        if (g * 64 < a.E && c < a.E) rows[g] = (int)(a.off[c] - (c ? a.off[c - 1] : 0));
+        uneven = uneven || __ballot((int64_t)rows[g] * a.E > 2 * L) != 0;
+      }
+    }
+    if (!uneven) {
+      int m_tile, m_loc, n_loc;
+      if (!rast.map<SN>(pid, m_tile, n, m_loc, n_loc)) return false;
+      e = __builtin_amdgcn_readfirstlane(m_tile / p_tiles);
+      m = m_tile - e * p_tiles;
+      return true;
+    }
+    const int x = pid & 7, i = pid >> 3;
+    int nth = __builtin_amdgcn_readfirstlane(i / chunk);
+    const int t = ((x + nth) & 7) * chunk + (i - nth * chunk);
+    if (nth >= a.E || t >= p_tiles * q_tiles) return false;
+    // the nth expert by the size of its load, in half powers of two
+    int size[GROUPS], most = 0;
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+      const int lg = 31 - __clz(max(rows[g], 1));
+      size[g] = rows[g] < 0 ? -1 : 2 * lg + (lg > 0 ? (rows[g] >> (lg - 1)) & 1 : 0);
+      most = max(most, size[g]);
+    }
+    e = 0;
+    for (int s = __builtin_amdgcn_readfirstlane(wave_max(most)); s >= 0 && nth >= 0; --s) {
+#pragma unroll
+      for (int g = 0; g < GROUPS; ++g) {
+        const unsigned long long q = __ballot(size[g] == s);
+        const int have = __popcll(q);
+        if (nth >= 0 && nth < have)
+          e = g * 64 + __ffsll((long long)__ballot(size[g] == s && __popcll(q & ((1ull << lane) - 1)) == nth)) - 1;
+        nth -= have;
+      }
+    }
+    e = __builtin_amdgcn_readfirstlane(e);
+    const int per_band = p_tiles * band;
+    const int b = __builtin_amdgcn_readfirstlane(t / per_band);
+    const int width = min(band, q_tiles - b * band), in = t - b * per_band;
+    m = __builtin_amdgcn_readfirstlane(in / width);
+    n = b * band + in - m * width;
+    return true;
+  }
+};
+
 template <typename T, class TL, bool GA, bool GB>
-__global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void xty_mfma_kernel(XtYPlan a, Raster rast, int p_tiles) {
-  __shared__ XtYLds<TL> s;
-  int m_tile, n_tile, m_loc, n_loc;
-  if (!rast.map(blockIdx.x, m_tile, n_tile, m_loc, n_loc)) return;
-  xty_tile<T, TL, GA, GB>(a, m_tile / p_tiles, (m_tile % p_tiles) * TL::BM, n_tile * TL::BN, s.lds, s.dst, s.rows, s.bias);
+__global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void xty_mfma_kernel(XtYPlan a, XtYOrder order) {
+  int e, m, n;
+  if constexpr (TL::PAIR) {
+    __shared__ __attribute__((aligned(16))) char lds[PAIR_LDS];
+    if (!order.map<TL::PAIR ? 2 * Raster::SN : Raster::SN>(a, blockIdx.x, e, m, n)) return;
+    xty_tile<T, TL, GA, GB>(a, e, m * TL::BM, n * TL::BN, lds, (int64_t*)(lds + PAIR_B), nullptr, nullptr);
+  } else {
+    __shared__ XtYLds<TL> s;
+    if (!order.map<TL::PAIR ? 2 * Raster::SN : Raster::SN>(a, blockIdx.x, e, m, n)) return;
+    xty_tile<T, TL, GA, GB>(a, e, m * TL::BM, n * TL::BN, s.lds, s.dst, s.rows, s.bias);
+  }
 }
 
 }  // namespace smoe
@@ -2118,15 +2327,19 @@ template <typename T, class TL>
 static int launch_xty(const XtYArgs& a, hipStream_t st) {
   const bool k_contig = a.sdwk == 1;
   const XtYPlan p = xty_plan(a);
-  const int p_tiles = (p.np + TL::BM - 1) / TL::BM;
-  const int q_tiles = (p.nq + TL::BN - 1) / TL::BN;
-  const Raster r = make_raster((int64_t)a.E * p_tiles, q_tiles, GM_XTY);
-  const int64_t grid = r.grid();
+  XtYOrder r;
+  r.p_tiles = (p.np + TL::BM - 1) / TL::BM;
+  r.q_tiles = (p.nq + TL::BN - 1) / TL::BN;
+  r.band = TL::PAIR ? 2 * Raster::SN : Raster::SN;
+  r.rast = make_raster((int64_t)a.E * r.p_tiles, r.q_tiles, GM_XTY, r.band);
+  const int64_t chunk = ((int64_t)r.p_tiles * r.q_tiles + 7) / 8;
+  const int64_t grid = std::max(r.rast.grid(), chunk * a.E * 8);
   if (grid > 0x7fffffffLL) { set_error("smoe_groupXtY: grid too large"); return SMOE_ERR_RANGE; }
-  if constexpr (TL::RS) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, false>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r, p_tiles);
-  else if (a.idx == nullptr) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, false>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r, p_tiles);
-  else if (k_contig) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, true>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r, p_tiles);
-  else hipLaunchKernelGGL((xty_mfma_kernel<T, TL, true, false>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r, p_tiles);
+  r.chunk = (int)chunk;
+  if constexpr (TL::RS) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, false>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r);
+  else if (a.idx == nullptr) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, false>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r);
+  else if (k_contig) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, true>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r);
+  else hipLaunchKernelGGL((xty_mfma_kernel<T, TL, true, false>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r);
   return launch_status("xty_mfma_kernel");
 }
 
@@ -2194,16 +2407,45 @@ static bool xty_held(const XtYArgs& a) {
   return (int64_t)a.E * ((a.N + 255) / 256) * ((a.K + 255) / 256) >= 256 && xty_rows_fits(xty_plan(a));
 }
 
+// Between them: 256 x 128 tiles, two workgroups per CU (mainloop_pair), or the small tiles again, against eight waves per
+// 256 x 256 tile over 2000 random launches of 257 to 2047 rows per expert (4 to 128 experts, K and N from 256 to 8000, gathered
+// and not; even / Zipf-like loads, each in the order of XtYOrder).  256 x 128, 257 to 700 rows 1.10 / 1.17 times as fast, to 1200
+// 1.06 / 1.14, to 2047 1.03 / 1.11 (beyond 20 rounds of them 0.98 / 1.02, there from 1200 rows on they are not taken); from
+// 2048 rows on, where the operands are gathered or the bias gradient is wanted, only up to two rounds (1.05 / 1.17; beyond
+// 0.95 to 0.99 / 1.05), the one-wave-per-SIMD form otherwise (0.98).  Small tiles against 256 x 128 while the operands
+// come from the memory-side cache, beyond one round: 257 to 700 rows, up to eight rounds 1.07 / 1.02, to 1200 rows, up to four
+// 1.07 / 1.02, to 2047 rows, up to two 1.07 / 1.02.
+// us, 32 experts x 500 rows, 2880 x 2880 346 -> 309; 32 x 300, 2880 x 5760 gathered 504 -> 467; 16 x 1000, 1024 x 1024 35.8 -> 34.4.
+// Same bits in every class.
+static constexpr int XTY_PAIR_ROUND = 2 * NUM_CU;
+static int64_t xty_pair_tiles(const XtYPlan& p) { return (int64_t)p.E * ((p.np + 255) / 256) * ((p.nq + 127) / 128); }
+static bool xty_small_again(const XtYArgs& a) {
+  const int64_t rows = a.L / a.E, tiles = xty_pair_tiles(xty_plan(a));
+  if (rows <= XTY_SMALL_ROWS || rows >= RS_XTY_MIN_ROWS || (int64_t)a.L * (a.N + a.K) * 2 > (256ll << 20)) return false;
+  return tiles > XTY_PAIR_ROUND && tiles <= XTY_PAIR_ROUND * (rows < 700 ? 8 : rows < 1200 ? 4 : 2);
+}
+static bool xty_pairs(const XtYArgs& a, bool rs_form) {
+  const XtYPlan p = xty_plan(a);
+  const int64_t rows = a.L / a.E, tiles = xty_pair_tiles(p);
+  if (rs_form || rows < XTY_STORE_ROWS || tiles > XTY_PAIR_ROUND * (rows >= RS_XTY_MIN_ROWS ? 2 : rows >= 1200 ? 20 : 1 << 20)) return false;
+  // Output pieces of 16 bytes; rows that do not overlap (the descriptors end with the last one) and, gathered, a source below
+  // 2 GiB.
+  if (((uintptr_t)p.OUT & 15) != 0 || ((p.soe | p.sop | p.nq) & 7) != 0 || p.ldp < p.np || p.ldq < p.nq) return false;
+  return a.idx == nullptr || (p.x_rows + 1) * a.sxm + a.K < (1ll << 30);
+}
+
 template <typename T>
 static int dispatch_xty(const XtYArgs& a, bool rs_form, hipStream_t st) {
   typedef Tile<128, 128, 2, 2, 1, false, 4> Small;
   typedef Tile<256, 256, 2, 4> Large;
-  const bool small = xty_idle_chip(a, rs_form) || xty_few_rows(a);
+  const bool small = xty_idle_chip(a, rs_form) || xty_few_rows(a) || xty_small_again(a);
   int rc;
   if (xty_held(a)) {
     rc = launch_xty_rows<T>(xty_plan(a), a.L, st);
   } else if (small) {
     rc = launch_xty<T, Small>(a, st);
+  } else if (xty_pairs(a, rs_form)) {
+    rc = launch_xty<T, PairTile>(a, st);
   } else {
     rc = rs_form ? launch_xty<T, Tile<256, 256, 2, 2, 2, true>>(a, st) : launch_xty<T, Large>(a, st);
   }

@@ -4,26 +4,6 @@
 
 namespace smoe {
 
-// 16 bytes per lane from global memory into LDS through a buffer descriptor: as load_to_lds16, but a lane whose offset lies
-// beyond the descriptor's range reads zeros (the rows behind an expert's last one, without a branch and without a second
-// write to LDS).  `soff`: a scalar byte offset on top of the lanes' own.
-__device__ __forceinline__ void buffer_to_lds16(i32x4 rsrc, unsigned off, unsigned soff, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :
-               : "s"(lds_addr), "v"(off), "s"(rsrc), "s"(soff)
-               : "memory", "m0");
-}
-__device__ __forceinline__ i32x4 buffer_rsrc(const void* base, unsigned bytes) {
-  const uint64_t v = (uint64_t)base;
-  i32x4 r = {(int)__builtin_amdgcn_readfirstlane((unsigned)v), (int)__builtin_amdgcn_readfirstlane((unsigned)(v >> 32)),
-             (int)__builtin_amdgcn_readfirstlane(bytes), 0x00020000};
-  asm volatile("s_nop 4" : "+s"(r));      // an assembly load may follow: five wait states behind the instructions above
-  return r;
-}
-
-// A lane offset that every descriptor of this kernel rejects, with any instruction or scalar offset on top of it (ranges stay
-// below 2 GiB, see xty_rows_fits).
-static constexpr unsigned OUT_OF_RANGE = 0x80000000u;
 static constexpr int XTY_ROWS_MAX = 256;       // rows of an expert whose operand is held: four 64-row slices in registers
 static constexpr int XR_P = 256, XR_Q = 64;    // output rows of a workgroup's panel, output columns of a step
 static constexpr int XR_RING = 64 * 1024, XR_OUT = 16 * 1024;      // LDS of a workgroup, two of them per CU: operand stages, output
