@@ -62,7 +62,9 @@ bool try_xty_mfma(const XtYArgs& a, int dtype, hipStream_t st, int& rc) {
   // (128 experts, 768 x 2048 and 2048 x 1536 outputs) 0.81 -> 0.77 and 1.55 -> 1.51 ms, 1024 rows per expert even.
   const bool out16 = (((uintptr_t)a.DW & 15) == 0) && ((a.sdwe | (a.sdwk == 1 ? a.sdwn : a.sdwk) | (a.sdwk == 1 ? a.K : a.N)) & 7) == 0;
   const bool db_in_loop = a.Db != nullptr && a.sdwk == 1;
-  const bool rs_form = a.idx == nullptr && !db_in_loop && out16 && a.L / a.E >= RS_XTY_MIN_ROWS;
+  // (its buffer descriptors end with an operand's last row: rows that overlap, as those of an expanded tensor, would read as zeros)
+  const bool apart = a.sdym >= a.N && a.sxm >= a.K;
+  const bool rs_form = a.idx == nullptr && !db_in_loop && out16 && apart && a.L / a.E >= RS_XTY_MIN_ROWS;
   rc = dtype == SMOE_BF16 ? dispatch_xty_bf16(a, rs_form, st) : dispatch_xty_f16(a, rs_form, st);
   return true;
 }

@@ -1901,7 +1901,10 @@ static bool takes_pairs(const S2SArgs& a) { return a.K < RS_MIN_K && whole_piece
 
 template <typename T>
 static int launch_main_class(const S2SArgs& a, bool b_tr, hipStream_t st) {
-  if (a.K >= RS_MIN_K && whole_pieces(a))
+  // (its buffer descriptors end with the last row of a strided operand: rows that overlap, as those of an expanded tensor, would
+  // read as zeros)
+  const bool apart = !b_tr || a.swk >= (a.glu == 1 ? 2 : 1) * (int64_t)a.N;
+  if (a.K >= RS_MIN_K && whole_pieces(a) && apart)
     return launch_s2s<T, Tile<256, 256, 2, 2, 2, true>>(a, b_tr, st);
   return launch_s2s<T, Tile<256, 256, 2, 4>>(a, b_tr, st);
 }
