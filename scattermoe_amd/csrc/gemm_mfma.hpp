@@ -2181,10 +2181,11 @@ struct XtYLds {
 // workgroup of index i runs on XCD i % 8 whatever else that one has to do: where an expert has more than twice the average
 // rows, every XCD takes an eighth of every expert's tiles, one contiguous piece in bands of `band` columns, the experts with
 // the most rows first.  In super tiles one XCD has all its CUs in the heaviest expert while others have none of its tiles
-// (us, super tiles -> this: 32 experts, 1 / rank^1.8 of 32768 rows, 2880 x 2880 256 x 256 tiles 877 -> 627, 256 x 128 915 ->
-// 582, 128 x 128 652 -> 591; 2880 x 5760 gathered 1541 -> 1266, 1576 -> 1290, 1385 -> 1293).  Even loads keep the super tiles:
-// an expert's rows shared by all XCDs are read by each of them (128 x 2048 rows, 2048 x 1536 1600 -> 1640; 64 x 400,
-// 1024 x 2048 138 -> 148).
+// (us, super tiles -> this, loads of a router with logits shifted by -1.8 log(rank), experts in any order: 32 experts, 32768 rows,
+// 2880 x 2880 in 256 x 256 tiles 786 -> 626, 256 x 128 723 -> 579, 128 x 128 732 -> 640; 2880 x 5760 gathered 1692 -> 1315, 1582 ->
+// 1210, 1355 -> 1246; 128 experts, 131072 rows, 2048 x 1536 gathered 1562 -> 1034, 1581 -> 1012.  The experts as they come instead
+// of the largest first: 0.8 to 1.04 times as fast).  Even loads keep the super tiles: an expert's rows shared by all XCDs are
+// read by each of them (128 x 2048 rows, 2048 x 1536 1600 -> 1640; 64 x 400, 1024 x 2048 138 -> 148).
 struct XtYOrder {
   static constexpr int GROUPS = 4;         // more than 256 experts: always super tiles
   Raster rast;
@@ -2215,18 +2216,18 @@ struct XtYOrder {
     int nth = __builtin_amdgcn_readfirstlane(i / chunk);
     const int t = ((x + nth) & 7) * chunk + (i - nth * chunk);
     if (nth >= a.E || t >= p_tiles * q_tiles) return false;
-    // the nth expert by the size of its load, in half powers of two
+    // the nth expert by the power of two its load reaches (finer steps and groups that hold no expert cost each tile 1.5 us)
     int size[GROUPS], most = 0;
 #pragma unroll
     for (int g = 0; g < GROUPS; ++g) {
-      const int lg = 31 - __clz(max(rows[g], 1));
-      size[g] = rows[g] < 0 ? -1 : 2 * lg + (lg > 0 ? (rows[g] >> (lg - 1)) & 1 : 0);
+      size[g] = rows[g] < 0 ? -1 : 32 - __clz(rows[g]);
       most = max(most, size[g]);
     }
     e = 0;
     for (int s = __builtin_amdgcn_readfirstlane(wave_max(most)); s >= 0 && nth >= 0; --s) {
 #pragma unroll
       for (int g = 0; g < GROUPS; ++g) {
+        if (g * 64 >= a.E) break;
         const unsigned long long q = __ballot(size[g] == s);
         const int have = __popcll(q);
         if (nth >= 0 && nth < have)
@@ -2413,9 +2414,10 @@ static bool xty_held(const XtYArgs& a) {
 // Between them: 256 x 128 tiles, two workgroups per CU (mainloop_pair), or the small tiles again, against eight waves per
 // 256 x 256 tile over 2000 random launches of 257 to 2047 rows per expert (4 to 128 experts, K and N from 256 to 8000, gathered
 // and not; even / Zipf-like loads, each in the order of XtYOrder).  256 x 128, 257 to 700 rows 1.10 / 1.17 times as fast, to 1200
-// 1.06 / 1.14, to 2047 1.03 / 1.11 (beyond 20 rounds of them 0.98 / 1.02, there from 1200 rows on they are not taken); from
-// 2048 rows on, where the operands are gathered or the bias gradient is wanted, only up to two rounds (1.05 / 1.17; beyond
-// 0.95 to 0.99 / 1.05), the one-wave-per-SIMD form otherwise (0.98).  Small tiles against 256 x 128 while the operands
+// 1.06 / 1.14, to 2047 1.03 / 1.11.  Not beyond 20 rounds of them from 1200 rows on (0.99 / 1.04), with gathered rows, whose
+// lookups come twice as often, beyond eight (0.97 / 1.02).  From 2048 rows on,
+// where an operand is gathered or the bias gradient is wanted, only up to two rounds (1.05 / 1.17; beyond 0.95 to 0.99 /
+// 1.05), the one-wave-per-SIMD form otherwise (0.98).  Small tiles against 256 x 128 while the operands
 // come from the memory-side cache, beyond one round: 257 to 700 rows, up to eight rounds 1.07 / 1.02, to 1200 rows, up to four
 // 1.07 / 1.02, to 2047 rows, up to two 1.07 / 1.02.
 // us, 32 experts x 500 rows, 2880 x 2880 346 -> 309; 32 x 300, 2880 x 5760 gathered 504 -> 467; 16 x 1000, 1024 x 1024 35.8 -> 34.4.
@@ -2430,11 +2432,14 @@ static bool xty_small_again(const XtYArgs& a) {
 static bool xty_pairs(const XtYArgs& a, bool rs_form) {
   const XtYPlan p = xty_plan(a);
   const int64_t rows = a.L / a.E, tiles = xty_pair_tiles(p);
-  if (rs_form || rows < XTY_STORE_ROWS || tiles > XTY_PAIR_ROUND * (rows >= RS_XTY_MIN_ROWS ? 2 : rows >= 1200 ? 20 : 1 << 20)) return false;
+  if (rs_form || rows < XTY_STORE_ROWS) return false;
+  const bool gathered = a.idx != nullptr;
+  const int64_t rounds = rows >= RS_XTY_MIN_ROWS ? 2 : rows >= 1200 ? (gathered ? 8 : 20) : 1 << 20;
+  if (tiles > XTY_PAIR_ROUND * rounds) return false;
   // Output pieces of 16 bytes; rows that do not overlap (the descriptors end with the last one) and, gathered, a source below
   // 2 GiB.
   if (((uintptr_t)p.OUT & 15) != 0 || ((p.soe | p.sop | p.nq) & 7) != 0 || p.ldp < p.np || p.ldq < p.nq) return false;
-  return a.idx == nullptr || (p.x_rows + 1) * a.sxm + a.K < (1ll << 30);
+  return !gathered || (p.x_rows + 1) * a.sxm + a.K < (1ll << 30);
 }
 
 template <typename T>
