@@ -2187,15 +2187,16 @@ struct XtYLds {
 // of the largest first: 0.8 to 1.04 times as fast).  Even loads keep the super tiles: an expert's rows shared by all XCDs are
 // read by each of them (128 x 2048 rows, 2048 x 1536 1600 -> 1640; 64 x 400, 1024 x 2048 138 -> 148).
 struct XtYOrder {
-  static constexpr int GROUPS = 4;         // more than 256 experts: always super tiles
+  static constexpr int GROUPS = 4;         // groups of 64 experts that are looked through
   Raster rast;
   int p_tiles, q_tiles, band, chunk;       // chunk: tiles of an expert per XCD
+  int by_rows;                             // 0: always super tiles
   template <int SN>
   __device__ __forceinline__ bool map(const XtYPlan& a, int pid, int& e, int& m, int& n) const {
     const int lane = lane_id();
     int rows[GROUPS];
     bool uneven = false;
-    if (a.E <= 64 * GROUPS) {
+    if (by_rows) {
       const int64_t L = a.off[a.E - 1];
 #pragma unroll
       for (int g = 0; g < GROUPS; ++g) {
@@ -2327,6 +2328,8 @@ static XtYPlan xty_plan(const XtYArgs& a) {
   return p;
 }
 
+static constexpr int XTY_STORE_ROWS = 96;        // rows per expert below which a weight gradient is bound by its stores
+
 template <typename T, class TL>
 static int launch_xty(const XtYArgs& a, hipStream_t st) {
   const bool k_contig = a.sdwk == 1;
@@ -2340,6 +2343,9 @@ static int launch_xty(const XtYArgs& a, hipStream_t st) {
   const int64_t grid = std::max(r.rast.grid(), chunk * a.E * 8);
   if (grid > 0x7fffffffLL) { set_error("smoe_groupXtY: grid too large"); return SMOE_ERR_RANGE; }
   r.chunk = (int)chunk;
+  // Below 96 rows per expert stores are what a tile costs, its expert's rows little (128 x 24 rows, 2048 x 1536, loads as 1 /
+  // rank^0.84 145 -> 158 in the order by rows).
+  r.by_rows = a.E <= 64 * XtYOrder::GROUPS && a.L / a.E >= XTY_STORE_ROWS;
   if constexpr (TL::RS) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, false>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r);
   else if (a.idx == nullptr) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, false>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r);
   else if (k_contig) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, true>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r);
@@ -2361,7 +2367,7 @@ static constexpr int XTY_SMALL_ROWS = 256;
 // memory is written in) share one at every tile edge; twice the edges cost more than small tiles save, in launches of more than
 // 512 large tiles: 50 random ones of 2 to 96 rows per expert 256 x 256 -> small 0.92 times as fast (161 of whole pieces 1.28;
 // us: 16 experts x 22 rows, (11024, 2416) 278 -> 311, 128 x 34, (1064, 4144) 384 -> 475).
-static constexpr int XTY_STORE_ROWS = 96, XTY_STORE_TILES = 512;
+static constexpr int XTY_STORE_TILES = 512;
 static bool xty_few_rows(const XtYArgs& a) {
   const int64_t rows = a.L / a.E, tiles = (int64_t)a.E * ((a.N + 255) / 256) * ((a.K + 255) / 256);
   if (rows > XTY_SMALL_ROWS) return false;

@@ -70,7 +70,7 @@ def test_pairs_remainders(rows):
 
 
 # small tiles (few rows; two rounds of the larger ones), eight waves (gathered, many tiles), one wave per SIMD
-@pytest.mark.parametrize("E,K,N,rows,gather", [(30, 264, 136, 60, True), (8, 2056, 1544, 400, True), (3, 3080, 5128, 2048, True),
+@pytest.mark.parametrize("E,K,N,rows,gather", [(30, 264, 136, 100, True), (8, 2056, 1544, 400, True), (3, 3080, 5128, 2048, True),
                                                (2, 3080, 2568, 2048, False)])
 @pytest.mark.parametrize("kind", ["even", "last", "halves"])
 @pytest.mark.parametrize("layout", ["nk", "kn"])
@@ -82,4 +82,4 @@ def test_other_classes(E, K, N, rows, gather, kind, layout):
 @pytest.mark.parametrize("E", [1, 2, 64, 65, 130, 256, 257])
 @pytest.mark.parametrize("kind", ["last", "halves"])
 def test_numbers_of_experts(E, kind):
-    _run(E, 136, 264, 70, kind, "nk", True, True, torch.bfloat16)
+    _run(E, 136, 264, 100, kind, "nk", True, True, torch.bfloat16)
