@@ -1896,8 +1896,25 @@ static bool whole_pieces(const S2SArgs& a) {
 // forms are held by the power cap there: a launch of K = 64 takes what its stores take, and every slice adds 63 us, 1.1 PFLOP/s.)
 // Longer contractions: the one-wave-per-SIMD form reads half as much from LDS per product; K from 2048 0.97, 8 x 4096 rows,
 // 14336 -> 4096 2957 -> 3216.
+// Tiles half as wide have twice the edges, and where output rows are no whole number of 64-byte pieces (the unit memory is written
+// in) two tiles share one at every edge.  What the gated units write, up to three times as wide as their products, then costs more
+// than the tiles save, the more the shorter the contraction.  4400 random launches of more than half a round, times as fast (more
+// than 3 % slower), even loads, rows of whole pieces / ragged: gated forward that saves its pre-activation 1.09 (3 of 357) /
+// 0.97 (373 of 816; 64 experts x 230 rows, 64 -> 6952 325 -> 509 us, 32 x 699, 64 -> 2632 155 -> 223), its gradient 1.10 (2 of 328) /
+// 1.02 (211 of 772; below 400 0.95), the interleaved unit's forward 1.12 (2 of 115) / 1.04 (8 of 64; from 1024 on 1.06, below 0.99), its
+// gradient 1.10 / 1.08, forward passes that save nothing 1.15 / 1.11, plain 1.14 (9 of 492) / 1.08 (32 of 908; contractions of up to 128
+// 1.05, 7 of 49).  Loads as 1 / rank^0.84 and 1 / rank^1.8: whole pieces 1.03 to 1.11, ragged 0.91 to 0.97 gated, 1.03 to 1.07 the others.
 typedef Tile<256, 128, 2, 2, 2, false, 2, true> PairTile;
-static bool takes_pairs(const S2SArgs& a) { return a.K < RS_MIN_K && whole_pieces(a); }
+static bool takes_pairs(const S2SArgs& a) {
+  if (a.K >= RS_MIN_K || !whole_pieces(a)) return false;
+  const bool saves = a.Y != nullptr;
+  int64_t in = (int64_t)((uintptr_t)a.Y & 63) >> 1 | (saves ? a.sym : 0);              // elements; whole pieces: multiples of 32
+  if (a.glu == 1 || a.glu == 3) in |= (int64_t)((uintptr_t)a.H & 63) >> 1 | a.shm;
+  if (a.glu == 1 || a.glu == 2) in |= a.N;                                        // the second half's first column
+  if ((in & 31) == 0) return true;
+  if ((a.glu == 1 && saves) || a.glu == 2) return false;
+  return a.K >= (a.glu == 3 && saves ? 1024 : 192);
+}
 
 template <typename T>
 static int launch_main_class(const S2SArgs& a, bool b_tr, hipStream_t st) {

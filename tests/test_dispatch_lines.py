@@ -1,0 +1,74 @@
+"""Which tiles a launch goes in, asked of the launchers' own rules: a host-only build of the kernels' header (no GPU, no device
+code).  The lines that a launch must not cross, each with the launch that was slower beyond it, and the classes that the GPU tests
+mean to run."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from scattermoe_amd import _build
+
+pytestmark = pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="needs hipcc")
+
+SOURCE = """
+#include "%s/gemm_mfma.hpp"
+using namespace smoe;
+static void* at(int64_t offset) { return (void*)(0x10000 + offset); }
+extern "C" int s2s_pairs(int64_t K, int64_t N, int glu, int64_t pitch, int64_t h_pitch, int64_t y_at, int saved) {
+  S2SArgs a{};
+  a.K = (int)K, a.N = (int)N, a.glu = glu;
+  a.Y = saved ? at(y_at) : nullptr, a.H = at(0), a.aux = at(0);
+  a.sym = a.saux = pitch, a.shm = h_pitch;
+  return takes_pairs(a);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    src, lib = d / "rules.hip", d / "rules.so"
+    src.write_text(SOURCE % _build.CSRC)
+    subprocess.run([_build._hipcc(), "--cuda-host-only", "-x", "hip", "-std=c++17", "-O1", "-fPIC", "-shared",
+                    "-Wno-unused-command-line-argument", "-o", str(lib), str(src)], check=True)
+    return ctypes.CDLL(str(lib))
+
+
+def _pairs(rules, K, N, glu=0, pitch=None, y_at=0, saved=True):
+    width = 2 * N if glu in (1, 2, 4) else N
+    return bool(rules.s2s_pairs(*(ctypes.c_int64(v) for v in (K, N)), glu, ctypes.c_int64(pitch or width),
+                                ctypes.c_int64(N // 2 if glu == 3 else N), ctypes.c_int64(y_at), int(saved)))
+
+
+@pytest.mark.parametrize("glu", [1, 2])
+def test_gated_products_of_ragged_rows_keep_wide_tiles(rules, glu):
+    """Rows that are no whole number of 64-byte pieces share one at every edge of a tile (64 experts x 230 rows, 64 -> 6952: 325
+    us in 256 x 256 tiles, 509 in 256 x 128)."""
+    for K, N in ((64, 6952), (192, 2152), (1536, 592), (1728, 1000)):
+        assert not _pairs(rules, K, N, glu), (K, N)
+        assert _pairs(rules, K, N // 32 * 32, glu), (K, N)
+    assert not _pairs(rules, 64, 2048, glu, y_at=32) and _pairs(rules, 64, 2048, glu, y_at=64)
+    assert not _pairs(rules, 64, 2048, glu, pitch=4096 + 8)
+
+
+def test_interleaved_gated_products(rules):
+    assert _pairs(rules, 64, 2 * 2048, 3) and _pairs(rules, 64, 2064, 4)
+    assert not _pairs(rules, 960, 2 * 2056, 3) and _pairs(rules, 1024, 2 * 2056, 3)
+    assert not _pairs(rules, 128, 2056, 4) and _pairs(rules, 192, 2056, 4)
+
+
+def test_forward_that_saves_nothing(rules):
+    assert _pairs(rules, 64, 2048, 1, pitch=4096 + 8, saved=False)
+    assert not _pairs(rules, 128, 2056, 1, saved=False) and _pairs(rules, 192, 2056, 1, saved=False)
+    assert not _pairs(rules, 128, 2 * 2056, 3, saved=False) and _pairs(rules, 192, 2 * 2056, 3, saved=False)
+
+
+def test_plain_products(rules):
+    """Ragged rows cost a plain product of a short contraction as well (64 x 504 rows, 64 -> 2088: 64 -> 76 us)."""
+    assert _pairs(rules, 64, 2048) and not _pairs(rules, 64, 2088) and not _pairs(rules, 128, 2088)
+    assert _pairs(rules, 192, 2088) and _pairs(rules, 1728, 2088)
+    assert not _pairs(rules, 1792, 2048)                    # the one-wave-per-SIMD form
+    assert not _pairs(rules, 200, 2048)                     # whole 64-deep slices
+    assert not _pairs(rules, 192, 2048, y_at=8)             # 16-byte pieces
