@@ -5,8 +5,8 @@
 namespace smoe {
 
 int dispatch_s2s_f16(const S2SArgs& a, bool b_tr, hipStream_t st);
-int dispatch_xty_bf16(const XtYArgs& a, bool rs_form, hipStream_t st);
-int dispatch_xty_f16(const XtYArgs& a, bool rs_form, hipStream_t st);
+int dispatch_xty_bf16(const XtYArgs& a, hipStream_t st);
+int dispatch_xty_f16(const XtYArgs& a, hipStream_t st);
 
 int64_t s2s_workspace_floats(int64_t L, int64_t K, int64_t N, int E, int dtype) {
   if ((dtype != SMOE_BF16 && dtype != SMOE_F16) || E <= 0 || L / E < REMAINDER_MIN_AVG_ROWS) return 0;
@@ -56,16 +56,7 @@ bool try_xty_mfma(const XtYArgs& a, int dtype, hipStream_t st, int& rc) {
   // 31.3 -> 31.5 ms: wide layers keep the separate pass.
   // (The kernel that holds one operand looks every row up once per unit: always.)
   if (a.idx != nullptr && a.N > XTY_GATHER_MAX_N && !xty_held(a)) return false;
-  // One-wave-per-SIMD form: needs the LDS-staged epilogue; no gathered operand, no bias gradient in the main loop.
-  // Both operands are read transposed (two LDS reads per fragment), which leaves less to win than in
-  // scatter2scatter: Mixtral shape (4096 rows per expert) 3.28 -> 3.12 and 6.35 -> 6.20 ms, 2048 rows per expert
-  // (128 experts, 768 x 2048 and 2048 x 1536 outputs) 0.81 -> 0.77 and 1.55 -> 1.51 ms, 1024 rows per expert even.
-  const bool out16 = (((uintptr_t)a.DW & 15) == 0) && ((a.sdwe | (a.sdwk == 1 ? a.sdwn : a.sdwk) | (a.sdwk == 1 ? a.K : a.N)) & 7) == 0;
-  const bool db_in_loop = a.Db != nullptr && a.sdwk == 1;
-  // (its buffer descriptors end with an operand's last row: rows that overlap, as those of an expanded tensor, would read as zeros)
-  const bool apart = a.sdym >= a.N && a.sxm >= a.K;
-  const bool rs_form = a.idx == nullptr && !db_in_loop && out16 && apart && a.L / a.E >= RS_XTY_MIN_ROWS;
-  rc = dtype == SMOE_BF16 ? dispatch_xty_bf16(a, rs_form, st) : dispatch_xty_f16(a, rs_form, st);
+  rc = dtype == SMOE_BF16 ? dispatch_xty_bf16(a, st) : dispatch_xty_f16(a, st);
   return true;
 }
 

@@ -2437,12 +2437,12 @@ static bool xty_held(const XtYArgs& a) {
 // Between them: 256 x 128 tiles, two workgroups per CU (mainloop_pair), or the small tiles again, against eight waves per
 // 256 x 256 tile over 2000 random launches of 257 to 2047 rows per expert (4 to 128 experts, K and N from 256 to 8000, gathered
 // and not; even / Zipf-like loads, each in the order of XtYOrder).  256 x 128, 257 to 700 rows 1.10 / 1.17 times as fast, to 1200
-// 1.06 / 1.14, to 2047 1.03 / 1.11.  Not beyond 20 rounds of them from 1200 rows on (0.99 / 1.04), with gathered rows, whose
-// lookups come twice as often, beyond eight (0.97 / 1.02).  From 2048 rows on,
-// where an operand is gathered or the bias gradient is wanted, only up to two rounds (1.05 / 1.17; beyond 0.95 to 0.99 /
-// 1.05), the one-wave-per-SIMD form otherwise (0.98).  Small tiles against 256 x 128 while the operands
-// come from the memory-side cache, beyond one round: 257 to 700 rows, up to eight rounds 1.07 / 1.02, to 1200 rows, up to four
-// 1.07 / 1.02, to 2047 rows, up to two 1.07 / 1.02.
+// 1.06 / 1.14, to 2047 1.03 / 1.11.  Not, gathered, beyond eight rounds from 1200 rows on (0.97 / 1.02: the lookups come twice as
+// often).  Not where an expert's output is one tile wide: two of 128 columns read the rows twice for it (30 random launches of 129 to 256
+// columns, even loads 0.96, 23 more than 3 % slower; us, 200 experts x 389 rows, 2752 x 256 177 -> 205, x 765, 3072 x 192 298 -> 339).  Not from 2048 rows on
+// (even loads 0.96, 17 of 27 more than 3 % slower; 200 x 3491 rows, 256 x 256 121 -> 137).  Small tiles against 256 x 128 while the
+// operands come from the memory-side cache, beyond one round: 257 to 700 rows, up to eight rounds 1.07 / 1.02, to 1200 rows, up to
+// four 1.07 / 1.02, to 2047 rows, up to two 1.07 / 1.02.
 // us, 32 experts x 500 rows, 2880 x 2880 346 -> 309; 32 x 300, 2880 x 5760 gathered 504 -> 467; 16 x 1000, 1024 x 1024 35.8 -> 34.4.
 // Same bits in every class.
 static constexpr int XTY_PAIR_ROUND = 2 * NUM_CU;
@@ -2452,33 +2452,48 @@ static bool xty_small_again(const XtYArgs& a) {
   if (rows <= XTY_SMALL_ROWS || rows >= RS_XTY_MIN_ROWS || (int64_t)a.L * (a.N + a.K) * 2 > (256ll << 20)) return false;
   return tiles > XTY_PAIR_ROUND && tiles <= XTY_PAIR_ROUND * (rows < 700 ? 8 : rows < 1200 ? 4 : 2);
 }
-static bool xty_pairs(const XtYArgs& a, bool rs_form) {
+static bool xty_pairs(const XtYArgs& a) {
   const XtYPlan p = xty_plan(a);
-  const int64_t rows = a.L / a.E, tiles = xty_pair_tiles(p);
-  if (rs_form || rows < XTY_STORE_ROWS) return false;
+  const int64_t rows = a.L / a.E;
   const bool gathered = a.idx != nullptr;
-  const int64_t rounds = rows >= RS_XTY_MIN_ROWS ? 2 : rows >= 1200 ? (gathered ? 8 : 20) : 1 << 20;
-  if (tiles > XTY_PAIR_ROUND * rounds) return false;
+  if (rows <= XTY_SMALL_ROWS || rows >= RS_XTY_MIN_ROWS || (p.nq > 128 && p.nq <= 256)) return false;
+  if (gathered && rows >= 1200 && xty_pair_tiles(p) > 8 * XTY_PAIR_ROUND) return false;
   // Output pieces of 16 bytes; rows that do not overlap (the descriptors end with the last one) and, gathered, a source below
   // 2 GiB.
   if (((uintptr_t)p.OUT & 15) != 0 || ((p.soe | p.sop | p.nq) & 7) != 0 || p.ldp < p.np || p.ldq < p.nq) return false;
   return !gathered || (p.x_rows + 1) * a.sxm + a.K < (1ll << 30);
 }
 
+// One-wave-per-SIMD form: needs the LDS-staged epilogue; no gathered operand, no bias gradient in the main loop.
+// Both operands are read transposed (two LDS reads per fragment), which leaves less to win than in
+// scatter2scatter: Mixtral shape (4096 rows per expert) 3.28 -> 3.12 and 6.35 -> 6.20 ms, 2048 rows per expert
+// (128 experts, 768 x 2048 and 2048 x 1536 outputs) 0.81 -> 0.77 and 1.55 -> 1.51 ms, 1024 rows per expert even.
+static bool xty_one_wave(const XtYArgs& a) {
+  const bool out16 = (((uintptr_t)a.DW & 15) == 0) && ((a.sdwe | (a.sdwk == 1 ? a.sdwn : a.sdwk) | (a.sdwk == 1 ? a.K : a.N)) & 7) == 0;
+  const bool db_in_loop = a.Db != nullptr && a.sdwk == 1;
+  // (its buffer descriptors end with an operand's last row: rows that overlap, as those of an expanded tensor, would read as zeros)
+  const bool apart = a.sdym >= a.N && a.sxm >= a.K;
+  return a.idx == nullptr && !db_in_loop && out16 && apart && a.L / a.E >= RS_XTY_MIN_ROWS;
+}
+
+enum class XtYClass { held, small, pairs, one_wave, large };
+static XtYClass xty_class(const XtYArgs& a) {
+  const bool rs_form = xty_one_wave(a);
+  if (xty_held(a)) return XtYClass::held;
+  if (xty_idle_chip(a, rs_form) || xty_few_rows(a) || xty_small_again(a)) return XtYClass::small;
+  if (xty_pairs(a)) return XtYClass::pairs;
+  return rs_form ? XtYClass::one_wave : XtYClass::large;
+}
+
 template <typename T>
-static int dispatch_xty(const XtYArgs& a, bool rs_form, hipStream_t st) {
-  typedef Tile<128, 128, 2, 2, 1, false, 4> Small;
-  typedef Tile<256, 256, 2, 4> Large;
-  const bool small = xty_idle_chip(a, rs_form) || xty_few_rows(a) || xty_small_again(a);
-  int rc;
-  if (xty_held(a)) {
-    rc = launch_xty_rows<T>(xty_plan(a), a.L, st);
-  } else if (small) {
-    rc = launch_xty<T, Small>(a, st);
-  } else if (xty_pairs(a, rs_form)) {
-    rc = launch_xty<T, PairTile>(a, st);
-  } else {
-    rc = rs_form ? launch_xty<T, Tile<256, 256, 2, 2, 2, true>>(a, st) : launch_xty<T, Large>(a, st);
+static int dispatch_xty(const XtYArgs& a, hipStream_t st) {
+  int rc = 0;
+  switch (xty_class(a)) {
+    case XtYClass::held: rc = launch_xty_rows<T>(xty_plan(a), a.L, st); break;
+    case XtYClass::small: rc = launch_xty<T, Tile<128, 128, 2, 2, 1, false, 4>>(a, st); break;
+    case XtYClass::pairs: rc = launch_xty<T, PairTile>(a, st); break;
+    case XtYClass::one_wave: rc = launch_xty<T, Tile<256, 256, 2, 2, 2, true>>(a, st); break;
+    case XtYClass::large: rc = launch_xty<T, Tile<256, 256, 2, 4>>(a, st); break;
   }
   if (rc == 0 && a.Db != nullptr && a.sdwk != 1) {
     hipLaunchKernelGGL(colsum_kernel<T>, dim3((a.N + 255) / 256, a.E), dim3(256), 0, st, (const T*)a.DY,

@@ -4,7 +4,7 @@
 
 namespace smoe {
 
-int dispatch_xty_bf16(const XtYArgs& a, bool rs_form, hipStream_t st) { return dispatch_xty<bf16_t>(a, rs_form, st); }
-int dispatch_xty_f16(const XtYArgs& a, bool rs_form, hipStream_t st) { return dispatch_xty<f16_t>(a, rs_form, st); }
+int dispatch_xty_bf16(const XtYArgs& a, hipStream_t st) { return dispatch_xty<bf16_t>(a, st); }
+int dispatch_xty_f16(const XtYArgs& a, hipStream_t st) { return dispatch_xty<f16_t>(a, st); }
 
 }  // namespace smoe

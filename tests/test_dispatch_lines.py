@@ -23,7 +23,18 @@ extern "C" int s2s_pairs(int64_t K, int64_t N, int glu, int64_t pitch, int64_t h
   a.sym = a.saux = pitch, a.shm = h_pitch;
   return takes_pairs(a);
 }
+extern "C" int xty_tiles(int64_t E, int64_t K, int64_t N, int64_t L, int gathered, int bias, int n_contiguous, int64_t dy_pitch,
+                         int64_t x_pitch) {
+  XtYArgs a{};
+  a.DY = at(0), a.X = at(0), a.DW = at(0), a.Db = bias ? at(0) : nullptr;
+  a.E = (int)E, a.K = (int)K, a.N = (int)N, a.L = (int)L;
+  a.sdyn = a.sxk = 1, a.sdym = dy_pitch, a.sxm = x_pitch, a.sdwe = K * N;
+  a.sdwk = n_contiguous ? N : 1, a.sdwn = n_contiguous ? 1 : K;
+  if (gathered) a.idx = (const int64_t*)at(0), a.fan_out = 2;
+  return (int)xty_class(a);
+}
 """
+XTY_CLASSES = ("held", "small", "pairs", "one wave", "large")
 
 
 @pytest.fixture(scope="module")
@@ -72,3 +83,24 @@ def test_plain_products(rules):
     assert not _pairs(rules, 1792, 2048)                    # the one-wave-per-SIMD form
     assert not _pairs(rules, 200, 2048)                     # whole 64-deep slices
     assert not _pairs(rules, 192, 2048, y_at=8)             # 16-byte pieces
+
+
+def _xty(rules, E, K, N, rows, layout="nk", gathered=False, bias=False, dy_pitch=None, x_pitch=None):
+    i64 = ctypes.c_int64
+    return XTY_CLASSES[rules.xty_tiles(i64(E), i64(K), i64(N), i64(E * rows), int(gathered), int(bias), int(layout == "kn"),
+                                       i64(N if dy_pitch is None else dy_pitch), i64(K if x_pitch is None else x_pitch))]
+
+
+def test_weight_gradients_of_one_tile_column_keep_wide_tiles(rules):
+    """Two tiles of 128 columns in place of one of 256 read the rows twice (200 x 389 rows, 2752 x 256: 177 -> 205 us)."""
+    assert _xty(rules, 200, 256, 2752, 389) == "large" and _xty(rules, 200, 3072, 192, 765, "kn") == "large"
+    assert _xty(rules, 200, 264, 2752, 389) == "pairs" and _xty(rules, 200, 3072, 264, 765, "kn") == "pairs"
+    assert _xty(rules, 200, 128, 2752, 600) == "pairs"
+
+
+def test_weight_gradients_of_many_rows_keep_wide_tiles(rules):
+    """200 x 3491 rows, 256 x 256: 121 us in 256 x 256 tiles, 137 in 256 x 128."""
+    for gathered, bias in ((True, False), (False, True)):
+        assert _xty(rules, 4, 2056, 1544, 2048, gathered=gathered, bias=bias) == "large"
+        assert _xty(rules, 4, 2056, 1544, 2047, gathered=gathered, bias=bias) == "pairs"
+    assert _xty(rules, 4, 2056, 1544, 2048) == "one wave"
