@@ -18,7 +18,7 @@ from scattermoe_amd import _build
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 VMEM = re.compile(r"\b(global_load|buffer_load|global_store|buffer_store)\w*\b")
-SBASE = re.compile(r"\bs\[(\d+):(\d+)\]")
+SCALAR = re.compile(r"\bs(?:(\d+)\b|\[(\d+):(\d+)\])")      # base, descriptor, scalar offset
 VALU_TO_SGPR = re.compile(r"v_\w+ s(?:(\d+)|\[(\d+):(\d+)\])")      # a vector instruction whose destination is scalar
 
 
@@ -34,11 +34,12 @@ def _hazards(text):
             continue
         if not (inside and VMEM.search(line)):
             continue
-        m = SBASE.search(line)
-        if not m:
+        regs = set()
+        for m in SCALAR.finditer(line):
+            regs |= set(range(int(m[1] or m[2]), int(m[1] or m[3]) + 1))
+        if not regs:
             continue
         loads += 1
-        regs = set(range(int(m.group(1)), int(m.group(2)) + 1))
         k, states = i - 1, 0
         while k >= 0 and states < 6:
             t = lines[k].strip()
@@ -61,6 +62,10 @@ def test_scanner_sees_a_hazard_and_its_fix():
     for writer in ("v_readlane_b32 s3, v20, s9", "v_cmp_lt_u32_e64 s[2:3], v1, v2", "v_readlane_b32 s2, v20, 63"):
         assert _hazards(bad.replace("v_readfirstlane_b32 s2, v20", writer))[1], writer
     assert not _hazards(bad.replace("v_readfirstlane_b32 s2, v20", "v_readlane_b32 s4, v20, s2"))[1]
+    for load in ("buffer_load_dwordx4 v1, s[4:7], s2 offen lds", "buffer_load_dwordx4 v1, s[0:3], s6 offen lds"):
+        assert _hazards(bad.replace("global_load_dword v1, v2, s[2:3]", load))[1], load
+        assert not _hazards(good.replace("global_load_dword v1, v2, s[2:3]", load))[1], load
+    assert not _hazards(bad.replace("global_load_dword v1, v2, s[2:3]", "buffer_load_dwordx4 v1, s[4:7], s3 offen lds"))[1]
 
 
 def _sources():
