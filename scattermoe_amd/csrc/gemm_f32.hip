@@ -7,12 +7,14 @@
 // operands stored [k][row] so that an MFMA operand (lane = row, lanes 32..63 the second k) is one conflict-free
 // ds_read_b32.  Global loads are 16 bytes per thread, fetched into registers one slice ahead of the MFMAs; an
 // operand with contiguous contraction axis is transposed on its way into LDS.  The fp32 matrix pipe is 16 times
-// slower than the bf16 one, so this simple pipeline already keeps it busy.  Launches of fewer such tiles than CUs, and
-// operands whose rows are not 16-byte aligned, go in tiles of 32 x 32 instead (s2s_f32_small_kernel, xty_f32_small_kernel).
+// slower than the bf16 one, so this simple pipeline already keeps it busy.  Launches of few such tiles, and
+// operands whose rows are not 16-byte aligned, go in tiles of 32 x 32 where those are faster (s2s_small, xty_small).
 //
 // Counterparts in the reference: _scatter2scatter (scattermoe/kernels/ops.py:50-118) and _groupXtY
 // (ops.py:242-366) with float32 tensors (where Triton would use TF32 products under ALLOW_TF32).
 #include "common.hpp"
+
+#include <algorithm>
 
 namespace smoe {
 
@@ -187,11 +189,29 @@ __global__ __launch_bounds__(FNT) void s2s_f32_kernel(S2SArgs a, int n_tiles) {
 // 11.7 -> 5.3; 112 rows, 600 -> 1200 70 -> 36, 1200 -> 600 124 -> 35; 583 rows, 512 -> 512 62 -> 44; 34 rows, 100 -> 100
 // 19.5 -> 5.4.
 static constexpr int SMALL = 32, SMALL_WAVES = FNT / 64;
-// The line: products up to 256 expected tiles of 128 x 128 (192 62 -> 55, 320 141 -> 129, 448 115 -> 118 and 96 -> 113), weight
-// gradients, of which both operands come a float per lane and load, up to 128 (64 13.5 -> 9.5 and, of 12 rows, 8.2 -> 7.9; 128
-// 17.2 -> 14.7, of 583 rows 58 -> 49; 192 21 -> 30).  Rows that are not 16-byte aligned: always, in place of the any-layout
-// kernels (8 x 410 rows, 682 -> 512 137 -> 45, its weight gradient 158 -> 51).
-static constexpr int64_t S2S_SMALL_TILES = 256, XTY_SMALL_TILES = 128;
+// Where the line lies: 7600 random products and 6500 weight gradients (1 to 128 experts, 1 to 5000 rows each, K and N from 16 to
+// 4500, even and Zipf-like loads) against the 128 x 128 tiles or, operands whose rows are not 16-byte aligned, the any-layout
+// kernels; times as fast (more than 3 % slower).
+// Products: a short contraction leaves a wave of the four a chunk or two, and the stores of 16 times as many tiles weigh more than
+// what is saved.  Aligned, K 16 / 32 / 64 / 128: up to 2 K tiles (64 at the least) 1.3 / 1.4 / 1.6 / 1.8, beyond them up to 256
+// 1.08 (18 of 63) / 1.1 (24 of 94) / 1.1 (18 of 53) / 1.4; 256 and more 1.6 to 8.  From 256 tiles on the large ones fill the chip
+// (320 141 -> 129 us, 448 115 -> 118 and 96 -> 113).  Not aligned, up to 2 K 1.0 to 1.4 (K 16 to 64) and 1.6 (128), up to twice as
+// many 0.95 to 1.1, four times 0.8 to 0.95; K 256 up to 1024 tiles 1.3, up to 4096 1.1; 384 and more 1.05 to 10.
+static bool s2s_small(const S2SArgs& a, bool aligned) {
+  // (128 x 128 tiles; an expert's last one is half full on average)
+  const int64_t tiles = (cdiv64(a.L, FBM) + a.E / 2) * ((a.N + FBN - 1) / FBN);
+  const int64_t line = std::max<int64_t>(64, (aligned || a.K < 256 ? 2 : 4) * (int64_t)a.K);
+  return aligned ? tiles <= std::min<int64_t>(256, line) : a.K >= 384 || tiles <= line;
+}
+// Weight gradients: up to 1024 tiles of 32 x 32 never slower; more of them cost more than few rows' products do.  Aligned, up to 128
+// tiles of 128 x 128 (192 21 -> 30 us): 1 to 32 rows per expert 0.95 (66 of 129), 32 to 48 1.15 (7 of 20), then 1.3 to 1.5.  Not aligned: 1
+// to 16 rows 0.7 to 1.0, 16 to 32 1.02 (43 of 116), then 1.3 to 6.
+static bool xty_small(const XtYArgs& a, bool aligned) {
+  auto tiles = [&](int64_t t) { return a.E * ((a.K + t - 1) / t) * ((a.N + t - 1) / t); };
+  const int64_t rows = a.L / a.E;
+  if (aligned && tiles(FBM) > 128) return false;
+  return tiles(SMALL) <= 1024 || rows >= (aligned ? 48 : 32);
+}
 
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));      // 16-byte loads need dword alignment only
 
@@ -307,8 +327,9 @@ bool try_s2s_f32(const S2SArgs& a, hipStream_t st, int& rc) {
   const bool aligned = a.K % 4 == 0 && a.sxm % 4 == 0 && al16(a.X) && al16(a.W) && a.swe % 4 == 0 &&
                        (w_kc || (a.swn == 1 && a.swk % 4 == 0 && a.N % 4 == 0));
   const int n_tiles = (a.N + FBN - 1) / FBN;
-  // (an expert's last tile is half full on average)
-  if (!aligned || (cdiv64(a.L, FBM) + a.E / 2) * n_tiles <= S2S_SMALL_TILES) {
+  const bool small = s2s_small(a, aligned);
+  if (!aligned && !small) return false;
+  if (small) {
     if (!aligned) w_kc = a.swk == 1;
     const int cols = (a.N + SMALL - 1) / SMALL;
     const int64_t grid = max_tiles(a.L, a.E, SMALL) * cols;
@@ -449,7 +470,8 @@ bool try_xty_f32(const XtYArgs& a, hipStream_t st, int& rc) {
   const bool nk = a.sdwk == 1;                     // output rows = N index, K contiguous; else rows = K index, N contiguous
   const bool aligned = a.sdym % 4 == 0 && a.sxm % 4 == 0 && a.K % 4 == 0 && a.N % 4 == 0 && al16(a.DY) && al16(a.X) &&
                        al16(a.DW) && a.sdwe % 4 == 0 && (nk ? a.sdwn : a.sdwk) % 4 == 0;
-  if (!aligned && a.E > 65535) return false;       // (the bias gradient's grid)
+  const bool small = xty_small(a, aligned);
+  if (!aligned && (!small || a.E > 65535)) return false;       // (the bias gradient's grid)
   XtYPlanF32 p;
   if (nk) {
     p.P = (const float*)a.DY; p.ldp = a.sdym; p.np = a.N;
@@ -464,11 +486,11 @@ bool try_xty_f32(const XtYArgs& a, hipStream_t st, int& rc) {
   const int p_tiles = (p.np + FBM - 1) / FBM, q_tiles = (p.nq + FBN - 1) / FBN;
   const int64_t grid = (int64_t)a.E * p_tiles * q_tiles;
   if (grid > 0x7fffffffLL) { set_error("smoe_groupXtY: grid too large"); rc = SMOE_ERR_RANGE; return true; }
-  if (grid > 0 && (!aligned || grid <= XTY_SMALL_TILES)) {
+  if (grid > 0 && small) {
     const int pt = (p.np + SMALL - 1) / SMALL, qt = (p.nq + SMALL - 1) / SMALL;
-    const int64_t small = (int64_t)a.E * pt * qt;
-    if (small > 0x7fffffffLL) return false;
-    hipLaunchKernelGGL(xty_f32_small_kernel, dim3((unsigned)small), dim3(FNT), 0, st, p, pt, qt);
+    const int64_t cells = (int64_t)a.E * pt * qt;
+    if (cells > 0x7fffffffLL) return false;
+    hipLaunchKernelGGL(xty_f32_small_kernel, dim3((unsigned)cells), dim3(FNT), 0, st, p, pt, qt);
     rc = launch_status("xty_f32_small_kernel");
     if (rc != 0) return true;
   } else if (grid > 0) {

@@ -12,10 +12,50 @@ from scattermoe_amd import _build
 
 pytestmark = pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="needs hipcc")
 
+# Launches are noted (the launching function's name with its tile, the kernel, the workgroups) instead of being made.
 SOURCE = """
-#include "%s/gemm_mfma.hpp"
+#include <hip/hip_runtime.h>
+#include <string>
+static std::string launched;
+static void note(const char* from, const char* kernel, unsigned grid) {
+  launched += std::string(from) + " / " + kernel + " / " + std::to_string(grid) + "\\n";
+}
+#undef __global__
+#define __global__ static __device__ __attribute__((unused))
+#undef __launch_bounds__
+#define __launch_bounds__(...)
+#undef hipLaunchKernelGGL
+#define hipLaunchKernelGGL(kernel, grid, ...) note(__PRETTY_FUNCTION__, #kernel, dim3(grid).x)
+#include "%(csrc)s/gemm_mfma.hpp"
+#include "%(csrc)s/gemm_f32.hip"
+namespace smoe {
+int launch_status(const char*) { return 0; }
+void set_error(const char*, ...) {}
+}
 using namespace smoe;
 static void* at(int64_t offset) { return (void*)(0x10000 + offset); }
+static S2SArgs s2s_args(int64_t E, int64_t K, int64_t N, int64_t L, int n_contiguous, int64_t pad) {
+  S2SArgs a{};
+  a.X = at(0), a.W = at(0), a.Y = at(0);
+  a.E = (int)E, a.K = (int)K, a.N = (int)N, a.L = (int)L, a.fan_out = 1, a.x_grouped = a.y_grouped = 1;
+  a.sxk = a.syn = 1, a.sxm = K + pad, a.sym = N;
+  if (n_contiguous) a.swn = 1, a.swk = N + pad, a.swe = K * (N + pad);
+  else a.swk = 1, a.swn = K + pad, a.swe = N * (K + pad);
+  return a;
+}
+extern "C" const char* s2s_launch(int64_t E, int64_t K, int64_t N, int64_t L, int n_contiguous, int64_t expanded) {
+  launched.clear();
+  S2SArgs a = s2s_args(E, K, N, L, n_contiguous, 0);
+  if (expanded) a.swk = 0;
+  dispatch_s2s<bf16_t>(a, n_contiguous, 0);
+  return launched.c_str();
+}
+extern "C" const char* s2s_f32_launch(int64_t E, int64_t K, int64_t N, int64_t L, int n_contiguous, int64_t pad) {
+  launched.clear();
+  int rc;
+  if (!try_s2s_f32(s2s_args(E, K, N, L, n_contiguous, pad), 0, rc)) launched = "any layout";
+  return launched.c_str();
+}
 extern "C" int s2s_pairs(int64_t K, int64_t N, int glu, int64_t pitch, int64_t h_pitch, int64_t y_at, int saved) {
   S2SArgs a{};
   a.K = (int)K, a.N = (int)N, a.glu = glu;
@@ -33,6 +73,16 @@ extern "C" int xty_tiles(int64_t E, int64_t K, int64_t N, int64_t L, int gathere
   if (gathered) a.idx = (const int64_t*)at(0), a.fan_out = 2;
   return (int)xty_class(a);
 }
+extern "C" const char* xty_f32_launch(int64_t E, int64_t K, int64_t N, int64_t L, int64_t pad) {
+  launched.clear();
+  XtYArgs a{};
+  a.DY = at(0), a.X = at(0), a.DW = at(0);
+  a.E = (int)E, a.K = (int)K, a.N = (int)N, a.L = (int)L;
+  a.sdyn = a.sxk = a.sdwk = 1, a.sdym = N + pad, a.sxm = K + pad, a.sdwn = K, a.sdwe = N * K;
+  int rc;
+  if (!try_xty_f32(a, 0, rc)) launched = "any layout";
+  return launched.c_str();
+}
 """
 XTY_CLASSES = ("held", "small", "pairs", "one wave", "large")
 
@@ -41,10 +91,12 @@ XTY_CLASSES = ("held", "small", "pairs", "one wave", "large")
 def rules(tmp_path_factory):
     d = tmp_path_factory.mktemp("rules")
     src, lib = d / "rules.hip", d / "rules.so"
-    src.write_text(SOURCE % _build.CSRC)
+    src.write_text(SOURCE % {"csrc": _build.CSRC})
     subprocess.run([_build._hipcc(), "--cuda-host-only", "-x", "hip", "-std=c++17", "-O1", "-fPIC", "-shared",
                     "-Wno-unused-command-line-argument", "-o", str(lib), str(src)], check=True)
-    return ctypes.CDLL(str(lib))
+    lib = ctypes.CDLL(str(lib))
+    lib.s2s_launch.restype = lib.s2s_f32_launch.restype = lib.xty_f32_launch.restype = ctypes.c_char_p
+    return lib
 
 
 def _pairs(rules, K, N, glu=0, pitch=None, y_at=0, saved=True):
@@ -104,3 +156,32 @@ def test_weight_gradients_of_many_rows_keep_wide_tiles(rules):
         assert _xty(rules, 4, 2056, 1544, 2048, gathered=gathered, bias=bias) == "large"
         assert _xty(rules, 4, 2056, 1544, 2047, gathered=gathered, bias=bias) == "pairs"
     assert _xty(rules, 4, 2056, 1544, 2048) == "one wave"
+
+
+def _f32(launch, *sizes):
+    text = launch(*(ctypes.c_int64(v) for v in sizes)).decode()
+    return "small" if "small_kernel" in text else "any layout" if text == "any layout" else "large"
+
+
+def test_float32_products(rules):
+    """Times of the launch in 32 x 32 tiles against the other kind that it would go in."""
+    def tiles(E, K, N, rows, pad=0, n_contiguous=0):
+        return _f32(rules.s2s_f32_launch, E, K, N, E * rows, n_contiguous, pad)
+    assert tiles(8, 512, 512, 64) == tiles(8, 4096, 1024, 256) == "small"
+    assert tiles(8, 1024, 4096, 256) == "large"
+    # short contractions: 64 x 909 rows, 16 -> 168 24 -> 54 us; 16 x 2296, 48 -> 1248 109 -> 252
+    assert tiles(64, 16, 168, 909, 1) == tiles(16, 48, 1248, 2296, 1) == tiles(128, 28, 420, 1962, 1) == "any layout"
+    assert tiles(8, 32, 512, 1024) == "large" and tiles(8, 32, 512, 128) == tiles(8, 128, 512, 256) == "small"
+    assert tiles(8, 256, 2048, 256, 1) == tiles(32, 768, 768, 4096, 1) == "small"
+    assert tiles(8, 256, 4096, 4096, 1) == "any layout"
+    assert tiles(8, 256, 2048, 256, 1, 1) == "small"
+
+
+def test_float32_weight_gradients(rules):
+    def tiles(E, K, N, rows, pad=0):
+        return _f32(rules.xty_f32_launch, E, K, N, E * rows, pad)
+    # 8 x 16 rows, 512 x 512 8 -> 11 us; 32 x 4, 1592 x 4368, rows of no whole 16 bytes, 452 -> 706
+    assert tiles(8, 512, 512, 16) == "large" and tiles(8, 512, 512, 48) == "small"
+    assert tiles(8, 256, 512, 1) == tiles(8, 128, 512, 16) == tiles(8, 256, 512, 1, 1) == "small"       # up to 1024 of them
+    assert tiles(32, 1592, 4368, 4, 1) == tiles(8, 512, 512, 31, 1) == "any layout" and tiles(8, 512, 512, 32, 1) == "small"
+    assert tiles(8, 1024, 1024, 4096) == "large" and tiles(8, 1024, 1024, 4096, 1) == "small"

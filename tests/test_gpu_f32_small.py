@@ -61,7 +61,7 @@ def test_weight_gradients(K, N, layout):
 
 def test_unaligned_operands():
     """Operands and outputs that begin one element into wider matrices; more tiles than the aligned ones may have."""
-    for K, N in ((68, 3300), (67, 3301)):
+    for K, N in ((68, 3300), (67, 3301), (131, 3301)):      # 182 tiles of 128 x 128: the last goes in 32 x 32 ones
         g, E, L, eid, idx, off, X, W, b = _inputs(K + 1, N + 1, 1)
         X, W = X[:, 1:], W[:, 1:, 1:]
         DY = torch.randn(L, N + 1, generator=g, device=DEV)[:, 1:]
