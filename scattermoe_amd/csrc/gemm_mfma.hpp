@@ -2347,22 +2347,30 @@ static XtYPlan xty_plan(const XtYArgs& a) {
 
 static constexpr int XTY_STORE_ROWS = 96;        // rows per expert below which a weight gradient is bound by its stores
 
-template <typename T, class TL>
-static int launch_xty(const XtYArgs& a, hipStream_t st) {
-  const bool k_contig = a.sdwk == 1;
-  const XtYPlan p = xty_plan(a);
+// `grid`: workgroups.  Each order has its own number; a launch that may take either has to cover both.
+template <class TL>
+static XtYOrder xty_order(const XtYPlan& p, int64_t L, int64_t& grid) {
   XtYOrder r;
   r.p_tiles = (p.np + TL::BM - 1) / TL::BM;
   r.q_tiles = (p.nq + TL::BN - 1) / TL::BN;
   r.band = TL::PAIR ? 2 * Raster::SN : Raster::SN;
-  r.rast = make_raster((int64_t)a.E * r.p_tiles, r.q_tiles, GM_XTY, r.band);
-  const int64_t chunk = ((int64_t)r.p_tiles * r.q_tiles + 7) / 8;
-  const int64_t grid = std::max(r.rast.grid(), chunk * a.E * 8);
-  if (grid > 0x7fffffffLL) { set_error("smoe_groupXtY: grid too large"); return SMOE_ERR_RANGE; }
-  r.chunk = (int)chunk;
+  r.rast = make_raster((int64_t)p.E * r.p_tiles, r.q_tiles, GM_XTY, r.band);
   // Below 96 rows per expert stores are what a tile costs, its expert's rows little (128 x 24 rows, 2048 x 1536, loads as 1 /
   // rank^0.84 145 -> 158 in the order by rows).
-  r.by_rows = a.E <= 64 * XtYOrder::GROUPS && a.L / a.E >= XTY_STORE_ROWS;
+  r.by_rows = p.E <= 64 * XtYOrder::GROUPS && L / p.E >= XTY_STORE_ROWS;
+  const int64_t chunk = ((int64_t)r.p_tiles * r.q_tiles + 7) / 8;
+  r.chunk = (int)chunk;
+  grid = r.by_rows ? std::max(r.rast.grid(), chunk * p.E * 8) : r.rast.grid();
+  return r;
+}
+
+template <typename T, class TL>
+static int launch_xty(const XtYArgs& a, hipStream_t st) {
+  const bool k_contig = a.sdwk == 1;
+  const XtYPlan p = xty_plan(a);
+  int64_t grid;
+  const XtYOrder r = xty_order<TL>(p, a.L, grid);
+  if (grid > 0x7fffffffLL) { set_error("smoe_groupXtY: grid too large"); return SMOE_ERR_RANGE; }
   if constexpr (TL::RS) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, false>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r);
   else if (a.idx == nullptr) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, false>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r);
   else if (k_contig) hipLaunchKernelGGL((xty_mfma_kernel<T, TL, false, true>), dim3((unsigned)grid), dim3(TL::NT), 0, st, p, r);

@@ -83,6 +83,14 @@ extern "C" const char* xty_f32_launch(int64_t E, int64_t K, int64_t N, int64_t L
   if (!try_xty_f32(a, 0, rc)) launched = "any layout";
   return launched.c_str();
 }
+extern "C" int64_t xty_workgroups(int64_t E, int64_t np, int64_t nq, int64_t L, int wide) {
+  XtYPlan p{};
+  p.E = (int)E, p.np = (int)np, p.nq = (int)nq;
+  int64_t grid;
+  if (wide) xty_order<Tile<256, 256, 2, 4>>(p, L, grid);
+  else xty_order<Tile<128, 128, 2, 2, 1, false, 4>>(p, L, grid);
+  return grid;
+}
 """
 XTY_CLASSES = ("held", "small", "pairs", "one wave", "large")
 
@@ -95,6 +103,7 @@ def rules(tmp_path_factory):
     subprocess.run([_build._hipcc(), "--cuda-host-only", "-x", "hip", "-std=c++17", "-O1", "-fPIC", "-shared",
                     "-Wno-unused-command-line-argument", "-o", str(lib), str(src)], check=True)
     lib = ctypes.CDLL(str(lib))
+    lib.xty_workgroups.restype = ctypes.c_int64
     lib.s2s_launch.restype = lib.s2s_f32_launch.restype = lib.xty_f32_launch.restype = ctypes.c_char_p
     return lib
 
@@ -185,3 +194,19 @@ def test_float32_weight_gradients(rules):
     assert tiles(8, 256, 512, 1) == tiles(8, 128, 512, 16) == tiles(8, 256, 512, 1, 1) == "small"       # up to 1024 of them
     assert tiles(32, 1592, 4368, 4, 1) == tiles(8, 512, 512, 31, 1) == "any layout" and tiles(8, 512, 512, 32, 1) == "small"
     assert tiles(8, 1024, 1024, 4096) == "large" and tiles(8, 1024, 1024, 4096, 1) == "small"
+
+
+def _workgroups(rules, E, np_, nq, rows, wide):
+    return rules.xty_workgroups(*(ctypes.c_int64(v) for v in (E, np_, nq, E * rows)), int(wide))
+
+
+def test_weight_gradients_that_keep_super_tiles_have_their_grid_only(rules):
+    """The order by rows gives every expert a whole number of workgroups per XCD, eight for an expert of one tile; launches that never
+    take it (few rows, more experts than are looked through) start none of those."""
+    for wide, tile in ((True, 256), (False, 128)):
+        assert _workgroups(rules, 256, tile, tile, 95, wide) == 8 * 256 // 2        # super tiles of 8 x 4, of which one column exists
+        assert _workgroups(rules, 256, tile, tile, 96, wide) == 8 * 256
+        assert _workgroups(rules, 257, tile, tile, 300, wide) < 8 * 257
+        # (each covers its own order)
+        assert _workgroups(rules, 40, 9 * tile, 5 * tile, 95, wide) >= 40 * 45
+        assert _workgroups(rules, 40, 9 * tile, 5 * tile, 96, wide) >= 40 * 48
