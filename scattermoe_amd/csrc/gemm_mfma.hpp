@@ -2211,9 +2211,16 @@ struct XtYOrder {
   template <int SN>
   __device__ __forceinline__ bool map(const XtYPlan& a, int pid, int& e, int& m, int& n) const {
     const int lane = lane_id();
-    int rows[GROUPS];
+    int m_tile, m_loc, n_loc;
+    const bool in_super = rast.map<SN>(pid, m_tile, n, m_loc, n_loc);
+    const int x = pid & 7, i = pid >> 3;
+    int nth = 0, t = 0, rows[GROUPS];
     bool uneven = false;
     if (by_rows) {
+      nth = __builtin_amdgcn_readfirstlane(i / chunk);
+      t = ((x + nth) & 7) * chunk + (i - nth * chunk);
+      const bool in_chunk = nth < a.E && t < p_tiles * q_tiles;
+      if (!in_super && !in_chunk) return false;              // (narrow outputs: three quarters of the super tiles' workgroups)
       const int64_t L = a.off[a.E - 1];
 #pragma unroll
       for (int g = 0; g < GROUPS; ++g) {
@@ -2222,18 +2229,14 @@ struct XtYOrder {
         if (g * 64 < a.E && c < a.E) rows[g] = (int)(a.off[c] - (c ? a.off[c - 1] : 0));
         uneven = uneven || __ballot((int64_t)rows[g] * a.E > 2 * L) != 0;
       }
+      if (uneven && !in_chunk) return false;
     }
     if (!uneven) {
-      int m_tile, m_loc, n_loc;
-      if (!rast.map<SN>(pid, m_tile, n, m_loc, n_loc)) return false;
+      if (!in_super) return false;
       e = __builtin_amdgcn_readfirstlane(m_tile / p_tiles);
       m = m_tile - e * p_tiles;
       return true;
     }
-    const int x = pid & 7, i = pid >> 3;
-    int nth = __builtin_amdgcn_readfirstlane(i / chunk);
-    const int t = ((x + nth) & 7) * chunk + (i - nth * chunk);
-    if (nth >= a.E || t >= p_tiles * q_tiles) return false;
     // the nth expert by the power of two its load reaches (finer steps and groups that hold no expert cost each tile 1.5 us)
     int size[GROUPS], most = 0;
 #pragma unroll
@@ -2346,6 +2349,7 @@ static XtYPlan xty_plan(const XtYArgs& a) {
 }
 
 static constexpr int XTY_STORE_ROWS = 96;        // rows per expert below which a weight gradient is bound by its stores
+static constexpr int XTY_SMALL_ROWS = 256;       // ... and up to which it goes in small tiles (xty_few_rows)
 
 // `grid`: workgroups.  Each order has its own number; a launch that may take either has to cover both.
 template <class TL>
@@ -2355,9 +2359,10 @@ static XtYOrder xty_order(const XtYPlan& p, int64_t L, int64_t& grid) {
   r.q_tiles = (p.nq + TL::BN - 1) / TL::BN;
   r.band = TL::PAIR ? 2 * Raster::SN : Raster::SN;
   r.rast = make_raster((int64_t)p.E * r.p_tiles, r.q_tiles, GM_XTY, r.band);
-  // Below 96 rows per expert stores are what a tile costs, its expert's rows little (128 x 24 rows, 2048 x 1536, loads as 1 /
-  // rank^0.84 145 -> 158 in the order by rows).
-  r.by_rows = p.E <= 64 * XtYOrder::GROUPS && L / p.E >= XTY_STORE_ROWS;
+  // Few rows are little of what a tile costs, and to ask whether loads are even is the more of it: up to 256 rows per expert, even loads
+  // 0.94 to 0.99 of the time without the order (78 of 176 random launches more than 3 % slower), as 1 / rank^0.84 and ^1.8 0.97 to 1.07
+  // (128 x 24 rows, 2048 x 1536 145 -> 158 us).  So is one column of 256 wide tiles, each alone on its CU: 0.96 (41 of 72), uneven 1.02.
+  r.by_rows = p.E <= 64 * XtYOrder::GROUPS && L / p.E > XTY_SMALL_ROWS && !(TL::BN == 256 && r.q_tiles == 1);
   const int64_t chunk = ((int64_t)r.p_tiles * r.q_tiles + 7) / 8;
   r.chunk = (int)chunk;
   grid = r.by_rows ? std::max(r.rast.grid(), chunk * p.E * 8) : r.rast.grid();
@@ -2387,7 +2392,6 @@ static int launch_xty(const XtYArgs& a, hipStream_t st) {
 // 257 -> 191, 316 -> 270, 390 -> 370, 480 -> 489.  Inside a training step, at its lower clock: 32 x 188 rows, 2880 x 2880
 // 248 -> 212; even at 280).  Gathered rows as well: 34 random launches of 128 to 256 rows per expert 256 x 256 -> small
 // 1.23 times as fast.
-static constexpr int XTY_SMALL_ROWS = 256;
 // But with few rows per expert the launch is all stores.  Output rows that are no whole number of 64-byte pieces (the unit
 // memory is written in) share one at every tile edge; twice the edges cost more than small tiles save, in launches of more than
 // 512 large tiles: 50 random ones of 2 to 96 rows per expert 256 x 256 -> small 0.92 times as fast (161 of whole pieces 1.28;

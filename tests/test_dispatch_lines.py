@@ -200,13 +200,15 @@ def _workgroups(rules, E, np_, nq, rows, wide):
     return rules.xty_workgroups(*(ctypes.c_int64(v) for v in (E, np_, nq, E * rows)), int(wide))
 
 
-def test_weight_gradients_that_keep_super_tiles_have_their_grid_only(rules):
-    """The order by rows gives every expert a whole number of workgroups per XCD, eight for an expert of one tile; launches that never
-    take it (few rows, more experts than are looked through) start none of those."""
+def test_weight_gradients_that_keep_super_tiles(rules):
+    """Up to 256 rows per expert, more experts than are looked through, one column of 256 wide tiles: no order by rows, which costs even
+    loads a look at all experts per tile (8 x 200 rows, 256 x 20000: 6 %).  Such launches have the super tiles' grid only; the
+    order by rows gives every expert a whole number of workgroups per XCD, eight for an expert of one tile."""
+    small = 8 * 256 // 2                                    # super tiles of 8 x 4, of which one column exists
+    assert _workgroups(rules, 256, 128, 128, 256, False) == small and _workgroups(rules, 256, 128, 128, 257, False) == 8 * 256
+    assert _workgroups(rules, 256, 256, 256, 2000, True) == small
     for wide, tile in ((True, 256), (False, 128)):
-        assert _workgroups(rules, 256, tile, tile, 95, wide) == 8 * 256 // 2        # super tiles of 8 x 4, of which one column exists
-        assert _workgroups(rules, 256, tile, tile, 96, wide) == 8 * 256
-        assert _workgroups(rules, 257, tile, tile, 300, wide) < 8 * 257
+        assert _workgroups(rules, 257, tile, 2 * tile, 300, wide) < 8 * 257
         # (each covers its own order)
-        assert _workgroups(rules, 40, 9 * tile, 5 * tile, 95, wide) >= 40 * 45
-        assert _workgroups(rules, 40, 9 * tile, 5 * tile, 96, wide) >= 40 * 48
+        assert _workgroups(rules, 40, 9 * tile, 5 * tile, 256, wide) >= 40 * 45
+        assert _workgroups(rules, 40, 9 * tile, 5 * tile, 257, wide) >= 40 * 48
