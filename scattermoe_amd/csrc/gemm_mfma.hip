@@ -53,9 +53,11 @@ bool try_xty_mfma(const XtYArgs& a, int dtype, hipStream_t st, int& rc) {
   // Looking the rows up costs the kernel about 4 % of its time; the gathered copy it saves costs 4 K bytes of HBM
   // traffic per row against 2 K N flops, i.e. a share of the kernel time that shrinks with N.  Measured per training
   // step: N = 1536 (Qwen-like, top-8) 9.12 -> 8.90 ms, N = 5760 (gpt-oss-like) 6.07 -> 6.03 ms, N = 28672 (Mixtral)
-  // 31.3 -> 31.5 ms: wide layers keep the separate pass.
-  // (The kernel that holds one operand looks every row up once per unit: always.)
-  if (a.idx != nullptr && a.N > XTY_GATHER_MAX_N && !xty_held(a)) return false;
+  // 31.3 -> 31.5 ms: wide layers keep the separate pass.  Not where X is streamed past a held operand, which looks every row up
+  // once per unit (the experts of more than 256 rows do so in every slice of a tile, all the same): random launches of N from
+  // 6200 on, even loads / as 1 / rank^0.42, ^0.84, ^1.8, against the copy and 128 x 128 tiles 1.42 / 1.17 / 1.05 / 0.99; where X
+  // is held (N contiguous) 1.3 / 1.0 / 0.90 / 0.88 with lookups, 1.27 / 1.02 / 0.94 / 0.93 over the copy.
+  if (a.idx != nullptr && a.N > XTY_GATHER_MAX_N && !(xty_held(a) && a.sdwk == 1)) return false;
   rc = dtype == SMOE_BF16 ? dispatch_xty_bf16(a, st) : dispatch_xty_f16(a, st);
   return true;
 }

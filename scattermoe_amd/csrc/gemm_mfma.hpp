@@ -2438,12 +2438,18 @@ static bool xty_idle_chip(const XtYArgs& a, bool rs_form) {
 // 0.96 (both are bound by their stores there), 64 to 96 1.00 to 1.07.  Up to 224: experts beyond 256 rows go in tiles, two
 // workgroups per CU where a launch of nothing but tiles has four (even loads of 250 rows, half of them beyond: 0.95, 1190
 // rows 0.85).  At least 256 tiles of 256 x 256: smaller launches have too few units (16 x 142 rows, 1472 x 512 11 -> 13).
-// Uneven loads of such an average (1 / rank^0.84, 1 / rank^1.8): 0.95 and 1.2, the heavy experts then start first.
-static constexpr int XTY_HELD_MIN_ROWS = 96, XTY_HELD_MAX_ROWS = 224;
+// 5650 random launches within those lines, even loads / as 1 / rank^0.42, ^0.84, ^1.8 (more than 3 % slower): the held operand is a
+// panel of 256 output rows, of which narrow outputs leave most empty, two thirds and more of them multiplied for nothing; and
+// what unevenness puts beyond 256 rows is then a chain of slices for a few workgroups.  Up to 128 rows 0.80 / 0.66 / 0.76 / 1.1 (100 of 102, 104
+// of 121 ...), to 256 0.99 / 0.80 / 0.85 / 1.1, to 384 1.15 / 0.95 / 1.01 / 1.14, beyond 1.21 to 1.38 / 1.0 to 1.16 / 1.0 to 1.06 / 1.2 to 1.3.
+// With few experts one of them has most of the rows: 8 experts 1.24 / 1.05 / 0.94 (53 of 85) / 0.96, 4 1.23 / 1.10 / 1.02 / 0.92, 16
+// 1.24 / 1.04 / 0.97 / 1.08, 32 1.25 / 1.04 / 1.03 / 1.18, more 1.23 to 1.3 / 1.1 / 1.1 / 1.2.
+static constexpr int XTY_HELD_MIN_ROWS = 96, XTY_HELD_MAX_ROWS = 224, XTY_HELD_MIN_PANEL = 384, XTY_HELD_MIN_EXPERTS = 16;
 static bool xty_held(const XtYArgs& a) {
+  const XtYPlan p = xty_plan(a);
   const int64_t rows = a.L / a.E;
-  if (rows < XTY_HELD_MIN_ROWS || rows > XTY_HELD_MAX_ROWS) return false;
-  return (int64_t)a.E * ((a.N + 255) / 256) * ((a.K + 255) / 256) >= 256 && xty_rows_fits(xty_plan(a));
+  if (rows < XTY_HELD_MIN_ROWS || rows > XTY_HELD_MAX_ROWS || a.E < XTY_HELD_MIN_EXPERTS || p.np < XTY_HELD_MIN_PANEL) return false;
+  return (int64_t)a.E * ((a.N + 255) / 256) * ((a.K + 255) / 256) >= 256 && xty_rows_fits(p);
 }
 
 // Between them: 256 x 128 tiles, two workgroups per CU (mainloop_pair), or the small tiles again, against eight waves per

@@ -569,6 +569,14 @@ def _xty_launch(E, DW, Db, DY, X, expert_offsets):
     _backend.xty(DY, X, DW, Db, _as_i64(expert_offsets).contiguous(), E)
 
 
+def _xty_holds_rows(DW, X, L):
+    """Whether the library holds the gathered rows in registers for a gradient with N contiguous of more than 512 tiles of 256 x 256
+    (`xty_held` in csrc/gemm_mfma.hpp; the tests compare the two)."""
+    E, K, _ = DW.shape
+    return (96 * E <= L < 225 * E and E >= 16 and K >= 384 and (DW.stride(0) | DW.stride(1)) % 64 == 0
+            and X.size(0) * X.stride(0) + K + 256 < 2 ** 30)
+
+
 def _xty_gathered_launch(E, DW, Db, DY, X, idx, fan_out, expert_offsets):
     """groupXtY over X[idx // fan_out]: one launch that reads the rows of X through idx where the library has one,
     else the gathered copy and the plain launch."""
@@ -577,12 +585,11 @@ def _xty_gathered_launch(E, DW, Db, DY, X, idx, fan_out, expert_offsets):
     # fast, 0.94 to 1.17; d = F = 2880, 32 experts, 50 / 188 rows: 219 -> 201, 377 -> 369 us).  Everything else looks the rows
     # up inside the launch: of up to 512 tiles the copy's launch is what counts (20 rows: 11 us against 19), and with K
     # contiguous the copy is never faster (87 random launches 0.93; 128 experts x 100 rows, 2048 x 1536 201 against 249 us).
-    # Nor is it where the rows held in registers are looked up once per workgroup (96 to 224 rows per expert, output rows on
-    # 128-byte lines: 188 rows, 2880 x 2880 / 5760, lookups 156 / 266 us, plain 154 / 255, the copy 9).
-    held = 96 * E <= DY.size(0) < 225 * E and (DW.stride(0) | DW.stride(1)) % 64 == 0
-    copy_rows = (DW.stride(2) == 1 and DY.size(0) <= 256 * E and DY.size(1) >= 2048 and not held
-                 and E * DY.size(1) * X.size(1) > 512 * 256 * 256)
+    # Nor is it where the rows held in registers are looked up once per workgroup (188 rows, 2880 x 2880 / 5760, lookups 156 /
+    # 266 us, plain 154 / 255, the copy 9).
     lookups = DY.is_cuda and hasattr(_backend, "xty_gathered") and DY.dtype in (torch.bfloat16, torch.float16)
+    copy_rows = (lookups and DW.stride(2) == 1 and DY.size(0) <= 256 * E and DY.size(1) >= 2048
+                 and E * DY.size(1) * X.size(1) > 512 * 256 * 256 and not _xty_holds_rows(DW, X, DY.size(0)))
     if lookups and not copy_rows:
         _same_dtype("group_bwd_W", DY, X, DW, Db)
         if _backend.xty_gathered(DY, X, _as_i64(idx).contiguous(), fan_out, DW, Db,

@@ -3,6 +3,7 @@ code).  The lines that a launch must not cross, each with the launch that was sl
 mean to run."""
 import ctypes
 import os
+import random
 import shutil
 import subprocess
 
@@ -26,11 +27,14 @@ static void note(const char* from, const char* kernel, unsigned grid) {
 #define __launch_bounds__(...)
 #undef hipLaunchKernelGGL
 #define hipLaunchKernelGGL(kernel, grid, ...) note(__PRETTY_FUNCTION__, #kernel, dim3(grid).x)
-#include "%(csrc)s/gemm_mfma.hpp"
+#include "%(csrc)s/gemm_mfma.hip"
+#include "%(csrc)s/gemm_mfma_xty.hip"
 #include "%(csrc)s/gemm_f32.hip"
 namespace smoe {
 int launch_status(const char*) { return 0; }
 void set_error(const char*, ...) {}
+int dispatch_s2s_f16(const S2SArgs&, bool, hipStream_t) { return 0; }
+bool try_s2s_rowdot(const S2SArgs&, int, hipStream_t, int&) { return false; }
 }
 using namespace smoe;
 static void* at(int64_t offset) { return (void*)(0x10000 + offset); }
@@ -63,15 +67,24 @@ extern "C" int s2s_pairs(int64_t K, int64_t N, int glu, int64_t pitch, int64_t h
   a.sym = a.saux = pitch, a.shm = h_pitch;
   return takes_pairs(a);
 }
-extern "C" int xty_tiles(int64_t E, int64_t K, int64_t N, int64_t L, int gathered, int bias, int n_contiguous, int64_t dy_pitch,
-                         int64_t x_pitch) {
+static XtYArgs xty_args(int64_t E, int64_t K, int64_t N, int64_t L, int gathered, int n_contiguous) {
   XtYArgs a{};
-  a.DY = at(0), a.X = at(0), a.DW = at(0), a.Db = bias ? at(0) : nullptr;
+  a.DY = at(0), a.X = at(0), a.DW = at(0), a.off = (const int64_t*)at(0);
   a.E = (int)E, a.K = (int)K, a.N = (int)N, a.L = (int)L;
-  a.sdyn = a.sxk = 1, a.sdym = dy_pitch, a.sxm = x_pitch, a.sdwe = K * N;
+  a.sdyn = a.sxk = 1, a.sdym = N, a.sxm = K, a.sdwe = K * N;
   a.sdwk = n_contiguous ? N : 1, a.sdwn = n_contiguous ? 1 : K;
   if (gathered) a.idx = (const int64_t*)at(0), a.fan_out = 2;
+  return a;
+}
+extern "C" int xty_tiles(int64_t E, int64_t K, int64_t N, int64_t L, int gathered, int bias, int n_contiguous, int64_t dy_pitch,
+                         int64_t x_pitch) {
+  XtYArgs a = xty_args(E, K, N, L, gathered, n_contiguous);
+  a.Db = bias ? at(0) : nullptr, a.sdym = dy_pitch, a.sxm = x_pitch;
   return (int)xty_class(a);
+}
+extern "C" int xty_gathers(int64_t E, int64_t K, int64_t N, int64_t L, int n_contiguous) {
+  int rc;
+  return try_xty_mfma(xty_args(E, K, N, L, 1, n_contiguous), SMOE_BF16, 0, rc);
 }
 extern "C" const char* xty_f32_launch(int64_t E, int64_t K, int64_t N, int64_t L, int64_t pad) {
   launched.clear();
@@ -212,3 +225,45 @@ def test_weight_gradients_that_keep_super_tiles(rules):
         # (each covers its own order)
         assert _workgroups(rules, 40, 9 * tile, 5 * tile, 256, wide) >= 40 * 45
         assert _workgroups(rules, 40, 9 * tile, 5 * tile, 257, wide) >= 40 * 48
+
+
+def test_held_operand(rules):
+    """One operand in registers: not for narrow panels (300 x 180 rows, 64 x 6080 231 -> 595 us under loads as 1 / rank^0.84), not with
+    few experts, one of which has most of the rows when loads differ (8 x 209 rows, 256 x 25344: 53 -> 86)."""
+    for layout in ("nk", "kn"):
+        shape = lambda panel, other: (panel, other) if layout == "kn" else (other, panel)
+        assert _xty(rules, 32, *shape(384, 2880), 188, layout) == "held" and _xty(rules, 32, *shape(320, 2880), 188, layout) == "small"
+        assert _xty(rules, 16, *shape(2048, 1536), 96, layout) == "held" and _xty(rules, 16, *shape(2048, 1536), 95, layout) == "small"
+        assert _xty(rules, 16, *shape(2048, 1536), 224, layout) == "held" and _xty(rules, 16, *shape(2048, 1536), 225, layout) == "small"
+        assert _xty(rules, 15, *shape(4096, 2048), 188, layout) == "small"
+        assert _xty(rules, 128, *shape(768, 64), 188, layout) == "held"
+
+
+def test_wide_gradients_look_rows_up_only_where_they_are_streamed(rules):
+    """Beyond 6144 columns the caller copies the gathered rows, unless they are streamed past the held operand."""
+    def gathers(N, rows, layout):
+        return bool(rules.xty_gathers(*(ctypes.c_int64(v) for v in (32, 2048, N, 32 * rows)), int(layout == "kn")))
+    assert gathers(6144, 188, "nk") and gathers(6144, 188, "kn") and gathers(6144, 300, "kn")
+    assert gathers(14336, 188, "nk") and not gathers(14336, 188, "kn") and not gathers(14336, 300, "nk")
+
+
+def test_python_side_of_the_held_operand_agrees(rules):
+    """The caller asks the same question before it decides on a copy (gradients with N contiguous, more than 512 tiles)."""
+    from types import SimpleNamespace
+    from scattermoe_amd.kernels import ops
+    rng, held = random.Random(1), 0
+    for _ in range(4000):
+        E, rows = rng.choice((8, 15, 16, 17, 64)), rng.choice((95, 96, 150, 224, 225))
+        K, N = rng.choice((376, 384, 1024, 2880)), rng.choice((2048, 2080, 2880, 6144))
+        L = E * rows + rng.choice((0, rng.randrange(E)))
+        L += L % 2
+        x_pitch = K + rng.choice((0, 0, 8, 2 ** 30 // (L // 2) // 8 * 8))
+        if E * -(-K // 256) * -(-N // 256) <= 512:
+            continue
+        DW = SimpleNamespace(shape=(E, K, N), stride=lambda i: (K * N, N, 1)[i])
+        X = SimpleNamespace(size=lambda i: (L // 2, K)[i], stride=lambda i: (x_pitch, 1)[i])
+        want = XTY_CLASSES[rules.xty_tiles(*(ctypes.c_int64(v) for v in (E, K, N, L)), 1, 0, 1, ctypes.c_int64(N),
+                                           ctypes.c_int64(x_pitch))] == "held"
+        assert ops._xty_holds_rows(DW, X, L) == want, (E, K, N, L, x_pitch)
+        held += want
+    assert 200 < held < 3000

@@ -81,6 +81,6 @@ def test_other_classes(E, K, N, rows, gather, kind, layout):
 # one group of 64 experts exactly, two, the most that are sorted, one more
 @pytest.mark.parametrize("E", [1, 2, 64, 65, 130, 256, 257])
 @pytest.mark.parametrize("kind", ["last", "halves"])
-@pytest.mark.parametrize("K,rows", [(136, 100), (392, 258)])      # super tiles whatever the loads; 256 x 128 tiles (64 experts and more)
+@pytest.mark.parametrize("K,rows", [(136, 100), (392, 258)])      # super tiles whatever the loads; by rows
 def test_numbers_of_experts(E, K, rows, kind):
     _run(E, K, 264, rows, kind, "nk", True, True, torch.bfloat16)
