@@ -2456,11 +2456,13 @@ static bool xty_held(const XtYArgs& a) {
 // 256 x 256 tile over 2000 random launches of 257 to 2047 rows per expert (4 to 128 experts, K and N from 256 to 8000, gathered
 // and not; even / Zipf-like loads, each in the order of XtYOrder).  256 x 128, 257 to 700 rows 1.10 / 1.17 times as fast, to 1200
 // 1.06 / 1.14, to 2047 1.03 / 1.11.  Not, gathered, beyond eight rounds from 1200 rows on (0.97 / 1.02: the lookups come twice as
-// often).  Not where an expert's output is one tile wide: two of 128 columns read the rows twice for it (30 random launches of 129 to 256
-// columns, even loads 0.96, 23 more than 3 % slower; us, 200 experts x 389 rows, 2752 x 256 177 -> 205, x 765, 3072 x 192 298 -> 339).  Not from 2048 rows on
-// (even loads 0.96, 17 of 27 more than 3 % slower; 200 x 3491 rows, 256 x 256 121 -> 137).  Small tiles against 256 x 128 while the
-// operands come from the memory-side cache, beyond one round: 257 to 700 rows, up to eight rounds 1.07 / 1.02, to 1200 rows, up to
-// four 1.07 / 1.02, to 2047 rows, up to two 1.07 / 1.02.
+// often), nor where the gathered operand is a single tile row (0.98 / 1.14, 10 of 29 even ones more than 3 % slower; us, 64 experts x 857
+// rows, 176 x 2520 98 -> 113); nor, a single tile row, with more experts than XtYOrder looks through (uneven loads of 300 0.81 to 0.96).
+// Not where an expert's output is one tile wide: two of 128 columns read the rows twice for it (30 random launches of 129 to 256
+// columns, even loads 0.96, 23 more than 3 % slower; 200 x 389 rows, 2752 x 256 177 -> 205, x 765, 3072 x 192 298 -> 339).  Not from
+// 2048 rows on (even loads 0.96, 17 of 27 more than 3 % slower; 200 x 3491 rows, 256 x 256 121 -> 137).  Small tiles against 256 x 128
+// while the operands come from the memory-side cache, beyond one round: 257 to 700 rows, up to eight rounds 1.07 / 1.02, to 1200
+// rows, up to four 1.07 / 1.02, to 2047 rows, up to two 1.07 / 1.02.
 // us, 32 experts x 500 rows, 2880 x 2880 346 -> 309; 32 x 300, 2880 x 5760 gathered 504 -> 467; 16 x 1000, 1024 x 1024 35.8 -> 34.4.
 // Same bits in every class.
 static constexpr int XTY_PAIR_ROUND = 2 * NUM_CU;
@@ -2475,6 +2477,7 @@ static bool xty_pairs(const XtYArgs& a) {
   const int64_t rows = a.L / a.E;
   const bool gathered = a.idx != nullptr;
   if (rows <= XTY_SMALL_ROWS || rows >= RS_XTY_MIN_ROWS || (p.nq > 128 && p.nq <= 256)) return false;
+  if (p.np <= 256 && ((gathered && !p.db_from_p) || p.E > 64 * XtYOrder::GROUPS)) return false;
   if (gathered && rows >= 1200 && xty_pair_tiles(p) > 8 * XTY_PAIR_ROUND) return false;
   // Output pieces of 16 bytes; rows that do not overlap (the descriptors end with the last one) and, gathered, a source below
   // 2 GiB.

@@ -172,6 +172,15 @@ def test_weight_gradients_of_one_tile_column_keep_wide_tiles(rules):
     assert _xty(rules, 200, 128, 2752, 600) == "pairs"
 
 
+def test_weight_gradients_of_one_tile_row_keep_wide_tiles(rules):
+    """Gathered rows that are looked up for every 128 columns of a single tile row (64 x 857 rows, 176 x 2520: 98 -> 113 us); uneven loads
+    of more experts than the order by rows looks through (300 x 663, 24 x 4168: 2490 -> 3070)."""
+    assert _xty(rules, 64, 176, 2520, 857, "kn", gathered=True) == "large"
+    assert _xty(rules, 64, 176, 2520, 857, "kn") == _xty(rules, 64, 264, 2520, 857, "kn", gathered=True) == "pairs"
+    assert _xty(rules, 64, 2520, 176, 857, "nk", gathered=True) == "pairs"
+    assert _xty(rules, 300, 4168, 24, 1200) == "large" and _xty(rules, 256, 4168, 24, 1200) == "pairs"
+
+
 def test_weight_gradients_of_many_rows_keep_wide_tiles(rules):
     """200 x 3491 rows, 256 x 256: 121 us in 256 x 256 tiles, 137 in 256 x 128."""
     for gathered, bias in ((True, False), (False, True)):
