@@ -276,3 +276,30 @@ def test_python_side_of_the_held_operand_agrees(rules):
         assert ops._xty_holds_rows(DW, X, L) == want, (E, K, N, L, x_pitch)
         held += want
     assert 200 < held < 3000
+
+
+@pytest.mark.parametrize("layout", ["nk", "kn"])
+def test_classes_that_the_gpu_tests_mean_to_run(rules, layout):
+    """test_gpu_xty_order and test_gpu_expanded_operands: the loads differ there, the averages are these."""
+    ask = lambda *sizes, **kw: _xty(rules, *sizes, layout, **kw)
+    for gathered, bias in ((False, True), (True, True)):
+        assert ask(8, 1288, 1032, 298, gathered=gathered, bias=bias) == "pairs"
+    for rows in (258, 700, 2046):
+        assert ask(4, 2056, 1544, rows, gathered=True, bias=True) == "pairs" and ask(2, 2824, 2568, rows, gathered=True, bias=True) == "small"
+    assert ask(12, 2056, 1544, 1200, bias=True) == "pairs"
+    assert ask(30, 264, 136, 100, gathered=True) == ask(8, 2056, 1544, 400, gathered=True) == ask(2, 3080, 2568, 2048) == "small"
+    assert ask(3, 3080, 5128, 2048, gathered=True) == "large" and ask(4, 2056, 1544, 2048) == "one wave"
+    for width in (64, 128, 192, 320):                      # test_gpu_xty_held
+        K, N = (width, 512) if layout == "nk" else (512, width)
+        assert ask(140, K, N, 148, gathered=True, bias=True) == "held"
+    assert ask(20, 832, 1024, 148) == ask(20, 832, 1024, 148, dy_pitch=0) == ask(20, 832, 1024, 148, x_pitch=0) == "held"
+    # rows on top of each other: neither descriptors that end with an operand's last row
+    for rows, other in ((300, "pairs"), (2048, "one wave")):
+        assert ask(4, 2056, 1544, rows) == other and ask(4, 2056, 1544, rows, dy_pitch=0) == ask(4, 2056, 1544, rows, x_pitch=0) == "large"
+
+
+def test_overlapping_weights_leave_the_one_wave_form(rules):
+    def tile(K, expanded):
+        return rules.s2s_launch(*(ctypes.c_int64(v) for v in (2, K, 14336, 1200)), 1, ctypes.c_int64(expanded)).decode()
+    assert "<256, 256, 2, 2, 2, true>" in tile(2048, 0) and "<256, 256, 2, 4>" in tile(2048, 1)
+    assert "<256, 128, 2, 2, 2, false, 2, true>" in tile(1024, 0) and "<256, 128, 2, 2, 2, false, 2, true>" in tile(1024, 1)

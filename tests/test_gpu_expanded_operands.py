@@ -8,15 +8,18 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("rows", [300, 2048])              # 256 x 128 tiles and the form of many rows
+# Shapes whose copies go in 256 x 128 tiles (300 rows) and in the form of many rows (2048): see test_dispatch_lines, which asks the
+# rules; 264 tiles of 256 x 256 leave the chip idle in a second round and go in small tiles, which take any rows
+@pytest.mark.parametrize("E,K,N", [(4, 2056, 1544), (2, 2568, 2824)])
+@pytest.mark.parametrize("rows", [300, 2048])
 @pytest.mark.parametrize("which", ["DY", "X"])
-def test_weight_gradient(rows, which):
+def test_weight_gradient(rows, which, E, K, N):
     g = torch.Generator(device=DEV).manual_seed(rows)
-    E, K, N = 2, 2568, 2824
-    off = torch.tensor([rows - 7, 2 * rows], device=DEV)
-    t = {"DY": torch.randn(2 * rows, N, generator=g, device=DEV).bfloat16(),
-         "X": torch.randn(2 * rows, K, generator=g, device=DEV).bfloat16()}
-    t[which] = t[which][:1].expand(2 * rows, -1)
+    L = E * rows
+    off = torch.tensor([rows - 7, 2 * rows, 3 * rows + 1, L][:E - 1] + [L], device=DEV)
+    t = {"DY": torch.randn(L, N, generator=g, device=DEV).bfloat16(),
+         "X": torch.randn(L, K, generator=g, device=DEV).bfloat16()}
+    t[which] = t[which][:1].expand(L, -1)
     c = {n: v.contiguous() for n, v in t.items()}
     a, _ = ops.group_bwd_W(t["DY"], t["X"], off, E)
     b, _ = ops.group_bwd_W(c["DY"], c["X"], off, E)

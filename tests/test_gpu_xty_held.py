@@ -18,11 +18,11 @@ def _check(got, want, mass, n, dtype):
     assert bool(((got.double() - want).abs() <= bound).all())
 
 
-def _inputs(K, N, dtype, k=2):
+def _inputs(K, N, dtype, k=2, loads=LOADS):
     g = torch.Generator(device=DEV).manual_seed(K + N)
-    E, L = len(LOADS), sum(LOADS)
+    E, L = len(loads), sum(loads)
     assert L % k == 0 and 96 <= L // E <= 224 and E * -(-K // 256) * -(-N // 256) >= 256
-    experts = torch.repeat_interleave(torch.arange(E, device=DEV), torch.tensor(LOADS, device=DEV))
+    experts = torch.repeat_interleave(torch.arange(E, device=DEV), torch.tensor(loads, device=DEV))
     experts = experts[torch.randperm(L, generator=g, device=DEV)].view(L // k, k)
     _, idx, off = ops.route(experts, E)
     X = torch.randn(L // k, K, generator=g, device=DEV).to(dtype)
@@ -78,3 +78,28 @@ def test_infinities_stay_with_their_expert(layout):
     keep = [e for e in range(E) if e != bad]
     assert torch.equal(DW[keep], want[keep]) and torch.equal(Db[keep], want_b[keep])
     assert bool(DW[bad].isnan().all())
+
+
+# column steps of 64: one, two, three (fewer than there are stages), five
+@pytest.mark.parametrize("width", [64, 128, 192, 320])
+@pytest.mark.parametrize("layout", ["nk", "kn"])
+def test_few_steps_and_more_experts_than_a_wave_has_lanes(width, layout):
+    """Experts of more than 256 rows in every group of 64."""
+    K, N = (width, 512) if layout == "nk" else (512, width)
+    E, X, DY, idx, off, k = _inputs(K, N, torch.bfloat16, loads=LOADS * 7)
+    like = torch.empty(E, K, N, dtype=torch.bfloat16, device=DEV) if layout == "kn" else None
+    DW, Db = ops.group_bwd_W(DY, X, off, E, has_bias=True, like=like, gather=(idx, k))
+    _check_all(DW, Db, ops.group(X, idx, fan_out=k), DY, off, torch.bfloat16)
+
+
+@pytest.mark.parametrize("which", ["DY", "X"])
+@pytest.mark.parametrize("layout", ["nk", "kn"])
+def test_rows_on_top_of_each_other(which, layout):
+    """An expanded row as either operand: the same bits as of a copy."""
+    E, X, DY, idx, off, k = _inputs(832, 1024, torch.bfloat16)
+    t = {"DY": DY, "X": ops.group(X, idx, fan_out=k)}
+    t[which] = t[which][:1].expand(DY.size(0), -1)
+    like = torch.empty(E, 832, 1024, dtype=torch.bfloat16, device=DEV) if layout == "kn" else None
+    DW, _ = ops.group_bwd_W(t["DY"], t["X"], off, E, like=like)
+    want, _ = ops.group_bwd_W(t["DY"].contiguous(), t["X"].contiguous(), off, E, like=like)
+    assert torch.equal(DW, want)

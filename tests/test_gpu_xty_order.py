@@ -64,14 +64,21 @@ def test_pairs(kind, layout, gather, bias, dtype):
     _run(8, 1288, 1032, 298, kind, layout, gather, bias, dtype)
 
 
-@pytest.mark.parametrize("rows", [96, 257, 700, 2047])
-def test_pairs_remainders(rows):
-    _run(2, 2824, 2568, rows + rows % 2, "halves", "nk", True, True, torch.bfloat16)
+# (252 of 256 x 256: 256 x 128 tiles at every one of these; 264 leave the chip idle in a second round and go in small tiles)
+@pytest.mark.parametrize("E,K,N", [(4, 2056, 1544), (2, 2824, 2568)])
+@pytest.mark.parametrize("rows", [96, 257, 700, 2046])
+def test_pairs_remainders(rows, E, K, N):
+    _run(E, K, N, rows + rows % 2, "halves", "nk", True, True, torch.bfloat16)
 
 
-# small tiles (few rows; two rounds of the larger ones), eight waves (gathered, many tiles), one wave per SIMD
-@pytest.mark.parametrize("E,K,N,rows,gather", [(30, 264, 136, 100, True), (8, 2056, 1544, 400, True), (3, 3080, 5128, 2048, True),
-                                               (2, 3080, 2568, 2048, False)])
+# more than a round of 256 x 128 tiles, beyond what goes in small ones
+def test_pairs_of_more_rounds():
+    _run(12, 2056, 1544, 1200, "halves", "kn", False, True, torch.bfloat16)
+
+
+# small tiles (few rows; two rounds of the larger ones; a second one partly filled), eight waves (gathered, 2048 rows), one wave per SIMD
+@pytest.mark.parametrize("E,K,N,rows,gather", [(30, 264, 136, 100, True), (8, 2056, 1544, 400, True), (2, 3080, 2568, 2048, False),
+                                               (3, 3080, 5128, 2048, True), (4, 2056, 1544, 2048, False)])
 @pytest.mark.parametrize("kind", ["even", "last", "halves"])
 @pytest.mark.parametrize("layout", ["nk", "kn"])
 def test_other_classes(E, K, N, rows, gather, kind, layout):
