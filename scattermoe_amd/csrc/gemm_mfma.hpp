@@ -2211,16 +2211,15 @@ struct XtYOrder {
   template <int SN>
   __device__ __forceinline__ bool map(const XtYPlan& a, int pid, int& e, int& m, int& n) const {
     const int lane = lane_id();
-    int m_tile, m_loc, n_loc;
-    const bool in_super = rast.map<SN>(pid, m_tile, n, m_loc, n_loc);
     const int x = pid & 7, i = pid >> 3;
-    int nth = 0, t = 0, rows[GROUPS];
+    int rows[GROUPS];
     bool uneven = false;
     if (by_rows) {
-      nth = __builtin_amdgcn_readfirstlane(i / chunk);
-      t = ((x + nth) & 7) * chunk + (i - nth * chunk);
-      const bool in_chunk = nth < a.E && t < p_tiles * q_tiles;
-      if (!in_super && !in_chunk) return false;              // (narrow outputs: three quarters of the super tiles' workgroups)
+      // (where most of a super tile's columns do not exist, workgroups with no tile in either order leave first)
+      if (2 * q_tiles <= SN && i / chunk >= a.E) {
+        int m_tile, m_loc, n_loc;
+        if (!rast.map<SN>(pid, m_tile, n, m_loc, n_loc)) return false;
+      }
       const int64_t L = a.off[a.E - 1];
 #pragma unroll
       for (int g = 0; g < GROUPS; ++g) {
@@ -2229,14 +2228,17 @@ struct XtYOrder {
         if (g * 64 < a.E && c < a.E) rows[g] = (int)(a.off[c] - (c ? a.off[c - 1] : 0));
         uneven = uneven || __ballot((int64_t)rows[g] * a.E > 2 * L) != 0;
       }
-      if (uneven && !in_chunk) return false;
     }
     if (!uneven) {
-      if (!in_super) return false;
+      int m_tile, m_loc, n_loc;
+      if (!rast.map<SN>(pid, m_tile, n, m_loc, n_loc)) return false;
       e = __builtin_amdgcn_readfirstlane(m_tile / p_tiles);
       m = m_tile - e * p_tiles;
       return true;
     }
+    int nth = __builtin_amdgcn_readfirstlane(i / chunk);
+    const int t = ((x + nth) & 7) * chunk + (i - nth * chunk);
+    if (nth >= a.E || t >= p_tiles * q_tiles) return false;
     // the nth expert by the power of two its load reaches (finer steps and groups that hold no expert cost each tile 1.5 us)
     int size[GROUPS], most = 0;
 #pragma unroll
