@@ -64,9 +64,10 @@ def test_pairs(kind, layout, gather, bias, dtype):
     _run(8, 1288, 1032, 298, kind, layout, gather, bias, dtype)
 
 
-# (252 of 256 x 256: 256 x 128 tiles at every one of these; 264 leave the chip idle in a second round and go in small tiles)
+# (252 of 256 x 256: 256 x 128 tiles up to 2046 rows, eight waves at 2048; 264 leave the chip idle in a second round and go in small
+# tiles)
 @pytest.mark.parametrize("E,K,N", [(4, 2056, 1544), (2, 2824, 2568)])
-@pytest.mark.parametrize("rows", [96, 257, 700, 2046])
+@pytest.mark.parametrize("rows", [96, 257, 700, 2046, 2047])
 def test_pairs_remainders(rows, E, K, N):
     _run(E, K, N, rows + rows % 2, "halves", "nk", True, True, torch.bfloat16)
 
