@@ -3,7 +3,7 @@
 // One workgroup owns one BM x BN output tile that never straddles two experts and walks the contraction in
 // slices of 64: global -> LDS directly (double buffered, or a ring of stages for the memory-bound small-row
 // classes), or global -> registers -> LDS in the one-wave-per-SIMD form of the 256 x 256 class (mainloop_rs)
-// -> MFMA 32x32x16 -> LDS-staged epilogue with 16-byte global accesses.
+// -> MFMA 16x16x32 -> LDS-staged epilogue with 16-byte global accesses.
 // Operands whose contraction axis is contiguous in memory ("direct": gathered X rows, weights stored
 // (N,K)) sit in LDS as [row][64] with a 16-byte XOR swizzle and are read with ds_read_b128; operands
 // whose contraction axis is strided ("transposed": weights stored (K,N), both operands of X^T dY) sit
@@ -53,16 +53,23 @@ namespace smoe {
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 static constexpr int BK = 64;               // contraction slice per stage
 
+// Products are 16 x 16 x 32, not 32 x 32 x 16: the launches run at the power cap, and the smaller shape moves a quarter of the
+// accumulators per instruction through the matrix cores for twice the operands.  Nothing but independent instructions on random
+// operands in registers, one wave per SIMD: 1.80 PFLOP/s with 32 x 32 x 16, 2.01 with 16 x 16 x 32.  One of these adds up its
+// 32 products in the order of two of those: the same bits.
 template <typename T> struct Mfma;
 template <> struct Mfma<bf16_t> {
-  static __device__ __forceinline__ f32x16 run(i32x4 a, i32x4 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  static __device__ __forceinline__ f32x4 run(i32x4 a, i32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ void in_place(i32x4 a, i32x4 b, f32x4& c) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
   }
   static __device__ __forceinline__ float sum8(i32x4 a) {
     const bf16x8 v = __builtin_bit_cast(bf16x8, a);
@@ -71,8 +78,11 @@ template <> struct Mfma<bf16_t> {
   }
 };
 template <> struct Mfma<f16_t> {
-  static __device__ __forceinline__ f32x16 run(i32x4 a, i32x4 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  static __device__ __forceinline__ f32x4 run(i32x4 a, i32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ void in_place(i32x4 a, i32x4 b, f32x4& c) {
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
   }
   static __device__ __forceinline__ float sum8(i32x4 a) {
     const f16x8 v = __builtin_bit_cast(f16x8, a);
@@ -80,6 +90,19 @@ template <> struct Mfma<f16_t> {
            (((float)v[4] + (float)v[5]) + ((float)v[6] + (float)v[7]));
   }
 };
+
+// The accumulators of a 32 x 32 block of the output: four 16 x 16 products, q[2 r + c] the one at (16 r, 16 c).  The MFMAs are
+// issued with the operands swapped (column operand first), so a lane holds, of group g, four consecutive columns of one row.
+struct Block {
+  f32x4 q[4];
+  __device__ __forceinline__ float operator[](int e) const { return q[e >> 2][e & 3]; }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) q[g] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+};
+__device__ __forceinline__ int block_row(int lane, int g) { return 16 * (g >> 1) + (lane & 15); }
+__device__ __forceinline__ int block_col(int lane, int g) { return 16 * (g & 1) + 4 * (lane >> 4); }
 
 typedef __attribute__((address_space(3))) char lds_char;
 
@@ -135,9 +158,11 @@ __device__ __forceinline__ const char* make_uniform(const char* p) {
 // the XOR swizzles below are applied on the global side.
 
 // ---- operand with contiguous contraction axis: LDS tile [EXT][64], 128 B per row ------------------------
-// piece p = (row, phys) holds contraction chunk c = phys ^ f(row); f makes the 16 lanes of a ds_read_b128
-// phase (16 consecutive rows, one chunk) hit 16 different 16-byte bank groups.
-__device__ __forceinline__ int direct_swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
+// piece p = (row, phys) holds contraction chunk c = phys ^ f(row).  A ds_read_b128 takes its lanes in groups of 16 that are not
+// consecutive (0-3, 12-15, 20-23, 24-27; 4-11, 16-19, 28-31; ...): of a fragment of 16 rows, eight rows of one chunk and the eight
+// others of the chunk next to it, which this f puts into 16 different 16-byte bank groups (16 cycles per fragment with four
+// waves reading; 32 with an f that separates 16 rows of one chunk).
+__device__ __forceinline__ int direct_swz(int row) { return row & 7; }
 
 template <int EXT, int NT, bool STREAM = false>
 struct DirectOp {
@@ -201,11 +226,10 @@ struct DirectOp {
       if (k0 + c * 8 >= kend) lds_write16(tile + p * 16, i32x4{0, 0, 0, 0});
     }
   }
-  // fragment of MFMA operand rows [base, base+32), contraction step ks (16 elements)
+  // fragment of MFMA operand rows [base, base+16), contraction step ks (32 elements)
   static __device__ __forceinline__ i32x4 frag(const char* tile, int base, int ks) {
     const int l = lane_id();
-    const int row = base + (l & 31);
-    return lds_read16(tile + row * 128 + (((2 * ks + (l >> 5)) ^ direct_swz(row)) << 4));
+    return lds_read16(tile + (base + (l & 15)) * 128 + (((4 * ks + (l >> 4)) ^ direct_swz(l & 15)) << 4));
   }
   // only operands that gather their contraction rows have anything to do here (see TransOp)
   __device__ __forceinline__ void fetch_rows(int, int) {}
@@ -215,15 +239,20 @@ struct DirectOp {
 
 // ---- operand with strided contraction axis: LDS tile [64][EXT], read transposed --------------------------
 // Row kr of the tile is EXT*2 bytes = G granules of 64 B (32 columns).  A ds_read_b64_tr_b16 phase touches
-// one granule column in 4 consecutive rows; storing granule g of row kr at position g ^ (kr & 3) spreads
-// those 4 accesses over all 64 banks.
+// half a granule (16 columns) in 4 consecutive rows and in the 4 rows 8 further down; storing granule g of row kr at position
+// g ^ (kr & 3), its halves exchanged in every second 8 rows, spreads those 8 accesses over all 64 banks.
+__device__ __forceinline__ int trans_piece(int kr, int phys) {      // logical 16-byte piece of row kr at position phys
+  return phys ^ ((kr & 3) << 2) ^ ((kr >> 2) & 2);
+}
 // GATHER: the contraction rows are not consecutive in memory but picked through an index vector (row r of the
 // operand is row rows[r] / fan of the source matrix).  The 64 rows of a slice are looked up once per workgroup, not
 // once per thread (vector-ALU work in this loop comes straight out of the matrix pipe's time): thread t < 64 fetches
 // the index of row t one slice ahead (`fetch_rows`, an ordinary load that the main loop's wait covers), turns it into
 // a byte offset and puts it into LDS before the loop's barrier (`stage_rows`); after the barrier every thread picks
 // the offsets of its own load slots up from there (`take_rows`).
-template <int EXT, int NT, bool STREAM = false, bool GATHER = false>
+// LEAN: one offset register for all load slots whose pieces differ by whole rows only, the rows between them added in scalar
+// registers (weight gradients: 128 registers per wave, or 256 accumulators, leave no room for one per slot).
+template <int EXT, int NT, bool STREAM = false, bool GATHER = false, bool LEAN = false>
 struct TransOp {
   static constexpr int CPR = EXT / 8;                  // 16-byte pieces per contraction row
   static constexpr int PIECES = 64 * CPR;
@@ -233,8 +262,13 @@ struct TransOp {
   static constexpr int LDS_BYTES = 64 * RS;
   static_assert(PIECES % NT == 0 && EXT % 128 == 0, "unsupported transposed tile width");
   const char* base;    // wave-uniform global address of (contraction 0, column 0 of the tile)
-  unsigned off[R];     // byte offset of this thread's piece of load slot j within the first slice
+  static constexpr int SLOT_ROWS = NT / CPR;           // contraction rows between load slots
+  static constexpr int OFFS = LEAN && !GATHER ? (SLOT_ROWS % 16 == 0 ? 1 : 2) : R;
+  static_assert(SLOT_ROWS % 8 == 0 || OFFS == R, "two kinds of rows");
+  unsigned off[OFFS];  // byte offset of this thread's piece of load slot j within the first slice
                        // (GATHER: within the slice that is issued next)
+  // (rot is 0 where OFFS < R) what load slot j adds to off[j % OFFS]
+  __device__ __forceinline__ unsigned slot_off(int j) const { return OFFS == R ? 0u : (unsigned)(j / OFFS * OFFS * SLOT_ROWS) * (unsigned)ld; }
   int rot = 0;         // load slot j carries round (j + rot) % R (see DirectOp)
   __device__ __forceinline__ int rnd(int j) const { const int r = j + rot; return r >= R ? r - R : r; }
   int64_t ld;          // bytes between contraction rows
@@ -242,8 +276,8 @@ struct TransOp {
   const int64_t* rows; // wave-uniform: index vector, already offset to the first contraction row
   unsigned fan;
   unsigned colb;       // byte offset of this thread's pieces inside their contraction rows (the rows of its load slots
-                       // differ by multiples of 4, which the swizzle does not see)
-  static_assert(!GATHER || NT / CPR % 4 == 0, "one column offset per thread");
+                       // differ by multiples of 16, which the swizzle does not see)
+  static_assert(!GATHER || NT / CPR % 16 == 0, "one column offset per thread");
   unsigned next_row;   // thread t < 64: index of contraction row t of the slice after the one being issued
   unsigned* srow;      // LDS, [2][64]: byte offsets of the rows of the slice to be issued next, by slice parity
   // contraction row inside a slice that load slot j of this thread carries
@@ -260,10 +294,10 @@ struct TransOp {
     ld = ld_bytes;
     const int t = threadIdx.x;
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
+    for (int j = 0; j < OFFS; ++j) {
       const int p = rnd(j) * NT + t;
       const int kr = p / CPR, phys = p % CPR;
-      const int cc = ((((phys >> 2) ^ (kr & 3)) << 2) | (phys & 3));      // logical 16-byte piece of the row
+      const int cc = trans_piece(kr, phys);
       if constexpr (GATHER) colb = (unsigned)col_of(cc * 8) * 2;
       else off[j] = (unsigned)(kr * ld_bytes) + (unsigned)col_of(cc * 8) * 2;
     }
@@ -307,7 +341,7 @@ struct TransOp {
   }
   __device__ __forceinline__ void issue_one(unsigned tile, int k0, int j) const {
     if constexpr (GATHER) load_to_lds16<STREAM>(make_uniform(base), off[j], tile + wave_uniform_id() * 1024 + rnd(j) * NT * 16);
-    else load_to_lds16<STREAM>(base + (int64_t)k0 * ld, off[j], tile + wave_uniform_id() * 1024 + rnd(j) * NT * 16);
+    else load_to_lds16<STREAM>(base + (int64_t)k0 * ld + slot_off(j), off[j % OFFS], tile + wave_uniform_id() * 1024 + rnd(j) * NT * 16);
   }
   // the same piece into registers (not for gathered rows), and where it belongs in the LDS tile
   // Contraction rows from `kend` on read as zeros: the buffer descriptor of the slice ends with row kend - 1
@@ -316,7 +350,7 @@ struct TransOp {
     const int64_t span = (int64_t)(kend - k0) * ld;
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(base + (int64_t)k0 * ld), 0, span < 0xffffffffLL ? (int)(unsigned)span : -1, 0x00020000);
-    return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off[j], 0, 0));
+    return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off[j % OFFS] + slot_off(j)), 0, 0));      // (a scalar offset would come off the range)
   }
   __device__ __forceinline__ int piece_lds(int j) const { return (rnd(j) * NT + (int)threadIdx.x) * 16; }
   __device__ __forceinline__ void issue(unsigned tile, int k0) const {
@@ -331,7 +365,7 @@ struct TransOp {
     } else {
       const int kr = slot_row(j);
       const bool ok = k0 + kr < kend;
-      load_to_lds16<STREAM>(base + (int64_t)k0 * ld, ok ? off[j] : off[j] - (unsigned)(kr * ld),
+      load_to_lds16<STREAM>(base + (int64_t)k0 * ld, off[j % OFFS] + slot_off(j) - (ok ? 0u : (unsigned)(kr * ld)),
                     tile + wave_uniform_id() * 1024 + rnd(j) * NT * 16);
     }
   }
@@ -348,15 +382,15 @@ struct TransOp {
     }
   }
   // Each 16-lane block transposes a 4 (contraction) x 16 (columns) patch: lane r of the block points at
-  // contraction row r/4, columns 4*(r%4)..+3 and receives column r, contraction 0..3.  Blocks 0/1 cover
-  // columns 0-15 / 16-31 of the 32-wide fragment, blocks 2/3 the contraction elements 8..15; a second
-  // read 4 rows further down completes the 8 elements per lane the MFMA expects (k = 8*(lane/32) + 0..7).
+  // contraction row r/4, columns 4*(r%4)..+3 and receives column r, contraction 0..3.  Block b covers the contraction
+  // elements 8*b..; a second read 4 rows further down completes the 8 elements per lane the MFMA expects
+  // (k = 8*(lane/16) + 0..7).
   static __device__ __forceinline__ i32x4 frag(const char* tile, int base, int ks) {
     const int l = lane_id();
     const int b = l >> 4, r = l & 15;
-    const int kr = ks * 16 + 8 * (b >> 1) + (r >> 2);
-    const int gran = (base >> 5) ^ (r >> 2);                       // (kr & 3) == r >> 2
-    const char* p = tile + kr * RS + (gran << 6) + (16 * (b & 1) + 4 * (r & 3)) * 2;
+    const int kr = ks * 32 + 8 * b + (r >> 2);
+    const int unit = (base >> 4) ^ ((r >> 2) << 1) ^ (b & 1);      // 32 bytes; (kr & 3) == r >> 2, (kr >> 3 & 1) == (b & 1)
+    const char* p = tile + kr * RS + (unit << 5) + (r & 3) * 8;
     const s16x4 lo = lds_read_tr(p);
     const s16x4 hi = lds_read_tr(p + 4 * RS);
     const s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -394,11 +428,12 @@ template <int EXT, int NT, bool GATHER>
 struct RowsOp {
   typedef TransOp<EXT, NT> Layout;
   static constexpr int R = Layout::R, LDS_BYTES = Layout::LDS_BYTES, DS_PER_FRAG = Layout::DS_PER_FRAG, CPR = Layout::CPR;
-  static_assert(NT / CPR % 4 == 0, "one column offset per thread");
+  static_assert(NT / CPR % 8 == 0, "one column offset per thread, or one for each of two kinds of load slots");
+  static constexpr int COLS = NT / CPR % 16 == 0 ? 1 : 2;
   const char* base;        // wave-uniform: (contraction 0, column 0 of the tile); GATHER: of the source matrix
   i32x4 rsrc;              // of the slice to be issued next
   unsigned off[R];
-  unsigned ld, colb;       // bytes
+  unsigned ld, colb[COLS]; // bytes (of load slot j: colb[j % COLS])
   int klen;
   // GATHER only
   const int64_t* rows;
@@ -407,14 +442,16 @@ struct RowsOp {
     base = make_uniform(b);
     ld = (unsigned)ld_bytes;
     klen = k;
-    const int kr = (int)threadIdx.x / CPR, phys = (int)threadIdx.x % CPR;
-    const int tc = ((((phys >> 2) ^ (kr & 3)) << 2) | (phys & 3)) * 8;
-    colb = tc < valid_cols ? tc * 2 : 0;                   // (such columns only feed outputs that are never stored)
+#pragma unroll
+    for (int j = 0; j < COLS; ++j) {
+      const int tc = trans_piece((j * NT + (int)threadIdx.x) / CPR, (int)threadIdx.x % CPR) * 8;
+      colb[j] = tc < valid_cols ? tc * 2 : 0;              // (such columns only feed outputs that are never stored)
+    }
   }
   __device__ __forceinline__ void init(const char* b, int64_t ld_bytes, int valid_cols, int k) {
     init_cols(b, ld_bytes, valid_cols, k);
 #pragma unroll
-    for (int j = 0; j < R; ++j) off[j] = (unsigned)((j * NT + (int)threadIdx.x) / CPR) * ld + colb;
+    for (int j = 0; j < R; ++j) off[j] = (unsigned)((j * NT + (int)threadIdx.x) / CPR) * ld + colb[j % COLS];
     take_rows(0);
   }
   // `span`: bytes from `b` to the end of the source matrix
@@ -455,7 +492,7 @@ struct RowsOp {
       asm volatile("" : "+v"(next_row));                   // (the compiler's wait for it: here, with nothing in flight)
 #pragma unroll
       for (int j = 0; j < R; ++j)
-        off[j] = (unsigned)__builtin_amdgcn_ds_bpermute((j * NT + (int)threadIdx.x) / CPR * 4, (int)row_off) + colb;
+        off[j] = (unsigned)__builtin_amdgcn_ds_bpermute((j * NT + (int)threadIdx.x) / CPR * 4, (int)row_off) + colb[j % COLS];
     } else {
       const int left = klen - slice * BK;
       rsrc = buffer_rsrc(base + (int64_t)slice * BK * ld, left > 0 ? (unsigned)min(left, BK) * ld : 0u);
@@ -503,19 +540,88 @@ struct Tile {
   static constexpr int WAVES_PER_SIMD = WG_ * NW / 4 > 0 ? WG_ * NW / 4 : 1;
   static constexpr int WTM = BM / WM, WTN = BN / WN;
   static constexpr int FM = WTM / 32, FN = WTN / 32;
-  static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile must be a multiple of the 32x32 MFMA");
+  static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile must be a multiple of a 32x32 block");
 };
+
+// A wave's products of a slice where fragments are read while others are multiplied.  A step of 32 contraction elements needs
+// 2 FM fragments of the row operand and 2 FN of the column operand (16 rows each), too many registers to hold twice.  It goes in
+// four quarters, each half of the row fragments times half of the column fragments, in an order in which a half is read during
+// the quarter before the one that needs it, into registers whose last use was the quarter before that: row halves 0 0 1 1,
+// column halves 0 1 1 0 in a slice's first step, 1 0 0 1 in its second.
+// Quarter Q = 0..7 of a slice:
+template <int Q>
+struct Quarter {
+  static constexpr int STEP = Q >> 2, C = Q & 3;
+  static constexpr int A = C >> 1, B = (C == 0 || C == 3 ? 0 : 1) ^ STEP;            // halves that it multiplies
+  // the half that is read meanwhile: of the row (else the column) operand, which half, of which step (2: next slice, step 0)
+  static constexpr bool READ_A = C == 1 || C == 2;
+  static constexpr int READ_HALF = READ_A ? (C == 1 ? 1 : 0) : 1 ^ STEP;
+  static constexpr int READ_STEP = C < 2 ? STEP : STEP + 1;
+};
+template <typename T, class TL, int Q>
+__device__ __forceinline__ void quarter_products(Block (&acc)[TL::FM][TL::FN], const i32x4 (&fa)[2 * TL::FM], const i32x4 (&fb)[2 * TL::FN]) {
+#pragma unroll
+  for (int u = 0; u < TL::FM * TL::FN; ++u) {
+    const int i = Quarter<Q>::A * TL::FM + u / TL::FN, j = Quarter<Q>::B * TL::FN + u % TL::FN;
+    f32x4& c = acc[i >> 1][j >> 1].q[2 * (i & 1) + (j & 1)];
+    c = Mfma<T>::run(fb[j], fa[i], c);
+  }
+}
+// Fragment number f of the half that is read in quarter Q, from the stage at `ta`, `tb`.
+template <class TL, class AOp, class BOp, int Q>
+__device__ __forceinline__ void quarter_read(const char* ta, const char* tb, int wm, int wn, int f, i32x4 (&fa)[2 * TL::FM],
+                                             i32x4 (&fb)[2 * TL::FN]) {
+  typedef Quarter<Q> Qu;
+  constexpr int step = Qu::READ_STEP & 1;
+  if constexpr (Qu::READ_A) {
+    const int i = Qu::READ_HALF * TL::FM + f;
+    fa[i] = AOp::frag(ta, wm * TL::WTM + i * 16, step);
+  } else {
+    const int j = Qu::READ_HALF * TL::FN + f;
+    fb[j] = BOp::frag(tb, wn * TL::WTN + j * 16, step);
+  }
+}
 
 // Main loop shared by both kernels.  acc[i][j] is the 32x32 block (i, j) of this wave's tile.
 // Full 64-deep slices travel global -> LDS directly (no registers, no ds_write) one slice ahead of the
 // MFMAs; a trailing partial slice is zero-filled in LDS after it has landed.
 // If `rowsum`, rs[i] additionally accumulates, per lane, the sum of the lane's own 8 contraction elements of
-// A-fragment i; adding lanes l and l+32 afterwards gives the sum over the contraction of A row l%32.
+// A-fragment i; adding lanes l, l+16, l+32 and l+48 afterwards gives the sum over the contraction of A row l%16.
+template <typename T, class TL, class AOp, class BOp, int Q, bool CAN_ROWSUM>
+__device__ __forceinline__ void mainloop_quarter(const char* ta, const char* tb, int wm, int wn, bool rowsum,
+                                                 Block (&acc)[TL::FM][TL::FN], float (&rs)[2 * TL::FM],
+                                                 i32x4 (&fa)[2 * TL::FM], i32x4 (&fb)[2 * TL::FN]) {
+  typedef Quarter<Q> Qu;
+  // (four workgroups per CU hide a wave's wait for its row fragments, and have no registers to read them ahead)
+  constexpr bool LATE_A = TL::WG > 2;
+  constexpr int NF = Qu::READ_STEP == 2 || (LATE_A && Qu::READ_A) ? 0 : Qu::READ_A ? TL::FM : TL::FN;
+  if constexpr (LATE_A && Q > 0 && (Qu::C & 1) == 0) {
+#pragma unroll
+    for (int i = 0; i < TL::FM; ++i)
+      fa[Qu::A * TL::FM + i] = AOp::frag(ta, wm * TL::WTM + (Qu::A * TL::FM + i) * 16, Qu::STEP);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int f = 0; f < NF; ++f) quarter_read<TL, AOp, BOp, Q>(ta, tb, wm, wn, f, fa, fb);
+  quarter_products<T, TL, Q>(acc, fa, fb);
+  if (CAN_ROWSUM && rowsum && (Qu::C & 1) == 0) {
+#pragma unroll
+    for (int i = 0; i < TL::FM; ++i) rs[Qu::A * TL::FM + i] += Mfma<T>::sum8(fa[Qu::A * TL::FM + i]);
+  }
+  // Interleave: the LDS reads are spread between the first MFMAs.
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    __builtin_amdgcn_sched_group_barrier(0x100, Qu::READ_A ? AOp::DS_PER_FRAG : BOp::DS_PER_FRAG, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+  }
+  if constexpr (TL::FM * TL::FN > NF) __builtin_amdgcn_sched_group_barrier(0x008, TL::FM * TL::FN - NF, 0);
+  __builtin_amdgcn_sched_barrier(0);
+}
 template <typename T, class TL, class AOp, class BOp, bool CAN_ROWSUM>
 __device__ __forceinline__ void mainloop(AOp& A, BOp& B, int klen, char* lds, bool rowsum,
-                                         f32x16 (&acc)[TL::FM][TL::FN], float (&rs)[TL::FM]) {
+                                         Block (&acc)[TL::FM][TL::FN], float (&rs)[2 * TL::FM]) {
   constexpr int STAGE = AOp::LDS_BYTES + BOp::LDS_BYTES;
-  const int wave = threadIdx.x >> 6;
+  const int wave = threadIdx.x >> 6, l = lane_id();
   const int wm = wave / TL::WN, wn = wave % TL::WN;
   const int nfull = klen / BK;
   const bool tail = (klen % BK) != 0;
@@ -559,45 +665,19 @@ __device__ __forceinline__ void mainloop(AOp& A, BOp& B, int klen, char* lds, bo
     }
     const char* ta = cur;
     const char* tb = cur + AOp::LDS_BYTES;
-    i32x4 fa[2][TL::FM], fb[2][TL::FN];
+    i32x4 fa[2 * TL::FM], fb[2 * TL::FN];
 #pragma unroll
-    for (int i = 0; i < TL::FM; ++i) fa[0][i] = AOp::frag(ta, wm * TL::WTM + i * 32, 0);
+    for (int i = 0; i < TL::FM; ++i) fa[i] = AOp::frag(ta, wm * TL::WTM + i * 16, 0);
 #pragma unroll
-    for (int j = 0; j < TL::FN; ++j) fb[0][j] = BOp::frag(tb, wn * TL::WTN + j * 32, 0);
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      const int c = ks & 1, n = c ^ 1;
-      if (ks + 1 < BK / 16) {
-#pragma unroll
-        for (int i = 0; i < TL::FM; ++i) fa[n][i] = AOp::frag(ta, wm * TL::WTM + i * 32, ks + 1);
-#pragma unroll
-        for (int j = 0; j < TL::FN; ++j) fb[n][j] = BOp::frag(tb, wn * TL::WTN + j * 32, ks + 1);
-      }
-#pragma unroll
-      for (int i = 0; i < TL::FM; ++i)
-#pragma unroll
-        for (int j = 0; j < TL::FN; ++j) acc[i][j] = Mfma<T>::run(fb[c][j], fa[c][i], acc[i][j]);
-      if (CAN_ROWSUM && rowsum) {
-#pragma unroll
-        for (int i = 0; i < TL::FM; ++i) rs[i] += Mfma<T>::sum8(fa[c][i]);
-      }
-      // Interleave: the LDS reads of step ks+1 are spread between the MFMAs of step ks.
-      if (ks + 1 < BK / 16) {
-#pragma unroll
-        for (int i = 0; i < TL::FM; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x100, AOp::DS_PER_FRAG, 0);
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        }
-#pragma unroll
-        for (int j = 0; j < TL::FN; ++j) {
-          __builtin_amdgcn_sched_group_barrier(0x100, BOp::DS_PER_FRAG, 0);
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        }
-        if constexpr (TL::FM * TL::FN > TL::FM + TL::FN)
-          __builtin_amdgcn_sched_group_barrier(0x008, TL::FM * TL::FN - TL::FM - TL::FN, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    for (int j = 0; j < TL::FN; ++j) fb[j] = BOp::frag(tb, wn * TL::WTN + j * 16, 0);
+    mainloop_quarter<T, TL, AOp, BOp, 0, CAN_ROWSUM>(ta, tb, wm, wn, rowsum, acc, rs, fa, fb);
+    mainloop_quarter<T, TL, AOp, BOp, 1, CAN_ROWSUM>(ta, tb, wm, wn, rowsum, acc, rs, fa, fb);
+    mainloop_quarter<T, TL, AOp, BOp, 2, CAN_ROWSUM>(ta, tb, wm, wn, rowsum, acc, rs, fa, fb);
+    mainloop_quarter<T, TL, AOp, BOp, 3, CAN_ROWSUM>(ta, tb, wm, wn, rowsum, acc, rs, fa, fb);
+    mainloop_quarter<T, TL, AOp, BOp, 4, CAN_ROWSUM>(ta, tb, wm, wn, rowsum, acc, rs, fa, fb);
+    mainloop_quarter<T, TL, AOp, BOp, 5, CAN_ROWSUM>(ta, tb, wm, wn, rowsum, acc, rs, fa, fb);
+    mainloop_quarter<T, TL, AOp, BOp, 6, CAN_ROWSUM>(ta, tb, wm, wn, rowsum, acc, rs, fa, fb);
+    mainloop_quarter<T, TL, AOp, BOp, 7, CAN_ROWSUM>(ta, tb, wm, wn, rowsum, acc, rs, fa, fb);
   }
 }
 
@@ -606,11 +686,11 @@ __device__ __forceinline__ void mainloop(AOp& A, BOp& B, int klen, char* lds, bo
 // the memory pipeline has taken all of them (it takes one 1 KB wave-load per ~17 cycles and CU), and loads spread over
 // the slice leave the late ones too little time to land when LDS is the only place they can land in: here every
 // thread's pieces of a slice (16 in a 256 x 256 tile) sit in registers for up to two slices, which LDS has no room for.
-//   set S = (kt + 1) & 1 holds slice kt + 1: its pieces are written to the other LDS stage during steps 0-2 of
-//   slice kt (ds_write_b128, spread evenly: behind every third MFMA) and each is reloaded with slice kt + 3 one step
-//   later (the last quarter of them in step 0 of the next slice), one load per 4 MFMAs throughout;
-//   one barrier per slice, after step 2: behind it the fragments of step 0 of slice kt + 1 are read while the
-//   MFMAs of step 3 run.
+//   set S = (kt + 1) & 1 holds slice kt + 1: its pieces are written to the other LDS stage during the first six of
+//   slice kt's eight quarters (ds_write_b128, spread evenly: behind every sixth MFMA) and each is reloaded with slice kt + 3 two
+//   quarters later (the last of them in the first two quarters of the next slice), one load per 8 MFMAs throughout;
+//   one barrier per slice, after six quarters: behind it the first fragments of slice kt + 1 are read while the
+//   last two quarters are multiplied.
 // Whole 64-deep slices only, at least two of them (the launcher checks); loads past the end re-read the last slice.
 //
 // A thread's pieces of a slice in the order they are written and reloaded: the operands alternate while the row
@@ -619,108 +699,92 @@ template <class TL, class AOp, class BOp>
 struct RsPlan {
   static_assert(AOp::R <= BOp::R && BOp::R == 8, "the column operand is the larger one");
   static constexpr int N = AOp::R + BOp::R;                       // pieces per thread and slice
-  static constexpr int NM = TL::FM * TL::FN;                      // MFMAs per step
-  static constexpr int L = (N + 3) / 4;                           // loads per step (step 0: what is left)
-  static_assert(N <= 3 * NM, "at most one LDS write behind an MFMA");
+  static constexpr int NM = TL::FM * TL::FN;                      // MFMAs per quarter of a step (Quarter), eight of them per slice
+  static constexpr int L = (N + 3) / 4;                           // loads per two quarters (the first two: what is left)
+  static_assert(N <= 6 * NM, "at most one LDS write behind an MFMA");
   static constexpr bool is_b(int q) { return q >= 2 * AOp::R || (q & 1); }
   static constexpr int index(int q) { return q < 2 * AOp::R ? q >> 1 : q - AOp::R; }
-  // pieces written before MFMA g of steps 0-2
-  static constexpr int written(int g) { return N * (g + 1) / (3 * NM); }
-  static_assert(written(0) == 0 && written(3 * NM) == N, "every piece is written once");
-  static_assert(written(NM) >= L && written(2 * NM) >= 2 * L && N >= 3 * L, "a piece is reloaded after it has been written");
-  // fragments of the next step read behind MFMA m: one behind each, the surplus of small tiles behind the first
-  static constexpr int NF = TL::FM + TL::FN, FIRST = NF > NM ? NF - NM + 1 : 1;
-  static constexpr int frags_before(int m) { return m == 0 ? 0 : FIRST + m - 1 < NF ? FIRST + m - 1 : NF; }
-  static constexpr int loads_before(int n, int m) { return n * m / NM; }
+  // pieces written before MFMA g of the first six quarters
+  static constexpr int written(int g) { return N * (g + 1) / (6 * NM); }
+  static_assert(written(0) == 0 && written(6 * NM) == N, "every piece is written once");
+  static_assert(written(2 * NM) >= L && written(4 * NM) >= 2 * L && N >= 3 * L, "a piece is reloaded after it has been written");
+  static constexpr int loads_before(int n, int m) { return n * m / (2 * NM); }
+  // LDS: the two stages of the row operand, then those of the column operand, so that the instructions' offset fields reach from
+  // one stage to the other (one set of addresses)
+  static constexpr int A_STAGE = AOp::LDS_BYTES, B0 = 2 * AOp::LDS_BYTES, B_STAGE = BOp::LDS_BYTES;
 };
 
-template <typename T, class TL, class AOp, class BOp, int P, int KS, int N>
-__device__ __forceinline__ void rs_step(const AOp& A, const BOp& B, const char* __restrict__ cur, char* __restrict__ nxt,
-                                        int k2, int k3, int kend, int wm, int wn,
-                                        f32x16 (&acc)[TL::FM][TL::FN], i32x4 (&g)[2][N],
-                                        i32x4 (&fa)[2][TL::FM], i32x4 (&fb)[2][TL::FN]) {
+template <typename T, class TL, class AOp, class BOp, int P, int Q, int N>
+__device__ __forceinline__ void rs_quarter(const AOp& A, const BOp& B, char* lds, int k2, int k3, int kend, int wm, int wn,
+                                           Block (&acc)[TL::FM][TL::FN], i32x4 (&g)[2][N],
+                                           i32x4 (&fa)[2 * TL::FM], i32x4 (&fb)[2 * TL::FN]) {
   typedef RsPlan<TL, AOp, BOp> Plan;
-  constexpr int FM = TL::FM, FN = TL::FN, NM = Plan::NM;
-  constexpr int S = P ^ 1;
-  constexpr int c = KS & 1, n = c ^ 1;
-  // LDS traffic of the step in the order it is to be issued in (the compiler keeps reads and writes of LDS in
-  // program order): the fragments of the next step behind the first MFMAs - from the stage being multiplied, in
-  // step 3 from the stage just filled - and the pieces of steps 0-2 spread evenly.
-  const char* src = KS < 3 ? cur : (const char*)nxt;
-  constexpr int fstep = KS < 3 ? KS + 1 : 0;
-#pragma unroll
-  for (int m = 0; m < NM; ++m) {
-#pragma unroll
-    for (int f = Plan::frags_before(m); f < Plan::frags_before(m + 1); ++f) {
-      if (f < FM) fa[n][f] = AOp::frag(src, wm * TL::WTM + f * 32, fstep);
-      else fb[n][f - FM] = BOp::frag(src + AOp::LDS_BYTES, wn * TL::WTN + (f - FM) * 32, fstep);
-    }
-    if (KS < 3 && Plan::written(KS * NM + m + 1) > Plan::written(KS * NM + m)) {
-      const int q = Plan::written(KS * NM + m);
-      if (Plan::is_b(q)) lds_write16(nxt + AOp::LDS_BYTES + B.piece_lds(Plan::index(q)), g[S][q]);
-      else lds_write16(nxt + A.piece_lds(Plan::index(q)), g[S][q]);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = Mfma<T>::run(fb[c][j], fa[c][i], acc[i][j]);
-  // pieces loaded in this step: the last ones of the other set (slice kt + 2), then a third each of the others of
+  typedef Quarter<Q> Qu;
+  constexpr int NM = Plan::NM, S = P ^ 1;
+  constexpr int NF = Qu::READ_A ? TL::FM : TL::FN;
+  static_assert(NF <= NM, "at most one fragment read behind an MFMA");
+  // LDS traffic of the quarter in the order it is to be issued in (the compiler keeps reads and writes of LDS in
+  // program order): the fragments that are read in it behind the first MFMAs - from the stage being multiplied, in
+  // the last two quarters from the stage just filled - and the pieces of the first six spread evenly.
+  constexpr int src = Qu::READ_STEP == 2 ? S : P;
+  // pieces loaded in two quarters: the last ones of the other set (slice kt + 2), then a third each of the others of
   // this one (slice kt + 3)
-  constexpr int SET = KS == 0 ? P : S;
-  constexpr int q0 = KS == 0 ? 3 * Plan::L : (KS - 1) * Plan::L, nl = KS == 0 ? N - 3 * Plan::L : Plan::L;
-#pragma unroll
-  for (int q = q0; q < q0 + nl; ++q) {
-    const int k0 = KS == 0 ? k2 : k3;
-    g[SET][q] = Plan::is_b(q) ? B.load_piece(k0, kend, Plan::index(q)) : A.load_piece(k0, kend, Plan::index(q));
-  }
+  constexpr int H = Q >> 1, SET = H == 0 ? P : S;
+  constexpr int q0 = H == 0 ? 3 * Plan::L : (H - 1) * Plan::L, nl = H == 0 ? N - 3 * Plan::L : Plan::L;
+  constexpr int m0 = (Q & 1) * NM;
+  const int k0 = H == 0 ? k2 : k3;
 #pragma unroll
   for (int m = 0; m < NM; ++m) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-#pragma unroll
-    for (int f = Plan::frags_before(m); f < Plan::frags_before(m + 1); ++f) {
-      if (f < FM) __builtin_amdgcn_sched_group_barrier(0x100, AOp::DS_PER_FRAG, 0);
-      else __builtin_amdgcn_sched_group_barrier(0x100, BOp::DS_PER_FRAG, 0);
+    const int i = Qu::A * TL::FM + m / TL::FN, j = Qu::B * TL::FN + m % TL::FN;
+    Mfma<T>::in_place(fb[j], fa[i], acc[i >> 1][j >> 1].q[2 * (i & 1) + (j & 1)]);
+    if (m < NF) quarter_read<TL, AOp, BOp, Q>(lds + src * Plan::A_STAGE, lds + Plan::B0 + src * Plan::B_STAGE, wm, wn, m, fa, fb);
+    if (Q < 6 && Plan::written(Q * NM + m + 1) > Plan::written(Q * NM + m)) {
+      const int q = Plan::written(Q * NM + m);
+      if (Plan::is_b(q)) lds_write16(lds + Plan::B0 + S * Plan::B_STAGE + B.piece_lds(Plan::index(q)), g[S][q]);
+      else lds_write16(lds + S * Plan::A_STAGE + A.piece_lds(Plan::index(q)), g[S][q]);
     }
-    if (KS < 3 && Plan::written(KS * NM + m + 1) > Plan::written(KS * NM + m)) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-    if (Plan::loads_before(nl, m + 1) > Plan::loads_before(nl, m)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+    if (Plan::loads_before(nl, m0 + m + 1) > Plan::loads_before(nl, m0 + m)) {
+      const int q = q0 + Plan::loads_before(nl, m0 + m);
+      g[SET][q] = Plan::is_b(q) ? B.load_piece(k0, kend, Plan::index(q)) : A.load_piece(k0, kend, Plan::index(q));
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (KS == 2) {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // this thread's pieces are in LDS, its reads of `cur` done
+  if constexpr (Q == 5) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // this thread's pieces are in LDS, its reads of this stage done
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
 template <typename T, class TL, class AOp, class BOp, int P, int N>
-__device__ __forceinline__ void rs_slice(const AOp& A, const BOp& B, const char* cur, char* nxt,
-                                         int kt, int last_k0, int kend, int wm, int wn,
-                                         f32x16 (&acc)[TL::FM][TL::FN], i32x4 (&g)[2][N],
-                                         i32x4 (&fa)[2][TL::FM], i32x4 (&fb)[2][TL::FN]) {
+__device__ __forceinline__ void rs_slice(const AOp& A, const BOp& B, char* lds, int kt, int last_k0, int kend, int wm, int wn,
+                                         Block (&acc)[TL::FM][TL::FN], i32x4 (&g)[2][N],
+                                         i32x4 (&fa)[2 * TL::FM], i32x4 (&fb)[2 * TL::FN]) {
   const int k2 = min((kt + 2) * BK, last_k0), k3 = min((kt + 3) * BK, last_k0);
   __builtin_amdgcn_sched_barrier(0);
-  rs_step<T, TL, AOp, BOp, P, 0, N>(A, B, cur, nxt, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_step<T, TL, AOp, BOp, P, 1, N>(A, B, cur, nxt, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_step<T, TL, AOp, BOp, P, 2, N>(A, B, cur, nxt, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_step<T, TL, AOp, BOp, P, 3, N>(A, B, cur, nxt, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 0, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 1, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 2, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 3, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 4, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 5, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 6, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 7, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
 }
 
 template <typename T, class TL, class AOp, class BOp>
-__device__ __forceinline__ void mainloop_rs(const AOp& A, const BOp& B, int klen, char* lds,
-                                            f32x16 (&acc)[TL::FM][TL::FN]) {
+__device__ __forceinline__ void mainloop_rs(const AOp& A, const BOp& B, int klen, char* lds, Block (&acc)[TL::FM][TL::FN]) {
   typedef RsPlan<TL, AOp, BOp> Plan;
   constexpr int N = Plan::N;
-  static_assert(BK == 64, "four steps per slice");
-  constexpr int STAGE = AOp::LDS_BYTES + BOp::LDS_BYTES;
-  const int wave = threadIdx.x >> 6;
+  static_assert(BK == 64, "eight quarters per slice");
+  const int wave = threadIdx.x >> 6, l = lane_id();
   const int wm = wave / TL::WN, wn = wave % TL::WN;
   // A partial last slice only with operands that zero-fill (TransOp); without any contraction rows one slice of
   // zeros is multiplied (no branch around the loop: 256 accumulator registers would have to be merged behind it).
   const int nk = max(1, (klen + BK - 1) / BK);
   const int last_k0 = (nk - 1) * BK;
   i32x4 g[2][N];
-  i32x4 fa[2][TL::FM], fb[2][TL::FN];
+  i32x4 fa[2 * TL::FM], fb[2 * TL::FN];
   const int k1 = min(BK, last_k0), k2 = min(2 * BK, last_k0);
   auto load = [&](int k0, int q) {
     return Plan::is_b(q) ? B.load_piece(k0, klen, Plan::index(q)) : A.load_piece(k0, klen, Plan::index(q));
@@ -731,7 +795,7 @@ __device__ __forceinline__ void mainloop_rs(const AOp& A, const BOp& B, int klen
   for (int q = 0; q < N; ++q) g[1][q] = load(k1, q);
 #pragma unroll
   for (int q = 0; q < N; ++q) {
-    if (Plan::is_b(q)) lds_write16(lds + AOp::LDS_BYTES + B.piece_lds(Plan::index(q)), g[0][q]);
+    if (Plan::is_b(q)) lds_write16(lds + Plan::B0 + B.piece_lds(Plan::index(q)), g[0][q]);
     else lds_write16(lds + A.piece_lds(Plan::index(q)), g[0][q]);
   }
 #pragma unroll
@@ -739,22 +803,20 @@ __device__ __forceinline__ void mainloop_rs(const AOp& A, const BOp& B, int klen
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
+  // what the first quarter multiplies
 #pragma unroll
-  for (int i = 0; i < TL::FM; ++i) fa[0][i] = AOp::frag(lds, wm * TL::WTM + i * 32, 0);
+  for (int i = 0; i < TL::FM; ++i) fa[i] = AOp::frag(lds, wm * TL::WTM + i * 16, 0);
 #pragma unroll
-  for (int j = 0; j < TL::FN; ++j) fb[0][j] = BOp::frag(lds + AOp::LDS_BYTES, wn * TL::WTN + j * 32, 0);
-  // The second stage starts 64 KB into LDS (in a 256-row tile), beyond what the offset field of an LDS instruction can
-  // add: its addresses are formed from a base of their own (kept from being folded into constants), not with one
-  // vector-ALU instruction per access.
-  unsigned second = STAGE;
-  asm volatile("" : "+v"(second));
-  char* lds1 = lds + second;
+  for (int j = 0; j < TL::FN; ++j) fb[j] = BOp::frag(lds + Plan::B0, wn * TL::WTN + j * 16, 0);
   int kt = 0;
   for (; kt + 1 < nk; kt += 2) {
-    rs_slice<T, TL, AOp, BOp, 0, N>(A, B, lds, lds1, kt, last_k0, klen, wm, wn, acc, g, fa, fb);
-    rs_slice<T, TL, AOp, BOp, 1, N>(A, B, lds1, lds, kt + 1, last_k0, klen, wm, wn, acc, g, fa, fb);
+    rs_slice<T, TL, AOp, BOp, 0, N>(A, B, lds, kt, last_k0, klen, wm, wn, acc, g, fa, fb);
+    rs_slice<T, TL, AOp, BOp, 1, N>(A, B, lds, kt + 1, last_k0, klen, wm, wn, acc, g, fa, fb);
   }
-  if (kt < nk) rs_slice<T, TL, AOp, BOp, 0, N>(A, B, lds, lds1, kt, last_k0, klen, wm, wn, acc, g, fa, fb);
+  if (kt < nk) rs_slice<T, TL, AOp, BOp, 0, N>(A, B, lds, kt, last_k0, klen, wm, wn, acc, g, fa, fb);
+  // (the compiler does not know how long the products above, being assembly, take to write their accumulators: 19 wait states at
+  // the most; they are read by assembly, see stage_accumulators)
+  asm volatile("s_nop 15\n\ts_nop 3");
 }
 
 // Main loop of the class with two workgroups of four waves per CU (256 x 128 tiles, wave tiles of up to 128 x 64).  Its
@@ -768,11 +830,11 @@ __device__ __forceinline__ void mainloop_rs(const AOp& A, const BOp& B, int klen
 // `rowsum` and rs as in mainloop.
 static constexpr int PAIR_STAGE = 32 * 1024, PAIR_B = 2 * PAIR_STAGE, PAIR_LDS = PAIR_B + 16 * 1024;
 template <typename T, class TL, class AOp, class BOp, bool ROWS>
-__device__ __forceinline__ void mainloop_pair(AOp& A, BOp& B, int klen, char* lds, bool rowsum, f32x16 (&acc)[TL::FM][TL::FN],
-                                              float (&rs)[TL::FM]) {
+__device__ __forceinline__ void mainloop_pair(AOp& A, BOp& B, int klen, char* lds, bool rowsum, Block (&acc)[TL::FM][TL::FN],
+                                              float (&rs)[2 * TL::FM]) {
   static_assert(AOp::LDS_BYTES <= PAIR_STAGE && BOp::LDS_BYTES <= PAIR_LDS - PAIR_B, "LDS");
-  constexpr int KS = BK / 16, LOADS = AOp::R + BOp::R, PER_STEP = (LOADS + KS - 2) / (KS - 1);      // (all of them up front: 2 % slower)
-  const int wave = threadIdx.x >> 6;
+  constexpr int KS = 2 * (BK / 32), LOADS = AOp::R + BOp::R, PER_STEP = (LOADS + KS - 2) / (KS - 1);      // (all of them up front: 2 % slower)
+  const int wave = threadIdx.x >> 6, l = lane_id();
   const int wm = wave / TL::WN, wn = wave % TL::WN;
   const unsigned lds_u = lds_address(lds);
   const int nk = ROWS ? max(1, (klen + BK - 1) / BK) : klen / BK;      // (no rows: one slice of zeros)
@@ -792,15 +854,15 @@ __device__ __forceinline__ void mainloop_pair(AOp& A, BOp& B, int klen, char* ld
       A.take_rows(kt + 1);
       B.take_rows(kt + 1);
     }
-    i32x4 fa[2][TL::FM], fb[KS][TL::FN];
+    // half of the row fragments of a step of 32 at a time, the next half read meanwhile
+    i32x4 fa[2][TL::FM], fb[BK / 32][2 * TL::FN];
+    auto row_frag = [&](int h, int i) { return AOp::frag(ta, wm * TL::WTM + ((h & 1) * TL::FM + i) * 16, h >> 1); };
 #pragma unroll
-    for (int j = 0; j < TL::FN; ++j) fb[0][j] = BOp::frag(tb, wn * TL::WTN + j * 32, 0);
+    for (int j = 0; j < 2 * TL::FN; ++j) fb[0][j] = BOp::frag(tb, wn * TL::WTN + j * 16, 0);
 #pragma unroll
-    for (int i = 0; i < TL::FM; ++i) fa[0][i] = AOp::frag(ta, wm * TL::WTM + i * 32, 0);
+    for (int i = 0; i < TL::FM; ++i) fa[0][i] = row_frag(0, i);
 #pragma unroll
-    for (int ks = 1; ks < KS; ++ks)
-#pragma unroll
-      for (int j = 0; j < TL::FN; ++j) fb[ks][j] = BOp::frag(tb, wn * TL::WTN + j * 32, ks);
+    for (int j = 0; j < 2 * TL::FN; ++j) fb[1][j] = BOp::frag(tb, wn * TL::WTN + j * 16, 1);
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // everyone has the column operand's fragments
     __builtin_amdgcn_sched_barrier(0);
@@ -828,15 +890,19 @@ __device__ __forceinline__ void mainloop_pair(AOp& A, BOp& B, int klen, char* ld
       }
       if (ks + 1 < KS) {
 #pragma unroll
-        for (int i = 0; i < TL::FM; ++i) fa[n][i] = AOp::frag(ta, wm * TL::WTM + i * 32, ks + 1);
+        for (int i = 0; i < TL::FM; ++i) fa[n][i] = row_frag(ks + 1, i);
       }
 #pragma unroll
       for (int i = 0; i < TL::FM; ++i)
 #pragma unroll
-        for (int j = 0; j < TL::FN; ++j) acc[i][j] = Mfma<T>::run(fb[ks][j], fa[c][i], acc[i][j]);
+        for (int j = 0; j < 2 * TL::FN; ++j) {
+          const int r = c * TL::FM + i;
+          f32x4& d = acc[r >> 1][j >> 1].q[2 * (r & 1) + (j & 1)];
+          d = Mfma<T>::run(fb[ks >> 1][j], fa[c][i], d);
+        }
       if (ROWS && rowsum) {
 #pragma unroll
-        for (int i = 0; i < TL::FM; ++i) rs[i] += Mfma<T>::sum8(fa[c][i]);
+        for (int i = 0; i < TL::FM; ++i) rs[c * TL::FM + i] += Mfma<T>::sum8(fa[c][i]);
       }
       if (ks + 1 < KS) {
 #pragma unroll
@@ -844,7 +910,7 @@ __device__ __forceinline__ void mainloop_pair(AOp& A, BOp& B, int klen, char* ld
           __builtin_amdgcn_sched_group_barrier(0x100, AOp::DS_PER_FRAG, 0);
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         }
-        if constexpr (TL::FM * TL::FN > TL::FM) __builtin_amdgcn_sched_group_barrier(0x008, TL::FM * TL::FN - TL::FM, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 2 * TL::FM * TL::FN - TL::FM, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -858,12 +924,12 @@ __device__ __forceinline__ void mainloop_pair(AOp& A, BOp& B, int klen, char* ld
 // slices travel through a ring of NS stages; NS-1 slices are on their way while one is being multiplied.
 template <typename T, class TL, class AOp, class BOp>
 __device__ __forceinline__ void mainloop_ring(const AOp& A, const BOp& B, int klen, char* lds,
-                                              f32x16 (&acc)[TL::FM][TL::FN]) {
+                                              Block (&acc)[TL::FM][TL::FN]) {
   constexpr int STAGE = AOp::LDS_BYTES + BOp::LDS_BYTES;
   constexpr int NS = TL::NS;
   constexpr int LOADS = AOp::R + BOp::R;               // direct loads per thread and slice
   static_assert((NS - 2) * LOADS <= 63, "vmcnt cannot count that many loads in flight");
-  const int wave = threadIdx.x >> 6;
+  const int wave = threadIdx.x >> 6, l = lane_id();
   const int wm = wave / TL::WN, wn = wave % TL::WN;
   const int nfull = klen / BK;
   const bool tail = (klen % BK) != 0;
@@ -891,32 +957,32 @@ __device__ __forceinline__ void mainloop_ring(const AOp& A, const BOp& B, int kl
     __syncthreads();                 // everyone's part of slice kt is there; everyone is done with slice kt-1
     const int prev = slot == 0 ? NS - 1 : slot - 1;
     SMOE_RING_ISSUE(kt + NS - 1, prev);
-    i32x4 fa[BK / 16][TL::FM], fb[BK / 16][TL::FN];
+    i32x4 fa[BK / 32][2 * TL::FM], fb[BK / 32][2 * TL::FN];
 #pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
+    for (int ks = 0; ks < BK / 32; ++ks) {
 #pragma unroll
-      for (int i = 0; i < TL::FM; ++i) fa[ks][i] = AOp::frag(cur, wm * TL::WTM + i * 32, ks);
+      for (int i = 0; i < 2 * TL::FM; ++i) fa[ks][i] = AOp::frag(cur, wm * TL::WTM + i * 16, ks);
 #pragma unroll
-      for (int j = 0; j < TL::FN; ++j) fb[ks][j] = BOp::frag(cur + AOp::LDS_BYTES, wn * TL::WTN + j * 32, ks);
+      for (int j = 0; j < 2 * TL::FN; ++j) fb[ks][j] = BOp::frag(cur + AOp::LDS_BYTES, wn * TL::WTN + j * 16, ks);
     }
 #pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks)
+    for (int ks = 0; ks < BK / 32; ++ks)
 #pragma unroll
-      for (int i = 0; i < TL::FM; ++i)
+      for (int i = 0; i < 2 * TL::FM; ++i)
 #pragma unroll
-        for (int j = 0; j < TL::FN; ++j) acc[i][j] = Mfma<T>::run(fb[ks][j], fa[ks][i], acc[i][j]);
+        for (int j = 0; j < 2 * TL::FN; ++j) {
+          f32x4& c = acc[i >> 1][j >> 1].q[2 * (i & 1) + (j & 1)];
+          c = Mfma<T>::run(fb[ks][j], fa[ks][i], c);
+        }
     slot = slot + 1 == NS ? 0 : slot + 1;
   }
 #undef SMOE_RING_ISSUE
 }
 
-// Store the wave's accumulators.  The MFMAs are issued with the operands swapped (column operand first), so
-// acc[i][j] holds the TRANSPOSE of output block (i, j): a lane owns output row i*32 + lane%32 and, per group
-// g of four registers, the four consecutive columns j*32 + 8*g + 4*(lane/32) + 0..3 - one 8-byte store per
-// group instead of four 2-byte stores.  dst[m] is the element offset of output row m of the tile (or -1),
+// Store the wave's accumulators: per group of four (see Block) one 8-byte store instead of four 2-byte stores.  dst[m] is the element offset of output row m of the tile (or -1),
 // columns n0 + [0, BN) clipped to ncols (contiguous); optional bias (already offset to the expert), stride sb.
 template <typename T, class TL>
-__device__ __forceinline__ void epilogue(const f32x16 (&acc)[TL::FM][TL::FN], T* __restrict__ out,
+__device__ __forceinline__ void epilogue(const Block (&acc)[TL::FM][TL::FN], T* __restrict__ out,
                                          const int64_t* dst, int n0, int ncols,
                                          const T* __restrict__ bias, int64_t sb) {
   typedef T T4 __attribute__((ext_vector_type(4)));
@@ -925,12 +991,12 @@ __device__ __forceinline__ void epilogue(const f32x16 (&acc)[TL::FM][TL::FN], T*
   const bool base_ok = ((uintptr_t)out & 7) == 0;
 #pragma unroll
   for (int i = 0; i < TL::FM; ++i) {
-    const int64_t d = dst[wm * TL::WTM + i * 32 + (l & 31)];
 #pragma unroll
-    for (int j = 0; j < TL::FN; ++j) {
+    for (int g = 0; g < 4; ++g) {
+      const int64_t d = dst[wm * TL::WTM + i * 32 + block_row(l, g)];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n = n0 + wn * TL::WTN + j * 32 + g * 8 + (l >> 5) * 4;
+      for (int j = 0; j < TL::FN; ++j) {
+        const int n = n0 + wn * TL::WTN + j * 32 + block_col(l, g);
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -976,28 +1042,43 @@ __device__ __forceinline__ int staged_addr(int row, int col) {
   return row * (TL::BN * 2) + ((((col >> 3) ^ row) & (CPR - 1)) << 4) + ((col & 7) << 1);
 }
 
+// The thread's index, for what comes behind the main loop: the one-wave-per-SIMD form, and four workgroups per CU, have no
+// registers to hold what the compiler would derive from it ahead of the loop.
+template <class TL>
+__device__ __forceinline__ int late_thread() {
+  int t = (int)threadIdx.x;
+  if constexpr (TL::RS || TL::WG > 2) asm volatile("" : "+v"(t));
+  return t;
+}
 // `bias_of(tile_col)` returns the value to add to that column (0 without bias).
 template <typename T, class TL, typename BF>
-__device__ __forceinline__ void stage_accumulators(const f32x16 (&acc)[TL::FM][TL::FN], char* lds, BF bias_of,
+__device__ __forceinline__ void stage_accumulators(const Block (&acc)[TL::FM][TL::FN], char* lds, BF bias_of,
                                                    float* sbias) {
   typedef T T4 __attribute__((ext_vector_type(4)));
-  const int wave = threadIdx.x >> 6, l = lane_id();
+  const int tx = late_thread<TL>(), wave = tx >> 6, l = tx & 63;
   const int wm = wave / TL::WN, wn = wave % TL::WN;
   // One wave per SIMD: the additions per column come from LDS (written here, one column per thread), so that the
   // walk over the 256 accumulator registers below is one straight piece of code without loads or branches.
   if constexpr (TL::RS) {
-    for (int t = threadIdx.x; t < TL::BN; t += TL::NT) sbias[t] = bias_of(t);
+    for (int t = tx; t < TL::BN; t += TL::NT) sbias[t] = bias_of(t);
   }
   __syncthreads();                                   // every wave is done reading operands
+  // One wave per SIMD: accumulators leave their registers where they are used (left to the compiler, all of them are copied ahead),
+  // behind the wait at the main loop's end.
+  auto value = [](float x) {
+    if constexpr (!TL::RS) return x;
+    float v;
+    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(x));
+    return v;
+  };
 #pragma unroll
   for (int j = 0; j < TL::FN; ++j) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int col = wn * TL::WTN + j * 32 + g * 8 + (l >> 5) * 4;
+    for (int c = 0; c < 2; ++c) {
+      const int col = wn * TL::WTN + j * 32 + block_col(l, c);
       float bv[4];
       if constexpr (TL::RS) {
-        typedef float f32x4_t __attribute__((ext_vector_type(4)));
-        const f32x4_t b4 = *(const f32x4_t*)(sbias + col);
+        const f32x4 b4 = *(const f32x4*)(sbias + col);
 #pragma unroll
         for (int e = 0; e < 4; ++e) bv[e] = b4[e];
       } else {
@@ -1005,16 +1086,29 @@ __device__ __forceinline__ void stage_accumulators(const f32x16 (&acc)[TL::FM][T
         for (int e = 0; e < 4; ++e) bv[e] = bias_of(col + e);
       }
 #pragma unroll
-      for (int i = 0; i < TL::FM; ++i) {
-        const int row = wm * TL::WTM + i * 32 + (l & 31);
+      for (int i = 0; i < 2 * TL::FM; ++i) {
+        const int g = 2 * (i & 1) + c, row = wm * TL::WTM + (i >> 1) * 32 + block_row(l, g);
         T4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = from_f32<T>(acc[i][j][g * 4 + e] + bv[e]);
+        for (int e = 0; e < 4; ++e) v[e] = from_f32<T>(value(acc[i >> 1][j].q[g][e]) + bv[e]);
         *(T4*)(lds + staged_addr<TL>(row, col)) = v;
       }
     }
   }
   __syncthreads();
+}
+
+// What is added to output column n; to column tc of a tile of the fused forward GLU (hidden columns from nh0).
+template <typename T>
+__device__ __forceinline__ float plain_bias(const T* __restrict__ bias, int64_t sb, int ncols, int n) {
+  return bias != nullptr && n < ncols ? to_f32(bias[(int64_t)n * sb]) : 0.0f;
+}
+template <typename T, class TL>
+__device__ __forceinline__ float glu_bias(const S2SArgs& a, const T* __restrict__ bias, int nh0, int tc) {
+  constexpr int HALF = TL::WTN / 2;
+  const int j = tc % TL::WTN;
+  const int hc = nh0 + (tc / TL::WTN) * HALF + j % HALF;
+  return bias != nullptr && hc < a.N ? to_f32(bias[(int64_t)(hc + (j >= HALF ? a.N : 0)) * a.sbn]) : 0.0f;
 }
 
 // Fused gated-linear-unit epilogues (rows in grouped order: output row = row0 + m).
@@ -1023,7 +1117,7 @@ __device__ __forceinline__ void stage_accumulators(const f32x16 (&acc)[TL::FM][T
 // rounded to the storage type first and the hidden value is computed from the rounded values, i.e. the same
 // arithmetic as storing the pre-activation and running the stand-alone pass over it.
 template <typename T, class TL>
-__device__ __forceinline__ void epilogue_glu_fwd(const f32x16 (&acc)[TL::FM][TL::FN], const S2SArgs& a, int row0,
+__device__ __forceinline__ void epilogue_glu_fwd(const Block (&acc)[TL::FM][TL::FN], const S2SArgs& a, int row0,
                                                  int rows, int nh0, const T* __restrict__ bias) {
   if constexpr (TL::FN % 2 == 0) {
     typedef T T4 __attribute__((ext_vector_type(4)));
@@ -1037,13 +1131,13 @@ __device__ __forceinline__ void epilogue_glu_fwd(const f32x16 (&acc)[TL::FM][TL:
     const bool vec_ok = (((uintptr_t)pre | (uintptr_t)hid) & 7) == 0 && ((a.sym | a.shm | F) & 3) == 0;
 #pragma unroll
     for (int i = 0; i < TL::FM; ++i) {
-      const int m = wm * TL::WTM + i * 32 + (l & 31);
-      const int64_t row = row0 + m;
 #pragma unroll
       for (int j = 0; j < FH; ++j) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          const int n = nh0 + wn * (TL::WTN / 2) + j * 32 + g * 8 + (l >> 5) * 4;
+          const int m = wm * TL::WTM + i * 32 + block_row(l, g);
+          const int64_t row = row0 + m;
+          const int n = nh0 + wn * (TL::WTN / 2) + j * 32 + block_col(l, g);
           T first[4], second[4], h[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
@@ -1084,7 +1178,7 @@ __device__ __forceinline__ void epilogue_glu_fwd(const f32x16 (&acc)[TL::FM][TL:
 // Backward: the product is d(hidden); it is rounded to the storage type and turned into d(pre-activation)
 // with the saved pre-activation, exactly as the stand-alone pass would do from a stored d(hidden).
 template <typename T, class TL>
-__device__ __forceinline__ void epilogue_glu_bwd(const f32x16 (&acc)[TL::FM][TL::FN], const S2SArgs& a, int row0,
+__device__ __forceinline__ void epilogue_glu_bwd(const Block (&acc)[TL::FM][TL::FN], const S2SArgs& a, int row0,
                                                  int rows, int n0) {
   typedef T T4 __attribute__((ext_vector_type(4)));
   const int wave = threadIdx.x >> 6, l = lane_id();
@@ -1096,15 +1190,14 @@ __device__ __forceinline__ void epilogue_glu_bwd(const f32x16 (&acc)[TL::FM][TL:
   const bool vec_ok = (((uintptr_t)pre | (uintptr_t)dpre) & 7) == 0 && ((a.sym | a.saux | F) & 3) == 0;
 #pragma unroll
   for (int i = 0; i < TL::FM; ++i) {
-    const int m = wm * TL::WTM + i * 32 + (l & 31);
-    if (m >= rows) continue;
-    const int64_t row = row0 + m;
 #pragma unroll
     for (int j = 0; j < TL::FN; ++j) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int n = n0 + wn * TL::WTN + j * 32 + g * 8 + (l >> 5) * 4;
-        if (n >= F) continue;
+        const int m = wm * TL::WTM + i * 32 + block_row(l, g);
+        const int64_t row = row0 + m;
+        const int n = n0 + wn * TL::WTN + j * 32 + block_col(l, g);
+        if (m >= rows || n >= F) continue;
         const bool vec = vec_ok && n + 3 < F;
         T p1[4], p2[4], o1[4], o2[4];
         if (vec) {
@@ -1171,15 +1264,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rows_rsrc(void* base, int
 }
 
 template <typename T, class TL>
-__device__ __forceinline__ void epilogue_staged(const f32x16 (&acc)[TL::FM][TL::FN], T* __restrict__ out,
+__device__ __forceinline__ void epilogue_staged(const Block (&acc)[TL::FM][TL::FN], T* __restrict__ out,
                                                 const int64_t* dst, int n0, int ncols, const T* __restrict__ bias,
-                                                int64_t sb, char* lds, float* sbias = nullptr) {
+                                                int64_t sb, char* lds) {
+  const int tx = late_thread<TL>();
   typedef T T8 __attribute__((ext_vector_type(8)));
   constexpr int CPR = TL::BN / 8, PIECES = TL::BM * CPR, PP = PIECES / TL::NT;
   static_assert(PIECES % TL::NT == 0, "pieces must divide evenly");
-  stage_accumulators<T, TL>(acc, lds, [&](int tc) {
-    return bias != nullptr && n0 + tc < ncols ? to_f32(bias[(int64_t)(n0 + tc) * sb]) : 0.0f;
-  }, sbias);
+  if constexpr (!TL::RS)
+    stage_accumulators<T, TL>(acc, lds, [&](int tc) { return plain_bias<T>(bias, sb, ncols, n0 + tc); }, nullptr);
   // In groups: the row offsets of a group, then its pieces, are read from LDS back to back before the first of its
   // stores (written as one conditional store per piece, every piece would wait for two LDS round trips of its own)
   constexpr int GRP = PP % 16 == 0 ? 16 : PP % 8 == 0 ? 8 : PP;
@@ -1189,17 +1282,17 @@ __device__ __forceinline__ void epilogue_staged(const f32x16 (&acc)[TL::FM][TL::
     int64_t d[GRP];
     T8 v[GRP];
 #pragma unroll
-    for (int g = 0; g < GRP; ++g) d[g] = dst[((q0 + g) * TL::NT + threadIdx.x) / CPR];
+    for (int g = 0; g < GRP; ++g) d[g] = dst[((q0 + g) * TL::NT + tx) / CPR];
 #pragma unroll
     for (int g = 0; g < GRP; ++g) {
-      const int p = (q0 + g) * TL::NT + threadIdx.x;
+      const int p = (q0 + g) * TL::NT + tx;
       v[g] = *(const T8*)(lds + staged_addr<TL>(p / CPR, (p % CPR) * 8));
     }
 #pragma unroll
     for (int g = 0; g < GRP; ++g) asm volatile("" : "+v"(v[g]), "+v"(d[g]));      // keeps the reads above the branches
 #pragma unroll
     for (int g = 0; g < GRP; ++g) {
-      const int n = n0 + (((q0 + g) * TL::NT + threadIdx.x) % CPR) * 8;
+      const int n = n0 + (((q0 + g) * TL::NT + tx) % CPR) * 8;
       if (d[g] >= 0 && n < ncols) stream_store(v[g], (T8*)(out + d[g] + n));
     }
   }
@@ -1208,20 +1301,17 @@ __device__ __forceinline__ void epilogue_staged(const f32x16 (&acc)[TL::FM][TL::
 // Forward GLU through LDS: both halves staged (tile column order: per wave block WTN/2 first-half columns, then
 // the matching second-half columns); per 16-byte piece of hidden columns two LDS reads, three coalesced stores.
 template <typename T, class TL>
-__device__ __forceinline__ void epilogue_glu_fwd_staged(const f32x16 (&acc)[TL::FM][TL::FN], const S2SArgs& a,
+__device__ __forceinline__ void epilogue_glu_fwd_staged(const Block (&acc)[TL::FM][TL::FN], const S2SArgs& a,
                                                         int row0, int rows, int nh0, const T* __restrict__ bias,
-                                                        char* lds, float* sbias = nullptr) {
+                                                        char* lds) {
   {
+    const int tx = late_thread<TL>();
     typedef T T8 __attribute__((ext_vector_type(8)));
     constexpr int HALF = TL::WTN / 2;
     constexpr int CPR = TL::BN / 16, PIECES = TL::BM * CPR, PP = PIECES / TL::NT;
     static_assert(PIECES % TL::NT == 0 && HALF % 8 == 0, "pieces must divide evenly");
     const int F = a.N;
-    stage_accumulators<T, TL>(acc, lds, [&](int tc) {
-      const int j = tc % TL::WTN;
-      const int hc = nh0 + (tc / TL::WTN) * HALF + j % HALF;
-      return bias != nullptr && hc < F ? to_f32(bias[(int64_t)(hc + (j >= HALF ? F : 0)) * a.sbn]) : 0.0f;
-    }, sbias);
+    if constexpr (!TL::RS) stage_accumulators<T, TL>(acc, lds, [&](int tc) { return glu_bias<T, TL>(a, bias, nh0, tc); }, nullptr);
     T* pre = (T*)a.Y;
     T* hid = (T*)a.H;
     // a group's LDS reads are issued back to back ahead of its arithmetic and stores (see epilogue_staged)
@@ -1236,7 +1326,7 @@ __device__ __forceinline__ void epilogue_glu_fwd_staged(const f32x16 (&acc)[TL::
       T8 v1[GRP], v2[GRP];
 #pragma unroll
       for (int g = 0; g < GRP; ++g) {
-        const int p = (q0 + g) * TL::NT + threadIdx.x;
+        const int p = (q0 + g) * TL::NT + tx;
         const int row = p / CPR, hc = (p % CPR) * 8;          // hidden column inside the tile
         const int tc = (hc / HALF) * TL::WTN + hc % HALF;     // tile column of the first-half value
         v1[g] = *(const T8*)(lds + staged_addr<TL>(row, tc));
@@ -1246,7 +1336,7 @@ __device__ __forceinline__ void epilogue_glu_fwd_staged(const f32x16 (&acc)[TL::
       for (int g = 0; g < GRP; ++g) asm volatile("" : "+v"(v1[g]), "+v"(v2[g]));
 #pragma unroll
       for (int g = 0; g < GRP; ++g) {
-        const int p = (q0 + g) * TL::NT + threadIdx.x;
+        const int p = (q0 + g) * TL::NT + tx;
         const int row = p / CPR, n = nh0 + (p % CPR) * 8;
         if (row >= rows || n >= F) continue;
         const T8 first = v1[g], second = v2[g];
@@ -1275,13 +1365,14 @@ __device__ __forceinline__ void epilogue_glu_fwd_staged(const f32x16 (&acc)[TL::
 // Backward through LDS: d(hidden) tile staged, then every thread handles 16-byte pieces (8 columns of one row):
 // two coalesced 16-byte loads of the saved pre-activation, two coalesced 16-byte stores of its gradient.
 template <typename T, class TL>
-__device__ __forceinline__ void epilogue_glu_bwd_staged(const f32x16 (&acc)[TL::FM][TL::FN], const S2SArgs& a,
-                                                        int row0, int rows, int n0, char* lds, float* sbias = nullptr) {
+__device__ __forceinline__ void epilogue_glu_bwd_staged(const Block (&acc)[TL::FM][TL::FN], const S2SArgs& a,
+                                                        int row0, int rows, int n0, char* lds) {
+  const int tx = late_thread<TL>();
   typedef T T8 __attribute__((ext_vector_type(8)));
   constexpr int CPR = TL::BN / 8, PIECES = TL::BM * CPR, PP = PIECES / TL::NT;
   constexpr int GRP = PP % 8 == 0 ? 4 : PP % 4 == 0 ? 2 : (PP >= 2 ? PP / 2 : 1);    // pieces per group, two in flight
   static_assert(PIECES % TL::NT == 0 && (PP == 1 || PP % (2 * GRP) == 0), "pieces must divide evenly");
-  stage_accumulators<T, TL>(acc, lds, [](int) { return 0.0f; }, sbias);
+  if constexpr (!TL::RS) stage_accumulators<T, TL>(acc, lds, [](int) { return 0.0f; }, nullptr);
   const int F = a.N;
   const T* pre = (const T*)a.aux;
   T* dpre = (T*)a.Y;
@@ -1295,7 +1386,7 @@ __device__ __forceinline__ void epilogue_glu_bwd_staged(const f32x16 (&acc)[TL::
   auto fetch = [&](auto buf, int q0) {
 #pragma unroll
     for (int u = 0; u < GRP; ++u) {
-      const int p = (q0 + u) * TL::NT + threadIdx.x;
+      const int p = (q0 + u) * TL::NT + tx;
       const int row = p / CPR, n = n0 + (p % CPR) * 8;
       const T* src = pre + (int64_t)(row0 + (row < rows ? row : 0)) * a.saux + (n < F ? n : 0);
       // read exactly once per step: the non-temporal hint keeps it from displacing operand panels in the L2 (-0.3 %)
@@ -1307,12 +1398,12 @@ __device__ __forceinline__ void epilogue_glu_bwd_staged(const f32x16 (&acc)[TL::
     T8 dh[GRP];
 #pragma unroll
     for (int u = 0; u < GRP; ++u) {
-      const int p = (q0 + u) * TL::NT + threadIdx.x;
+      const int p = (q0 + u) * TL::NT + tx;
       dh[u] = *(const T8*)(lds + staged_addr<TL>(p / CPR, (p % CPR) * 8));
     }
 #pragma unroll
     for (int u = 0; u < GRP; ++u) {
-      const int p = (q0 + u) * TL::NT + threadIdx.x;
+      const int p = (q0 + u) * TL::NT + tx;
       const int row = p / CPR, n = n0 + (p % CPR) * 8;
       T8 o1, o2;
 #pragma unroll
@@ -1352,16 +1443,16 @@ __device__ __forceinline__ void epilogue_glu_bwd_staged(const f32x16 (&acc)[TL::
 // pairs per row; per 16-byte piece one LDS read, one 16-byte store of the pre-activation (if wanted) and one
 // 8-byte store of four hidden values.
 template <typename T, class TL>
-__device__ __forceinline__ void epilogue_oss_fwd_staged(const f32x16 (&acc)[TL::FM][TL::FN], const S2SArgs& a,
+__device__ __forceinline__ void epilogue_oss_fwd_staged(const Block (&acc)[TL::FM][TL::FN], const S2SArgs& a,
                                                         int row0, int rows, int n0, const T* __restrict__ bias,
-                                                        char* lds, float* sbias = nullptr) {
+                                                        char* lds) {
+  const int tx = late_thread<TL>();
   typedef T T8 __attribute__((ext_vector_type(8)));
   typedef T T4 __attribute__((ext_vector_type(4)));
   constexpr int CPR = TL::BN / 8, PIECES = TL::BM * CPR, PP = PIECES / TL::NT;
   static_assert(PIECES % TL::NT == 0, "pieces must divide evenly");
-  stage_accumulators<T, TL>(acc, lds, [&](int tc) {
-    return bias != nullptr && n0 + tc < a.N ? to_f32(bias[(int64_t)(n0 + tc) * a.sbn]) : 0.0f;
-  }, sbias);
+  if constexpr (!TL::RS)
+    stage_accumulators<T, TL>(acc, lds, [&](int tc) { return plain_bias<T>(bias, a.sbn, a.N, n0 + tc); }, nullptr);
   T* pre = (T*)a.Y;
   T* hid = (T*)a.H;
   constexpr int GRP = PP % 16 == 0 ? 16 : PP % 8 == 0 ? 8 : PP;      // LDS reads of a group back to back (see epilogue_staged)
@@ -1371,14 +1462,14 @@ __device__ __forceinline__ void epilogue_oss_fwd_staged(const f32x16 (&acc)[TL::
     T8 vs[GRP];
 #pragma unroll
     for (int g = 0; g < GRP; ++g) {
-      const int p = (q0 + g) * TL::NT + threadIdx.x;
+      const int p = (q0 + g) * TL::NT + tx;
       vs[g] = *(const T8*)(lds + staged_addr<TL>(p / CPR, (p % CPR) * 8));
     }
 #pragma unroll
     for (int g = 0; g < GRP; ++g) asm volatile("" : "+v"(vs[g]));
 #pragma unroll
     for (int g = 0; g < GRP; ++g) {
-      const int p = (q0 + g) * TL::NT + threadIdx.x;
+      const int p = (q0 + g) * TL::NT + tx;
       const int row = p / CPR, n = n0 + (p % CPR) * 8;
       if (row >= rows || n >= a.N) continue;
       const T8 v = vs[g];
@@ -1397,13 +1488,14 @@ __device__ __forceinline__ void epilogue_oss_fwd_staged(const f32x16 (&acc)[TL::
 // gpt-oss backward through LDS: d(hidden) tile staged; per piece of 8 hidden columns two 16-byte loads of the saved
 // pre-activation pairs and two 16-byte stores of their gradient.
 template <typename T, class TL>
-__device__ __forceinline__ void epilogue_oss_bwd_staged(const f32x16 (&acc)[TL::FM][TL::FN], const S2SArgs& a,
-                                                        int row0, int rows, int n0, char* lds, float* sbias = nullptr) {
+__device__ __forceinline__ void epilogue_oss_bwd_staged(const Block (&acc)[TL::FM][TL::FN], const S2SArgs& a,
+                                                        int row0, int rows, int n0, char* lds) {
+  const int tx = late_thread<TL>();
   typedef T T8 __attribute__((ext_vector_type(8)));
   constexpr int CPR = TL::BN / 8, PIECES = TL::BM * CPR, PP = PIECES / TL::NT;
   constexpr int GRP = PP % 8 == 0 ? 4 : PP % 4 == 0 ? 2 : (PP >= 2 ? PP / 2 : 1);    // pieces per group, two in flight
   static_assert(PIECES % TL::NT == 0 && (PP == 1 || PP % (2 * GRP) == 0), "pieces must divide evenly");
-  stage_accumulators<T, TL>(acc, lds, [](int) { return 0.0f; }, sbias);
+  if constexpr (!TL::RS) stage_accumulators<T, TL>(acc, lds, [](int) { return 0.0f; }, nullptr);
   const int F = a.N;
   const T* pre = (const T*)a.aux;
   T* dpre = (T*)a.Y;
@@ -1413,7 +1505,7 @@ __device__ __forceinline__ void epilogue_oss_bwd_staged(const f32x16 (&acc)[TL::
   auto fetch = [&](auto buf, int q0) {
 #pragma unroll
     for (int u = 0; u < GRP; ++u) {
-      const int p = (q0 + u) * TL::NT + threadIdx.x;
+      const int p = (q0 + u) * TL::NT + tx;
       const int row = p / CPR, n = n0 + (p % CPR) * 8;
       const T* src = pre + (int64_t)(row0 + (row < rows ? row : 0)) * a.saux + 2 * (n < F ? n : 0);
       p1[decltype(buf)::value][u] = *(const T8*)src;
@@ -1424,12 +1516,12 @@ __device__ __forceinline__ void epilogue_oss_bwd_staged(const f32x16 (&acc)[TL::
     T8 dh[GRP];
 #pragma unroll
     for (int u = 0; u < GRP; ++u) {
-      const int p = (q0 + u) * TL::NT + threadIdx.x;
+      const int p = (q0 + u) * TL::NT + tx;
       dh[u] = *(const T8*)(lds + staged_addr<TL>(p / CPR, (p % CPR) * 8));
     }
 #pragma unroll
     for (int u = 0; u < GRP; ++u) {
-      const int p = (q0 + u) * TL::NT + threadIdx.x;
+      const int p = (q0 + u) * TL::NT + tx;
       const int row = p / CPR, n = n0 + (p % CPR) * 8;
       const T8 v1 = p1[decltype(buf)::value][u], v2 = p2[decltype(buf)::value][u];
       T8 o1, o2;
@@ -1562,7 +1654,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   // out of the L2s (hint extended from the 32-/64-row classes to all ring classes: Mixtral layer forward at 256 /
   // 384 / 448 tokens 0.539 -> 0.505 / 0.559 -> 0.526 / 0.711 -> 0.688 ms, neutral from 768 tokens on)
   constexpr bool W_ONCE = TL::NS > 2 || (TL::WG > 1 && !TL::PAIR);
-  typedef typename std::conditional<B_TR, TransOp<TL::BN, TL::NT, W_ONCE>, DirectOp<TL::BN, TL::NT, W_ONCE>>::type BOp;
+  typedef typename std::conditional<B_TR, TransOp<TL::BN, TL::NT, W_ONCE, false, TL::RS>, DirectOp<TL::BN, TL::NT, W_ONCE>>::type BOp;
   constexpr bool CAN_SPLIT = TL::BM == 128 && TL::BN == 256 && TL::NS == 3;
   const int glu = TL::RS ? __builtin_amdgcn_readfirstlane(a.glu) : -1;      // (as for the tile in s2s_mfma_kernel)
   const int e = t.e, row0 = t.row0, rows = t.rows, n0 = t.n0;
@@ -1601,14 +1693,12 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
     B.init(Wb, [&](int row) { const int n = n0 + row < N ? n0 + row : N - 1; return (int64_t)n * swn * 2; });
   }
 
-  f32x16 acc[TL::FM][TL::FN];
-  float rs[TL::FM];
+  Block acc[TL::FM][TL::FN];
+  float rs[2 * TL::FM];
 #pragma unroll
   for (int i = 0; i < TL::FM; ++i)
 #pragma unroll
-    for (int j = 0; j < TL::FN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    for (int j = 0; j < TL::FN; ++j) acc[i][j].clear();
   if constexpr (TL::RS) mainloop_rs<T, TL, AOp, BOp>(A, B, a.K, lds, acc);
   else if constexpr (TL::PAIR) mainloop_pair<T, TL, AOp, BOp, false>(A, B, a.K, lds, false, acc, rs);
   else if constexpr (TL::NS > 2) mainloop_ring<T, TL, AOp, BOp>(A, B, t.klen, lds, acc);
@@ -1618,8 +1708,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
     if (a.ksplit > 1) {
       // This part's accumulators as they lie in the registers, 16 bytes per lane and store (whole 1 KB runs per
       // wave); splitk_reduce_kernel knows which output element each of them belongs to.
-      typedef float f32x4_t __attribute__((ext_vector_type(4)));
-      f32x4_t* P = (f32x4_t*)a.partial +
+      f32x4* P = (f32x4*)a.partial +
                    (((int64_t)e * n_tiles + t.n_tile) * a.ksplit + t.part) * (TL::FM * TL::FN * 4 * TL::NT);
 #pragma unroll
       for (int i = 0; i < TL::FM; ++i)
@@ -1627,8 +1716,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
         for (int j = 0; j < TL::FN; ++j)
 #pragma unroll
           for (int g = 0; g < 4; ++g)
-            P[((i * TL::FN + j) * 4 + g) * TL::NT + threadIdx.x] =
-                f32x4_t{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+            P[((i * TL::FN + j) * 4 + g) * TL::NT + threadIdx.x] = acc[i][j].q[g];
       return;
     }
   }
@@ -1644,11 +1732,16 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   // 16-byte pieces need every row start 16-byte aligned; otherwise the lane-wise epilogues are used (the
   // one-wave-per-SIMD class is only launched on aligned outputs)
   if constexpr (TL::RS) {
-    if (glu == 0) epilogue_staged<T, TL>(acc, (T*)a.Y, sDst, n0, a.N, bias, a.sbn, lds, sBias);
-    else if (glu == 1) epilogue_glu_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds, sBias);
-    else if (glu == 2) epilogue_glu_bwd_staged<T, TL>(acc, a, row0, rows, n0, lds, sBias);
-    else if (glu == 3) epilogue_oss_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds, sBias);
-    else epilogue_oss_bwd_staged<T, TL>(acc, a, row0, rows, n0, lds, sBias);
+    // (staged here, once for all epilogues: a copy of the walk over 256 accumulators in each costs registers ahead of them)
+    stage_accumulators<T, TL>(acc, lds, [&](int tc) {
+      if (glu == 1) return glu_bias<T, TL>(a, bias, n0, tc);
+      return glu == 0 || glu == 3 ? plain_bias<T>(bias, a.sbn, a.N, n0 + tc) : 0.0f;
+    }, sBias);
+    if (glu == 0) epilogue_staged<T, TL>(acc, (T*)a.Y, sDst, n0, a.N, bias, a.sbn, lds);
+    else if (glu == 1) epilogue_glu_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds);
+    else if (glu == 2) epilogue_glu_bwd_staged<T, TL>(acc, a, row0, rows, n0, lds);
+    else if (glu == 3) epilogue_oss_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds);
+    else epilogue_oss_bwd_staged<T, TL>(acc, a, row0, rows, n0, lds);
   } else if (a.glu == 0) {
     const bool al16 = (((uintptr_t)a.Y & 15) == 0) && ((a.sym | a.N) & 7) == 0;
     if (al16) epilogue_staged<T, TL>(acc, (T*)a.Y, sDst, n0, a.N, bias, a.sbn, lds);
@@ -1757,31 +1850,30 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
 template <typename T>
 __global__ __launch_bounds__(512) void splitk_reduce_kernel(S2SArgs a, int n_tiles) {
   typedef Tile<128, 256, 2, 4, 3> TL;
-  typedef float f32x4_t __attribute__((ext_vector_type(4)));
   typedef T T4 __attribute__((ext_vector_type(4)));
   const int e = blockIdx.y, n_tile = blockIdx.x;
   int row0, rows;
   if (!find_remainder<256>(a.off, a.E, e, TL::BM, row0, rows)) return;
   const int wave = threadIdx.x >> 6, l = lane_id();
   const int wm = wave / TL::WN, wn = wave % TL::WN;
-  const f32x4_t* P = (const f32x4_t*)a.partial + ((int64_t)e * n_tiles + n_tile) * a.ksplit * (TL::FM * TL::FN * 4 * TL::NT);
+  const f32x4* P = (const f32x4*)a.partial + ((int64_t)e * n_tiles + n_tile) * a.ksplit * (TL::FM * TL::FN * 4 * TL::NT);
   const T* bias = a.b ? (const T*)a.b + (int64_t)e * a.sbe : nullptr;
   T* out = (T*)a.Y;
   const bool base_ok = ((uintptr_t)out & 7) == 0;
 #pragma unroll
   for (int i = 0; i < TL::FM; ++i) {
-    const int m = wm * TL::WTM + i * 32 + (l & 31);
-    if (m >= rows) continue;
-    const int64_t row = row0 + m;
-    const int64_t d = (a.y_grouped ? row : a.idx[row]) * a.sym;
 #pragma unroll
-    for (int j = 0; j < TL::FN; ++j) {
+    for (int g = 0; g < 4; ++g) {
+      const int m = wm * TL::WTM + i * 32 + block_row(l, g);
+      if (m >= rows) continue;
+      const int64_t row = row0 + m;
+      const int64_t d = (a.y_grouped ? row : a.idx[row]) * a.sym;
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n = n_tile * TL::BN + wn * TL::WTN + j * 32 + g * 8 + (l >> 5) * 4;
+      for (int j = 0; j < TL::FN; ++j) {
+        const int n = n_tile * TL::BN + wn * TL::WTN + j * 32 + block_col(l, g);
         if (n >= a.N) continue;
         const int slot = ((i * TL::FN + j) * 4 + g) * TL::NT + threadIdx.x;
-        f32x4_t v = P[slot];
+        f32x4 v = P[slot];
         for (int c = 1; c < a.ksplit; ++c) v += P[(int64_t)c * (TL::FM * TL::FN * 4 * TL::NT) + slot];
         if (bias != nullptr) {
 #pragma unroll
@@ -2119,12 +2211,18 @@ struct XtYPlan {
   int64_t x_rows;                         // rows of the matrix X is gathered from
 };
 
+// Sum over the four lanes that hold a row's shares of the contraction.
+__device__ __forceinline__ float sum_of_lane_groups(float v) {
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+
 // One output tile: rows p0, columns q0 of expert e.
 template <typename T, class TL, bool GA, bool GB>
 __device__ __forceinline__ void xty_tile(const XtYPlan& a, int e, int p0, int q0, char* lds, int64_t* sDst, unsigned* sRows,
                                          float* sBias) {
-  typedef std::conditional_t<TL::PAIR, RowsOp<TL::BM, TL::NT, GA>, TransOp<TL::BM, TL::NT, false, GA>> AOp;
-  typedef std::conditional_t<TL::PAIR, RowsOp<TL::BN, TL::NT, GB>, TransOp<TL::BN, TL::NT, false, GB>> BOp;
+  typedef std::conditional_t<TL::PAIR, RowsOp<TL::BM, TL::NT, GA>, TransOp<TL::BM, TL::NT, false, GA, (TL::WG > 2 || TL::RS)>> AOp;
+  typedef std::conditional_t<TL::PAIR, RowsOp<TL::BN, TL::NT, GB>, TransOp<TL::BN, TL::NT, false, GB, (TL::WG > 2 || TL::RS)>> BOp;
   const int r_lo = e ? (int)a.off[e - 1] : 0;
   const int r_hi = (int)a.off[e];
 
@@ -2150,15 +2248,13 @@ __device__ __forceinline__ void xty_tile(const XtYPlan& a, int e, int p0, int q0
   else if constexpr (GB) B.init_gather((const char*)a.Q + (int64_t)q0 * 2, a.ldq * 2, a.nq - q0, a.idx + r_lo, a.fan_out, r_hi - r_lo, sRows);
   else B.init((const char*)a.Q + ((int64_t)r_lo * a.ldq + q0) * 2, a.ldq * 2, a.nq - q0);
 
-  f32x16 acc[TL::FM][TL::FN];
-  float rs[TL::FM];
+  Block acc[TL::FM][TL::FN];
+  float rs[2 * TL::FM];
 #pragma unroll
   for (int i = 0; i < TL::FM; ++i) {
-    rs[i] = 0.0f;
+    rs[2 * i] = rs[2 * i + 1] = 0.0f;
 #pragma unroll
-    for (int j = 0; j < TL::FN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    for (int j = 0; j < TL::FN; ++j) acc[i][j].clear();
   }
   const bool want_db = a.Db != nullptr && a.db_from_p && q0 == 0;
   if constexpr (TL::RS) mainloop_rs<T, TL, AOp, BOp>(A, B, r_hi - r_lo, lds, acc);      // no bias gradient, no gather
@@ -2166,20 +2262,21 @@ __device__ __forceinline__ void xty_tile(const XtYPlan& a, int e, int p0, int q0
   else mainloop<T, TL, AOp, BOp, true>(A, B, r_hi - r_lo, lds, want_db, acc, rs);
   if constexpr (TL::PAIR) output_rows();                 // (into the column stage, which nobody reads any more)
 
+  if constexpr (TL::RS) stage_accumulators<T, TL>(acc, lds, [](int) { return 0.0f; }, sBias);
   if (TL::RS || TL::PAIR || ((((uintptr_t)a.OUT & 15) == 0) && ((a.soe | a.sop | a.nq) & 7) == 0))
-    epilogue_staged<T, TL>(acc, (T*)a.OUT, sDst, q0, a.nq, nullptr, 0, lds, sBias);
+    epilogue_staged<T, TL>(acc, (T*)a.OUT, sDst, q0, a.nq, nullptr, 0, lds);
   else
     epilogue<T, TL>(acc, (T*)a.OUT, sDst, q0, a.nq, nullptr, 0);
 
   if (want_db) {
-    // lanes l and l+32 hold the two contraction halves of row l%32; the first wave column writes the sums
+    // lanes l, l+16, l+32 and l+48 hold a quarter of the contraction of row l%16 each; the first wave column writes the sums
     const int wave = threadIdx.x >> 6, l = lane_id();
     const int wm = wave / TL::WN, wn = wave % TL::WN;
 #pragma unroll
-    for (int i = 0; i < TL::FM; ++i) {
-      const float tot = rs[i] + __shfl_xor(rs[i], 32, 64);
-      const int p = p0 + wm * TL::WTM + i * 32 + l;
-      if (wn == 0 && l < 32 && p < a.np) ((T*)a.Db)[(int64_t)e * a.sdbe + (int64_t)p * a.sdbn] = from_f32<T>(tot);
+    for (int i = 0; i < 2 * TL::FM; ++i) {
+      const float tot = sum_of_lane_groups(rs[i]);
+      const int p = p0 + wm * TL::WTM + i * 16 + l;
+      if (wn == 0 && l < 16 && p < a.np) ((T*)a.Db)[(int64_t)e * a.sdbe + (int64_t)p * a.sdbn] = from_f32<T>(tot);
     }
   }
 }

@@ -64,11 +64,11 @@ __device__ __forceinline__ void xty_rows_unit(const XtYPlan& a, int e, int r_lo,
   };
 
   // ---- the held operand: two slices at a time through LDS, then as fragments in registers
-  i32x4 fa[NSL * 4][2];
+  i32x4 fa[NSL * 2][4];
   {
     const i32x4 rp = rsrc_of(std::integral_constant<bool, GP>(), a.P, a.ldp, a.np);
     const int kr = t >> 5, phys = t & 31;                // piece j of this thread: row j * 8 + kr of the slice
-    const unsigned col = (unsigned)p0 * 2 + (((((phys >> 2) ^ (kr & 3)) << 2) | (phys & 3)) << 4);
+    const unsigned col[2] = {(unsigned)p0 * 2 + (trans_piece(kr, phys) << 4), (unsigned)p0 * 2 + (trans_piece(8 + kr, phys) << 4)};
 #pragma unroll
     for (int s0 = 0; s0 < NSL; s0 += 2) {
       if (s0 > 0) __syncthreads();                       // the first two slices have been read
@@ -76,37 +76,38 @@ __device__ __forceinline__ void xty_rows_unit(const XtYPlan& a, int e, int r_lo,
       for (int s = s0; s < s0 + 2 && s < NSL; ++s)
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          buffer_to_lds16(rp, row_off(std::integral_constant<bool, GP>(), s * 64 + j * 8 + kr, a.ldp) + col, 0,
+          buffer_to_lds16(rp, row_off(std::integral_constant<bool, GP>(), s * 64 + j * 8 + kr, a.ldp) + col[j & 1], 0,
                           lds_u + (s - s0) * POp::LDS_BYTES + j * 4096 + wave * 1024);
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
 #pragma unroll
       for (int s = s0; s < s0 + 2 && s < NSL; ++s)
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
+        for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-          for (int i = 0; i < 2; ++i) fa[s * 4 + ks][i] = POp::frag(lds + (s - s0) * POp::LDS_BYTES, wave * 64 + i * 32, ks);
+          for (int i = 0; i < 4; ++i) fa[s * 2 + ks][i] = POp::frag(lds + (s - s0) * POp::LDS_BYTES, wave * 64 + i * 16, ks);
     }
   }
   if (want_db) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < 4; ++i) {
       float rs = 0.0f;
 #pragma unroll
-      for (int q = 0; q < NSL * 4; ++q) rs += Mfma<T>::sum8(fa[q][i]);
-      const float tot = rs + __shfl_xor(rs, 32, 64);
-      const int p = p0 + wave * 64 + i * 32 + l;
-      if (l < 32 && p < a.np) ((T*)a.Db)[(int64_t)e * a.sdbe + (int64_t)p * a.sdbn] = from_f32<T>(tot);
+      for (int q = 0; q < NSL * 2; ++q) rs += Mfma<T>::sum8(fa[q][i]);
+      const float tot = sum_of_lane_groups(rs);
+      const int p = p0 + wave * 64 + i * 16 + l;
+      if (l < 16 && p < a.np) ((T*)a.Db)[(int64_t)e * a.sdbe + (int64_t)p * a.sdbn] = from_f32<T>(tot);
     }
   }
 
-  // ---- the streamed operand: rows of 128 bytes per step, the two 64-byte granules of a row swapped in every second pair
-  // of rows (a transposing read touches one granule of four consecutive rows)
+  // ---- the streamed operand: rows of 128 bytes per step, the two 64-byte granules of a row exchanged in every second pair
+  // of rows, the halves of a granule in every second eight rows (a transposing read touches half a granule of four consecutive
+  // rows and of the four rows 8 further down)
   const i32x4 rq = rsrc_of(std::integral_constant<bool, GQ>(), a.Q, a.ldq, a.nq);
   unsigned qoff[LOADS];
   {
     const int kr = t >> 3, phys = t & 7;
-    const unsigned col = ((((phys >> 2) ^ ((kr >> 1) & 1)) << 2) | (phys & 3)) << 4;
+    const unsigned col = (phys ^ ((kr << 1) & 4) ^ ((kr >> 2) & 2)) << 4;
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) qoff[j] = row_off(std::integral_constant<bool, GQ>(), j * 32 + kr, a.ldq) + col;
   }
@@ -115,13 +116,12 @@ __device__ __forceinline__ void xty_rows_unit(const XtYPlan& a, int e, int r_lo,
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) buffer_to_lds16(rq, qoff[j], (unsigned)(step0 + step) * (XR_Q * 2), dst + j * 4096);
   };
-  // fragment (columns 32 j .. 32 j + 31, contraction step q) of a stage
+  // fragment (columns 16 j .. 16 j + 15, contraction step q) of a stage
   const int b = l >> 4, r4 = (l & 15) >> 2;
-  const int krow = 8 * (b >> 1) + r4;
-  const char* fbase = lds + krow * 128 + (16 * (b & 1) + 4 * (l & 3)) * 2;
-  const int gran = (r4 >> 1) << 6;
+  const char* fbase = lds + (8 * b + r4) * 128 + (l & 3) * 8;
+  const int unit = ((r4 & 2) << 5) ^ ((b & 1) << 5);
   auto frag = [&](int stage, int j, int q) {
-    const char* p = fbase + stage * STAGE + q * 2048 + ((j << 6) ^ gran);
+    const char* p = fbase + stage * STAGE + q * 4096 + ((j << 5) ^ unit);
     const s16x4 lo = lds_read_tr(p), hi = lds_read_tr(p + 512);
     return __builtin_bit_cast(i32x4, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
@@ -134,8 +134,8 @@ __device__ __forceinline__ void xty_rows_unit(const XtYPlan& a, int e, int r_lo,
                                                    ((int64_t)(valid - 1) * a.sop + a.nq) * 2);
   const int64_t pitch = a.sop * 2;
   const unsigned ooff = (unsigned)((wave * 64 + (l >> 3)) * pitch) + ((l & 7) << 4);
-  char* wr = out_lds + (l & 31) * 128;
-  const int wsw = (l >> 1) & 7, wch = l >> 5;
+  char* wr = out_lds + (l & 15) * 128;
+  const int wsw = (l >> 1) & 7, wch = 2 * (b & 1) + (b >> 1);
   const int rdrow = (l >> 3) * 128, rdch = (l & 7) ^ (l >> 4);                        // row 8 q + l / 8
   const char* rd[2] = {out_lds + rdrow + (rdch << 4), out_lds + rdrow + ((rdch ^ 4) << 4)};      // of even and odd q
 
@@ -157,30 +157,31 @@ __device__ __forceinline__ void xty_rows_unit(const XtYPlan& a, int e, int r_lo,
     }
     __syncthreads();                                     // everyone's have, and everyone is done with the step before
     if (step + NST - 1 < nsteps) issue(step + NST - 1, stage == 0 ? NST - 1 : stage - 1);
-    f32x16 acc[2][2];
+    Block acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-    i32x4 fb[2][2];
+      for (int j = 0; j < 2; ++j) acc[i][j].clear();
+    i32x4 fb[2][2];                                      // two of the four fragments of a step of 32, the next two meanwhile
     fb[0][0] = frag(stage, 0, 0);
     fb[0][1] = frag(stage, 1, 0);
 #pragma unroll
-    for (int q = 0; q < NSL * 4; ++q) {
-      const int c = q & 1, n = c ^ 1;
-      if (q + 1 < NSL * 4) {
-        fb[n][0] = frag(stage, 0, q + 1);
-        fb[n][1] = frag(stage, 1, q + 1);
+    for (int h = 0; h < NSL * 4; ++h) {
+      const int c = h & 1, n = c ^ 1;
+      if (h + 1 < NSL * 4) {
+        fb[n][0] = frag(stage, 2 * n, (h + 1) >> 1);
+        fb[n][1] = frag(stage, 2 * n + 1, (h + 1) >> 1);
       }
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) acc[i][j] = Mfma<T>::run(fb[c][j], fa[q][i], acc[i][j]);
+        for (int i = 0; i < 4; ++i) {
+          f32x4& d = acc[i >> 1][c].q[2 * (i & 1) + j];
+          d = Mfma<T>::run(fb[c][j], fa[h >> 1][i], d);
+        }
     }
-    // A lane holds, per group of four accumulators, four consecutive columns of its output row, the lane 32 further the
-    // four next to them.  Exchanging halves between two neighbouring groups leaves each lane with eight columns.
+    // A lane holds, per group of four accumulators, four consecutive columns of its output row, the lane 16 further the
+    // four next to them.  Exchanging every second 16 lanes between two neighbouring groups leaves each lane with eight columns.
     const int n0 = (step0 + step) * XR_Q;
     const bool whole = n0 + XR_Q <= a.nq;
     const unsigned off = whole || n0 + ((l & 7) << 3) < a.nq ? ooff + (unsigned)n0 * 2 : OUT_OF_RANGE;
@@ -192,17 +193,17 @@ __device__ __forceinline__ void xty_rows_unit(const XtYPlan& a, int e, int r_lo,
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int g = 0; g < 4; g += 2) {
+        for (int r = 0; r < 2; ++r) {
           T4 lo, hi;
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
-            set_pair<T>(lo, h, acc[i][j][g * 4 + 2 * h], acc[i][j][g * 4 + 2 * h + 1]);
-            set_pair<T>(hi, h, acc[i][j][g * 4 + 4 + 2 * h], acc[i][j][g * 4 + 4 + 2 * h + 1]);
+            set_pair<T>(lo, h, acc[i][j][r * 8 + 2 * h], acc[i][j][r * 8 + 2 * h + 1]);
+            set_pair<T>(hi, h, acc[i][j][r * 8 + 4 + 2 * h], acc[i][j][r * 8 + 4 + 2 * h + 1]);
           }
           const u32x2_t u = __builtin_bit_cast(u32x2_t, lo), v = __builtin_bit_cast(u32x2_t, hi);
-          const auto s0 = __builtin_amdgcn_permlane32_swap(u[0], v[0], false, false);
-          const auto s1 = __builtin_amdgcn_permlane32_swap(u[1], v[1], false, false);
-          *(u32x4_t*)(wr + (((j * 4 + g + wch) ^ wsw) << 4)) = u32x4_t{s0[0], s1[0], s0[1], s1[1]};
+          const auto s0 = __builtin_amdgcn_permlane16_swap(u[0], v[0], false, false);
+          const auto s1 = __builtin_amdgcn_permlane16_swap(u[1], v[1], false, false);
+          *(u32x4_t*)(wr + r * 2048 + (((j * 4 + wch) ^ wsw) << 4)) = u32x4_t{s0[0], s1[0], s0[1], s1[1]};
         }
       u32x4_t w[4];
 #pragma unroll

@@ -75,6 +75,59 @@ def _sources():
     return names
 
 
+VECTOR = re.compile(r"\b([av])(?:(\d+)\b|\[(\d+):(\d+)\])")
+
+
+def _vector_registers(text):
+    return {(m[1], k) for m in VECTOR.finditer(text) for k in range(int(m[2] or m[3]), int(m[2] or m[4]) + 1)}
+
+
+def _product_hazards(text):
+    """Products issued from assembly blocks, which the compiler's hazard recogniser does not look into: a vector instruction
+    must not write one of their operands within the two wait states before them, and nothing but a product may touch their
+    result within the 19 states that the longest of them takes to write it (followed in program order, as the code falls
+    through)."""
+    code, inside = [], False
+    for n, line in enumerate(text.split("\n")):
+        t = line.strip()
+        if "ASMSTART" in t or "ASMEND" in t:
+            inside = "ASMSTART" in t
+        elif t and t[0] not in ".;" and not t.split(";")[0].strip().endswith(":"):
+            code.append((n + 1, t.split(";")[0].strip(), inside))
+    states = lambda t: int(t.split()[1]) + 1 if t.startswith("s_nop") else 1
+    products, found = 0, []
+    for i, (n, t, in_asm) in enumerate(code):
+        if not (in_asm and t.startswith("v_mfma")):
+            continue
+        products += 1
+        operands = t.split(None, 1)[1].split(",")
+        result, sources = _vector_registers(operands[0]), _vector_registers(",".join(operands[1:]))
+        k, passed = i - 1, 0
+        while k >= 0 and passed < 2:
+            u = code[k][1]
+            if u.startswith("v_") and not u.startswith("v_mfma") and _vector_registers(u.split(",")[0]) & sources:
+                found.append((n, t, code[k]))
+            passed, k = passed + states(u), k - 1
+        k, passed = i + 1, 0
+        while k < len(code) and passed < 19 and not code[k][1].startswith(("s_branch", "s_endpgm", "s_setpc")):
+            u = code[k][1]
+            if not u.startswith("v_mfma") and _vector_registers(u) & result:
+                found.append((n, t, code[k]))
+            passed, k = passed + states(u), k + 1
+    return products, found
+
+
+def test_scanner_sees_an_early_access_of_a_product():
+    product = "\t;;#ASMSTART\n\tv_mfma_f32_16x16x32_bf16 a[0:3], v[8:11], v[4:7], a[0:3]\n\t;;#ASMEND\n"
+    for bad in ("\tv_mov_b32_e32 v5, v1\n" + product, "\tv_accvgpr_write_b32 a3, 0\n\ts_nop 0\n" + product,
+                product + "\tv_accvgpr_read_b32 v1, a2\n", product + "\ts_nop 15\n\tscratch_store_dword off, a3, off\n",
+                product + ".LBB0_1:\n\tv_mov_b32_e32 v9, v1\n\tv_accvgpr_read_b32 v1, a0\n"):
+        assert _product_hazards(bad)[1], bad
+    for good in ("\tv_mov_b32_e32 v5, v1\n\ts_nop 1\n" + product, product + product, "\tv_mov_b32_e32 v3, v5\n" + product,
+                 product + "\ts_nop 15\n\ts_nop 3\n\tv_accvgpr_read_b32 v1, a2\n", product + "\tds_read_b128 v[8:11], v1\n"):
+        assert _product_hazards(good) == (good.count("v_mfma"), []), good
+
+
 needs_hipcc = pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"),
                                  reason="needs hipcc")
 
@@ -100,6 +153,16 @@ def test_no_inline_assembly_load_reads_a_freshly_written_scalar_base(assembly):
         loads, found = _hazards(text)
         assert loads > 100, "%s: no inline-assembly loads found: the scan is looking at the wrong text" % name
         assert not found, (name, found[:5])
+
+
+@needs_hipcc
+def test_products_of_assembly_blocks_keep_their_distance(assembly):
+    seen = 0
+    for name, text in assembly.items():
+        products, found = _product_hazards(text)
+        seen += products
+        assert not found, (name, found[:5])
+    assert seen > 1000, "no inline-assembly products found: the scan is looking at the wrong text"
 
 
 def _scratch_of_kernels(text):
