@@ -126,7 +126,8 @@ int smoe_scatter2scatter(const void* X, int64_t sxm, int64_t sxk,
  * 8 experts x 16 tile columns) those tiles are too few to fill the chip and each walks the whole contraction.
  * With `workspace` of at least smoe_scatter2scatter_workspace_bytes(L, K, N, E, dtype) bytes (16-byte aligned)
  * their contraction is cut into parts that run side by side; a second small launch adds the float32 partial
- * sums in a fixed order and writes the rows.  Results are the same on every run, and within float32 rounding
+ * sums in a fixed order and writes the rows.  So is that of whole products whose tiles would leave half of the chip
+ * idle (8 experts x 194 rows, 14336 -> 4096: 128 tiles).  Results are the same on every run, and within float32 rounding
  * of - not bit-identical to - the product without workspace (the additions are grouped differently).
  * workspace == NULL, too small or not 16-byte aligned: exactly smoe_scatter2scatter (the workspace is then not
  * touched; no error).  The workspace is free again when the launches

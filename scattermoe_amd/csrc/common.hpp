@@ -143,6 +143,16 @@ __device__ __forceinline__ bool find_tile(const int64_t* __restrict__ off, int E
   return false;
 }
 
+// Number of tile rows of height BM that the experts have.
+template <int BM>
+__device__ __forceinline__ int count_tile_rows(const int64_t* __restrict__ off, int E) {
+  int n = 0;
+  for (int e = lane_id(); e < E; e += 64) n += ((int)(off[e] - (e ? off[e - 1] : 0)) + BM - 1) / BM;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) n += __shfl_xor(n, d, 64);
+  return __builtin_amdgcn_readfirstlane(n);
+}
+
 // Largest of the wave's values, in a scalar register: six row shifts and row broadcasts (lanes without a source keep
 // their own value).
 __device__ __forceinline__ int wave_max(int v) {
@@ -293,10 +303,11 @@ struct S2SArgs {
   // Products whose experts end in a partly filled tile (MFMA path only).  1: this launch leaves out every expert's
   // last tile when it holds at most 128 rows; 2: this launch takes exactly those rows, one tile row per expert.
   int tail_mode = 0;
-  // tail_mode 2 only: the contraction of every tile is cut into `ksplit` equal parts, one workgroup each, which
-  // leave their float32 accumulators in `partial` (see splitk_floats); a second launch adds the parts up in a
-  // fixed order and writes the output rows.  `partial` / `partial_floats`: the caller's workspace, may be NULL / 0.
-  int ksplit = 1, k_part = 0;           // k_part = K / ksplit
+  // The contraction of every tile is cut into `ksplit` parts of `k_part` (the last may be shorter), one workgroup each, which
+  // leave their float32 sums in `partial` (tail_mode 2: accumulators, see splitk_floats; whole products: rows, see
+  // parts_sum_kernel); a second launch adds the parts up in a fixed order and writes the output rows.
+  // `partial` / `partial_floats`: the caller's workspace, may be NULL / 0.
+  int ksplit = 1, k_part = 0;
   float* partial = nullptr;
   int64_t partial_floats = 0;
 };

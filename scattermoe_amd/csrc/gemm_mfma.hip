@@ -9,7 +9,9 @@ int dispatch_xty_bf16(const XtYArgs& a, hipStream_t st);
 int dispatch_xty_f16(const XtYArgs& a, hipStream_t st);
 
 int64_t s2s_workspace_floats(int64_t L, int64_t K, int64_t N, int E, int dtype) {
-  if ((dtype != SMOE_BF16 && dtype != SMOE_F16) || E <= 0 || L / E < REMAINDER_MIN_AVG_ROWS) return 0;
+  if ((dtype != SMOE_BF16 && dtype != SMOE_F16) || E <= 0) return 0;
+  if (const int parts = whole_parts_for(L, K, N, E); parts > 1) return L * N * parts;
+  if (L / E < REMAINDER_MIN_AVG_ROWS) return 0;
   if (2.0 * (double)L * K * N < REMAINDER_MIN_FLOP) return 0;
   const int ks = tail_ksplit_for(K, N, E, 0);
   return ks > 1 ? splitk_floats(N, E, ks) : 0;

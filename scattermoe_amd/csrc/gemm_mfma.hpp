@@ -1050,6 +1050,21 @@ __device__ __forceinline__ int late_thread() {
   if constexpr (TL::RS || TL::WG > 2) asm volatile("" : "+v"(t));
   return t;
 }
+// Four accumulators where they are used.  One wave per SIMD: assembly, behind the wait at the main loop's end (left to the compiler,
+// all accumulators are copied to vector registers ahead of it).
+template <class TL>
+__device__ __forceinline__ f32x4 accumulators(const f32x4& q) {
+  if constexpr (!TL::RS) return q;
+  f32x4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float x;
+    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(q[e]));
+    v[e] = x;
+  }
+  return v;
+}
+
 // `bias_of(tile_col)` returns the value to add to that column (0 without bias).
 template <typename T, class TL, typename BF>
 __device__ __forceinline__ void stage_accumulators(const Block (&acc)[TL::FM][TL::FN], char* lds, BF bias_of,
@@ -1063,14 +1078,6 @@ __device__ __forceinline__ void stage_accumulators(const Block (&acc)[TL::FM][TL
     for (int t = tx; t < TL::BN; t += TL::NT) sbias[t] = bias_of(t);
   }
   __syncthreads();                                   // every wave is done reading operands
-  // One wave per SIMD: accumulators leave their registers where they are used (left to the compiler, all of them are copied ahead),
-  // behind the wait at the main loop's end.
-  auto value = [](float x) {
-    if constexpr (!TL::RS) return x;
-    float v;
-    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(x));
-    return v;
-  };
 #pragma unroll
   for (int j = 0; j < TL::FN; ++j) {
 #pragma unroll
@@ -1088,9 +1095,10 @@ __device__ __forceinline__ void stage_accumulators(const Block (&acc)[TL::FM][TL
 #pragma unroll
       for (int i = 0; i < 2 * TL::FM; ++i) {
         const int g = 2 * (i & 1) + c, row = wm * TL::WTM + (i >> 1) * 32 + block_row(l, g);
+        const f32x4 q = accumulators<TL>(acc[i >> 1][j].q[g]);
         T4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = from_f32<T>(value(acc[i >> 1][j].q[g][e]) + bv[e]);
+        for (int e = 0; e < 4; ++e) v[e] = from_f32<T>(q[e] + bv[e]);
         *(T4*)(lds + staged_addr<TL>(row, col)) = v;
       }
     }
@@ -1655,10 +1663,11 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   // 384 / 448 tokens 0.539 -> 0.505 / 0.559 -> 0.526 / 0.711 -> 0.688 ms, neutral from 768 tokens on)
   constexpr bool W_ONCE = TL::NS > 2 || (TL::WG > 1 && !TL::PAIR);
   typedef typename std::conditional<B_TR, TransOp<TL::BN, TL::NT, W_ONCE, false, TL::RS>, DirectOp<TL::BN, TL::NT, W_ONCE>>::type BOp;
-  constexpr bool CAN_SPLIT = TL::BM == 128 && TL::BN == 256 && TL::NS == 3;
+  constexpr bool LAST_TILES = TL::BM == 128 && TL::BN == 256 && TL::NS == 3;
+  constexpr bool CAN_SPLIT = LAST_TILES || TL::RS;
   const int glu = TL::RS ? __builtin_amdgcn_readfirstlane(a.glu) : -1;      // (as for the tile in s2s_mfma_kernel)
   const int e = t.e, row0 = t.row0, rows = t.rows, n0 = t.n0;
-  const int k_first = CAN_SPLIT ? t.part * t.klen : 0;
+  const int k_first = CAN_SPLIT ? t.part * a.k_part : 0;
 
   AOp A;
   A.rot = TL::RS ? 0 : (t.n_loc * AOp::R / (TL::PAIR ? 2 * Raster::SN : Raster::SN)) % AOp::R;    // the row panel has SN sharers
@@ -1699,12 +1708,32 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   for (int i = 0; i < TL::FM; ++i)
 #pragma unroll
     for (int j = 0; j < TL::FN; ++j) acc[i][j].clear();
-  if constexpr (TL::RS) mainloop_rs<T, TL, AOp, BOp>(A, B, a.K, lds, acc);
+  if constexpr (TL::RS) mainloop_rs<T, TL, AOp, BOp>(A, B, t.klen, lds, acc);
   else if constexpr (TL::PAIR) mainloop_pair<T, TL, AOp, BOp, false>(A, B, a.K, lds, false, acc, rs);
   else if constexpr (TL::NS > 2) mainloop_ring<T, TL, AOp, BOp>(A, B, t.klen, lds, acc);
   else mainloop<T, TL, AOp, BOp, false>(A, B, a.K, lds, false, acc, rs);
 
-  if constexpr (CAN_SPLIT) {
+  if constexpr (TL::RS) {
+    if (a.ksplit > 1) {
+      // This part's sums of the tile's rows, in float32 (parts_sum_kernel adds the parts)
+      const int tx = late_thread<TL>(), wave = tx >> 6, l = tx & 63;
+      const int wm = wave / TL::WN, wn = wave % TL::WN;
+      float* P = a.partial + ((int64_t)t.part * a.L + row0) * a.N + n0;
+#pragma unroll
+      for (int i = 0; i < 2 * TL::FM; ++i) {
+        const int m = wm * TL::WTM + i * 16 + (l & 15);
+        if (m >= rows) continue;
+#pragma unroll
+        for (int j = 0; j < 2 * TL::FN; ++j) {
+          const int n = wn * TL::WTN + (j >> 1) * 32 + block_col(l, j & 1);
+          const f32x4 v = accumulators<TL>(acc[i >> 1][j >> 1].q[2 * (i & 1) + (j & 1)]);
+          if (n0 + n < a.N) *(f32x4*)(P + (int64_t)m * a.N + n) = v;
+        }
+      }
+      return;
+    }
+  }
+  if constexpr (LAST_TILES) {
     if (a.ksplit > 1) {
       // This part's accumulators as they lie in the registers, 16 bytes per lane and store (whole 1 KB runs per
       // wave); splitk_reduce_kernel knows which output element each of them belongs to.
@@ -1776,24 +1805,36 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
   int* sSrc = TL::PAIR ? (int*)(lds + PAIR_STAGE) : sSrc_;
   float* sBias = TL::PAIR ? nullptr : sBias_;
 
-  // Contraction parts (the class of the experts' last tiles only): the grid is `ksplit` copies of the raster, copy
-  // c multiplies the c-th part of the contraction (a raster is a multiple of 8 workgroups, so the XCD of a workgroup
-  // is still its first index modulo 8)
-  constexpr bool CAN_SPLIT = TL::BM == 128 && TL::BN == 256 && TL::NS == 3;
+  // Contraction parts of the experts' last tiles: the grid is `ksplit` copies of the raster, copy c multiplies the c-th part of the
+  // contraction (a raster is a multiple of 8 workgroups, so the XCD of a workgroup is still its first index modulo 8)
+  constexpr bool LAST_TILES = TL::BM == 128 && TL::BN == 256 && TL::NS == 3;
   // (the parts are the grid's second dimension; no division here: the compiler would do it in the vector unit and
   // everything derived from it, loop counters and LDS addresses included, would leave the scalar registers)
   S2STile t;
-  t.part = CAN_SPLIT ? (int)blockIdx.y : 0;
-  t.klen = CAN_SPLIT && a.ksplit > 1 ? a.k_part : a.K;
+  t.part = LAST_TILES ? (int)blockIdx.y : 0;
   int m_tile;
   int found = -1;
-  if (rast.chunked) {
+  if (TL::RS && a.ksplit > 1) {
+    // Contraction parts of a whole product, at most a round of workgroups: the tiles that there are, one part after another, so
+    // that every XCD, and every shader engine in it, has its share (workgroups without a tile between them, or columns in
+    // stripes, and some CUs have two: 4 experts x 628 rows, 8512 -> 1664, 252 workgroups 163, 144 -> 113 us)
+    const int tiles = count_tile_rows<TL::BM>(a.off, a.E) * rast.n_tiles;
+    t.part = __builtin_amdgcn_readfirstlane(tiles > 0 ? (int)blockIdx.x / tiles : a.ksplit);
+    if (t.part >= a.ksplit) return;
+    const int in = (int)blockIdx.x - t.part * tiles;
+    m_tile = __builtin_amdgcn_readfirstlane(in / rast.n_tiles);
+    t.n_tile = in - m_tile * rast.n_tiles;
+    t.m_loc = t.n_loc = 0;
+    found = find_tile<TL::BM>(a.off, a.E, m_tile, t.e, t.row0, t.rows) ? 1 : 0;
+    if (found == 0) return;
+  } else if (rast.chunked) {
     t.m_loc = t.n_loc = 0;
     found = find_tile_chunked<TL::BM, TL::BM == 256 && (TL::BN == 256 || TL::PAIR)>(a.off, a.E, blockIdx.x, rast.n_tiles,
                                                                       rast.chunked == 2 ? TL::WG * 256 : 0,
                                                                       t.e, t.row0, t.rows, t.n_tile);
     if (found == 0) return;
   }
+  t.klen = (LAST_TILES || TL::RS) && a.ksplit > 1 ? min(a.k_part, a.K - t.part * a.k_part) : a.K;
   if (found < 0 && !rast.map<TL::PAIR ? 2 * Raster::SN : Raster::SN>(blockIdx.x, m_tile, t.n_tile, t.m_loc, t.n_loc)) return;
   if (found > 0) {
     // looked up above
@@ -1892,32 +1933,36 @@ __global__ __launch_bounds__(512) void splitk_reduce_kernel(S2SArgs a, int n_til
   }
 }
 
-template <typename T, class TL>
-static int launch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
-  const int bn = a.glu == 1 ? TL::BN / 2 : TL::BN;     // output columns per tile
-  const int n_tiles = (a.N + bn - 1) / bn;
-  const int64_t m_tiles = a.tail_mode == 2 ? a.E : std::min<int64_t>(max_tiles(a.L, a.E, TL::BM) - a.m_begin, a.m_count);
-  // With only a few tile rows per expert no weight panel is shared by the tile rows of a super tile; the striped
-  // order at least keeps the tile rows of one expert together on one XCD.
-  const bool striped = TL::NS > 2 || a.L / a.E < STRIPE_BELOW;
-  Raster r = striped ? make_striped(m_tiles, n_tiles, GM_RING) : make_raster(m_tiles, n_tiles, GM_S2S, TL::PAIR ? 2 * Raster::SN : Raster::SN);
-  const bool whole = a.m_begin == 0 && a.m_count == 0x7fffffff && a.tail_mode == 0;
-  const int64_t chunked = chunked_grid(m_tiles * n_tiles);
-  if (whole && a.L / a.E < CHUNK_BELOW && chunked <= 0x7fffffffLL) {
-    r.chunked = TL::NS > 2 || (TL::WG > 1 && !TL::PAIR) || a.L / a.E < ROWS256_BELOW ? 1 : 2;
-    r.grid_size = std::max(r.grid_size, chunked);
+// Second half of a product whose contraction was cut into parts as a whole: one wave per 512 columns of a row adds the parts up in
+// ascending order (the same result on every run), then bias, rounding and the scatter of the row.
+template <typename T>
+__global__ __launch_bounds__(256) void parts_sum_kernel(S2SArgs a) {
+  typedef T T8 __attribute__((ext_vector_type(8)));
+  const int pieces = (a.N + 511) / 512;                               // per row, one per wave
+  const int w = (int)(blockIdx.x * 4 + wave_uniform_id());
+  const int row = __builtin_amdgcn_readfirstlane(w / pieces);
+  const int n = ((w - row * pieces) * 64 + lane_id()) * 8;
+  if (row >= (int)a.off[a.E - 1]) return;                             // (rows without an expert are written by nobody)
+  int e = 0;
+  if (a.b != nullptr) {
+    for (int c = 0; c < a.E; c += 64) e += __popcll(__ballot(c + lane_id() < a.E && a.off[c + lane_id()] <= row));
   }
-  const int64_t grid = r.grid();
-  const unsigned parts = a.ksplit > 1 ? (unsigned)a.ksplit : 1u;
-  if (grid > 0x7fffffffLL || m_tiles > 0x7fffffffLL) { set_error("smoe_scatter2scatter: grid too large"); return SMOE_ERR_RANGE; }
-  if constexpr (TL::BN % 128 == 0) {
-    if (b_tr) {
-      hipLaunchKernelGGL((s2s_mfma_kernel<T, TL, true>), dim3((unsigned)grid, parts), dim3(TL::NT), 0, st, a, r);
-      return launch_status("s2s_mfma_kernel");
-    }
+  if (n >= a.N) return;
+  const float* P = a.partial + (int64_t)row * a.N + n;
+  f32x4 v[2] = {*(const f32x4*)P, *(const f32x4*)(P + 4)};
+  for (int c = 1; c < a.ksplit; ++c) {
+    P += (int64_t)a.L * a.N;
+    v[0] += *(const f32x4*)P;
+    v[1] += *(const f32x4*)(P + 4);
   }
-  hipLaunchKernelGGL((s2s_mfma_kernel<T, TL, false>), dim3((unsigned)grid, parts), dim3(TL::NT), 0, st, a, r);
-  return launch_status("s2s_mfma_kernel");
+  T8 y;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    float x = v[q >> 2][q & 3];
+    if (a.b != nullptr) x += to_f32(((const T*)a.b)[(int64_t)e * a.sbe + (int64_t)(n + q) * a.sbn]);
+    y[q] = from_f32<T>(x);
+  }
+  *(T8*)((T*)a.Y + (a.y_grouped ? (int64_t)row : a.idx[row]) * a.sym + n) = y;
 }
 
 static constexpr int NUM_CU = 256;
@@ -1936,6 +1981,36 @@ static double expected_row_tiles(int64_t L, int E, int skip_small = 0) {
       per_expert -= above(j * 256.0 + 0.5) - above(j * 256.0 + skip_small + 0.5);
   }
   return nearbyint(per_expert * E);
+}
+
+template <typename T, class TL>
+static int launch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
+  const int bn = a.glu == 1 ? TL::BN / 2 : TL::BN;     // output columns per tile
+  const int n_tiles = (a.N + bn - 1) / bn;
+  const int64_t m_tiles = a.tail_mode == 2 ? a.E : std::min<int64_t>(max_tiles(a.L, a.E, TL::BM) - a.m_begin, a.m_count);
+  // With only a few tile rows per expert no weight panel is shared by the tile rows of a super tile; the striped
+  // order at least keeps the tile rows of one expert together on one XCD.
+  const bool striped = TL::NS > 2 || a.L / a.E < STRIPE_BELOW;
+  Raster r = striped ? make_striped(m_tiles, n_tiles, GM_RING) : make_raster(m_tiles, n_tiles, GM_S2S, TL::PAIR ? 2 * Raster::SN : Raster::SN);
+  const bool whole = a.m_begin == 0 && a.m_count == 0x7fffffff && a.tail_mode == 0;
+  const int64_t chunked = chunked_grid(m_tiles * n_tiles);
+  const bool whole_parts = TL::RS && a.ksplit > 1;                      // (parts one after another, see s2s_mfma_kernel)
+  if (whole_parts) r.grid_size = m_tiles * n_tiles * a.ksplit;
+  else if (whole && a.L / a.E < CHUNK_BELOW && chunked <= 0x7fffffffLL) {
+    r.chunked = TL::NS > 2 || (TL::WG > 1 && !TL::PAIR) || a.L / a.E < ROWS256_BELOW ? 1 : 2;
+    r.grid_size = std::max(r.grid_size, chunked);
+  }
+  const int64_t grid = r.grid();
+  const unsigned parts = a.ksplit > 1 && !whole_parts ? (unsigned)a.ksplit : 1u;
+  if (grid > 0x7fffffffLL || m_tiles > 0x7fffffffLL) { set_error("smoe_scatter2scatter: grid too large"); return SMOE_ERR_RANGE; }
+  if constexpr (TL::BN % 128 == 0) {
+    if (b_tr) {
+      hipLaunchKernelGGL((s2s_mfma_kernel<T, TL, true>), dim3((unsigned)grid, parts), dim3(TL::NT), 0, st, a, r);
+      return launch_status("s2s_mfma_kernel");
+    }
+  }
+  hipLaunchKernelGGL((s2s_mfma_kernel<T, TL, false>), dim3((unsigned)grid, parts), dim3(TL::NT), 0, st, a, r);
+  return launch_status("s2s_mfma_kernel");
 }
 
 // A launch of a few whole rounds plus a remainder of up to half a round pays a whole round for the remainder.
@@ -2071,6 +2146,47 @@ static int launch_tails(const S2SArgs& a, bool b_tr, hipStream_t st) {
   return launch_status("splitk_reduce_kernel");
 }
 
+// Products of few tiles and a long contraction: the contraction of every tile is cut into parts, one workgroup of the
+// one-wave-per-SIMD form each, which leave float32 sums; a second launch adds them up in a fixed order (parts_sum_kernel).  Without
+// parts at most half of the CUs have a 256 x 256 tile, and 256 x 128 ring tiles hold a quarter of the loads in flight that the
+// weights' stream needs.  The number of parts, and whether any, by the time that the parts and the classes below would take, in us:
+// a slice of 64 costs 1.25 in a whole tile and 0.95 in a ring tile, or what the weights' stream does (5.2 and 4 TB/s); a
+// workgroup's set-up and store 14 and 4; the sums their bytes at 4.5 TB/s, written and read.  Measured, us, without -> with (parts):
+// 8 experts x 194 rows, 14336 -> 4096 241 -> 220 (2), 28672 -> 4096 478 -> 397 (2); 4 x 300, 14336 -> 4096 239 -> 196 (2); 2 x 500,
+// 8192 -> 4096 116 -> 73 (4); 1 x 609, 10240 -> 1472 155 -> 47 (8); 8 x 200, 2048 -> 2048 33 -> 39, so not; a second round of
+// workgroups loses as well (8 x 250, 14336 -> 4096 316 -> 361).
+static constexpr int PARTS_MAX = 8;
+static int part_length(int64_t K, int parts) { return (int)((K / BK + parts - 1) / parts) * BK; }
+static int whole_parts_for(int64_t L, int64_t K, int64_t N, int E) {
+  if (L / E < ROWS128_BELOW || K < RS_MIN_K || K % BK != 0 || N % 8 != 0) return 1;
+  const double tiles = expected_row_tiles(L, E) * ((N + 255) / 256), weights = 2.0 * E * K * N * 1e-6, slices = (double)(K / BK);
+  double least = 0.92 * (std::max(slices * 0.95, weights / 4.0) + 4);
+  int best = 1;
+  for (int p = 2; p <= PARTS_MAX && tiles * p <= NUM_CU; ++p) {
+    const int len = part_length(K, p);
+    if ((K + len - 1) / len != p) continue;                           // (no part is empty)
+    const double t = std::max(len / BK * 1.25, weights / 5.2) + 14 + 8e-6 * L * N * p / 4.5;
+    if (t < least) least = t, best = p;
+  }
+  return best;
+}
+static int whole_parts(const S2SArgs& a, bool b_tr) {
+  const bool whole = a.m_begin == 0 && a.m_count == 0x7fffffff && a.tail_mode == 0;
+  if (a.glu != 0 || !whole || a.partial == nullptr || !whole_pieces(a) || (b_tr && a.swk < a.N)) return 1;
+  const int p = whole_parts_for(a.L, a.K, a.N, a.E);
+  return a.partial_floats >= (int64_t)a.L * a.N * p ? p : 1;
+}
+template <typename T>
+static int launch_parts(const S2SArgs& a, int parts, bool b_tr, hipStream_t st) {
+  S2SArgs m = a;
+  m.ksplit = parts;
+  m.k_part = part_length(a.K, parts);
+  if (const int rc = launch_s2s<T, Tile<256, 256, 2, 2, 2, true>>(m, b_tr, st)) return rc;
+  const int64_t waves = (int64_t)a.L * ((a.N + 511) / 512);
+  hipLaunchKernelGGL(parts_sum_kernel<T>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, m);
+  return launch_status("parts_sum_kernel");
+}
+
 // A whole product in the 256-row classes: one launch, or whole rounds of 256 x 256 tiles plus a remainder of 256 x 128
 // tiles (tail_split), the experts' sparsely filled last tiles apart (cut_tails).
 template <typename T>
@@ -2173,6 +2289,7 @@ static int dispatch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
   // 52 rows on where it makes one round of what the 128-row tiles do in two (16 x 90, 2048 -> 2 x 1408 56 -> 42; paired
   // tiles, of which twice as many make a round, up to two: 17 random launches of 52 to 112 rows 1.15 times as fast), and
   // from 224 rows on whatever the number of tiles, unless half-width ones fit one round.
+  if (const int parts = whole_parts(a, b_tr); parts > 1) return launch_parts<T>(a, parts, b_tr, st);
   const int64_t tiles = (int64_t)a.E * ((a.N + (a.glu == 1 ? 127 : 255)) / (a.glu == 1 ? 128 : 256));
   if (avg >= ROWS256_BELOW && one_round_of_halves(a)) return launch_s2s<T, Tile<256, 128, 4, 2, 3>>(a, b_tr, st);
   if (avg >= ROWS256_BELOW || (avg >= ROWS128_BELOW && tiles >= MAIN_MIN_TILES) ||
