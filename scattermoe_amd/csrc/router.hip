@@ -6,7 +6,10 @@
 // every Hugging Face MoE block the reference patches computes its routing weights this way.
 //
 // One wave per token.  Lane l holds logits l, l+64, ... (at most 8 per lane, i.e. E <= 512).  Selection is k
-// rounds of a wave-wide arg-max; among equal values the lowest expert id wins.  All arithmetic in fp32.
+// rounds of a wave-wide maximum and a search for its first holder; among equal values the lowest expert id wins.  All
+// arithmetic in fp32.  The rounds follow one another, so what bounds the kernel is the latency of one: row shifts and
+// broadcasts between lanes (probabilities are never negative, so they order as their bits do) and ballots, no shuffles
+// through LDS.
 // Every id written is a valid expert id whatever the logits hold: a NaN logit counts as -inf, and a row without
 // any usable logit is routed as if all its logits were equal.
 #include "common.hpp"
@@ -49,19 +52,20 @@ __global__ __launch_bounds__(256) void topk_softmax_kernel(const T* __restrict__
   float picked = 0.0f;          // lane j keeps the j-th selected probability (k <= 64)
   float sel_sum = 0.0f;
   for (int j = 0; j < k; ++j) {
-    float best = -1.0f;
-    int be = 0x7fffffff;
+    int most = __float_as_int(v[0]);                            // (-1, no candidate, is a negative integer as well)
+#pragma unroll
+    for (int q = 1; q < ROUTER_MAX_PER_LANE; ++q) most = max(most, __float_as_int(v[q]));
+    most = wave_max(most);
+    int be = 0;
+    unsigned long long holders = 0;
 #pragma unroll
     for (int q = 0; q < ROUTER_MAX_PER_LANE; ++q) {
-      const int e = q * 64 + lane;
-      if (v[q] > best) { best = v[q]; be = e; }                // ascending e inside a lane: first maximum wins
+      if (holders == 0 && q * 64 < E) {
+        holders = __ballot(__float_as_int(v[q]) == most);
+        be = q * 64 + __ffsll((long long)holders) - 1;
+      }
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ob = __shfl_xor(best, o, 64);
-      const int oe = __shfl_xor(be, o, 64);
-      if (ob > best || (ob == best && oe < be)) { best = ob; be = oe; }
-    }
+    const float best = __int_as_float(most);
     const float pr = best * inv;
     if (lane == j) picked = pr;
     sel_sum += pr;
