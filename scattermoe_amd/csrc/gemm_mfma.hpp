@@ -193,11 +193,13 @@ struct DirectOp {
   __device__ __forceinline__ void issue_one(unsigned tile, int k0, int j) const {
     load_to_lds16<STREAM>(base + (int64_t)k0 * 2, off[j], tile + wave_uniform_id() * 1024 + rnd(j) * NT * 16);
   }
-  // the same piece into registers, and where it belongs in the LDS tile
-  // (whole slices only: `kend` is not looked at)
-  __device__ __forceinline__ i32x4 load_piece(int k0, int, int j) const {
-    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)(base + (int64_t)k0 * 2), 0, -1, 0x00020000);
-    return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off[j], 0, 0));
+  // The same pieces into registers: what the loads of a slice have in common, here its byte offset (whole slices only; past the
+  // last one: that one again), and where a piece belongs in the LDS tile
+  typedef int Slice;
+  __device__ __forceinline__ Slice slice(int k0, int kend) const { return min(k0, kend - BK) * 2; }
+  __device__ __forceinline__ i32x4 load_piece(Slice s, int j) const {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, -1, 0x00020000);
+    return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off[j], s, 0));
   }
   __device__ __forceinline__ int piece_lds(int j) const { return (rnd(j) * NT + (int)threadIdx.x) * 16; }
   __device__ __forceinline__ void issue(unsigned tile, int k0) const {
@@ -343,13 +345,15 @@ struct TransOp {
     if constexpr (GATHER) load_to_lds16<STREAM>(make_uniform(base), off[j], tile + wave_uniform_id() * 1024 + rnd(j) * NT * 16);
     else load_to_lds16<STREAM>(base + (int64_t)k0 * ld + slot_off(j), off[j % OFFS], tile + wave_uniform_id() * 1024 + rnd(j) * NT * 16);
   }
-  // the same piece into registers (not for gathered rows), and where it belongs in the LDS tile
-  // Contraction rows from `kend` on read as zeros: the buffer descriptor of the slice ends with row kend - 1
-  // (a row's pieces lie inside its first `ld` bytes).
-  __device__ __forceinline__ i32x4 load_piece(int k0, int kend, int j) const {
-    const int64_t span = (int64_t)(kend - k0) * ld;
-    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(base + (int64_t)k0 * ld), 0, span < 0xffffffffLL ? (int)(unsigned)span : -1, 0x00020000);
+  // The same pieces into registers (not for gathered rows): what the loads of a slice have in common, here a buffer descriptor
+  // that ends with row kend - 1, so that contraction rows from there on read as zeros (a row's pieces lie inside its first `ld`
+  // bytes; past the last slice: an empty one), and where a piece belongs in the LDS tile
+  struct Slice { const char* base; int bytes; };
+  __device__ __forceinline__ Slice slice(int k0, int kend) const {
+    return Slice{make_uniform(base + (int64_t)k0 * ld), __builtin_amdgcn_readfirstlane(min(max(kend - k0, 0), BK) * (int)ld)};
+  }
+  __device__ __forceinline__ i32x4 load_piece(Slice s, int j) const {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)s.base, 0, s.bytes, 0x00020000);
     return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off[j % OFFS] + slot_off(j)), 0, 0));      // (a scalar offset would come off the range)
   }
   __device__ __forceinline__ int piece_lds(int j) const { return (rnd(j) * NT + (int)threadIdx.x) * 16; }
@@ -701,21 +705,32 @@ struct RsPlan {
   static constexpr int N = AOp::R + BOp::R;                       // pieces per thread and slice
   static constexpr int NM = TL::FM * TL::FN;                      // MFMAs per quarter of a step (Quarter), eight of them per slice
   static constexpr int L = (N + 3) / 4;                           // loads per two quarters (the first two: what is left)
-  static_assert(N <= 6 * NM, "at most one LDS write behind an MFMA");
   static constexpr bool is_b(int q) { return q >= 2 * AOp::R || (q & 1); }
   static constexpr int index(int q) { return q < 2 * AOp::R ? q >> 1 : q - AOp::R; }
-  // pieces written before MFMA g of the first six quarters
-  static constexpr int written(int g) { return N * (g + 1) / (6 * NM); }
-  static_assert(written(0) == 0 && written(6 * NM) == N, "every piece is written once");
-  static_assert(written(2 * NM) >= L && written(4 * NM) >= 2 * L && N >= 3 * L, "a piece is reloaded after it has been written");
-  static constexpr int loads_before(int n, int m) { return n * m / (2 * NM); }
+  // pieces written before quarter Q, the first six
+  static constexpr int written(int Q) { return N * Q / 6; }
+  static_assert(written(2) >= L && written(4) >= 2 * L && N >= 3 * L, "a piece is reloaded after it has been written");
+  // Places in a quarter: behind which MFMA fragment, write or load number i is issued.  An MFMA takes four issue slots, one of them
+  // its own, so memory instructions, their waits and scalar work go behind different ones.
+  static constexpr int read_at(int i, int NF) { return 2 * NF <= NM ? 2 * i : i; }
+  static constexpr int write_at(int i) { return NM - 2 - 3 * i > 0 ? NM - 2 - 3 * i : 0; }
+  static constexpr int load_at(int i) { return NM * (2 * i + 1) / 4 + (NM >= 8 ? 1 : 0); }
   // LDS: the two stages of the row operand, then those of the column operand, so that the instructions' offset fields reach from
   // one stage to the other (one set of addresses)
   static constexpr int A_STAGE = AOp::LDS_BYTES, B0 = 2 * AOp::LDS_BYTES, B_STAGE = BOp::LDS_BYTES;
 };
 
+// What the loads of the next slices have in common: at the start of slice kt of parity P, a[P], b[P] of slice kt + 2, the other
+// ones of slice kt + 3.
+template <class AOp, class BOp>
+struct RsSlices {
+  typename AOp::Slice a[2];
+  typename BOp::Slice b[2];
+};
+
 template <typename T, class TL, class AOp, class BOp, int P, int Q, int N>
-__device__ __forceinline__ void rs_quarter(const AOp& A, const BOp& B, char* lds, int k2, int k3, int kend, int wm, int wn,
+__device__ __forceinline__ void rs_quarter(const AOp& A, const BOp& B, char* lds, char* lds_b, int kt, int kend,
+                                           RsSlices<AOp, BOp>& sl, int wm, int wn,
                                            Block (&acc)[TL::FM][TL::FN], i32x4 (&g)[2][N],
                                            i32x4 (&fa)[2 * TL::FM], i32x4 (&fb)[2 * TL::FN]) {
   typedef RsPlan<TL, AOp, BOp> Plan;
@@ -723,30 +738,38 @@ __device__ __forceinline__ void rs_quarter(const AOp& A, const BOp& B, char* lds
   constexpr int NM = Plan::NM, S = P ^ 1;
   constexpr int NF = Qu::READ_A ? TL::FM : TL::FN;
   static_assert(NF <= NM, "at most one fragment read behind an MFMA");
-  // LDS traffic of the quarter in the order it is to be issued in (the compiler keeps reads and writes of LDS in
-  // program order): the fragments that are read in it behind the first MFMAs - from the stage being multiplied, in
-  // the last two quarters from the stage just filled - and the pieces of the first six spread evenly.
+  // fragments are read from the stage being multiplied, in the last two quarters from the stage just filled
   constexpr int src = Qu::READ_STEP == 2 ? S : P;
-  // pieces loaded in two quarters: the last ones of the other set (slice kt + 2), then a third each of the others of
-  // this one (slice kt + 3)
+  // pieces written to the other stage; pieces loaded in two quarters: the last ones of the other set (slice kt + 2), then a third
+  // each of the others of this one (slice kt + 3)
+  constexpr int w0 = Plan::written(Q), nw = Q < 6 ? Plan::written(Q + 1) - w0 : 0;
   constexpr int H = Q >> 1, SET = H == 0 ? P : S;
-  constexpr int q0 = H == 0 ? 3 * Plan::L : (H - 1) * Plan::L, nl = H == 0 ? N - 3 * Plan::L : Plan::L;
-  constexpr int m0 = (Q & 1) * NM;
-  const int k0 = H == 0 ? k2 : k3;
+  constexpr int q0 = H == 0 ? 3 * Plan::L : (H - 1) * Plan::L, nl2 = H == 0 ? N - 3 * Plan::L : Plan::L;
+  constexpr int l0 = q0 + nl2 * (Q & 1) / 2, nl = q0 + nl2 * ((Q & 1) + 1) / 2 - l0;
+  static_assert(nw <= 3 && nl <= 2, "places");
 #pragma unroll
   for (int m = 0; m < NM; ++m) {
     const int i = Qu::A * TL::FM + m / TL::FN, j = Qu::B * TL::FN + m % TL::FN;
     Mfma<T>::in_place(fb[j], fa[i], acc[i >> 1][j >> 1].q[2 * (i & 1) + (j & 1)]);
-    if (m < NF) quarter_read<TL, AOp, BOp, Q>(lds + src * Plan::A_STAGE, lds + Plan::B0 + src * Plan::B_STAGE, wm, wn, m, fa, fb);
-    if (Q < 6 && Plan::written(Q * NM + m + 1) > Plan::written(Q * NM + m)) {
-      const int q = Plan::written(Q * NM + m);
-      if (Plan::is_b(q)) lds_write16(lds + Plan::B0 + S * Plan::B_STAGE + B.piece_lds(Plan::index(q)), g[S][q]);
-      else lds_write16(lds + S * Plan::A_STAGE + A.piece_lds(Plan::index(q)), g[S][q]);
-    }
-    if (Plan::loads_before(nl, m0 + m + 1) > Plan::loads_before(nl, m0 + m)) {
-      const int q = q0 + Plan::loads_before(nl, m0 + m);
-      g[SET][q] = Plan::is_b(q) ? B.load_piece(k0, kend, Plan::index(q)) : A.load_piece(k0, kend, Plan::index(q));
-    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      if (Plan::read_at(f, NF) == m)
+        quarter_read<TL, AOp, BOp, Q>(lds + src * Plan::A_STAGE, lds_b + src * Plan::B_STAGE, wm, wn, f, fa, fb);
+#pragma unroll
+    for (int f = 0; f < nw; ++f)
+      if (Plan::write_at(nw - 1 - f) == m) {
+        const int q = w0 + f;
+        if (Plan::is_b(q)) lds_write16(lds_b + S * Plan::B_STAGE + B.piece_lds(Plan::index(q)), g[S][q]);
+        else lds_write16(lds + S * Plan::A_STAGE + A.piece_lds(Plan::index(q)), g[S][q]);
+      }
+#pragma unroll
+    for (int f = 0; f < nl; ++f)
+      if (Plan::load_at(f) == m) {
+        const int q = l0 + f;
+        g[SET][q] = Plan::is_b(q) ? B.load_piece(sl.b[SET], Plan::index(q)) : A.load_piece(sl.a[SET], Plan::index(q));
+      }
+    if (Q == 2 && m == NM / 2 - 1) sl.a[P] = A.slice((kt + 4) * BK, kend);
+    if (Q == 3 && m == NM / 2 - 1) sl.b[P] = B.slice((kt + 4) * BK, kend);
     __builtin_amdgcn_sched_barrier(0);
   }
   if constexpr (Q == 5) {
@@ -757,19 +780,19 @@ __device__ __forceinline__ void rs_quarter(const AOp& A, const BOp& B, char* lds
 }
 
 template <typename T, class TL, class AOp, class BOp, int P, int N>
-__device__ __forceinline__ void rs_slice(const AOp& A, const BOp& B, char* lds, int kt, int last_k0, int kend, int wm, int wn,
+__device__ __forceinline__ void rs_slice(const AOp& A, const BOp& B, char* lds, char* lds_b, int kt, int kend,
+                                         RsSlices<AOp, BOp>& sl, int wm, int wn,
                                          Block (&acc)[TL::FM][TL::FN], i32x4 (&g)[2][N],
                                          i32x4 (&fa)[2 * TL::FM], i32x4 (&fb)[2 * TL::FN]) {
-  const int k2 = min((kt + 2) * BK, last_k0), k3 = min((kt + 3) * BK, last_k0);
   __builtin_amdgcn_sched_barrier(0);
-  rs_quarter<T, TL, AOp, BOp, P, 0, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_quarter<T, TL, AOp, BOp, P, 1, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_quarter<T, TL, AOp, BOp, P, 2, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_quarter<T, TL, AOp, BOp, P, 3, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_quarter<T, TL, AOp, BOp, P, 4, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_quarter<T, TL, AOp, BOp, P, 5, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_quarter<T, TL, AOp, BOp, P, 6, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
-  rs_quarter<T, TL, AOp, BOp, P, 7, N>(A, B, lds, k2, k3, kend, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 0, N>(A, B, lds, lds_b, kt, kend, sl, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 1, N>(A, B, lds, lds_b, kt, kend, sl, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 2, N>(A, B, lds, lds_b, kt, kend, sl, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 3, N>(A, B, lds, lds_b, kt, kend, sl, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 4, N>(A, B, lds, lds_b, kt, kend, sl, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 5, N>(A, B, lds, lds_b, kt, kend, sl, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 6, N>(A, B, lds, lds_b, kt, kend, sl, wm, wn, acc, g, fa, fb);
+  rs_quarter<T, TL, AOp, BOp, P, 7, N>(A, B, lds, lds_b, kt, kend, sl, wm, wn, acc, g, fa, fb);
 }
 
 template <typename T, class TL, class AOp, class BOp>
@@ -782,24 +805,30 @@ __device__ __forceinline__ void mainloop_rs(const AOp& A, const BOp& B, int klen
   // A partial last slice only with operands that zero-fill (TransOp); without any contraction rows one slice of
   // zeros is multiplied (no branch around the loop: 256 accumulator registers would have to be merged behind it).
   const int nk = max(1, (klen + BK - 1) / BK);
-  const int last_k0 = (nk - 1) * BK;
   i32x4 g[2][N];
   i32x4 fa[2 * TL::FM], fb[2 * TL::FN];
-  const int k1 = min(BK, last_k0), k2 = min(2 * BK, last_k0);
-  auto load = [&](int k0, int q) {
-    return Plan::is_b(q) ? B.load_piece(k0, klen, Plan::index(q)) : A.load_piece(k0, klen, Plan::index(q));
+  RsSlices<AOp, BOp> sl = {{A.slice(0, klen), A.slice(BK, klen)}, {B.slice(0, klen), B.slice(BK, klen)}};
+  auto load = [&](int set, int q) {
+    return Plan::is_b(q) ? B.load_piece(sl.b[set], Plan::index(q)) : A.load_piece(sl.a[set], Plan::index(q));
   };
+  // the column operand's stages from an address of their own (kept from being folded into constants): an instruction's offset
+  // field does not reach them from the row operand's
+  unsigned second = Plan::B0;
+  asm volatile("" : "+v"(second));
+  char* lds_b = lds + second;
 #pragma unroll
   for (int q = 0; q < N; ++q) g[0][q] = load(0, q);
 #pragma unroll
-  for (int q = 0; q < N; ++q) g[1][q] = load(k1, q);
+  for (int q = 0; q < N; ++q) g[1][q] = load(1, q);
+  sl.a[0] = A.slice(2 * BK, klen), sl.b[0] = B.slice(2 * BK, klen);
+  sl.a[1] = A.slice(3 * BK, klen), sl.b[1] = B.slice(3 * BK, klen);
 #pragma unroll
   for (int q = 0; q < N; ++q) {
-    if (Plan::is_b(q)) lds_write16(lds + Plan::B0 + B.piece_lds(Plan::index(q)), g[0][q]);
+    if (Plan::is_b(q)) lds_write16(lds_b + B.piece_lds(Plan::index(q)), g[0][q]);
     else lds_write16(lds + A.piece_lds(Plan::index(q)), g[0][q]);
   }
 #pragma unroll
-  for (int q = 0; q < 3 * Plan::L; ++q) g[0][q] = load(k2, q);
+  for (int q = 0; q < 3 * Plan::L; ++q) g[0][q] = load(0, q);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
@@ -807,13 +836,13 @@ __device__ __forceinline__ void mainloop_rs(const AOp& A, const BOp& B, int klen
 #pragma unroll
   for (int i = 0; i < TL::FM; ++i) fa[i] = AOp::frag(lds, wm * TL::WTM + i * 16, 0);
 #pragma unroll
-  for (int j = 0; j < TL::FN; ++j) fb[j] = BOp::frag(lds + Plan::B0, wn * TL::WTN + j * 16, 0);
+  for (int j = 0; j < TL::FN; ++j) fb[j] = BOp::frag(lds_b, wn * TL::WTN + j * 16, 0);
   int kt = 0;
   for (; kt + 1 < nk; kt += 2) {
-    rs_slice<T, TL, AOp, BOp, 0, N>(A, B, lds, kt, last_k0, klen, wm, wn, acc, g, fa, fb);
-    rs_slice<T, TL, AOp, BOp, 1, N>(A, B, lds, kt + 1, last_k0, klen, wm, wn, acc, g, fa, fb);
+    rs_slice<T, TL, AOp, BOp, 0, N>(A, B, lds, lds_b, kt, klen, sl, wm, wn, acc, g, fa, fb);
+    rs_slice<T, TL, AOp, BOp, 1, N>(A, B, lds, lds_b, kt + 1, klen, sl, wm, wn, acc, g, fa, fb);
   }
-  if (kt < nk) rs_slice<T, TL, AOp, BOp, 0, N>(A, B, lds, kt, last_k0, klen, wm, wn, acc, g, fa, fb);
+  if (kt < nk) rs_slice<T, TL, AOp, BOp, 0, N>(A, B, lds, lds_b, kt, klen, sl, wm, wn, acc, g, fa, fb);
   // (the compiler does not know how long the products above, being assembly, take to write their accumulators: 19 wait states at
   // the most; they are read by assembly, see stage_accumulators)
   asm volatile("s_nop 15\n\ts_nop 3");
