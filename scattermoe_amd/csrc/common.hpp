@@ -98,6 +98,28 @@ __device__ __forceinline__ void oss_grad(float gate, float up, float dh, float a
 }
 
 // ---- expert-aligned tile lookup -------------------------------------------------------------------
+// Inclusive sums over the wave's lanes: row shifts and row broadcasts (a lane without a source adds 0).  The lookups below stand at
+// the head of every tile, where nothing hides them, and are nothing but latency: a scan through six LDS shuffles takes about 700
+// cycles, this one about 60.
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);       // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);       // lane 15 of a row to the next row
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);       // lane 31 to the upper half
+  return v;
+}
+// Rows [lo, hi) of expert e0 + lane (none beyond the last one).
+__device__ __forceinline__ void load_expert_rows(const int64_t* __restrict__ off, int E, int e0, int& lo, int& hi) {
+  const int e = e0 + lane_id();
+  lo = hi = 0;
+  if (e < E) {
+    hi = (int)off[e];
+    lo = e ? (int)off[e - 1] : 0;
+  }
+}
+
 // Rows are expert-sorted; expert e owns rows [off[e-1], off[e]).  Tiles of height BM never straddle
 // two experts: expert e contributes ceil(count_e / BM) tiles and tiles are numbered expert-major.
 // Every wave of the block runs this redundantly and gets the same (uniform) answer.
@@ -108,24 +130,15 @@ __device__ __forceinline__ void oss_grad(float gate, float up, float dh, float a
 template <int BM>
 __device__ __forceinline__ bool find_tile(const int64_t* __restrict__ off, int E, int t,
                                           int& expert, int& row_start, int& rows, int skip_small = 0) {
-  const int lane = lane_id();
-  int tiles_before = 0;
+  int tiles_before = 0, lo, hi;
+  load_expert_rows(off, E, 0, lo, hi);
   for (int e0 = 0; e0 < E; e0 += 64) {
-    const int e = e0 + lane;
-    int lo = 0, hi = 0;
-    if (e < E) {
-      hi = (int)off[e];
-      lo = e ? (int)off[e - 1] : 0;
-    }
+    int lo_next = 0, hi_next = 0;                               // of the next 64 experts: on their way meanwhile
+    if (e0 + 64 < E) load_expert_rows(off, E, e0 + 64, lo_next, hi_next);
     int nt = (hi - lo + BM - 1) / BM;
     const int rem = (hi - lo) % BM;
     if (rem != 0 && rem <= skip_small) nt -= 1;
-    int incl = nt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      int v = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += v;
-    }
+    const int incl = wave_scan(nt);
     const int cum = tiles_before + incl;
     const unsigned long long hit = __ballot(cum > t);
     if (hit) {
@@ -139,6 +152,7 @@ __device__ __forceinline__ bool find_tile(const int64_t* __restrict__ off, int E
       return true;
     }
     tiles_before += __builtin_amdgcn_readlane(incl, 63);
+    lo = lo_next, hi = hi_next;
   }
   return false;
 }
@@ -148,9 +162,7 @@ template <int BM>
 __device__ __forceinline__ int count_tile_rows(const int64_t* __restrict__ off, int E) {
   int n = 0;
   for (int e = lane_id(); e < E; e += 64) n += ((int)(off[e] - (e ? off[e - 1] : 0)) + BM - 1) / BM;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) n += __shfl_xor(n, d, 64);
-  return __builtin_amdgcn_readfirstlane(n);
+  return __builtin_amdgcn_readlane(wave_scan(n), 63);
 }
 
 // Largest of the wave's values, in a scalar register: six row shifts and row broadcasts (lanes without a source keep
@@ -179,24 +191,15 @@ __device__ __forceinline__ int wave_max(int v) {
 template <int BM, bool HEIGHTS>
 __device__ __forceinline__ int find_tile_chunked(const int64_t* __restrict__ off, int E, int pid, int n_tiles,
                                                  int round, int& expert, int& row_start, int& rows, int& column) {
-  const int lane = lane_id();
-  auto load = [&](int e0, int& lo, int& hi, int& nt) {        // experts e0 .. e0 + 63, one per lane
-    const int e = e0 + lane;
-    lo = hi = 0;
-    if (e < E) {
-      hi = (int)off[e];
-      lo = e ? (int)off[e - 1] : 0;
-    }
+  // experts e0 .. e0 + 63, one per lane; the first 128 are loaded once, side by side
+  int lo0, hi0, lo1 = 0, hi1 = 0;
+  load_expert_rows(off, E, 0, lo0, hi0);
+  if (E > 64) load_expert_rows(off, E, 64, lo1, hi1);
+  auto load = [&](int e0, int& lo, int& hi, int& nt) {
+    if (e0 == 0) lo = lo0, hi = hi0;
+    else if (e0 == 64) lo = lo1, hi = hi1;
+    else load_expert_rows(off, E, e0, lo, hi);
     nt = (hi - lo + BM - 1) / BM;
-  };
-  auto scan = [&](int nt) {                                   // inclusive sums
-    int incl = nt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      int v = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += v;
-    }
-    return incl;
   };
   int lo, hi, nt;
   load(0, lo, hi, nt);
@@ -215,12 +218,12 @@ __device__ __forceinline__ int find_tile_chunked(const int64_t* __restrict__ off
     return 4 * (most_ + wave_max(-least_)) > most_;
   };
   if (__ballot(most > 1) && differ(most, least) && (!HEIGHTS || differ(most_b, least_b))) return -1;
-  int incl = scan(nt);
+  int incl = wave_scan(nt);
   int total = __builtin_amdgcn_readlane(incl, 63);
   for (int e0 = 64; e0 < E; e0 += 64) {
     int l_, h_, n_;
     load(e0, l_, h_, n_);
-    total += __builtin_amdgcn_readlane(scan(n_), 63);
+    total += __builtin_amdgcn_readlane(wave_scan(n_), 63);
   }
   const unsigned tiles = (unsigned)total * n_tiles;
   const unsigned R = round && tiles >= round + round / 2u ? (tiles + round / 2u) / round : 1;
@@ -248,7 +251,7 @@ __device__ __forceinline__ int find_tile_chunked(const int64_t* __restrict__ off
     e0 += 64;
     if (e0 >= E) return 0;
     load(e0, lo, hi, nt);
-    incl = scan(nt);
+    incl = wave_scan(nt);
   }
 }
 // Workgroups of such a launch of at most `tiles` tiles: 8 R chunks round up by less than 8 R <= tiles / 32 + 8.
