@@ -16,7 +16,7 @@ LIB_PATH = os.path.join(PKG_DIR, "libscattermoe_amd.so")
 PROBE_SRC = os.path.join(CSRC, "bench", "mfma_probe.hip")
 PROBE_LIB_PATH = os.path.join(PKG_DIR, "libsmoe_bench_probe.so")
 
-SOURCES = ["capi.hip", "route.hip", "group.hip", "s2s_generic.hip", "xty_generic.hip", "gemm_mfma.hip", "gemm_mfma_f16.hip", "gemm_mfma_xty.hip", "fused.hip", "router.hip", "s2s_rowdot.hip", "gemm_f32.hip"]
+SOURCES = ["capi.hip", "route.hip", "group.hip", "s2s_generic.hip", "xty_generic.hip", "gemm_mfma.hip", "gemm_mfma_f16.hip", "gemm_mfma_f16_n.hip", "gemm_mfma_xty.hip", "fused.hip", "router.hip", "s2s_rowdot.hip", "gemm_f32.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

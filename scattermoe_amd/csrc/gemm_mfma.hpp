@@ -59,6 +59,11 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 static constexpr int BK = 64;               // contraction slice per stage
 
+// Weight layouts whose kernels a source instantiates: 1 K-contiguous, 2 N-contiguous, 3 both (sources compile side by side)
+#ifndef SMOE_LAYOUTS
+#define SMOE_LAYOUTS 3
+#endif
+
 // Products are 16 x 16 x 32, not 32 x 32 x 16: the launches run at the power cap, and the smaller shape moves a quarter of the
 // accumulators per instruction through the matrix cores for twice the operands.  Nothing but independent instructions on random
 // operands in registers, one wave per SIMD: 1.80 PFLOP/s with 32 x 32 x 16, 2.01 with 16 x 16 x 32.  One of these adds up its
@@ -199,7 +204,7 @@ struct DirectOp {
   __device__ __forceinline__ Slice slice(int k0, int kend) const { return min(k0, kend - BK) * 2; }
   __device__ __forceinline__ i32x4 load_piece(Slice s, int j) const {
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, -1, 0x00020000);
-    return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off[j], s, 0));
+    return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off[j], s, STREAM ? 2 : 0));
   }
   __device__ __forceinline__ int piece_lds(int j) const { return (rnd(j) * NT + (int)threadIdx.x) * 16; }
   __device__ __forceinline__ void issue(unsigned tile, int k0) const {
@@ -354,7 +359,7 @@ struct TransOp {
   }
   __device__ __forceinline__ i32x4 load_piece(Slice s, int j) const {
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)s.base, 0, s.bytes, 0x00020000);
-    return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off[j % OFFS] + slot_off(j)), 0, 0));      // (a scalar offset would come off the range)
+    return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off[j % OFFS] + slot_off(j)), 0, STREAM ? 2 : 0));      // (a scalar offset would come off the range)
   }
   __device__ __forceinline__ int piece_lds(int j) const { return (rnd(j) * NT + (int)threadIdx.x) * 16; }
   __device__ __forceinline__ void issue(unsigned tile, int k0) const {
@@ -531,15 +536,17 @@ __device__ __forceinline__ void issue_slice_tail(const AOp& A, const BOp& B, uns
 
 // WG_: workgroups per CU the registers have to leave room for (LDS permitting)
 // PAIR_: two workgroups per CU that fill its LDS between them (mainloop_pair)
-template <int BM_, int BN_, int WM_, int WN_, int NS_ = 2, bool RS_ = false, int WG_ = 1, bool PAIR_ = false>
+// ONCE_: the tile is its expert's only one in its column: nobody else reads its weights (see s2s_tile)
+template <int BM_, int BN_, int WM_, int WN_, int NS_ = 2, bool RS_ = false, int WG_ = 1, bool PAIR_ = false, bool ONCE_ = false>
 struct Tile {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_;
   static constexpr int NS = NS_;                      // LDS stages (2: double buffer, more: ring)
   static constexpr bool RS = RS_;                     // operands travel global -> registers -> LDS (mainloop_rs)
   static constexpr int WG = WG_;
-  static constexpr bool PAIR = PAIR_;
+  static constexpr bool PAIR = PAIR_, ONCE = ONCE_;
   // the same tile with U blocks of 32 rows per wave
-  template <int U> using Height = Tile<U * 32 * WM_, BN_, WM_, WN_, NS_, RS_, WG_, PAIR_>;
+  template <int U> using Height = Tile<U * 32 * WM_, BN_, WM_, WN_, NS_, RS_, WG_, PAIR_, ONCE_>;
+  typedef Tile<BM_, BN_, WM_, WN_, NS_, RS_, WG_, PAIR_, true> Once;
   static constexpr int NW = WM * WN, NT = NW * 64;
   static constexpr int WAVES_PER_SIMD = WG_ * NW / 4 > 0 ? WG_ * NW / 4 : 1;
   static constexpr int WTM = BM / WM, WTN = BN / WN;
@@ -1600,6 +1607,7 @@ struct Raster {
   int m_tiles, n_tiles, m_supers, n_supers, supers, gm;
   int striped;                             // 1: column-striped order of the memory-bound classes (see make_striped)
   int chunked = 0;                         // 1, 2: order of find_tile_chunked (2: in rounds) before this one
+  int once = 0;                            // weights of experts of one tile row bypass the caches (see reads_weights_once)
   int64_t grid_size;                       // host side only: number of workgroups (may exceed what a launch takes)
   __host__ int64_t grid() const { return grid_size; }
   // (ml, nl): position of the tile inside its super tile
@@ -1690,7 +1698,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   // once, and with the non-temporal hint it does not push the token rows, which every workgroup of a tile row reads,
   // out of the L2s (hint extended from the 32-/64-row classes to all ring classes: Mixtral layer forward at 256 /
   // 384 / 448 tokens 0.539 -> 0.505 / 0.559 -> 0.526 / 0.711 -> 0.688 ms, neutral from 768 tokens on)
-  constexpr bool W_ONCE = TL::NS > 2 || (TL::WG > 1 && !TL::PAIR);
+  constexpr bool W_ONCE = TL::ONCE || TL::NS > 2 || (TL::WG > 1 && !TL::PAIR);
   typedef typename std::conditional<B_TR, TransOp<TL::BN, TL::NT, W_ONCE, false, TL::RS>, DirectOp<TL::BN, TL::NT, W_ONCE>>::type BOp;
   constexpr bool LAST_TILES = TL::BM == 128 && TL::BN == 256 && TL::NS == 3;
   constexpr bool CAN_SPLIT = LAST_TILES || TL::RS;
@@ -1819,6 +1827,20 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   }
 }
 
+// A tile of at most TL::BM = 256 rows.  An expert's last tile is partly filled: it is multiplied at the height of its rows, in
+// steps of 64 (which keep the four waves, or the eight, equally busy), not as a whole tile.  (Same sums in the same order.)
+// What it buys is that such tiles need no launch of their own any more (see cut_tails); a training step with many
+// tiles per expert is the same with it (Mixtral shape, 16.5 tiles per expert).
+template <typename T, class TL, bool B_TR>
+__device__ __forceinline__ void s2s_tile_at_height(const S2SArgs& a, const S2STile& t, int n_tiles, char* lds, int64_t* sDst,
+                                                   const int* sSrc, float* sBias) {
+  const int h = (t.rows + 63) >> 6;
+  if (h == 4) s2s_tile<T, TL, B_TR>(a, t, n_tiles, lds, sDst, sSrc, sBias);
+  else if (h == 3) s2s_tile<T, typename TL::template Height<3>, B_TR>(a, t, n_tiles, lds, sDst, sSrc, sBias);
+  else if (h == 2) s2s_tile<T, typename TL::template Height<2>, B_TR>(a, t, n_tiles, lds, sDst, sSrc, sBias);
+  else s2s_tile<T, typename TL::template Height<1>, B_TR>(a, t, n_tiles, lds, sDst, sSrc, sBias);
+}
+
 template <typename T, class TL, bool B_TR>
 __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2SArgs a, Raster rast) {
   // (a workgroup that shares its CU's LDS with one other keeps its row tables where operands are to come: the source rows in
@@ -1899,15 +1921,13 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
   }
   __syncthreads();
   if constexpr (TL::BM == 256 && (TL::BN == 256 || TL::PAIR)) {
-    // An expert's last tile is partly filled: it is multiplied at the height of its rows, in steps of 64 (which keep
-    // the four waves, or the eight, equally busy), not as a whole tile.  (Same sums in the same order.)
-    // What it buys is that such tiles need no launch of their own any more (see cut_tails); a training step with many
-    // tiles per expert is the same with it (Mixtral shape, 16.5 tiles per expert).
-    const int h = (t.rows + 63) >> 6;
-    if (h == 4) s2s_tile<T, TL, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
-    else if (h == 3) s2s_tile<T, typename TL::template Height<3>, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
-    else if (h == 2) s2s_tile<T, typename TL::template Height<2>, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
-    else s2s_tile<T, typename TL::template Height<1>, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
+    if constexpr (TL::RS || TL::PAIR) {
+      if (rast.once && (int)a.off[t.e] - (t.e ? (int)a.off[t.e - 1] : 0) <= TL::BM) {
+        s2s_tile_at_height<T, typename TL::Once, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
+        return;
+      }
+    }
+    s2s_tile_at_height<T, TL, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
   } else {
     s2s_tile<T, TL, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
   }
@@ -2012,6 +2032,19 @@ static double expected_row_tiles(int64_t L, int E, int skip_small = 0) {
   return nearbyint(per_expert * E);
 }
 
+// An expert of one tile row has each weight read by one workgroup; with the non-temporal hint they leave the token rows in the L2s,
+// as in the ring classes.  Only where the weights are more than the 256 MB of the memory-side cache: a program whose other data
+// leaves them there finds them there (16 experts x 133 rows, 1024 -> 4960, 162 MB, launched again and again 46 -> 60 us; 64 x 120,
+// 1024 -> 2048, 268 MB 57 -> 61).  An expert of several tile rows reads them from the L2 as often (8 x 300 rows, 4096 -> 14336 with the
+// hint on its last tile 387 -> 447 us), hence by expert, asked where at least some are expected to have one.  us, without -> with the
+// hint: 128 x 188 rows, 2048 -> 1536 209 -> 191, 768 -> 2048 122 -> 115; 128 x 250 rows 255 -> 230, 141 -> 130, gated 263 -> 240;
+// 32 x 188 rows, 2880 -> 2880 148 -> 137, 2880 -> 5760 232 -> 227; 8 x 120 rows, 4096 -> 28672 364 -> 351, 8 x 194 475 -> 475.
+static constexpr int64_t ONCE_MIN_WEIGHTS = 320ll << 20;
+static constexpr int ONCE_BELOW_ROWS = 640;
+static bool reads_weights_once(const S2SArgs& a) {
+  return a.L / a.E < ONCE_BELOW_ROWS && (int64_t)a.E * a.K * 2 * (a.glu == 1 ? 2 : 1) * a.N >= ONCE_MIN_WEIGHTS;
+}
+
 template <typename T, class TL>
 static int launch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
   const int bn = a.glu == 1 ? TL::BN / 2 : TL::BN;     // output columns per tile
@@ -2029,16 +2062,17 @@ static int launch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
     r.chunked = TL::NS > 2 || (TL::WG > 1 && !TL::PAIR) || a.L / a.E < ROWS256_BELOW ? 1 : 2;
     r.grid_size = std::max(r.grid_size, chunked);
   }
+  r.once = reads_weights_once(a);
   const int64_t grid = r.grid();
   const unsigned parts = a.ksplit > 1 && !whole_parts ? (unsigned)a.ksplit : 1u;
   if (grid > 0x7fffffffLL || m_tiles > 0x7fffffffLL) { set_error("smoe_scatter2scatter: grid too large"); return SMOE_ERR_RANGE; }
-  if constexpr (TL::BN % 128 == 0) {
+  if constexpr (TL::BN % 128 == 0 && (SMOE_LAYOUTS & 2)) {
     if (b_tr) {
       hipLaunchKernelGGL((s2s_mfma_kernel<T, TL, true>), dim3((unsigned)grid, parts), dim3(TL::NT), 0, st, a, r);
       return launch_status("s2s_mfma_kernel");
     }
   }
-  hipLaunchKernelGGL((s2s_mfma_kernel<T, TL, false>), dim3((unsigned)grid, parts), dim3(TL::NT), 0, st, a, r);
+  if constexpr (SMOE_LAYOUTS & 1) hipLaunchKernelGGL((s2s_mfma_kernel<T, TL, false>), dim3((unsigned)grid, parts), dim3(TL::NT), 0, st, a, r);
   return launch_status("s2s_mfma_kernel");
 }
 
