@@ -708,12 +708,12 @@ __device__ __forceinline__ void mainloop(AOp& A, BOp& B, int klen, char* lds, bo
 // operand (the smaller one in a tile of fewer than 256 rows) has pieces left.
 template <class TL, class AOp, class BOp>
 struct RsPlan {
-  static_assert(AOp::R <= BOp::R && BOp::R == 8, "the column operand is the larger one");
+  static constexpr int BOTH = AOp::R < BOp::R ? AOp::R : BOp::R;
   static constexpr int N = AOp::R + BOp::R;                       // pieces per thread and slice
   static constexpr int NM = TL::FM * TL::FN;                      // MFMAs per quarter of a step (Quarter), eight of them per slice
   static constexpr int L = (N + 3) / 4;                           // loads per two quarters (the first two: what is left)
-  static constexpr bool is_b(int q) { return q >= 2 * AOp::R || (q & 1); }
-  static constexpr int index(int q) { return q < 2 * AOp::R ? q >> 1 : q - AOp::R; }
+  static constexpr bool is_b(int q) { return q >= 2 * BOTH ? BOp::R > AOp::R : (q & 1) != 0; }
+  static constexpr int index(int q) { return q < 2 * BOTH ? q >> 1 : q - BOTH; }
   // pieces written before quarter Q, the first six
   static constexpr int written(int Q) { return N * Q / 6; }
   static_assert(written(2) >= L && written(4) >= 2 * L && N >= 3 * L, "a piece is reloaded after it has been written");
@@ -1070,12 +1070,13 @@ __device__ __forceinline__ void set_pair(V& v, int k, float a, float b) {
 // After the main loop the operand buffers are free.  The accumulators (transposed blocks, see `epilogue`) are
 // rounded to the storage type and written to LDS as a row-major BM x BN tile, so that the global traffic of the
 // epilogue can be 16 bytes per lane with a wave covering whole 128-byte lines: 16-byte piece c of row r sits at
-// chunk c ^ (r & (CPR-1)) of the row, which keeps both the 8-byte column-strided writes and the 16-byte
+// chunk c ^ (r & (CPR-1)) of the row (192 columns: c ^ (r & 7)), which keeps both the 8-byte column-strided writes and the 16-byte
 // row-major reads free of bank conflicts.
 template <class TL>
 __device__ __forceinline__ int staged_addr(int row, int col) {
   constexpr int CPR = TL::BN / 8;
-  return row * (TL::BN * 2) + ((((col >> 3) ^ row) & (CPR - 1)) << 4) + ((col & 7) << 1);
+  constexpr int SWZ = (CPR & (CPR - 1)) == 0 ? CPR - 1 : 7;
+  return row * (TL::BN * 2) + (((col >> 3) ^ (row & SWZ)) << 4) + ((col & 7) << 1);
 }
 
 // The thread's index, for what comes behind the main loop: the one-wave-per-SIMD form, and four workgroups per CU, have no
@@ -1319,7 +1320,7 @@ __device__ __forceinline__ void epilogue_staged(const Block (&acc)[TL::FM][TL::F
     stage_accumulators<T, TL>(acc, lds, [&](int tc) { return plain_bias<T>(bias, sb, ncols, n0 + tc); }, nullptr);
   // In groups: the row offsets of a group, then its pieces, are read from LDS back to back before the first of its
   // stores (written as one conditional store per piece, every piece would wait for two LDS round trips of its own)
-  constexpr int GRP = PP % 16 == 0 ? 16 : PP % 8 == 0 ? 8 : PP;
+  constexpr int GRP = PP % 16 == 0 ? 16 : PP % 8 == 0 ? 8 : PP % 6 == 0 ? 6 : PP;
   static_assert(PP % GRP == 0, "groups must divide the pieces");
 #pragma unroll
   for (int q0 = 0; q0 < PP; q0 += GRP) {
@@ -1414,7 +1415,7 @@ __device__ __forceinline__ void epilogue_glu_bwd_staged(const Block (&acc)[TL::F
   const int tx = late_thread<TL>();
   typedef T T8 __attribute__((ext_vector_type(8)));
   constexpr int CPR = TL::BN / 8, PIECES = TL::BM * CPR, PP = PIECES / TL::NT;
-  constexpr int GRP = PP % 8 == 0 ? 4 : PP % 4 == 0 ? 2 : (PP >= 2 ? PP / 2 : 1);    // pieces per group, two in flight
+  constexpr int GRP = PP % 8 == 0 ? 4 : PP % 4 == 0 ? 2 : PP % 6 == 0 ? 3 : (PP >= 2 ? PP / 2 : 1);    // pieces per group, two in flight
   static_assert(PIECES % TL::NT == 0 && (PP == 1 || PP % (2 * GRP) == 0), "pieces must divide evenly");
   if constexpr (!TL::RS) stage_accumulators<T, TL>(acc, lds, [](int) { return 0.0f; }, nullptr);
   const int F = a.N;
@@ -1537,7 +1538,7 @@ __device__ __forceinline__ void epilogue_oss_bwd_staged(const Block (&acc)[TL::F
   const int tx = late_thread<TL>();
   typedef T T8 __attribute__((ext_vector_type(8)));
   constexpr int CPR = TL::BN / 8, PIECES = TL::BM * CPR, PP = PIECES / TL::NT;
-  constexpr int GRP = PP % 8 == 0 ? 4 : PP % 4 == 0 ? 2 : (PP >= 2 ? PP / 2 : 1);    // pieces per group, two in flight
+  constexpr int GRP = PP % 8 == 0 ? 4 : PP % 4 == 0 ? 2 : PP % 6 == 0 ? 3 : (PP >= 2 ? PP / 2 : 1);    // pieces per group, two in flight
   static_assert(PIECES % TL::NT == 0 && (PP == 1 || PP % (2 * GRP) == 0), "pieces must divide evenly");
   if constexpr (!TL::RS) stage_accumulators<T, TL>(acc, lds, [](int) { return 0.0f; }, nullptr);
   const int F = a.N;
@@ -1689,6 +1690,11 @@ struct S2STile {
   int slot;                     // thread m < BM: slot of row m of the tile, where one is needed
 };
 
+// Columns of a tile's column operand in LDS, if it is read transposed: tiles of 192 columns keep the layout of 256 and do not
+// multiply the last 64 (which repeat column 0: one more request of a piece that is there).
+template <class TL>
+static constexpr int column_extent = TL::BN == 192 ? 256 : TL::BN;
+
 // One output tile; TL::BM >= rows.
 template <typename T, class TL, bool B_TR>
 __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int n_tiles, char* lds, int64_t* sDst,
@@ -1699,7 +1705,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   // out of the L2s (hint extended from the 32-/64-row classes to all ring classes: Mixtral layer forward at 256 /
   // 384 / 448 tokens 0.539 -> 0.505 / 0.559 -> 0.526 / 0.711 -> 0.688 ms, neutral from 768 tokens on)
   constexpr bool W_ONCE = TL::ONCE || TL::NS > 2 || (TL::WG > 1 && !TL::PAIR);
-  typedef typename std::conditional<B_TR, TransOp<TL::BN, TL::NT, W_ONCE, false, TL::RS>, DirectOp<TL::BN, TL::NT, W_ONCE>>::type BOp;
+  typedef typename std::conditional<B_TR, TransOp<column_extent<TL>, TL::NT, W_ONCE, false, TL::RS>, DirectOp<TL::BN, TL::NT, W_ONCE>>::type BOp;
   constexpr bool LAST_TILES = TL::BM == 128 && TL::BN == 256 && TL::NS == 3;
   constexpr bool CAN_SPLIT = LAST_TILES || TL::RS;
   const int glu = TL::RS ? __builtin_amdgcn_readfirstlane(a.glu) : -1;      // (as for the tile in s2s_mfma_kernel)
@@ -1732,7 +1738,7 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
       B.init(Wb, [&](int row) { return (int64_t)wcol(row) * swn * 2; });
     }
   } else if constexpr (B_TR) {
-    B.init(Wb + (int64_t)n0 * 2, a.swk * 2, a.N - n0);
+    B.init(Wb + (int64_t)n0 * 2, a.swk * 2, TL::BN == 192 ? min(a.N - n0, TL::BN) : a.N - n0);
   } else {
     const int64_t swn = a.swn;
     const int N = a.N;
@@ -1800,14 +1806,18 @@ __device__ __forceinline__ void s2s_tile(const S2SArgs& a, const S2STile& t, int
   if constexpr (TL::RS) {
     // (staged here, once for all epilogues: a copy of the walk over 256 accumulators in each costs registers ahead of them)
     stage_accumulators<T, TL>(acc, lds, [&](int tc) {
-      if (glu == 1) return glu_bias<T, TL>(a, bias, n0, tc);
+      if constexpr (TL::BN != 192) {
+        if (glu == 1) return glu_bias<T, TL>(a, bias, n0, tc);
+      }
       return glu == 0 || glu == 3 ? plain_bias<T>(bias, a.sbn, a.N, n0 + tc) : 0.0f;
     }, sBias);
     if (glu == 0) epilogue_staged<T, TL>(acc, (T*)a.Y, sDst, n0, a.N, bias, a.sbn, lds);
-    else if (glu == 1) epilogue_glu_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds);
     else if (glu == 2) epilogue_glu_bwd_staged<T, TL>(acc, a, row0, rows, n0, lds);
-    else if (glu == 3) epilogue_oss_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds);
-    else epilogue_oss_bwd_staged<T, TL>(acc, a, row0, rows, n0, lds);
+    else if (glu == 4) epilogue_oss_bwd_staged<T, TL>(acc, a, row0, rows, n0, lds);
+    if constexpr (TL::BN != 192) {                          // (192 columns: not the forward units, see narrow_columns)
+      if (glu == 1) epilogue_glu_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds);
+      else if (glu == 3) epilogue_oss_fwd_staged<T, TL>(acc, a, row0, rows, n0, bias, lds);
+    }
   } else if (a.glu == 0) {
     const bool al16 = (((uintptr_t)a.Y & 15) == 0) && ((a.sym | a.N) & 7) == 0;
     if (al16) epilogue_staged<T, TL>(acc, (T*)a.Y, sDst, n0, a.N, bias, a.sbn, lds);
@@ -1846,7 +1856,7 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
   // (a workgroup that shares its CU's LDS with one other keeps its row tables where operands are to come: the source rows in
   // the second row stage, which is requested behind a barrier that follows their last reading, the output rows in the
   // column stage)
-  constexpr int STAGE = (TL::BM + TL::BN) * 128;
+  constexpr int STAGE = (TL::BM + (B_TR ? column_extent<TL> : TL::BN)) * 128;
   static_assert(TL::BM * TL::BN * 2 <= (TL::PAIR ? PAIR_B : TL::NS * STAGE), "staged tile must fit the operand buffers");
   __shared__ __attribute__((aligned(16))) char lds[TL::PAIR ? PAIR_LDS : TL::NS * STAGE];
   __shared__ int64_t sDst_[TL::PAIR ? 1 : TL::BM];
@@ -1880,7 +1890,7 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
     if (found == 0) return;
   } else if (rast.chunked) {
     t.m_loc = t.n_loc = 0;
-    found = find_tile_chunked<TL::BM, TL::BM == 256 && (TL::BN == 256 || TL::PAIR)>(a.off, a.E, blockIdx.x, rast.n_tiles,
+    found = find_tile_chunked<TL::BM, TL::BM == 256 && (TL::BN == 256 || TL::RS || TL::PAIR)>(a.off, a.E, blockIdx.x, rast.n_tiles,
                                                                       rast.chunked == 2 ? TL::WG * 256 : 0,
                                                                       t.e, t.row0, t.rows, t.n_tile);
     if (found == 0) return;
@@ -1920,7 +1930,7 @@ __global__ __launch_bounds__(TL::NT, TL::WAVES_PER_SIMD) void s2s_mfma_kernel(S2
     }
   }
   __syncthreads();
-  if constexpr (TL::BM == 256 && (TL::BN == 256 || TL::PAIR)) {
+  if constexpr (TL::BM == 256 && (TL::BN == 256 || TL::RS || TL::PAIR)) {
     if constexpr (TL::RS || TL::PAIR) {
       if (rast.once && (int)a.off[t.e] - (t.e ? (int)a.off[t.e - 1] : 0) <= TL::BM) {
         s2s_tile_at_height<T, typename TL::Once, B_TR>(a, t, rast.n_tiles, lds, sDst, sSrc, sBias);
@@ -2066,7 +2076,7 @@ static int launch_s2s(const S2SArgs& a, bool b_tr, hipStream_t st) {
   const int64_t grid = r.grid();
   const unsigned parts = a.ksplit > 1 && !whole_parts ? (unsigned)a.ksplit : 1u;
   if (grid > 0x7fffffffLL || m_tiles > 0x7fffffffLL) { set_error("smoe_scatter2scatter: grid too large"); return SMOE_ERR_RANGE; }
-  if constexpr (TL::BN % 128 == 0 && (SMOE_LAYOUTS & 2)) {
+  if constexpr ((TL::BN % 128 == 0 || TL::RS) && (SMOE_LAYOUTS & 2)) {
     if (b_tr) {
       hipLaunchKernelGGL((s2s_mfma_kernel<T, TL, true>), dim3((unsigned)grid, parts), dim3(TL::NT), 0, st, a, r);
       return launch_status("s2s_mfma_kernel");
@@ -2146,11 +2156,32 @@ static bool takes_pairs(const S2SArgs& a) {
   return a.K >= (a.glu == 3 && saves ? 1024 : 192);
 }
 
+// Few rows per expert: tiles of 192 columns in place of 256 where they take no more rounds of a workgroup per CU, a round being a
+// quarter shorter in products and weights.  Plain products and the gated units' gradients; the forward units' halves would not
+// be whole blocks.  us, 256 -> 192 columns (rounds): 32 experts x 188 rows, 2880 -> 2880 149 -> 131 (1.5 -> 1.9), 5760 -> 2880
+// 258 -> 240; 64 x 130, 2048 -> 2064 160 -> 146 (2.3 -> 2.8); 64 x 147, 2880 -> 1488 137 -> 120 (1.5 -> 2.0); 8 x 133, 4096 -> 5176
+// 87 -> 76 (0.7 -> 0.8).  A round more loses (64 x 139, 2048 -> 1816 135 -> 141; 32 x 188, 2880 -> 5760 240 -> 254), and with several
+// tile rows per expert the operands' LDS traffic per product counts (32 x 1024, 2880 -> 2880, 6 % less padding, 550 -> 574;
+// 128 x 438, 4096 -> 2288 1180 -> 1345).  48 random launches that take it: even loads 1.10 times as fast (1.01 to 1.23), as
+// 1 / rank^0.84 and ^1.8, whose tile rows nobody knows here, 1.03 (0.85 to 1.21).
+static constexpr int NARROW_MAX_ROUNDS = 4;
+static bool narrow_columns(const S2SArgs& a) {
+  if ((a.glu != 0 && a.glu != 2 && a.glu != 4) || a.m_begin != 0 || a.m_count != 0x7fffffff || a.tail_mode != 0) return false;
+  if (a.L / a.E >= ROWS256_BELOW) return false;
+  const double rows = expected_row_tiles(a.L, a.E);
+  const int64_t wide = (int64_t)(rows * ((a.N + 255) / 256)), narrow = (int64_t)(rows * ((a.N + 191) / 192));
+  const int64_t rounds = (narrow + NUM_CU - 1) / NUM_CU;
+  return rounds <= NARROW_MAX_ROUNDS && rounds == (wide + NUM_CU - 1) / NUM_CU;
+}
+template <typename T>
+int launch_narrow(const S2SArgs& a, bool b_tr, hipStream_t st);        // gemm_mfma_xty.hip
+
 template <typename T>
 static int launch_main_class(const S2SArgs& a, bool b_tr, hipStream_t st) {
   // (its buffer descriptors end with the last row of a strided operand: rows that overlap, as those of an expanded tensor, would
   // read as zeros)
   const bool apart = !b_tr || a.swk >= (a.glu == 1 ? 2 : 1) * (int64_t)a.N;
+  if (a.K >= RS_MIN_K && whole_pieces(a) && apart && narrow_columns(a)) return launch_narrow<T>(a, b_tr, st);
   if (a.K >= RS_MIN_K && whole_pieces(a) && apart)
     return launch_s2s<T, Tile<256, 256, 2, 2, 2, true>>(a, b_tr, st);
   return launch_s2s<T, Tile<256, 256, 2, 4>>(a, b_tr, st);
