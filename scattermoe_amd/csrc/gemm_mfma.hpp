@@ -2118,7 +2118,8 @@ static int tail_split(const S2SArgs& a) {
 // earn back: K = 768 is 5 % slower, K = 1536 even, K = 2048 is 5-8 % faster).
 // Both forms add up every output element in the same order: the same bits.
 static constexpr int RS_MIN_K = 1792;
-static constexpr int RS_XTY_MIN_ROWS = 2048;      // groupXtY: average rows per expert from which that form is used
+static constexpr int RS_XTY_MIN_ROWS = 2048;      // groupXtY: average rows per expert from which that form is used,
+static constexpr int RS_XTY_MIN_ROWS_ROUNDS = 1280, RS_XTY_ROUNDS = 4;      // and from which with so many rounds of tiles
 // Whole slices, and output pieces of 16 bytes: what the one-wave-per-SIMD form and the paired tiles take.
 static bool whole_pieces(const S2SArgs& a) {
   bool al16 = true;
@@ -2798,13 +2799,18 @@ static bool xty_pairs(const XtYArgs& a) {
 // One-wave-per-SIMD form: needs the LDS-staged epilogue; no gathered operand, no bias gradient in the main loop.
 // Both operands are read transposed (two LDS reads per fragment), which leaves less to win than in
 // scatter2scatter: Mixtral shape (4096 rows per expert) 3.28 -> 3.12 and 6.35 -> 6.20 ms, 2048 rows per expert
-// (128 experts, 768 x 2048 and 2048 x 1536 outputs) 0.81 -> 0.77 and 1.55 -> 1.51 ms, 1024 rows per expert even.
+// (128 experts, 768 x 2048 and 2048 x 1536 outputs) 0.81 -> 0.77 and 1.55 -> 1.51 ms.  Against 256 x 128 tiles, two workgroups per
+// CU, 90 random launches of 1280 to 2047 rows per expert under even and uneven loads: of four rounds and more 1.03 times as fast
+// (0.97 to 1.15; 32 x 2046 rows, 2880 x 3864 1549 -> 1432 us, 16 x 1983, 3128 x 4744 1054 -> 980), of fewer 1.00 (0.82 to 1.18); of 600 to
+// 1024 rows 0.95 (0.85 to 1.04).
 static bool xty_one_wave(const XtYArgs& a) {
   const bool out16 = (((uintptr_t)a.DW & 15) == 0) && ((a.sdwe | (a.sdwk == 1 ? a.sdwn : a.sdwk) | (a.sdwk == 1 ? a.K : a.N)) & 7) == 0;
   const bool db_in_loop = a.Db != nullptr && a.sdwk == 1;
   // (its buffer descriptors end with an operand's last row: rows that overlap, as those of an expanded tensor, would read as zeros)
   const bool apart = a.sdym >= a.N && a.sxm >= a.K;
-  return a.idx == nullptr && !db_in_loop && out16 && apart && a.L / a.E >= RS_XTY_MIN_ROWS;
+  const int64_t rows = a.L / a.E, tiles = (int64_t)a.E * ((a.N + 255) / 256) * ((a.K + 255) / 256);
+  return a.idx == nullptr && !db_in_loop && out16 && apart &&
+         (rows >= RS_XTY_MIN_ROWS || (rows >= RS_XTY_MIN_ROWS_ROUNDS && tiles >= RS_XTY_ROUNDS * NUM_CU));
 }
 
 enum class XtYClass { held, small, pairs, one_wave, large };
@@ -2812,8 +2818,8 @@ static XtYClass xty_class(const XtYArgs& a) {
   const bool rs_form = xty_one_wave(a);
   if (xty_held(a)) return XtYClass::held;
   if (xty_idle_chip(a, rs_form) || xty_few_rows(a) || xty_small_again(a)) return XtYClass::small;
-  if (xty_pairs(a)) return XtYClass::pairs;
-  return rs_form ? XtYClass::one_wave : XtYClass::large;
+  if (rs_form) return XtYClass::one_wave;
+  return xty_pairs(a) ? XtYClass::pairs : XtYClass::large;
 }
 
 template <typename T>
