@@ -1613,15 +1613,17 @@ struct Raster {
   __host__ int64_t grid() const { return grid_size; }
   // (ml, nl): position of the tile inside its super tile
   template <int SN_ = SN>
-  __device__ __forceinline__ bool map(int pid, int& m, int& n, int& ml, int& nl) const {
+  __host__ __device__ __forceinline__ bool map(int pid, int& m, int& n, int& ml, int& nl) const {
     const int x = pid & 7, i = pid >> 3;
     if (striped) {
-      // XCD x owns the tile columns n = x (mod 8) of every tile row; rows slowest, in groups of gm
-      // (the residue class an XCD owns moves on with every group of rows, so that a column count that is not a
-      // multiple of 8 does not leave the same XCDs short every time)
-      const int m_lo = i % gm, j = i / gm;
-      m = (j / n_supers) * gm + m_lo;
-      n = (j % n_supers) * 8 + ((x + j / n_supers) & 7);
+      // Every group of gm tile rows is dealt to the XCDs by columns, where the group before it left off: column n of group g is
+      // XCD (g * n_tiles + n) % 8's, so no XCD has more than one column group more than another.  (Moved on by one XCD per
+      // group, 12 columns gave the first XCDs two in each of the first four: 67 of 420 tiles where a round is 32 per XCD, so
+      // three rounds.  us, so -> this way: 8 experts x 584 rows, 21 tile rows in ten columns, 4640 -> 1272 179 -> 115; random launches
+      // with loads as 1 / rank^0.3 to ^1.8 times as fast: 4 to 112 rows per expert 1.03 to 1.05, 112 to 1000 1.03 to 1.07, 0.97 to 1.78.)
+      const int m_lo = i % gm, j = i / gm, g = j / n_supers;
+      m = g * gm + m_lo;
+      n = (j - g * n_supers) * 8 + ((x - g * n_tiles) & 7);
       ml = nl = 0;
       return m < m_tiles && n < n_tiles;
     }
@@ -2158,13 +2160,15 @@ static bool takes_pairs(const S2SArgs& a) {
 }
 
 // Few rows per expert: tiles of 192 columns in place of 256 where they take no more rounds of a workgroup per CU, a round being a
-// quarter shorter in products and weights.  Plain products and the gated units' gradients; the forward units' halves would not
-// be whole blocks.  us, 256 -> 192 columns (rounds): 32 experts x 188 rows, 2880 -> 2880 149 -> 131 (1.5 -> 1.9), 5760 -> 2880
+// quarter shorter in products and weights.  Plain products and the gated units' gradients; the forward units have not been measured in
+// them.  us, 256 -> 192 columns (rounds): 32 experts x 188 rows, 2880 -> 2880 149 -> 131 (1.5 -> 1.9), 5760 -> 2880
 // 258 -> 240; 64 x 130, 2048 -> 2064 160 -> 146 (2.3 -> 2.8); 64 x 147, 2880 -> 1488 137 -> 120 (1.5 -> 2.0); 8 x 133, 4096 -> 5176
 // 87 -> 76 (0.7 -> 0.8).  A round more loses (64 x 139, 2048 -> 1816 135 -> 141; 32 x 188, 2880 -> 5760 240 -> 254), and with several
 // tile rows per expert the operands' LDS traffic per product counts (32 x 1024, 2880 -> 2880, 6 % less padding, 550 -> 574;
-// 128 x 438, 4096 -> 2288 1180 -> 1345).  48 random launches that take it: even loads 1.10 times as fast (1.01 to 1.23), as
-// 1 / rank^0.84 and ^1.8, whose tile rows nobody knows here, 1.03 (0.85 to 1.21).
+// 128 x 438, 4096 -> 2288 1180 -> 1345).  16 launches that take it, most of them random, before the instruction and the order of this
+// class changed -> now: even loads 1.21 times as fast (1.09 to 1.32), as 1 / rank^0.3 1.16 (1.06 to 1.26), ^0.42 1.13 (0.92 to 1.26),
+// ^0.84 1.10 (0.93 to 1.21), ^1.8 1.08 (0.97 to 1.18).  Under uneven loads nobody knows the tile rows here: what loses are launches whose
+// last round was full to the brim (32 x 172, 3072 -> 2536, 37 tile rows for 32 expected, 518 tiles, 156 -> 169).
 static constexpr int NARROW_MAX_ROUNDS = 4;
 static bool narrow_columns(const S2SArgs& a) {
   if ((a.glu != 0 && a.glu != 2 && a.glu != 4) || a.m_begin != 0 || a.m_count != 0x7fffffff || a.tail_mode != 0) return false;
@@ -2310,8 +2314,8 @@ static constexpr int MAIN_MIN_TILES = 160;
 // the chip idle for as long (us, 256 x 256 -> 256 x 128: 4 experts x 332 rows, 1280 -> 3328 36 -> 26; 8 x 1829,
 // 10752 -> 448 224 -> 172; 32 x 438, 7616 -> 384 151 -> 118; 16 x 572, 10624 -> 448 191 -> 157; over 509 launches of
 // 224 to 4000 rows per expert, a quarter of them at this line, 5.5 % on average; a second round of them loses).  The line
-// is drawn for even loads: uneven ones go by column stripes, where a column's tiles share the 32 CUs of an XCD and may
-// take two rounds (8 x 584 rows on average, 4640 -> 1272, 21 tile rows in ten columns 109 -> 168).
+// is drawn for even loads; uneven ones go by column stripes (8 x 584 rows on average, 4640 -> 1272, 21 tile rows in ten
+// columns 115 us).
 static bool one_round_of_halves(const S2SArgs& a) {
   const int cols = a.glu == 1 ? 64 : 128;
   return expected_row_tiles(a.L, a.E) * ((a.N + cols - 1) / cols) <= NUM_CU;
@@ -2354,8 +2358,8 @@ static int dispatch_few_rows(const S2SArgs& a, bool b_tr, hipStream_t st) {
   if (!b_tr) {
     // K-contiguous weights: half-width tiles while 128-wide ones would not give every CU two workgroups (44 x 8 tiles
     // of K = 1024: 25 -> 17 us, 22 x 16 of K = 2048: 47 -> 39, 8 x 8 of K = 2816: 18 -> 16), and where 128-wide
-    // columns do not divide evenly among the 8 XCDs, as the stripes of uneven loads have to, at most 3/4 of the last
-    // row of eight in use (128 experts of K = 2048, uneven / evenly loaded, which take chunks: 9 columns 127 -> 116 /
+    // columns do not divide evenly among the 8 XCDs, at most 3/4 of the last
+    // row of eight in use (128 experts of K = 2048, uneven, before the stripes went on where they left off / evenly loaded, which take chunks: 9 columns 127 -> 116 /
     // 118 -> 106, 12 columns 164 -> 146 / 133 -> 131, 17 columns 214 -> 194 / 180 -> 179; 16 columns 213 -> 185 /
     // 165 -> 168, 32 columns 375 -> 356 / 329 -> 329: evenly loaded decides, being the ordinary case)
     if (wgs < 192) return launch_s2s<T, Tile<32, 64, 1, 2, 6>>(a, b_tr, st);
