@@ -192,3 +192,90 @@ def test_kernels_fit_their_registers(assembly):
             seen += one_wave
             assert scratch <= (12 if one_wave else 20), (name, kernel, scratch)
     assert seen == 4
+
+
+JUMP = re.compile(r"s_c?branch\w*\s+(\S+)")
+
+
+def _product_hazards_on_all_paths(text):
+    """As `_product_hazards`, along every path that the code can take: both ways of a branch, a loop's back edge among them, and every
+    jump that leads to a product."""
+    code, labels, inside = [], {}, False
+    for n, line in enumerate(text.split("\n")):
+        t = line.split(";")[0].strip()
+        if "ASMSTART" in line or "ASMEND" in line:
+            inside = "ASMSTART" in line
+        elif t.endswith(":"):
+            labels[t[:-1]] = len(code)
+        elif t and t[0] != ".":
+            code.append((n + 1, t, inside))
+    ends = lambda t: t.startswith(("s_branch", "s_endpgm", "s_setpc"))
+    jump = lambda t: JUMP.match(t) and labels[JUMP.match(t)[1]]
+    after, before = [], [[] for _ in code]
+    for i, (_, t, _) in enumerate(code):
+        to = [k for k in (None if ends(t) else i + 1, jump(t)) if k is not None and k < len(code)]
+        after.append(to)
+        for k in to:
+            before[k].append(i)
+    states = lambda t: int(t.split()[1]) + 1 if t.startswith("s_nop") else 1
+
+    def reached(start, edges, limit):
+        """Instructions that fewer than `limit` wait states lie between."""
+        least, todo = {}, [(k, 0) for k in edges[start]]
+        while todo:
+            k, passed = todo.pop()
+            if passed < limit and passed < least.get(k, limit):
+                least[k] = passed
+                todo += [(j, passed + states(code[k][1])) for j in edges[k]]
+        return least
+
+    products, found = 0, []
+    for i, (n, t, in_asm) in enumerate(code):
+        if not (in_asm and t.startswith("v_mfma")):
+            continue
+        products += 1
+        operands = t.split(None, 1)[1].split(",")
+        result, sources = _vector_registers(operands[0]), _vector_registers(",".join(operands[1:]))
+        found += [(n, t, code[k]) for k in reached(i, before, 2) if code[k][1].startswith("v_") and
+                  not code[k][1].startswith("v_mfma") and _vector_registers(code[k][1].split(",")[0]) & sources]
+        found += [(n, t, code[k]) for k in reached(i, after, 19)
+                  if not code[k][1].startswith("v_mfma") and _vector_registers(code[k][1]) & result]
+    return products, found
+
+
+def test_scanner_follows_branches():
+    product = "\t;;#ASMSTART\n\tv_mfma_f32_16x16x32_bf16 a[0:3], v[8:11], v[4:7], a[0:3]\n\t;;#ASMEND\n"
+    loop = ".LBB0_1:                                ; loop\n%s" + product + "%s\ts_cbranch_scc1 .LBB0_1\n%s\ts_endpgm\n"
+    skip = product + "\ts_cbranch_scc0 .LBB0_2\n\ts_nop 15\n\ts_nop 3\n%s.LBB0_2:\n%s\ts_endpgm\n"
+    enter = "\tv_mov_b32_e32 v5, v1\n\ts_branch .LBB0_3\n\ts_endpgm\n.LBB0_3:\n%s" + product
+    read, wait, write = "\tv_accvgpr_read_b32 v1, a2\n", "\ts_nop 15\n\ts_nop 3\n", "\tv_mov_b32_e32 v9, v1\n"
+    for bad in (loop % (read, "", wait + read), loop % ("", write, ""), loop % ("", "", read), skip % ("", read), enter % ""):
+        assert _product_hazards_on_all_paths(bad)[1], bad
+    # (the first two are beyond a scan of the code as it falls through)
+    assert not _product_hazards(loop % (read, "", wait + read))[1] and not _product_hazards(loop % ("", write, ""))[1]
+    for good in (loop % (wait + read, "", wait + read), loop % ("", write + "\ts_nop 1\n", ""), skip % (read, wait + read),
+                 enter % "\ts_nop 1\n", skip % (read, "")):
+        assert _product_hazards_on_all_paths(good) == (1, []), good
+
+
+@needs_hipcc
+def test_products_of_assembly_blocks_keep_their_distance_on_all_paths(assembly):
+    for name, text in assembly.items():
+        products, found = _product_hazards_on_all_paths(text)
+        assert products == _product_hazards(text)[0]
+        assert not found, (name, found[:5])
+
+
+@needs_hipcc
+def test_one_wave_per_simd_kernels_need_no_scratch_memory(assembly):
+    """Products in tiles of 256 and of 192 columns, and weight gradients: 256 (192) accumulators, two register sets of operands and
+    nothing in scratch memory."""
+    seen = {}
+    for name, text in assembly.items():
+        for kernel, scratch in _scratch_of_kernels(text):
+            tile = _tile(kernel)[:6]
+            if tile[2:] == (2, 2, 2, 1):
+                which = ("xty" if "xty_mfma_kernel" in kernel else "s2s", tile[1])
+                seen[which] = seen.get(which, 0) + 1
+                assert scratch == 0, (name, kernel, scratch)
+    assert seen == {("s2s", 256): 4, ("s2s", 192): 4, ("xty", 256): 2}, seen
