@@ -702,7 +702,9 @@ __device__ __forceinline__ void mainloop(AOp& A, BOp& B, int klen, char* lds, bo
 //   quarters later (the last of them in the first two quarters of the next slice), one load per 8 MFMAs throughout;
 //   one barrier per slice, after six quarters: behind it the first fragments of slice kt + 1 are read while the
 //   last two quarters are multiplied.
-// Whole 64-deep slices only, at least two of them (the launcher checks); loads past the end re-read the last slice.
+// Whole 64-deep slices (the launchers check) or operands that read as zeros behind their last contraction row.  One slice is
+// enough (a contraction part may have no more): what is loaded ahead past the last one, that one again (DirectOp) or zeros (TransOp),
+// is written to LDS and not multiplied.
 //
 // A thread's pieces of a slice in the order they are written and reloaded: the operands alternate while the row
 // operand (the smaller one in a tile of fewer than 256 rows) has pieces left.
@@ -2253,7 +2255,10 @@ static int launch_tails(const S2SArgs& a, bool b_tr, hipStream_t st) {
 // workgroup's set-up and store 14 and 4; the sums their bytes at 4.5 TB/s, written and read.  Measured, us, without -> with (parts):
 // 8 experts x 194 rows, 14336 -> 4096 241 -> 220 (2), 28672 -> 4096 478 -> 397 (2); 4 x 300, 14336 -> 4096 239 -> 196 (2); 2 x 500,
 // 8192 -> 4096 116 -> 73 (4); 1 x 609, 10240 -> 1472 155 -> 47 (8); 8 x 200, 2048 -> 2048 33 -> 39, so not; a second round of
-// workgroups loses as well (8 x 250, 14336 -> 4096 316 -> 361).
+// workgroups loses as well (8 x 250, 14336 -> 4096 316 -> 361).  22 launches that take parts, 19 of them random, against the state
+// before there were any: even loads 1.66 times as fast (1.00 to 3.05), as 1 / rank^0.3 1.73, ^0.42 1.72, ^0.84 1.69 (1.03 to 3.0), ^1.8
+// 1.66 (0.94 to 2.8): of the 110 one is slower, whose loads make three tile rows more than expected and so a second round (16 x 888 rows,
+// 11968 -> 280, 198 -> 211).
 static constexpr int PARTS_MAX = 8;
 static int part_length(int64_t K, int parts) { return (int)((K / BK + parts - 1) / parts) * BK; }
 static int whole_parts_for(int64_t L, int64_t K, int64_t N, int E) {

@@ -52,8 +52,8 @@ class HipBackend:
         lib = _C.load()
         sbe, sbn = (b.stride(0), b.stride(1)) if b is not None else (0, 0)
         code = _C.float_code(X.dtype)
-        # scratch for the products that split the contraction of their experts' last tiles (0 bytes for the others);
-        # torch's allocator hands the same block out again step after step
+        # scratch for the products that go in parts of the contraction, their experts' last tiles or, where there are few
+        # tiles, all of them (0 bytes for the others); torch's allocator hands the same block out again step after step
         need = lib.smoe_scatter2scatter_workspace_bytes(eid.numel(), X.size(1), Y.size(1), W.size(0), code)
         ws = torch.empty(need, dtype=torch.uint8, device=X.device) if need else None
         with _C.on_device(X.device):
