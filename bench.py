@@ -307,7 +307,7 @@ def mfma_sustained(torch):
             torch.cuda.synchronize()
             assert rc == 0, "smoe_bench_mfma_rate failed: %d" % rc
         res[name + "_tflops"] = round(flop.value / a.elapsed_time(b) / 1e9, 1)
-    res["kernel"] = "independent 32x32x16 bf16 MFMAs, one wave per SIMD on every CU, operands in registers"
+    res["kernel"] = "independent 16x16x32 bf16 MFMAs (the products' instruction), one wave per SIMD on every CU, operands in registers"
     return res
 
 
