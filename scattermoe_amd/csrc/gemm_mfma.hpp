@@ -1609,6 +1609,7 @@ struct Raster {
   static constexpr int SM = 8, SN = 4;
   int m_tiles, n_tiles, m_supers, n_supers, supers, gm;
   int striped;                             // 1: column-striped order of the memory-bound classes (see make_striped)
+  int shift = 0;                           // of that order: how many XCDs a group of tile rows is moved on
   int chunked = 0;                         // 1, 2: order of find_tile_chunked (2: in rounds) before this one
   int once = 0;                            // weights of experts of one tile row bypass the caches (see reads_weights_once)
   int64_t grid_size;                       // host side only: number of workgroups (may exceed what a launch takes)
@@ -1619,13 +1620,13 @@ struct Raster {
     const int x = pid & 7, i = pid >> 3;
     if (striped) {
       // Every group of gm tile rows is dealt to the XCDs by columns, where the group before it left off: column n of group g is
-      // XCD (g * n_tiles + n) % 8's, so no XCD has more than one column group more than another.  (Moved on by one XCD per
+      // XCD (n + g * shift) % 8's, so no XCD has more than one column group more than another.  (Moved on by one XCD per
       // group, 12 columns gave the first XCDs two in each of the first four: 67 of 420 tiles where a round is 32 per XCD, so
       // three rounds.  us, so -> this way: 8 experts x 584 rows, 21 tile rows in ten columns, 4640 -> 1272 179 -> 115; random launches
       // with loads as 1 / rank^0.3 to ^1.8 times as fast: 4 to 112 rows per expert 1.03 to 1.05, 112 to 1000 1.03 to 1.07, 0.97 to 1.78.)
       const int m_lo = i % gm, j = i / gm, g = j / n_supers;
       m = g * gm + m_lo;
-      n = (j - g * n_supers) * 8 + ((x - g * n_tiles) & 7);
+      n = (j - g * n_supers) * 8 + ((x - g * shift) & 7);
       ml = nl = 0;
       return m < m_tiles && n < n_tiles;
     }
@@ -1675,6 +1676,9 @@ static Raster make_striped(int64_t m_tiles, int n_tiles, int gm) {
   r.m_tiles = (int)m_tiles;
   r.n_tiles = n_tiles;
   r.gm = gm < 1 ? 1 : (gm > m_tiles ? (int)m_tiles : gm);
+  // (whole eights of columns are shared out whatever the shift; left where they are, an XCD has the same columns of all experts, which
+  // is slower: 16 experts, 346 rows as 1 / rank^1.8, 2688 -> 2 x 7168, 112 columns 144 -> 152 us)
+  r.shift = n_tiles % 8 ? n_tiles % 8 : 7;
   r.n_supers = (n_tiles + 7) / 8;                                        // tile columns per XCD
   r.m_supers = (int)((m_tiles + r.gm - 1) / r.gm);                       // groups of tile rows
   r.supers = 0;
