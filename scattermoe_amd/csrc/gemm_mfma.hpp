@@ -1609,7 +1609,6 @@ struct Raster {
   static constexpr int SM = 8, SN = 4;
   int m_tiles, n_tiles, m_supers, n_supers, supers, gm;
   int striped;                             // 1: column-striped order of the memory-bound classes (see make_striped)
-  int shift = 0;                           // of that order: how many XCDs a group of tile rows is moved on
   int chunked = 0;                         // 1, 2: order of find_tile_chunked (2: in rounds) before this one
   int once = 0;                            // weights of experts of one tile row bypass the caches (see reads_weights_once)
   int64_t grid_size;                       // host side only: number of workgroups (may exceed what a launch takes)
@@ -1619,14 +1618,15 @@ struct Raster {
   __host__ __device__ __forceinline__ bool map(int pid, int& m, int& n, int& ml, int& nl) const {
     const int x = pid & 7, i = pid >> 3;
     if (striped) {
-      // Every group of gm tile rows is dealt to the XCDs by columns, where the group before it left off: column n of group g is
-      // XCD (n + g * shift) % 8's, so no XCD has more than one column group more than another.  (Moved on by one XCD per
-      // group, 12 columns gave the first XCDs two in each of the first four: 67 of 420 tiles where a round is 32 per XCD, so
-      // three rounds.  us, so -> this way: 8 experts x 584 rows, 21 tile rows in ten columns, 4640 -> 1272 179 -> 115; random launches
-      // with loads as 1 / rank^0.3 to ^1.8 times as fast: 4 to 112 rows per expert 1.03 to 1.05, 112 to 1000 1.03 to 1.07, 0.97 to 1.78.)
-      const int m_lo = i % gm, j = i / gm, g = j / n_supers;
+      // Columns of a group of gm tile rows, one group after another, are dealt to the XCDs in eights, one each: no XCD has more
+      // than one column group more than another, and none has workgroups without a tile between those with one (they leave at
+      // once, but the CUs are dealt out by turns: 8 of every 16 put two tiles on every second CU).  Which of the eight an XCD takes
+      // moves on with the groups; an XCD that keeps the same columns of all experts is slower (16 experts, 346 rows as 1 / rank^1.8,
+      // 2688 -> 2 x 7168, 112 columns 144 -> 152 us).
+      const int m_lo = i % gm, j = i / gm;
+      const int u = 8 * j + ((x + 8 * j / n_tiles) & 7), g = u / n_tiles;
       m = g * gm + m_lo;
-      n = (j - g * n_supers) * 8 + ((x - g * shift) & 7);
+      n = u - g * n_tiles;
       ml = nl = 0;
       return m < m_tiles && n < n_tiles;
     }
@@ -1666,23 +1666,23 @@ static Raster make_raster(int64_t m_tiles, int n_tiles, int gm, int sn = Raster:
 }
 
 // Order of the memory-bound (ring) classes.  The grid covers an upper bound of the tile rows, so some rows are
-// empty, and which ones is known only on the device: every XCD therefore takes the same share of every tile row
-// (its own residue class of tile columns), and the empty rows, which come last, cost nothing but their launch.
-// `gm` consecutive tile rows visit a tile column back to back on one XCD, so that an expert with several tile
-// rows finds its weight panel in that XCD's L2.
+// empty, and which ones is known only on the device: every XCD therefore takes the same share of every group of `gm` tile
+// rows, and the empty rows, which come last, cost nothing but their launch.  The rows of a group visit a tile column back to
+// back on one XCD, so that an expert with several tile rows finds its weight panel in that XCD's L2.
+// us, when XCD x had the columns n = x + group (mod 8) of a group, existing or not -> now: 8 experts x 584 rows, 21 tile rows in
+// ten columns, 4640 -> 1272 179 -> 115 (the first XCDs had two columns in each of the groups, 42 tiles where a round is 32 per XCD);
+// random launches with loads as 1 / rank^0.3 to ^1.8 of 4 to 112 rows per expert 1.03 to 1.06 times as fast, of 112 to 1000 1.02 to
+// 1.07, in tiles of 192 columns 1.03 to 1.06, single ones 0.94 to 1.77; whole layers drawn at random 1.00 to 1.02 (0.98 to 1.52).
 static Raster make_striped(int64_t m_tiles, int n_tiles, int gm) {
   Raster r;
   r.striped = 1;
   r.m_tiles = (int)m_tiles;
   r.n_tiles = n_tiles;
   r.gm = gm < 1 ? 1 : (gm > m_tiles ? (int)m_tiles : gm);
-  // (whole eights of columns are shared out whatever the shift; left where they are, an XCD has the same columns of all experts, which
-  // is slower: 16 experts, 346 rows as 1 / rank^1.8, 2688 -> 2 x 7168, 112 columns 144 -> 152 us)
-  r.shift = n_tiles % 8 ? n_tiles % 8 : 7;
-  r.n_supers = (n_tiles + 7) / 8;                                        // tile columns per XCD
+  r.n_supers = 0;
   r.m_supers = (int)((m_tiles + r.gm - 1) / r.gm);                       // groups of tile rows
   r.supers = 0;
-  r.grid_size = (int64_t)r.m_supers * r.gm * r.n_supers * 8;
+  r.grid_size = ((int64_t)r.m_supers * n_tiles + 7) / 8 * 8 * r.gm;
   return r;
 }
 

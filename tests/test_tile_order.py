@@ -60,3 +60,15 @@ def test_stripes_share_the_tiles_out(order, n_tiles):
             whole, rest = divmod(rows, gm)
             per_xcd = [sum(x == xcd and m < rows for x, m, _ in tiles) for xcd in range(8)]
             assert max(per_xcd) <= -(-whole * n_tiles // 8) * gm + -(-n_tiles // 8) * rest, (m_tiles, rows, per_xcd)
+
+
+@pytest.mark.parametrize("n_tiles", [1, 3, 4, 8, 12, 22])
+def test_stripes_leave_no_gaps(order, n_tiles):
+    """An XCD's workgroups all have a tile until its last one of the whole groups of rows."""
+    for m_tiles in (8, 40, 136):
+        buf = (ctypes.c_int * (8 * (m_tiles + 16) * (n_tiles + 8)))()
+        grid = order.stripes(ctypes.c_int64(m_tiles), n_tiles, buf)
+        assert m_tiles * n_tiles <= grid < m_tiles * n_tiles + 8 * order.stripes_group()
+        for xcd in range(8):
+            has = [t >= 0 for t in buf[xcd:grid:8]]
+            assert all(has[:sum(has)]), (m_tiles, xcd)
